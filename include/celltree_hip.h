@@ -109,10 +109,36 @@ int64_t ct_max_nodes(int64_t n_elements);
 /* Device workspace, in bytes, that ct_build needs for n_elements and n_buckets. */
 size_t ct_build_workspace_bytes(int64_t n_elements, int32_t n_buckets);
 
-/* creation.py:384-413 initialize (+ build, :233-381): level-synchronous bucket-split
- * build on the device.  Writes nodes_out[0 .. *n_nodes) in the reference's DFS numbering
- * and bb_indices_out (n_elements).  n_nodes and depth are HOST outputs; the call
- * synchronizes the stream once per tree level. */
+/* Host results of ct_build_plan. */
+typedef struct ct_build_info {
+  int64_t n_nodes;
+  int32_t depth;
+  int32_t n_top;     /* for ct_build_emit */
+  int32_t n_small;   /* for ct_build_emit */
+  int32_t reserved;
+  double stats[5];   /* bbox_tree and the largest diagonal, as ct_bbox_stats */
+  int64_t flags[3];  /* the caller's flags array, or zeros */
+} ct_build_info;
+
+/* creation.py:384-413 initialize (+ build, :233-381) in two calls, so that the caller can
+ * allocate exactly what the tree needs in between.  ct_build_plan builds the tree in the
+ * workspace, writes bb_indices_out (n_elements) and, when `distances` is not null, the (n, 3)
+ * distances of ct_bbox_stats, and fills *info (HOST); it synchronizes the stream, once for all
+ * but very unbalanced trees.  `want_boxes`: also the tight node boxes.  `flags` (may be NULL): 3
+ * device int64 copied to info->flags, so that a caller's own check values arrive with the same
+ * synchronization; info is complete when the result is CT_OK or CT_ERR_DEGENERATE.
+ * ct_build_emit (asynchronous) writes nodes_out[0 .. info->n_nodes) in the reference's DFS
+ * numbering and, when node_boxes_out is not null (needs want_boxes), what ct_node_boxes writes. */
+int ct_build_plan(const double* bb_coords, int64_t n_elements, int32_t n_buckets,
+                  int32_t cells_per_leaf, int32_t want_boxes, void* workspace,
+                  size_t workspace_bytes, int32_t* bb_indices_out, double* distances,
+                  const int64_t* flags, ct_build_info* info, void* stream);
+int ct_build_emit(int64_t n_elements, int32_t n_buckets, void* workspace, size_t workspace_bytes,
+                  const ct_build_info* info, ct_node* nodes_out, double* node_boxes_out,
+                  void* stream);
+
+/* Both in one call, into arrays of the pessimistic capacity: writes nodes_out[0 .. *n_nodes)
+ * and bb_indices_out (n_elements).  n_nodes and depth are HOST outputs; synchronizes. */
 int ct_build(const double* bb_coords, int64_t n_elements, int32_t n_buckets,
              int32_t cells_per_leaf, void* workspace, size_t workspace_bytes,
              ct_node* nodes_out, int32_t* bb_indices_out, int64_t* n_nodes, int32_t* depth,

@@ -115,6 +115,20 @@ class CtRegridTopology(ctypes.Structure):
     ]
 
 
+class CtBuildInfo(ctypes.Structure):
+    """``ct_build_info``: host results of ct_build_plan."""
+
+    _fields_ = [
+        ("n_nodes", ctypes.c_int64),
+        ("depth", ctypes.c_int32),
+        ("n_top", ctypes.c_int32),
+        ("n_small", ctypes.c_int32),
+        ("reserved", ctypes.c_int32),
+        ("stats", ctypes.c_double * 5),
+        ("flags", ctypes.c_int64 * 3),
+    ]
+
+
 assert ctypes.sizeof(CtNode) == 32
 assert ctypes.sizeof(CtTree) == 152
 assert ctypes.sizeof(CtBatchTile) == 16
@@ -127,6 +141,7 @@ _SZ = ctypes.c_size_t
 _TP = ctypes.POINTER(CtTree)
 _BP = ctypes.POINTER(CtBatch)
 _RP = ctypes.POINTER(CtRegridTopology)
+_IP = ctypes.POINTER(CtBuildInfo)
 
 # name -> (restype, argtypes); mirrors include/celltree_hip.h one to one.
 SIGNATURES = {
@@ -143,6 +158,8 @@ SIGNATURES = {
         ctypes.c_int,
         [_P, _I64, _I32, _I32, _P, _SZ, _P, _P, ctypes.POINTER(_I64), ctypes.POINTER(_I32), _P],
     ),
+    "ct_build_plan": (ctypes.c_int, [_P, _I64, _I32, _I32, _I32, _P, _SZ, _P, _P, _P, _IP, _P]),
+    "ct_build_emit": (ctypes.c_int, [_I64, _I32, _P, _SZ, _IP, _P, _P, _P]),
     "ct_collect_node_bounds": (ctypes.c_int, [_P, _I64, ctypes.POINTER(_F64), _P, _P, _P]),
     "ct_validate_node_bounds": (ctypes.c_int, [_TP, _P, _P, _P]),
     "ct_locate_points": (ctypes.c_int, [_TP, _P, _I64, _F64, _P, _P]),

@@ -66,30 +66,38 @@ class CellTree2dBase:
         L = _native.lib()
         st = D.stream()
         ws = D.empty(int(L.ct_build_workspace_bytes(n, n_buckets)), torch.uint8)
-        cap = int(L.ct_max_nodes(n))
-        nodes_raw = D.empty(32 * cap, torch.uint8)
         bb_indices = D.empty(n, torch.int32)
-        n_nodes = ctypes.c_int64(0)
-        depth = ctypes.c_int32(0)
+        distances = D.empty((n, 3), torch.float64)
+        want_boxes = int(elements.shape[1]) >= 3
+        info = _native.CtBuildInfo()
         _native.call(
-            "ct_build", D.ptr(bb_coords), n, n_buckets, cells_per_leaf, D.ptr(ws), ws.numel(),
-            D.ptr(nodes_raw), D.ptr(bb_indices), ctypes.byref(n_nodes), ctypes.byref(depth), st,
+            "ct_build_plan", D.ptr(bb_coords), n, n_buckets, cells_per_leaf, int(want_boxes), D.ptr(ws), ws.numel(),
+            D.ptr(bb_indices), D.ptr(distances), None, ctypes.byref(info), st,
         )
+        nodes_raw = D.empty(32 * info.n_nodes, torch.uint8)
+        node_boxes = D.empty((info.n_nodes + 1, 4), torch.float64) if want_boxes else None
+        _native.call("ct_build_emit", n, n_buckets, D.ptr(ws), ws.numel(), ctypes.byref(info), D.ptr(nodes_raw),
+                     D.ptr(node_boxes), st)
         del ws
-        self._adopt(vertices, elements, bb_coords, nodes_raw[: 32 * n_nodes.value], bb_indices,
-                    int(n_nodes.value), int(depth.value), n_buckets, cells_per_leaf)
+        self._adopt(vertices, elements, bb_coords, nodes_raw, bb_indices, int(info.n_nodes), int(info.depth),
+                    n_buckets, cells_per_leaf, (distances, np.array(info.stats[:]), node_boxes))
 
     def _adopt(self, vertices: torch.Tensor, elements: torch.Tensor, bb_coords: torch.Tensor,
                nodes_raw: torch.Tensor, bb_indices: torch.Tensor, n_nodes: int, depth: int,
-               n_buckets: int, cells_per_leaf: int) -> None:
+               n_buckets: int, cells_per_leaf: int, built=None) -> None:
         """Takes a built (or imported) tree's device arrays and derives the rest: the bbox
-        statistics, the ct_tree descriptor and the device-only layouts."""
+        statistics, the ct_tree descriptor and the device-only layouts.  ``built``: the bbox
+        distances, the bbox statistics and the node boxes (None: not wanted) that a build has
+        already; an imported tree's are derived here."""
         n = int(elements.shape[0])
         st = D.stream()
-        distances = D.empty((n, 3), torch.float64)
-        stats = D.empty(5, torch.float64)
-        _native.call("ct_bbox_stats", D.ptr(bb_coords), n, D.ptr(distances), D.ptr(stats), st)
-        host = stats.cpu().numpy()
+        if built is not None:
+            distances, host, node_boxes = built
+        else:
+            distances = D.empty((n, 3), torch.float64)
+            stats = D.empty(5, torch.float64)
+            _native.call("ct_bbox_stats", D.ptr(bb_coords), n, D.ptr(distances), D.ptr(stats), st)
+            host, node_boxes = stats.cpu().numpy(), None
 
         self.n_buckets = n_buckets
         self.cells_per_leaf = cells_per_leaf
@@ -154,10 +162,12 @@ class CellTree2dBase:
         self.d_node_boxes = None
         if nmax >= 3:
             # Tight subtree boxes: segment-face queries skip subtrees a segment cannot reach.
-            self.d_node_boxes = D.empty((self.n_nodes + 1, 4), torch.float64)
-            scratch = D.empty(self.n_nodes, torch.int32)
-            _native.call("ct_node_boxes", self.tree_ref, D.ptr(scratch), D.ptr(self.d_node_boxes), st)
-            del scratch
+            if node_boxes is None:
+                node_boxes = D.empty((self.n_nodes + 1, 4), torch.float64)
+                scratch = D.empty(self.n_nodes, torch.int32)
+                _native.call("ct_node_boxes", self.tree_ref, D.ptr(scratch), D.ptr(node_boxes), st)
+                del scratch
+            self.d_node_boxes = node_boxes
             t.node_boxes = self.d_node_boxes.data_ptr()
 
     # ------------------------------------------------------------ export / import

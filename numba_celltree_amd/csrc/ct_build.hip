@@ -1,30 +1,42 @@
-// ct_build.hip -- level-synchronous GPU build of the Garth-Joy bucket-split cell tree.
+// ct_build.hip -- GPU build of the Garth-Joy bucket-split cell tree.
 //
-// The reference (creation.py:233-381) builds serially with a DFS stack.  Each node's
-// work depends only on its own cell range, so all nodes of one level are split at once:
+// The reference (creation.py:233-381) builds serially with a DFS stack.  Each node's work
+// depends only on its own cell range, so the nodes can be split in any order.  Two stages:
 //
-//   per level (A active nodes, one "slot" each; every cell position knows its slot):
-//     k_range      per position: min bb[2d] / max bb[2d+1] per slot      (get_bounds :153-171)
-//     k_bucket     per position: bucket id of the centroid               (centroid_test :44-51)
-//     k_rank_*     global exclusive scan of one-hot bucket counts -> stable rank of every
-//                  cell inside its (node, bucket) = the order sort_bbox_indices produces
-//                  with its repeated stable_partition (:54-151)
-//     k_scatter    per position: the stably partitioned permutation
-//     k_bbounds    per position: per-bucket Rmin/Lmax (the get_bounds loop :300-306)
-//     k_decide     per slot: special case (:312-320), empty-bucket merge (:322-341),
-//                  retry-other-dimension / degenerate leaf (:343-358), split_plane (:174-213),
-//                  children (:365-379)
-//     k_reseg      per position: slot of the child that now owns the position
+//   large nodes (more cells than one workgroup holds), level by level, three kernels a level:
+//     k_tile_count    per tile (<= kTile cells of ONE node): each cell's bucket, and the tile's
+//                     bucket counts and bucket bounds in both dimensions
+//     k_node_decide   per node: tile counts -> stable offsets, bucket bounds -> split (or
+//                     retry, or leaf); the children's extents are unions of bucket bounds, so no
+//                     pass over the cells computes them
+//     k_tile_scatter  per tile: the stably partitioned permutation
+//   small nodes (<= T cells): k_small, one workgroup per node, builds the whole subtree in LDS
+//   k_top             DFS ranks and tight boxes of the large nodes, in one workgroup
+//   k_emit            nodes (and tight boxes) to their reference indices
 //
-// Nodes are first numbered in creation order; a final pass renumbers them to the
-// reference's DFS numbering: the children of the k-th internal node in DFS preorder
-// (left first) sit at 1 + 2k (creation.py:373-379), so a bottom-up count of internal
-// nodes per subtree and a top-down prefix give every node its reference index.
+// What bounds it: the work per level is small (a permutation index, a 32-byte box and a byte per
+// cell), so a build is made of latencies: kernel boundaries, barriers, host round trips.  Half of
+// the levels lie below 1024 cells, where a workgroup's barriers replace kernel boundaries.  The
+// host launches as many large-node levels as a balanced tree has, plus two, without reading
+// anything back (an idle level costs three empty launches), and synchronizes once.  With a
+// sequence of 11 kernels and a host synchronization for each of the 22 levels, and the node boxes
+// in one launch a level, the constructor took 5.78 ms for 999,941 cells and 1.67 ms for 20,000;
+// now 1.42 and 0.43 ms.
+//
+// The stable partition is the order sort_bbox_indices (:54-151) produces with its repeated
+// stable_partition.  Per node as in the reference: special case (:312-320), empty-bucket merge
+// (:322-341), retry-other-dimension / degenerate leaf (:343-358), split_plane (:174-213),
+// children (:365-379).
+//
+// Nodes are first numbered in creation order.  The reference's DFS numbering puts the children
+// of the k-th internal node in DFS preorder (left first) at 1 + 2k (creation.py:373-379): a
+// bottom-up count of internal nodes per subtree and a top-down prefix give every node its
+// index, and a subtree whose root has rank r occupies the indices 2r + (its own numbering).
 //
 // Order-sensitive details kept from the reference: FP64 bucket bounds i*bl + Rmin and
 // (i+1)*bl + Rmin (no FMA), first strict minimum of the split cost, a node that retries
 // keeps its flipped dim even when it ends as a leaf.
-#include <vector>
+#include <algorithm>
 
 #include "ct_internal.h"
 #include "ct_primitives.h"
@@ -32,44 +44,72 @@
 namespace ct {
 namespace {
 
-constexpr int kRankItems = 4;
-constexpr int kRankTile = kBlock * kRankItems;
+using Key = unsigned long long;
+
+// Cells per tile of the large-node kernels: 4 per lane keep the tile count (and the prefix that
+// k_node_decide forms over a node's tiles) low; 999,941 cells are 977 workgroups.
+constexpr int kTileItems = 4;
+constexpr int kTile = kBlock * kTileItems;
+constexpr int kDecideBlock = 512;
 constexpr int kMaxBuckets = 64;
 
-enum Decision : int32_t { kLeaf = 0, kSplit = 1, kRetry = 2 };
+// Cells a workgroup's subtree stage takes, by bucket count: its LDS holds per-bucket bounds of
+// up to T / 2 nodes.
+int small_cells(int nb) { return nb <= 8 ? 1024 : nb <= 16 ? 512 : nb <= 32 ? 256 : 128; }
 
-struct Slots {  // active-node list, structure of arrays
+struct Slots {  // large nodes of one level, structure of arrays
   int32_t* id;     // creation-order node id
   int32_t* ptr;
   int32_t* size;
   int32_t* dim;
   int32_t* att;    // 0 first attempt, 1 after a dimension flip
   int32_t* depth;
+  int32_t* tile0;  // first tile; tiles of a node are consecutive
+  Key* range;      // 4 per node: min x, max x, min y, max y of its cells' boxes
+  int32_t* map;    // tile -> slot
+};
+
+struct Smalls {  // roots of the subtrees k_small builds
+  int32_t* id;
+  int32_t* ptr;
+  int32_t* size;
+  int32_t* dim;
+  int32_t* depth;
+};
+
+// Read back by the host in one transfer.
+struct Header {
+  int32_t next_id;    // nodes created by the large-node stage (and the root)
+  int32_t err;        // 1: a centroid in no bucket, 2: no finite split cost
+  int32_t depth;
+  int32_t n_small;
+  int32_t active[2];  // large nodes per level parity
+  int32_t tiles[2];
+  int32_t n_nodes;    // of the whole tree (k_top)
+  int32_t pad[3];
+  Key stats[5];       // as bbox_stat_keys leaves them: ~min x, max x, ~min y, max y, max diagonal
+  int64_t flags[3];   // the caller's check values, passed through
 };
 
 struct Work {
+  Header* head;
   int32_t* perm[2];
-  int32_t* seg;
-  int32_t* bid[2];
-  int32_t* rank;
-  int32_t* blockcnt;
+  uint8_t* bid;
+  int32_t* tilecnt;   // per tile and bucket: cells
+  int32_t* tilepre;   // per tile and bucket: cells of the node's earlier tiles
+  Key* tilebk;        // per tile, bucket: 4 bounds
+  int32_t* boff;      // per slot and bucket: first position
   Slots act[2];
-  unsigned long long* rmin;
-  unsigned long long* rmax;
-  int32_t* sstart;
-  int32_t* send;
-  int32_t* boff;
-  unsigned long long* bmin;
-  unsigned long long* bmax;
-  int32_t* decision;
-  int32_t* right_index;
-  int32_t* next_l;
-  int32_t* next_r;
-  ct_node* cnodes;  // creation-order nodes
+  Smalls small;
+  int32_t* group_end;  // creation-order ids at the start of every large-node level
+  ct_node* cnodes;     // large-node stage, creation order; child -2: a subtree k_small built
   int32_t* icount;
   int32_t* drank;
   int32_t* newidx;
-  int32_t* counters;  // [0] next node id, [1] next active count, [2] error, [3] max depth
+  double4* tbox;
+  ct_node* lnodes;     // subtrees: node x of the subtree at positions [p, ...) is entry 2p + x
+  int32_t* lmeta;      // its own DFS index | its internal rank << 16
+  double4* lbox;
 };
 
 struct Layout {
@@ -82,22 +122,26 @@ struct Layout {
   }
 };
 
+// Large nodes of a level hold more than small_cells(nb) cells each.
+int64_t max_active(int64_t n, int nb) { return n / (small_cells(nb) + 1) + 2; }
+int64_t max_tiles(int64_t n, int nb) { return n / kTile + max_active(n, nb) + 2; }
+
 // Carves the workspace; with base == nullptr it only measures.
 Work carve(char* base, int64_t n, int nb, size_t* total) {
   Layout L;
   Work w{};
-  const int64_t amax = n / 2 + 2;
+  const int64_t amax = max_active(n, nb), tmax = max_tiles(n, nb), smax = n / 2 + 2;
   const int64_t mmax = ct_max_nodes(n) + 2;
-  const int64_t nblk = (n + kRankTile - 1) / kRankTile + 1;
   auto P = [&](size_t off) { return base ? base + off : nullptr; };
 #define CT_TAKE(field, T, count) field = reinterpret_cast<T*>(P(L.take<T>(count)))
+  CT_TAKE(w.head, Header, 1);
   CT_TAKE(w.perm[0], int32_t, n);
   CT_TAKE(w.perm[1], int32_t, n);
-  CT_TAKE(w.seg, int32_t, n);
-  CT_TAKE(w.bid[0], int32_t, n);
-  CT_TAKE(w.bid[1], int32_t, n);
-  CT_TAKE(w.rank, int32_t, n);
-  CT_TAKE(w.blockcnt, int32_t, nblk * nb);
+  CT_TAKE(w.bid, uint8_t, n);
+  CT_TAKE(w.tilecnt, int32_t, tmax * nb);
+  CT_TAKE(w.tilepre, int32_t, tmax * nb);
+  CT_TAKE(w.tilebk, Key, tmax * nb * 4);
+  CT_TAKE(w.boff, int32_t, amax * nb);
   for (int k = 0; k < 2; ++k) {
     CT_TAKE(w.act[k].id, int32_t, amax);
     CT_TAKE(w.act[k].ptr, int32_t, amax);
@@ -105,429 +149,817 @@ Work carve(char* base, int64_t n, int nb, size_t* total) {
     CT_TAKE(w.act[k].dim, int32_t, amax);
     CT_TAKE(w.act[k].att, int32_t, amax);
     CT_TAKE(w.act[k].depth, int32_t, amax);
+    CT_TAKE(w.act[k].tile0, int32_t, amax);
+    CT_TAKE(w.act[k].range, Key, amax * 4);
+    CT_TAKE(w.act[k].map, int32_t, tmax);
   }
-  CT_TAKE(w.rmin, unsigned long long, amax);
-  CT_TAKE(w.rmax, unsigned long long, amax);
-  CT_TAKE(w.sstart, int32_t, amax * nb);
-  CT_TAKE(w.send, int32_t, amax * nb);
-  CT_TAKE(w.boff, int32_t, amax * nb);
-  CT_TAKE(w.bmin, unsigned long long, amax * nb);
-  CT_TAKE(w.bmax, unsigned long long, amax * nb);
-  CT_TAKE(w.decision, int32_t, amax);
-  CT_TAKE(w.right_index, int32_t, amax);
-  CT_TAKE(w.next_l, int32_t, amax);
-  CT_TAKE(w.next_r, int32_t, amax);
+  CT_TAKE(w.small.id, int32_t, smax);
+  CT_TAKE(w.small.ptr, int32_t, smax);
+  CT_TAKE(w.small.size, int32_t, smax);
+  CT_TAKE(w.small.dim, int32_t, smax);
+  CT_TAKE(w.small.depth, int32_t, smax);
+  CT_TAKE(w.group_end, int32_t, 2 * n + 8);
   CT_TAKE(w.cnodes, ct_node, mmax);
   CT_TAKE(w.icount, int32_t, mmax);
   CT_TAKE(w.drank, int32_t, mmax);
   CT_TAKE(w.newidx, int32_t, mmax);
-  CT_TAKE(w.counters, int32_t, 8);
+  CT_TAKE(w.tbox, double4, mmax);
+  CT_TAKE(w.lnodes, ct_node, 2 * n + 2);
+  CT_TAKE(w.lmeta, int32_t, 2 * n + 2);
+  CT_TAKE(w.lbox, double4, 2 * n + 2);
 #undef CT_TAKE
   *total = L.bytes + 256;
   return w;
 }
 
-__global__ void k_init(int32_t* __restrict__ perm, int32_t* __restrict__ seg, int n, int root_active,
-                       ct_node* __restrict__ cnodes, Slots act, int32_t* __restrict__ counters) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) {
-    perm[i] = i;
-    seg[i] = root_active ? 0 : -1;
-  }
-  if (i == 0) {
-    cnodes[0] = ct_node{-1.0, -1.0, -1, 0, n, 0};  // creation.py:400-401
-    act.id[0] = 0;
-    act.ptr[0] = 0;
-    act.size[0] = n;
-    act.dim[0] = 0;
-    act.att[0] = 0;
-    act.depth[0] = 0;
-    counters[0] = 1;
-    counters[1] = 0;
-    counters[2] = 0;
-    counters[3] = 0;
-  }
-}
-
-// Clears per-slot reduction targets for the A slots of this level and the next-level counter.
-__global__ void k_level_reset(int A, int nb, unsigned long long* __restrict__ rmin,
-                              unsigned long long* __restrict__ rmax,
-                              unsigned long long* __restrict__ bmin,
-                              unsigned long long* __restrict__ bmax, int32_t* __restrict__ counters) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < A) {
-    rmin[i] = ~0ull;
-    rmax[i] = 0ull;
-  }
-  if (i < A * nb) {
-    bmin[i] = ~0ull;
-    bmax[i] = 0ull;
-  }
-  if (i == 0) counters[1] = 0;
-}
-
-__global__ void __launch_bounds__(kBlock) k_range(int n, const int32_t* __restrict__ seg,
-                                                  const int32_t* __restrict__ perm,
-                                                  const int32_t* __restrict__ adim,
-                                                  const double* __restrict__ bb,
-                                                  unsigned long long* __restrict__ rmin,
-                                                  unsigned long long* __restrict__ rmax) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  int s = -1;
-  unsigned long long lo = ~0ull, hi = 0ull;
-  if (i < n) {
-    s = seg[i];
-    if (s >= 0) {
-      const int d = adim[s];
-      const double* row = bb + 4 * (int64_t)perm[i];
-      lo = dkey(row[2 * d]);
-      hi = dkey(row[2 * d + 1]);
-    }
-  }
-  wave_run_minmax(s, lo, hi, rmin, rmax);
+__device__ __forceinline__ double4 ld_box4(const double* __restrict__ bb, int c) {
+  return reinterpret_cast<const double4*>(bb)[c];
 }
 
 // creation.py:44-51 + the first-match bucket of sort_bbox_indices (:115-151).  Buckets
 // [i*bl + Rmin, (i+1)*bl + Rmin) share their bounding expressions, so the first matching
-// bucket is the only one.  No match: the reference indexes past its bucket list (error).
-__global__ void __launch_bounds__(kBlock) k_bucket(int n, int nb, const int32_t* __restrict__ seg,
-                                                   const int32_t* __restrict__ perm,
-                                                   const int32_t* __restrict__ adim,
-                                                   const double* __restrict__ bb,
-                                                   const unsigned long long* __restrict__ rmin,
-                                                   const unsigned long long* __restrict__ rmax,
-                                                   int32_t* __restrict__ bid,
-                                                   int32_t* __restrict__ counters) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int s = seg[i];
-  if (s < 0) return;
-  const int d = adim[s];
-  const double range_Rmin = dval(rmin[s]);
-  const double range_Lmax = dval(rmax[s]);
-  const double bl = (range_Lmax - range_Rmin) / (double)nb;  // creation.py:278
-  const double* row = bb + 4 * (int64_t)perm[i];
-  const double lo = row[2 * d], hi = row[2 * d + 1];
+// bucket is the only one.  No match (-1): the reference indexes past its bucket list (error).
+__device__ __forceinline__ int bucket_of(double lo, double hi, double range_Rmin, double bl, int nb) {
   const double centroid = lo + 0.5 * (hi - lo);
-  int b = -1;
   for (int k = 0; k < nb; ++k) {
     const double bmax = (double)(k + 1) * bl + range_Rmin;  // creation.py:286
     const double bmin = (double)k * bl + range_Rmin;        // creation.py:287
-    if ((centroid >= bmin) && (centroid < bmax)) {
-      b = k;
-      break;
+    if ((centroid >= bmin) && (centroid < bmax)) return k;
+  }
+  return -1;
+}
+
+// What creation.py:312-379 does with a node whose cells are sorted into buckets.  count(b),
+// rmin(b), lmax(b): cells and bounds of bucket b (bounds read only where count(b) > 0).  Empty
+// buckets are skipped where the reference merges them away (:322-341): only Rmin, Lmax, index and
+// size of the non-empty ones matter afterwards.
+enum Decision : int { kLeaf = 0, kSplit = 1, kRetry = 2 };
+
+struct Split {
+  int decision;
+  int plane;      // first bucket on the right
+  int left;       // cells on the left
+  double Lmax, Rmin;
+  bool bad_cost;  // no finite cost
+};
+
+template <typename C, typename R, typename L>
+__device__ __forceinline__ Split decide(int nb, int size, int att, double range_Rmin, double range_Lmax, C count,
+                                        R rmin, L lmax) {
+  Split s{kLeaf, -1, 0, -1.0, -1.0, false};
+  const double bl = (range_Lmax - range_Rmin) / (double)nb;
+  // creation.py:174-213 split_plane: the first strict minimum
+  double best = 1.7976931348623157e308, prev_L = 0.0;
+  int m = 0;
+  long long left = 0;
+  for (int b = 0; b < nb; ++b) {
+    const int c = count(b);
+    if (c == 0) continue;
+    if (m > 0) {
+      const long long right = (long long)size - left;
+      const double left_volume = (prev_L - range_Rmin) / bl;
+      const double right_volume = (range_Lmax - rmin(b)) / bl;
+      const double cost = left_volume * (double)left + right_volume * (double)right;
+      if (cost < best) {
+        best = cost;
+        s.plane = b;
+        s.left = (int)left;
+      }
+    }
+    left += c;
+    prev_L = lmax(b);
+    ++m;
+  }
+  if (m == 1) {  // creation.py:343-358: every cell in one bucket
+    s.decision = att == 0 ? kRetry : kLeaf;
+    return s;
+  }
+  if (s.plane < 0) {
+    s.bad_cost = true;
+    return s;
+  }
+  s.decision = kSplit;
+  s.Lmax = -1.7976931348623157e308;
+  s.Rmin = 1.7976931348623157e308;
+  for (int b = 0; b < nb; ++b) {
+    if (count(b) == 0) continue;
+    if (b < s.plane) {
+      if (lmax(b) > s.Lmax) s.Lmax = lmax(b);
+    } else {
+      if (rmin(b) < s.Rmin) s.Rmin = rmin(b);
     }
   }
-  if (b < 0) {
-    counters[2] = 1;
-    b = nb - 1;
-  }
-  bid[i] = b;
+  return s;
 }
 
-// Per-tile bucket histograms (positions of active nodes only).
-__global__ void __launch_bounds__(kBlock) k_rank_count(int n, int nb, const int32_t* __restrict__ seg,
-                                                       const int32_t* __restrict__ bid,
-                                                       int32_t* __restrict__ blockcnt) {
-  __shared__ int cnt[kMaxBuckets];
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) cnt[b] = 0;
-  __syncthreads();
-  const int base = blockIdx.x * kRankTile + threadIdx.x * kRankItems;
+// ------------------------------------------------------------------- large nodes
+// The root: a leaf (n <= cells_per_leaf), a subtree of k_small (n <= T) or the first large node.
+__global__ void __launch_bounds__(kBlock) k_init(int n, int nb, int cells_per_leaf, int T, Work w,
+                                                 int32_t* __restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) {
+    w.perm[0][i] = i;
+    out[i] = i;
+  }
+  const int tiles = (n + kTile - 1) / kTile;
+  if (n > T && i < tiles) w.act[0].map[i] = 0;
+  if (i == 0) {
+    w.cnodes[0] = ct_node{-1.0, -1.0, -1, 0, n, 0};  // creation.py:400-401
+    const bool large = n > cells_per_leaf && n > T, small = n > cells_per_leaf && n <= T;
+    const Slots& s = w.act[0];
+    s.id[0] = 0;
+    s.ptr[0] = 0;
+    s.size[0] = n;
+    s.dim[0] = 0;
+    s.att[0] = 0;
+    s.depth[0] = 0;
+    s.tile0[0] = 0;
+    Header& h = *w.head;
+    for (int k = 0; k < 4; ++k) s.range[k] = (k & 1) ? h.stats[k] : ~h.stats[k];
+    w.small.id[0] = 0;
+    w.small.ptr[0] = 0;
+    w.small.size[0] = n;
+    w.small.dim[0] = 0;
+    w.small.depth[0] = 0;
+    h.next_id = 1;
+    h.err = 0;
+    h.depth = 0;
+    h.n_small = small ? 1 : 0;
+    h.active[0] = large ? 1 : 0;
+    h.active[1] = 0;
+    h.tiles[0] = large ? tiles : 0;
+    h.tiles[1] = 0;
+    h.n_nodes = 0;
+    w.group_end[0] = 1;
+  }
+}
+
+// Buckets of a tile's cells, the tile's bucket counts and the bucket bounds in both dimensions
+// (LDS atomics: 16 lanes of a wavefront per address at 4 buckets, a few hundred cycles a tile).
+__global__ void __launch_bounds__(kBlock) k_tile_count(int nb, int level, int par, const double* __restrict__ bb,
+                                                       Work w) {
+  __shared__ int hist[kMaxBuckets];
+  __shared__ Key bnd[kMaxBuckets * 4];
+  Header* h = w.head;
+  const int t = blockIdx.x;
+  if (t == 0 && threadIdx.x == 0) {  // k_node_decide of this level fills the next level's lists
+    h->active[par ^ 1] = 0;
+    h->tiles[par ^ 1] = 0;
+    w.group_end[level] = h->next_id;
+  }
+  if (t >= h->tiles[par]) return;
+  const Slots& cur = w.act[par];
+  const int s = cur.map[t];
+  const int d = cur.dim[s];
+  const int begin = (t - cur.tile0[s]) * kTile;
+  const int count = min(kTile, cur.size[s] - begin);
+  const int base = cur.ptr[s] + begin;
+  const double range_Rmin = dval(cur.range[4 * s + 2 * d]);
+  const double range_Lmax = dval(cur.range[4 * s + 2 * d + 1]);
+  const double bl = (range_Lmax - range_Rmin) / (double)nb;  // creation.py:278
+  for (int k = threadIdx.x; k < 4 * nb; k += kBlock) bnd[k] = (k & 1) ? 0ull : ~0ull;
+  for (int k = threadIdx.x; k < nb; k += kBlock) hist[k] = 0;
+  const int32_t* __restrict__ perm = w.perm[par];
+  double4 box[kTileItems];
 #pragma unroll
-  for (int j = 0; j < kRankItems; ++j) {
-    const int p = base + j;
-    if (p < n && seg[p] >= 0) atomicAdd(&cnt[bid[p]], 1);
+  for (int j = 0; j < kTileItems; ++j) {
+    const int p = j * kBlock + threadIdx.x;
+    if (p < count) box[j] = ld_box4(bb, perm[base + p]);
   }
   __syncthreads();
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) blockcnt[blockIdx.x * nb + b] = cnt[b];
+#pragma unroll
+  for (int j = 0; j < kTileItems; ++j) {
+    const int p = j * kBlock + threadIdx.x;
+    if (p >= count) continue;
+    const double4 x = box[j];
+    int b = bucket_of(d ? x.z : x.x, d ? x.w : x.y, range_Rmin, bl, nb);
+    if (b < 0) {
+      h->err = 1;
+      b = nb - 1;
+    }
+    w.bid[base + p] = (uint8_t)b;
+    atomicAdd(&hist[b], 1);
+    atomicMin(&bnd[4 * b + 0], dkey(x.x));
+    atomicMax(&bnd[4 * b + 1], dkey(x.y));
+    atomicMin(&bnd[4 * b + 2], dkey(x.z));
+    atomicMax(&bnd[4 * b + 3], dkey(x.w));
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k < 4 * nb; k += kBlock) w.tilebk[(int64_t)t * 4 * nb + k] = bnd[k];
+  for (int k = threadIdx.x; k < nb; k += kBlock) w.tilecnt[(int64_t)t * nb + k] = hist[k];
 }
 
-// Exclusive scan of the tile histograms, per bucket, in one workgroup.
-__global__ void __launch_bounds__(kBlock) k_rank_scan(int nblk, int nb, int32_t* __restrict__ blockcnt) {
-  __shared__ int lds[kBlock / 64];
-  for (int b = 0; b < nb; ++b) {
-    int carry = 0;
-    for (int base = 0; base < nblk; base += kBlock) {
-      const int k = base + threadIdx.x;
-      const int v = (k < nblk) ? blockcnt[k * nb + b] : 0;
-      int total;
-      const int ex = block_exclusive_scan<int>(v, lds, &total);
-      if (k < nblk) blockcnt[k * nb + b] = carry + ex;
+// One workgroup per large node.
+__global__ void __launch_bounds__(kDecideBlock) k_node_decide(int nb, int cells_per_leaf, int T, int par, Work w) {
+  __shared__ Key bnd[kMaxBuckets * 4];
+  __shared__ int cnt[kMaxBuckets];
+  __shared__ Key lds[kDecideBlock / 64];
+  __shared__ int next_slot[2], next_tile[2], next_tiles[2];
+  Header* h = w.head;
+  const int s = blockIdx.x;
+  if (s >= h->active[par]) return;
+  const Slots& cur = w.act[par];
+  const Slots& nxt = w.act[par ^ 1];
+  const int X = cur.id[s], ptr = cur.ptr[s], size = cur.size[s], dim = cur.dim[s];
+  const int att = cur.att[s], depth = cur.depth[s], tile0 = cur.tile0[s];
+  const int ntiles = (size + kTile - 1) / kTile;
+  const int tid = threadIdx.x;
+  for (int k = tid; k < 4 * nb; k += kDecideBlock) bnd[k] = (k & 1) ? 0ull : ~0ull;
+  __syncthreads();
+  // bucket bounds over the node's tiles: a lane keeps to one of the 4 nb bounds
+  const int keys = 4 * nb, lanes = kDecideBlock / keys * keys;
+  if (tid < lanes) {
+    const int k = tid % keys;
+    Key v = (k & 1) ? 0ull : ~0ull;
+    for (int64_t i = tid; i < (int64_t)ntiles * keys; i += lanes) {
+      const Key x = w.tilebk[(int64_t)tile0 * keys + i];
+      v = (k & 1) ? (x > v ? x : v) : (x < v ? x : v);
+    }
+    if (k & 1) atomicMax(&bnd[k], v);
+    else atomicMin(&bnd[k], v);
+  }
+  // prefix of the tile counts, two buckets per scan (a node has fewer than 2^30 cells)
+  for (int b = 0; b < nb; b += 2) {
+    const bool two = b + 1 < nb;
+    Key carry = 0;
+    for (int t0 = 0; t0 < ntiles; t0 += kDecideBlock) {
+      const int t = t0 + tid;
+      const int64_t at = (int64_t)(tile0 + t) * nb + b;
+      Key v = 0;
+      if (t < ntiles) v = (Key)(unsigned)w.tilecnt[at] | (two ? (Key)(unsigned)w.tilecnt[at + 1] << 32 : 0ull);
+      Key total;
+      const Key e = carry + block_exclusive_scan<Key, kDecideBlock>(v, lds, &total);
+      if (t < ntiles) {
+        w.tilepre[at] = (int)(unsigned)e;
+        if (two) w.tilepre[at + 1] = (int)(unsigned)(e >> 32);
+      }
       carry += total;
     }
-  }
-}
-
-// Global prefix count of each position's bucket; node heads / tails record the prefix
-// vector at their segment start / end so k_scatter can rebase ranks per node.
-__global__ void __launch_bounds__(kBlock) k_rank_write(int n, int nb, const int32_t* __restrict__ seg,
-                                                       const int32_t* __restrict__ bid,
-                                                       const int32_t* __restrict__ blockcnt,
-                                                       const int32_t* __restrict__ aptr,
-                                                       const int32_t* __restrict__ asize,
-                                                       int32_t* __restrict__ rank,
-                                                       int32_t* __restrict__ sstart,
-                                                       int32_t* __restrict__ send) {
-  __shared__ int lds[kBlock / 64];
-  const int base = blockIdx.x * kRankTile + threadIdx.x * kRankItems;
-  int ps[kRankItems], pb[kRankItems];
-#pragma unroll
-  for (int j = 0; j < kRankItems; ++j) {
-    const int p = base + j;
-    ps[j] = (p < n) ? seg[p] : -1;
-    pb[j] = (ps[j] >= 0) ? bid[p] : -1;
-  }
-  for (int b = 0; b < nb; ++b) {
-    int c = 0;
-#pragma unroll
-    for (int j = 0; j < kRankItems; ++j) c += (pb[j] == b);
-    int total;
-    int run = blockcnt[blockIdx.x * nb + b] + block_exclusive_scan<int>(c, lds, &total);
-#pragma unroll
-    for (int j = 0; j < kRankItems; ++j) {
-      const int p = base + j;
-      const int s = ps[j];
-      if (s < 0) continue;
-      if (p == aptr[s]) sstart[s * nb + b] = run;
-      if (pb[j] == b) {
-        rank[p] = run;
-        ++run;
-      }
-      if (p == aptr[s] + asize[s] - 1) send[s * nb + b] = run;
+    if (tid == 0) {
+      cnt[b] = (int)(unsigned)carry;
+      if (two) cnt[b + 1] = (int)(unsigned)(carry >> 32);
     }
   }
-}
-
-// Per node: bucket start offsets relative to the node's first position.
-__global__ void k_offsets(int A, int nb, const int32_t* __restrict__ sstart,
-                          const int32_t* __restrict__ send, int32_t* __restrict__ boff) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= A) return;
-  int off = 0;
-  for (int b = 0; b < nb; ++b) {
-    boff[s * nb + b] = off;
-    off += send[s * nb + b] - sstart[s * nb + b];
-  }
-}
-
-__global__ void __launch_bounds__(kBlock) k_scatter(int n, int nb, const int32_t* __restrict__ seg,
-                                                    const int32_t* __restrict__ perm,
-                                                    const int32_t* __restrict__ bid,
-                                                    const int32_t* __restrict__ rank,
-                                                    const int32_t* __restrict__ aptr,
-                                                    const int32_t* __restrict__ sstart,
-                                                    const int32_t* __restrict__ boff,
-                                                    int32_t* __restrict__ perm2,
-                                                    int32_t* __restrict__ bid2) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  const int s = seg[p];
-  if (s < 0) {
-    perm2[p] = perm[p];
-    return;
-  }
-  const int b = bid[p];
-  const int q = aptr[s] + boff[s * nb + b] + (rank[p] - sstart[s * nb + b]);
-  perm2[q] = perm[p];
-  bid2[q] = b;
-}
-
-__global__ void __launch_bounds__(kBlock) k_bbounds(int n, int nb, const int32_t* __restrict__ seg,
-                                                    const int32_t* __restrict__ perm,
-                                                    const int32_t* __restrict__ bid,
-                                                    const int32_t* __restrict__ adim,
-                                                    const double* __restrict__ bb,
-                                                    unsigned long long* __restrict__ bmin,
-                                                    unsigned long long* __restrict__ bmax) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  int key = -1;
-  unsigned long long lo = ~0ull, hi = 0ull;
-  if (p < n) {
-    const int s = seg[p];
-    if (s >= 0) {
-      key = s * nb + bid[p];
-      const int d = adim[s];
-      const double* row = bb + 4 * (int64_t)perm[p];
-      lo = dkey(row[2 * d]);
-      hi = dkey(row[2 * d + 1]);
+  __syncthreads();
+  if (tid == 0) {
+    next_slot[0] = next_slot[1] = -1;
+    int off = ptr;
+    for (int b = 0; b < nb; ++b) {
+      w.boff[s * nb + b] = off;
+      off += cnt[b];
     }
-  }
-  wave_run_minmax(key, lo, hi, bmin, bmax);
-}
-
-__global__ void k_decide(int A, int nb, int cells_per_leaf, Slots cur, Slots nxt,
-                         const unsigned long long* __restrict__ rmin,
-                         const unsigned long long* __restrict__ rmax,
-                         const int32_t* __restrict__ sstart, const int32_t* __restrict__ send,
-                         const int32_t* __restrict__ boff,
-                         const unsigned long long* __restrict__ bminv,
-                         const unsigned long long* __restrict__ bmaxv,
-                         ct_node* __restrict__ cnodes, int32_t* __restrict__ decision,
-                         int32_t* __restrict__ right_index, int32_t* __restrict__ next_l,
-                         int32_t* __restrict__ next_r, int32_t* __restrict__ counters) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= A) return;
-  const int X = cur.id[s], ptr = cur.ptr[s], size = cur.size[s], dim = cur.dim[s];
-  const int att = cur.att[s], depth = cur.depth[s];
-  const double range_Rmin = dval(rmin[s]);
-  const double range_Lmax = dval(rmax[s]);
-  const double bl = (range_Lmax - range_Rmin) / (double)nb;
-  const int ndim = dim ? 0 : 1;
-
-  auto push_child = [&](int id, int cptr, int csize) -> int {
-    cnodes[id] = ct_node{-1.0, -1.0, -1, cptr, csize, ndim};  // creation.py:27-29
-    if (csize <= cells_per_leaf) return -1;
-    const int ns = atomicAdd(&counters[1], 1);
-    nxt.id[ns] = id;
-    nxt.ptr[ns] = cptr;
-    nxt.size[ns] = csize;
-    nxt.dim[ns] = ndim;
-    nxt.att[ns] = 0;
-    nxt.depth[ns] = depth + 1;
-    return ns;
-  };
-
-  if (cells_per_leaf == 1 && size == 2) {  // creation.py:312-320
-    cnodes[X].Lmax = range_Lmax;
-    cnodes[X].Rmin = range_Rmin;
-    const int c = atomicAdd(&counters[0], 2);
-    cnodes[X].child = c;
-    push_child(c, ptr, 1);
-    push_child(c + 1, ptr + 1, 1);
-    atomicMax(&counters[3], depth + 1);
-    decision[s] = kLeaf;  // both children are leaves: no position stays active
-    return;
-  }
-
-  // Non-empty buckets in order (creation.py:322-341 merges the empty ones away; only
-  // Rmin, Lmax, index and size matter afterwards).
-  double bR[kMaxBuckets], bL[kMaxBuckets];
-  int bI[kMaxBuckets], bS[kMaxBuckets];
-  int m = 0;
-  for (int b = 0; b < nb; ++b) {
-    const int cnt = send[s * nb + b] - sstart[s * nb + b];
-    if (cnt > 0) {
-      bR[m] = dval(bminv[s * nb + b]);
-      bL[m] = dval(bmaxv[s * nb + b]);
-      bI[m] = ptr + boff[s * nb + b];
-      bS[m] = cnt;
-      ++m;
-    }
-  }
-
-  if (m == 1) {  // creation.py:343-358: every cell in one bucket
-    if (att == 0) {
-      cnodes[X].dim = ndim;
-      const int ns = atomicAdd(&counters[1], 1);
-      nxt.id[ns] = X;
-      nxt.ptr[ns] = ptr;
-      nxt.size[ns] = size;
+    const Key* range = cur.range + 4 * s;
+    const double range_Rmin = dval(range[2 * dim]), range_Lmax = dval(range[2 * dim + 1]);
+    const Split sp = decide(
+        nb, size, att, range_Rmin, range_Lmax, [&](int b) { return cnt[b]; },
+        [&](int b) { return dval(bnd[4 * b + 2 * dim]); }, [&](int b) { return dval(bnd[4 * b + 2 * dim + 1]); });
+    const int ndim = dim ? 0 : 1;
+    auto push_large = [&](int which, int id, int cptr, int csize, int catt, int cdepth, const Key (&r)[4]) {
+      const int ns = atomicAdd(&h->active[par ^ 1], 1);
+      const int nt = (csize + kTile - 1) / kTile;
+      const int t0 = atomicAdd(&h->tiles[par ^ 1], nt);
+      nxt.id[ns] = id;
+      nxt.ptr[ns] = cptr;
+      nxt.size[ns] = csize;
       nxt.dim[ns] = ndim;
-      nxt.att[ns] = 1;
-      nxt.depth[ns] = depth;
-      decision[s] = kRetry;
-      next_l[s] = ns;
-    } else {
-      cnodes[X].Lmax = -1.0;
-      cnodes[X].Rmin = -1.0;
-      decision[s] = kLeaf;
+      nxt.att[ns] = catt;
+      nxt.depth[ns] = cdepth;
+      nxt.tile0[ns] = t0;
+      for (int k = 0; k < 4; ++k) nxt.range[4 * ns + k] = r[k];
+      next_slot[which] = ns;
+      next_tile[which] = t0;
+      next_tiles[which] = nt;
+    };
+    if (sp.bad_cost) h->err = 2;
+    if (sp.decision == kRetry) {
+      w.cnodes[X].dim = ndim;
+      const Key r[4] = {range[0], range[1], range[2], range[3]};
+      push_large(0, X, ptr, size, 1, depth, r);
+    } else if (sp.decision == kSplit) {
+      const int c = atomicAdd(&h->next_id, 2);
+      w.cnodes[X].Lmax = sp.Lmax;
+      w.cnodes[X].Rmin = sp.Rmin;
+      w.cnodes[X].child = c;
+      atomicMax(&h->depth, depth + 1);
+      for (int side = 0; side < 2; ++side) {
+        const int id = c + side, cptr = side ? ptr + sp.left : ptr, csize = side ? size - sp.left : sp.left;
+        w.cnodes[id] = ct_node{-1.0, -1.0, -1, cptr, csize, ndim};  // creation.py:27-29
+        if (csize <= cells_per_leaf) continue;
+        if (csize <= T) {
+          const int k = atomicAdd(&h->n_small, 1);
+          w.small.id[k] = id;
+          w.small.ptr[k] = cptr;
+          w.small.size[k] = csize;
+          w.small.dim[k] = ndim;
+          w.small.depth[k] = depth + 1;
+          continue;
+        }
+        Key r[4] = {~0ull, 0ull, ~0ull, 0ull};
+        for (int b = side ? sp.plane : 0; b < (side ? nb : sp.plane); ++b)
+          for (int k = 0; k < 4; ++k) {
+            const Key x = bnd[4 * b + k];  // the neutral key for an empty bucket
+            r[k] = (k & 1) ? (x > r[k] ? x : r[k]) : (x < r[k] ? x : r[k]);
+          }
+        push_large(side, id, cptr, csize, 0, depth + 1, r);
+      }
+    }
+  }
+  __syncthreads();
+  for (int k = 0; k < 2; ++k)
+    if (next_slot[k] >= 0)
+      for (int t = tid; t < next_tiles[k]; t += kDecideBlock) nxt.map[next_tile[k] + t] = next_slot[k];
+}
+
+// Bucket counts packed 16 bits each, four to a word: prefix and per-node totals of all buckets
+// of a tile (or a subtree's level) in one scan a word.
+__device__ __forceinline__ int packed(Key w, int b) { return (int)((w >> (16 * (b & 3))) & 0xffffu); }
+
+// The cells of a tile to their buckets, in order.  `out` always holds the latest order of every
+// position, whichever level a position is last touched at.
+__global__ void __launch_bounds__(kBlock) k_tile_scatter(int nb, int par, Work w, int32_t* __restrict__ out) {
+  __shared__ Key lds[kBlock / 64];
+  const int t = blockIdx.x;
+  if (t >= w.head->tiles[par]) return;
+  const Slots& cur = w.act[par];
+  const int s = cur.map[t];
+  const int begin = (t - cur.tile0[s]) * kTile;
+  const int count = min(kTile, cur.size[s] - begin);
+  const int base = cur.ptr[s] + begin;
+  int c[kTileItems], b[kTileItems];
+#pragma unroll
+  for (int j = 0; j < kTileItems; ++j) {
+    const int p = threadIdx.x * kTileItems + j;
+    c[j] = p < count ? w.perm[par][base + p] : -1;
+    b[j] = p < count ? (int)w.bid[base + p] : -4;
+  }
+  for (int word = 0; word < (nb + 3) / 4; ++word) {
+    Key v = 0;
+#pragma unroll
+    for (int j = 0; j < kTileItems; ++j)
+      if ((b[j] >> 2) == word) v += 1ull << (16 * (b[j] & 3));
+    Key total;
+    Key run = block_exclusive_scan<Key>(v, lds, &total);
+#pragma unroll
+    for (int j = 0; j < kTileItems; ++j) {
+      if ((b[j] >> 2) != word) continue;
+      const int q = w.boff[s * nb + b[j]] + w.tilepre[(int64_t)t * nb + b[j]] + packed(run, b[j]);
+      w.perm[par ^ 1][q] = c[j];
+      out[q] = c[j];
+      run += 1ull << (16 * (b[j] & 3));
+    }
+  }
+}
+
+// ------------------------------------------------------------------- subtrees in LDS
+__device__ __forceinline__ double4 box_union(double4 a, double4 b) {  // NaN poisons the union
+  const double nan = __builtin_nan("");
+  const bool bad = isnan(a.x) || isnan(a.y) || isnan(a.z) || isnan(a.w) || isnan(b.x) || isnan(b.y) ||
+                   isnan(b.z) || isnan(b.w);
+  if (bad) return make_double4(nan, nan, nan, nan);
+  return make_double4(b.x < a.x ? b.x : a.x, b.y > a.y ? b.y : a.y, b.z < a.z ? b.z : a.z,
+                      b.w > a.w ? b.w : a.w);
+}
+
+__device__ __forceinline__ double4 empty_box() {
+  const double inf = __builtin_inf();
+  return make_double4(inf, -inf, inf, -inf);
+}
+
+// One workgroup builds the whole subtree of a node of at most T cells: the levels of creation.py
+// run one after the other over the subtree's positions, T / THREADS of them per lane, with LDS
+// arrays and barriers where the large nodes have global arrays and kernels.  A cell's box is
+// gathered (16 bytes of it) once per level; everything else is in LDS.
+//   per level:  1 extents per node (a wavefront whose positions share one node reduces in
+//                 registers; otherwise LDS atomics)
+//               2 buckets, and the prefix over positions of the packed bucket counts
+//               3 the cells to their buckets; bucket bounds (LDS atomics)
+//               4 split decisions, one lane per node
+//               5 positions to the children's slots
+// NB: the bucket class (>= nb).
+template <int NB, int T, int THREADS>
+__global__ void __launch_bounds__(THREADS) k_small(int nb, int cells_per_leaf, int first, int want_boxes,
+                                                   const double* __restrict__ bb, Work w, int32_t* out) {
+  constexpr int IT = T / THREADS;
+  constexpr int W = NB / 4;
+  constexpr int S = T / 2;  // an active node has at least two cells
+  static_assert(T <= 1024 && IT * THREADS == T, "16-bit packed counts and node ids");
+  __shared__ int perm[T];
+  __shared__ short seg[T];
+  __shared__ Key pre[W][T + 1];
+  __shared__ Key rmin[S], rmax[S];
+  __shared__ Key bnd[2][S * NB];
+  __shared__ uint16_t sptr[2][S], ssize[2][S], sid[2][S], sdepth[2][S];
+  __shared__ uint8_t sdim[2][S], satt[2][S];
+  __shared__ uint16_t dright[S];
+  __shared__ short dl[S], dr[S];
+  __shared__ uint16_t child[2 * T];
+  __shared__ uint16_t gend[2 * T + 4];
+  __shared__ Key wave_tot[W][THREADS / 64];
+  __shared__ int next_id, n_next, max_depth, err;
+  // after the last level: node counts and ranks, where the bucket bounds were
+  uint16_t* ic = reinterpret_cast<uint16_t*>(&bnd[0][0]);
+  uint16_t* rk = ic + 2 * T;
+  uint16_t* li = rk + 2 * T;
+  static_assert(sizeof(bnd) >= 3 * 2 * T * sizeof(uint16_t), "node arrays fit the bucket bounds");
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+
+  for (int si = first + blockIdx.x; si < w.head->n_small; si += gridDim.x) {
+    const int root = w.small.id[si], base = w.small.ptr[si], m = w.small.size[si];
+    ct_node* ln = w.lnodes + 2 * (int64_t)base;
+    double4* lb = w.lbox + 2 * (int64_t)base;
+    auto node = [&](int x) { return x == 0 ? w.cnodes + root : ln + x; };
+    __syncthreads();  // the previous subtree's arrays are done with
+    for (int p = tid; p < T; p += THREADS) {
+      perm[p] = p < m ? out[base + p] : -1;
+      seg[p] = p < m ? 0 : -1;
+    }
+    if (tid == 0) {
+      sptr[0][0] = 0;
+      ssize[0][0] = (uint16_t)m;
+      sid[0][0] = 0;
+      sdepth[0][0] = 0;
+      sdim[0][0] = (uint8_t)w.small.dim[si];
+      satt[0][0] = 0;
+      next_id = 1;
+      n_next = 0;
+      max_depth = 0;
+      err = 0;
+      gend[0] = 1;
+      child[0] = 0;
+      rmin[0] = ~0ull;
+      rmax[0] = 0ull;
+    }
+    for (int k = tid; k < NB; k += THREADS) {
+      bnd[0][k] = ~0ull;
+      bnd[1][k] = 0ull;
+    }
+    int A = 1, cur = 0, G = 0;
+    __syncthreads();
+    while (A > 0) {
+      // 1: extents
+      int c[IT], s[IT];
+      Key lo[IT], hi[IT];
+#pragma unroll
+      for (int j = 0; j < IT; ++j) {
+        const int p = tid * IT + j;
+        s[j] = seg[p];
+        c[j] = perm[p];
+        lo[j] = ~0ull;
+        hi[j] = 0ull;
+        if (s[j] >= 0) {
+          const double2 x = reinterpret_cast<const double2*>(bb)[2 * (int64_t)c[j] + sdim[cur][s[j]]];
+          lo[j] = dkey(x.x);
+          hi[j] = dkey(x.y);
+        }
+      }
+      {
+        bool one = true;
+        const int s0 = __builtin_amdgcn_readfirstlane(s[0]);
+        Key l = lo[0], h = hi[0];
+#pragma unroll
+        for (int j = 0; j < IT; ++j) {
+          one = one && s[j] == s0;
+          l = lo[j] < l ? lo[j] : l;
+          h = hi[j] > h ? hi[j] : h;
+        }
+        if (__all(one)) {
+          if (s0 >= 0) {
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) {
+              const Key l2 = __shfl_xor(l, d, 64), h2 = __shfl_xor(h, d, 64);
+              l = l2 < l ? l2 : l;
+              h = h2 > h ? h2 : h;
+            }
+            if (lane == 0) {
+              atomicMin(&rmin[s0], l);
+              atomicMax(&rmax[s0], h);
+            }
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < IT; ++j) {
+            if (s[j] < 0) continue;
+            atomicMin(&rmin[s[j]], lo[j]);
+            atomicMax(&rmax[s[j]], hi[j]);
+          }
+        }
+      }
+      __syncthreads();
+      // 2: buckets and the prefix of their packed counts
+      int b[IT];
+      Key mine[W], incl[W];
+#pragma unroll
+      for (int k = 0; k < W; ++k) mine[k] = 0;
+#pragma unroll
+      for (int j = 0; j < IT; ++j) {
+        b[j] = -4;
+        if (s[j] < 0) continue;
+        const double range_Rmin = dval(rmin[s[j]]);
+        const double bl = (dval(rmax[s[j]]) - range_Rmin) / (double)nb;
+        b[j] = bucket_of(dval(lo[j]), dval(hi[j]), range_Rmin, bl, nb);
+        if (b[j] < 0) {
+          err = 1;
+          b[j] = nb - 1;
+        }
+#pragma unroll
+        for (int k = 0; k < W; ++k)
+          if ((b[j] >> 2) == k) mine[k] += 1ull << (16 * (b[j] & 3));
+      }
+#pragma unroll
+      for (int k = 0; k < W; ++k) {
+        Key x = mine[k];
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+          const Key y = __shfl_up(x, d, 64);
+          if (lane >= d) x += y;
+        }
+        incl[k] = x;
+        if (lane == 63) wave_tot[k][wave] = x;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < W; ++k) {
+        Key run = incl[k] - mine[k];
+        for (int v = 0; v < THREADS / 64; ++v)
+          if (v < wave) run += wave_tot[k][v];
+#pragma unroll
+        for (int j = 0; j < IT; ++j) {
+          pre[k][tid * IT + j] = run;
+          if ((b[j] >> 2) == k) run += 1ull << (16 * (b[j] & 3));
+        }
+        if (tid == THREADS - 1) pre[k][T] = run;
+      }
+      __syncthreads();
+      // 3: the cells to their buckets
+#pragma unroll
+      for (int j = 0; j < IT; ++j) {
+        if (s[j] < 0) continue;
+        const int p = tid * IT + j, sl = s[j];
+        const int a = sptr[cur][sl], e = a + ssize[cur][sl];
+        int q = a;
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+          const Key p0 = pre[k][a], tot = pre[k][e] - p0;
+#pragma unroll
+          for (int f = 0; f < 4; ++f)
+            if (4 * k + f < b[j]) q += packed(tot, f);
+          if ((b[j] >> 2) == k) q += packed(pre[k][p] - p0, b[j]);
+        }
+        perm[q] = c[j];
+        atomicMin(&bnd[0][sl * NB + b[j]], lo[j]);
+        atomicMax(&bnd[1][sl * NB + b[j]], hi[j]);
+      }
+      __syncthreads();
+      // 4: decisions
+      const int nx = cur ^ 1;
+      for (int sl = tid; sl < A; sl += THREADS) {
+        const int a = sptr[cur][sl], size = ssize[cur][sl], X = sid[cur][sl], dim = sdim[cur][sl];
+        const int depth = sdepth[cur][sl], ndim = dim ? 0 : 1;
+        const double range_Rmin = dval(rmin[sl]), range_Lmax = dval(rmax[sl]);
+        auto push = [&](int id, int cptr, int csize, int catt, int cdepth) -> int {
+          const int ns = atomicAdd(&n_next, 1);
+          sptr[nx][ns] = (uint16_t)cptr;
+          ssize[nx][ns] = (uint16_t)csize;
+          sid[nx][ns] = (uint16_t)id;
+          sdim[nx][ns] = (uint8_t)ndim;
+          satt[nx][ns] = (uint8_t)catt;
+          sdepth[nx][ns] = (uint16_t)cdepth;
+          return ns;
+        };
+        auto split = [&](double Lmax, double Rmin, int left) {
+          ct_node* nd = node(X);
+          const int ch = atomicAdd(&next_id, 2);
+          nd->Lmax = Lmax;
+          nd->Rmin = Rmin;
+          nd->child = X == 0 ? -2 : 1;  // linked by k_emit
+          child[X] = (uint16_t)ch;
+          child[ch] = child[ch + 1] = 0;
+          ln[ch] = ct_node{-1.0, -1.0, -1, base + a, left, ndim};  // creation.py:27-29
+          ln[ch + 1] = ct_node{-1.0, -1.0, -1, base + a + left, size - left, ndim};
+          dright[sl] = (uint16_t)(a + left);
+          dl[sl] = left > cells_per_leaf ? (short)push(ch, a, left, 0, depth + 1) : (short)-1;
+          dr[sl] = size - left > cells_per_leaf ? (short)push(ch + 1, a + left, size - left, 0, depth + 1) : (short)-1;
+          atomicMax(&max_depth, depth + 1);
+        };
+        dright[sl] = 0;
+        dl[sl] = dr[sl] = -1;
+        if (cells_per_leaf == 1 && size == 2) {  // creation.py:312-320
+          split(range_Lmax, range_Rmin, 1);
+          continue;
+        }
+        Key tot[W];
+#pragma unroll
+        for (int k = 0; k < W; ++k) tot[k] = pre[k][a + size] - pre[k][a];
+        const Split sp = decide(
+            nb, size, satt[cur][sl], range_Rmin, range_Lmax,
+            [&](int k) {
+              Key x = tot[0];
+#pragma unroll
+              for (int v = 1; v < W; ++v) x = (k >> 2) == v ? tot[v] : x;
+              return packed(x, k);
+            },
+            [&](int k) { return dval(bnd[0][sl * NB + k]); }, [&](int k) { return dval(bnd[1][sl * NB + k]); });
+        if (sp.bad_cost) err = 2;
+        if (sp.decision == kRetry) {
+          node(X)->dim = ndim;
+          dl[sl] = dr[sl] = (short)push(X, a, size, 1, depth);
+        } else if (sp.decision == kSplit) {
+          split(sp.Lmax, sp.Rmin, sp.left);
+        }
+      }
+      __syncthreads();
+      // 5: positions to their children's slots; the next level's reduction targets
+      const int An = n_next;
+#pragma unroll
+      for (int j = 0; j < IT; ++j) {
+        if (s[j] < 0) continue;
+        const int p = tid * IT + j;
+        seg[p] = p < (int)dright[s[j]] ? dl[s[j]] : dr[s[j]];
+      }
+      for (int k = tid; k < An; k += THREADS) {
+        rmin[k] = ~0ull;
+        rmax[k] = 0ull;
+      }
+      for (int k = tid; k < An * NB; k += THREADS) {
+        bnd[0][k] = ~0ull;
+        bnd[1][k] = 0ull;
+      }
+      __syncthreads();
+      ++G;
+      if (tid == 0) {
+        n_next = 0;
+        gend[G] = (uint16_t)next_id;
+      }
+      A = An;
+      cur = nx;
+    }
+    __syncthreads();
+    const int N = next_id;
+    for (int p = tid; p < m; p += THREADS) out[base + p] = perm[p];
+    // leaves, then internal nodes bottom-up: internal nodes per subtree, tight boxes
+    for (int x = tid; x < N; x += THREADS) {
+      if (child[x] != 0) continue;
+      ic[x] = 0;
+      if (!want_boxes) continue;
+      const ct_node nd = *node(x);
+      double4 u = empty_box();
+      for (int k = nd.ptr - base; k < nd.ptr - base + nd.size; ++k) u = box_union(u, ld_box4(bb, perm[k]));
+      (x == 0 ? w.tbox[root] : lb[x]) = u;
+    }
+    __syncthreads();
+    for (int g = G; g >= 0; --g) {
+      const int lo = g == 0 ? 0 : gend[g - 1], hi = gend[g];
+      for (int x = lo + tid; x < hi; x += THREADS) {
+        const int ch = child[x];
+        if (ch == 0) continue;
+        ic[x] = (uint16_t)(1 + ic[ch] + ic[ch + 1]);
+        if (want_boxes) (x == 0 ? w.tbox[root] : lb[x]) = box_union(lb[ch], lb[ch + 1]);
+      }
+      __syncthreads();
+    }
+    // top-down: ranks and DFS indices
+    if (tid == 0) {
+      rk[0] = 0;
+      li[0] = 0;
+    }
+    __syncthreads();
+    for (int g = 0; g <= G; ++g) {
+      const int lo = g == 0 ? 0 : gend[g - 1], hi = gend[g];
+      for (int x = lo + tid; x < hi; x += THREADS) {
+        const int ch = child[x];
+        if (ch == 0) continue;
+        const int r = rk[x];
+        li[ch] = (uint16_t)(1 + 2 * r);
+        li[ch + 1] = (uint16_t)(2 + 2 * r);
+        rk[ch] = (uint16_t)(r + 1);
+        rk[ch + 1] = (uint16_t)(r + 1 + ic[ch]);
+      }
+      __syncthreads();
+    }
+    for (int x = tid; x < N; x += THREADS)
+      if (x > 0) w.lmeta[2 * (int64_t)base + x] = (int)((unsigned)li[x] | ((unsigned)rk[x] << 16));
+    if (tid == 0) {
+      w.icount[root] = ic[0];
+      atomicMax(&w.head->depth, w.small.depth[si] + max_depth);
+      if (err) w.head->err = err;
+    }
+  }
+}
+
+// ------------------------------------------------------------------- numbering
+// The large-node stage's nodes: internal nodes per subtree and tight boxes bottom-up, DFS ranks
+// top-down, by creation level.  There are about 2 n / T of them, so one workgroup does it.
+constexpr int kTopBlock = 1024;
+
+__global__ void __launch_bounds__(kTopBlock) k_top(int levels, int want_boxes, const double* __restrict__ bb, Work w,
+                                                   const int32_t* __restrict__ cells,
+                                                   const int64_t* __restrict__ flags) {
+  const int tid = threadIdx.x, M = w.head->next_id;
+  ct_node* cn = w.cnodes;
+  // leaves: one wavefront each
+  for (int x = tid >> 6; x < M; x += kTopBlock / 64) {
+    const ct_node nd = cn[x];
+    if (nd.child != -1) continue;
+    double4 u = empty_box();
+    if (want_boxes) {
+      for (int k = nd.ptr + lane_id(); k < nd.ptr + nd.size; k += 64) u = box_union(u, ld_box4(bb, cells[k]));
+#pragma unroll
+      for (int d = 32; d >= 1; d >>= 1) {
+        const double4 v = make_double4(__shfl_xor(u.x, d, 64), __shfl_xor(u.y, d, 64), __shfl_xor(u.z, d, 64),
+                                       __shfl_xor(u.w, d, 64));
+        u = box_union(u, v);
+      }
+    }
+    if (lane_id() == 0) {
+      w.icount[x] = 0;
+      if (want_boxes) w.tbox[x] = u;
+    }
+  }
+  __syncthreads();
+  for (int g = levels; g >= 0; --g) {
+    const int lo = g == 0 ? 0 : w.group_end[g - 1], hi = g == levels ? M : w.group_end[g];
+    for (int x = lo + tid; x < hi; x += kTopBlock) {
+      const int c = cn[x].child;
+      if (c < 0) continue;
+      w.icount[x] = 1 + w.icount[c] + w.icount[c + 1];
+      if (want_boxes) w.tbox[x] = box_union(w.tbox[c], w.tbox[c + 1]);
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    w.drank[0] = 0;
+    w.newidx[0] = 0;
+  }
+  __syncthreads();
+  for (int g = 0; g <= levels; ++g) {
+    const int lo = g == 0 ? 0 : w.group_end[g - 1], hi = g == levels ? M : w.group_end[g];
+    for (int x = lo + tid; x < hi; x += kTopBlock) {
+      const int c = cn[x].child;
+      if (c < 0) continue;
+      const int r = w.drank[x];
+      w.newidx[c] = 1 + 2 * r;
+      w.newidx[c + 1] = 2 + 2 * r;
+      w.drank[c] = r + 1;
+      w.drank[c + 1] = r + 1 + w.icount[c];
+    }
+    __syncthreads();
+  }
+  if (tid == 0) w.head->n_nodes = 1 + 2 * w.icount[0];
+  if (tid < 3) w.head->flags[tid] = flags ? flags[tid] : 0;
+}
+
+// Nodes to their reference indices: workgroups below n_small copy a subtree each (its nodes are
+// 2 r + 1 ... 2 r + 2 * internal), the others the large-node stage's nodes.
+__global__ void __launch_bounds__(kBlock) k_emit(int n_small, int n_top, Work w, ct_node* __restrict__ nodes,
+                                                 double4* __restrict__ boxes) {
+  if ((int)blockIdx.x < n_small) {
+    const int root = w.small.id[blockIdx.x];
+    const int64_t at = 2 * (int64_t)w.small.ptr[blockIdx.x];
+    const int r = w.drank[root], count = 2 * w.icount[root];
+    for (int x = 1 + threadIdx.x; x <= count; x += kBlock) {
+      const unsigned meta = (unsigned)w.lmeta[at + x];
+      ct_node nd = w.lnodes[at + x];
+      nd.child = nd.child >= 0 ? 1 + 2 * (r + (int)(meta >> 16)) : -1;
+      const int64_t i = 2 * (int64_t)r + (meta & 0xffffu);
+      nodes[i] = nd;
+      if (boxes) boxes[i + 1] = w.lbox[at + x];
     }
     return;
   }
-
-  // creation.py:174-213 split_plane
-  double plane_min_cost = 1.7976931348623157e308;
-  int plane = -1;
-  long long left = 0;
-  for (int i = 1; i < m; ++i) {
-    left += bS[i - 1];
-    const long long right = (long long)size - left;
-    const double left_volume = (bL[i - 1] - range_Rmin) / bl;
-    const double right_volume = (range_Lmax - bR[i]) / bl;
-    const double cost = left_volume * (double)left + right_volume * (double)right;
-    if (cost < plane_min_cost) {
-      plane_min_cost = cost;
-      plane = i;
-    }
+  const int x = ((int)blockIdx.x - n_small) * kBlock + threadIdx.x;
+  if (x == 0 && boxes) {
+    const double nan = __builtin_nan("");
+    boxes[0] = make_double4(nan, nan, nan, nan);  // row 0 is not a node's
   }
-  if (plane < 0) {
-    counters[2] = 2;
-    decision[s] = kLeaf;
-    return;
+  if (x >= n_top) return;
+  ct_node nd = w.cnodes[x];
+  nd.child = nd.child == -1 ? -1 : 1 + 2 * w.drank[x];
+  nodes[w.newidx[x]] = nd;
+  if (boxes) boxes[w.newidx[x] + 1] = w.tbox[x];
+}
+
+int launch_small(int nb, int cells_per_leaf, int first, int want_boxes, const double* bb, const Work& w, int32_t* out,
+                 unsigned grid, hipStream_t st) {
+  if (nb <= 4) k_small<4, 1024, 512><<<grid, 512, 0, st>>>(nb, cells_per_leaf, first, want_boxes, bb, w, out);
+  else if (nb <= 8) k_small<8, 1024, 512><<<grid, 512, 0, st>>>(nb, cells_per_leaf, first, want_boxes, bb, w, out);
+  else if (nb <= 16) k_small<16, 512, 256><<<grid, 256, 0, st>>>(nb, cells_per_leaf, first, want_boxes, bb, w, out);
+  else if (nb <= 32) k_small<32, 256, 256><<<grid, 256, 0, st>>>(nb, cells_per_leaf, first, want_boxes, bb, w, out);
+  else k_small<64, 128, 128><<<grid, 128, 0, st>>>(nb, cells_per_leaf, first, want_boxes, bb, w, out);
+  CT_LAUNCH_CHECK();
+  return CT_OK;
+}
+
+int check_build(int64_t n, int32_t nb, int32_t cpl, size_t workspace_bytes) {
+  CT_REQUIRE(n >= 1 && n < (int64_t)1 << 30, "n_elements must be in [1, 2^30)");
+  CT_REQUIRE(nb >= 2 && nb <= kMaxBuckets, "n_buckets must be in [2, %d]", kMaxBuckets);
+  CT_REQUIRE(cpl >= 1, "cells_per_leaf must be >= 1");
+  size_t need = 0;
+  carve(nullptr, n, nb, &need);
+  if (workspace_bytes < need) {
+    set_error("build workspace too small: %zu < %zu", workspace_bytes, need);
+    return CT_ERR_WORKSPACE;
   }
-  double Lmax = -1.7976931348623157e308, Rmin = 1.7976931348623157e308;
-  for (int i = 0; i < plane; ++i)
-    if (bL[i] > Lmax) Lmax = bL[i];
-  for (int i = plane; i < m; ++i)
-    if (bR[i] < Rmin) Rmin = bR[i];
-  const int ridx = bI[plane];
-  const int rsize = ptr + size - ridx;
-  const int lsize = size - rsize;
-  cnodes[X].Lmax = Lmax;
-  cnodes[X].Rmin = Rmin;
-  const int c = atomicAdd(&counters[0], 2);
-  cnodes[X].child = c;
-  next_l[s] = push_child(c, ptr, lsize);
-  next_r[s] = push_child(c + 1, ridx, rsize);
-  right_index[s] = ridx;
-  decision[s] = kSplit;
-  atomicMax(&counters[3], depth + 1);
-}
-
-__global__ void __launch_bounds__(kBlock) k_reseg(int n, int32_t* __restrict__ seg,
-                                                  const int32_t* __restrict__ decision,
-                                                  const int32_t* __restrict__ right_index,
-                                                  const int32_t* __restrict__ next_l,
-                                                  const int32_t* __restrict__ next_r) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  const int s = seg[p];
-  if (s < 0) return;
-  const int dcs = decision[s];
-  int ns = -1;
-  if (dcs == kSplit) ns = (p < right_index[s]) ? next_l[s] : next_r[s];
-  else if (dcs == kRetry) ns = next_l[s];
-  seg[p] = ns;
-}
-
-// Bottom-up: number of internal nodes in each subtree (creation-order groups, reversed).
-__global__ void k_icount(int lo, int hi, const ct_node* __restrict__ cn, int32_t* __restrict__ icount) {
-  const int x = lo + blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= hi) return;
-  const int c = cn[x].child;
-  icount[x] = (c >= 0) ? 1 + icount[c] + icount[c + 1] : 0;
-}
-
-// Top-down: DFS preorder rank of internal nodes -> reference indices of their children.
-__global__ void k_dfs(int lo, int hi, const ct_node* __restrict__ cn, const int32_t* __restrict__ icount,
-                      int32_t* __restrict__ drank, int32_t* __restrict__ newidx) {
-  const int x = lo + blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= hi) return;
-  if (x == 0) {
-    newidx[0] = 0;
-    drank[0] = 0;
-  }
-  const int c = cn[x].child;
-  if (c < 0) return;
-  const int r = (x == 0) ? 0 : drank[x];
-  newidx[c] = 1 + 2 * r;
-  newidx[c + 1] = 2 + 2 * r;
-  drank[c] = r + 1;
-  drank[c + 1] = r + 1 + icount[c];
-}
-
-__global__ void k_emit(int total, const ct_node* __restrict__ cn, const int32_t* __restrict__ drank,
-                       const int32_t* __restrict__ newidx, ct_node* __restrict__ out) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= total) return;
-  ct_node nd = cn[x];
-  nd.child = (nd.child >= 0) ? 1 + 2 * drank[x] : -1;
-  out[newidx[x]] = nd;
-}
-
-__global__ void k_copy_i32(int n, const int32_t* __restrict__ a, int32_t* __restrict__ b) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) b[i] = a[i];
+  return CT_OK;
 }
 
 }  // namespace
@@ -549,111 +981,105 @@ int64_t ct_max_nodes(int64_t n_elements) {  // creation.py:216-230
 
 size_t ct_build_workspace_bytes(int64_t n_elements, int32_t n_buckets) {
   size_t total = 0;
-  carve(nullptr, n_elements < 1 ? 1 : n_elements, n_buckets < 2 ? 2 : n_buckets, &total);
+  const int nb = n_buckets < 2 ? 2 : (n_buckets > kMaxBuckets ? kMaxBuckets : n_buckets);
+  carve(nullptr, n_elements < 1 ? 1 : n_elements, nb, &total);
   return total;
+}
+
+int ct_build_plan(const double* bb_coords, int64_t n_elements, int32_t n_buckets, int32_t cells_per_leaf,
+                  int32_t want_boxes, void* workspace, size_t workspace_bytes, int32_t* bb_indices_out,
+                  double* distances, const int64_t* flags, ct_build_info* info, void* stream) {
+  int rc = check_build(n_elements, n_buckets, cells_per_leaf, workspace_bytes);
+  if (rc) return rc;
+  CT_REQUIRE(workspace && bb_indices_out && bb_coords && info, "null pointer");
+  hipStream_t st = as_stream(stream);
+  size_t need = 0;
+  const Work w = carve(static_cast<char*>(workspace), n_elements, n_buckets, &need);
+  const int n = (int)n_elements, nb = n_buckets, cpl = cells_per_leaf, T = small_cells(nb);
+
+  rc = bbox_stat_keys(bb_coords, n, distances, w.head->stats, st);
+  if (rc) return rc;
+  k_init<<<grid_for(n), kBlock, 0, st>>>(n, nb, cpl, T, w, bb_indices_out);
+  CT_LAUNCH_CHECK();
+
+  Header h{};
+  int levels = 0, done_small = 0;
+  // levels of a balanced tree above the subtrees, plus two; then more, in growing batches
+  int batch = 0;
+  if (n > T && n > cpl) {
+    batch = 2;
+    for (int64_t m = T; m < n; m *= 2) ++batch;
+  }
+  while (true) {
+    for (int k = 0; k < batch; ++k, ++levels) {
+      const int par = levels & 1;
+      const int64_t active = levels < 30 ? std::min((int64_t)1 << levels, max_active(n, nb)) : max_active(n, nb);
+      const unsigned tiles = (unsigned)std::min((int64_t)n / kTile + active + 1, max_tiles(n, nb));
+      k_tile_count<<<tiles, kBlock, 0, st>>>(nb, levels, par, bb_coords, w);
+      CT_LAUNCH_CHECK();
+      k_node_decide<<<(unsigned)active, kDecideBlock, 0, st>>>(nb, cpl, T, par, w);
+      CT_LAUNCH_CHECK();
+      k_tile_scatter<<<tiles, kBlock, 0, st>>>(nb, par, w, bb_indices_out);
+      CT_LAUNCH_CHECK();
+    }
+    const unsigned small_grid = (unsigned)std::min((int64_t)2048, (int64_t)n / 2 + 1);
+    rc = launch_small(nb, cpl, done_small, want_boxes, bb_coords, w, bb_indices_out, small_grid, st);
+    if (rc) return rc;
+    k_top<<<1, kTopBlock, 0, st>>>(levels, want_boxes, bb_coords, w, bb_indices_out, flags);
+    CT_LAUNCH_CHECK();
+    CT_HIP(hipMemcpyAsync(&h, w.head, sizeof(h), hipMemcpyDeviceToHost, st));
+    CT_HIP(hipStreamSynchronize(st));
+    done_small = h.n_small;
+    if (h.err != 0 || h.active[levels & 1] == 0) break;
+    // Children are strictly smaller than their parent and a node retries once, so the loop
+    // ends within 2 * n_elements levels (the length of group_end); the guard only protects it.
+    batch = std::min(std::max(2 * batch, 8), 64);
+    if (levels + batch > 2 * (int64_t)n + 4) batch = (int)(2 * (int64_t)n + 4 - levels);
+    if (batch <= 0) {
+      set_error("tree build did not converge");
+      return CT_ERR_DEGENERATE;
+    }
+  }
+  info->n_nodes = h.n_nodes;
+  info->depth = h.depth;
+  info->n_top = h.next_id;
+  info->n_small = h.n_small;
+  info->reserved = 0;
+  for (int k = 0; k < 5; ++k) info->stats[k] = dval((k == 0 || k == 2) ? ~h.stats[k] : h.stats[k]);
+  for (int k = 0; k < 3; ++k) info->flags[k] = h.flags[k];
+  if (h.err != 0) {
+    set_error(h.err == 1 ? "degenerate bucketing: a cell centroid falls outside every bucket"
+                         : "degenerate bucketing: no finite split cost");
+    return CT_ERR_DEGENERATE;
+  }
+  return CT_OK;
+}
+
+int ct_build_emit(int64_t n_elements, int32_t n_buckets, void* workspace, size_t workspace_bytes,
+                  const ct_build_info* info, ct_node* nodes_out, double* node_boxes_out, void* stream) {
+  int rc = check_build(n_elements, n_buckets, 1, workspace_bytes);
+  if (rc) return rc;
+  CT_REQUIRE(workspace && info && nodes_out && info->n_top >= 1 && info->n_small >= 0, "bad arguments");
+  size_t need = 0;
+  const Work w = carve(static_cast<char*>(workspace), n_elements, n_buckets, &need);
+  k_emit<<<(unsigned)info->n_small + grid_for(info->n_top), kBlock, 0, as_stream(stream)>>>(
+      info->n_small, info->n_top, w, nodes_out, reinterpret_cast<double4*>(node_boxes_out));
+  CT_LAUNCH_CHECK();
+  return CT_OK;
 }
 
 int ct_build(const double* bb_coords, int64_t n_elements, int32_t n_buckets, int32_t cells_per_leaf,
              void* workspace, size_t workspace_bytes, ct_node* nodes_out, int32_t* bb_indices_out,
              int64_t* n_nodes, int32_t* depth, void* stream) {
-  CT_REQUIRE(n_elements >= 1 && n_elements < (int64_t)1 << 30, "n_elements must be in [1, 2^30)");
-  CT_REQUIRE(n_buckets >= 2 && n_buckets <= kMaxBuckets, "n_buckets must be in [2, %d]", kMaxBuckets);
-  CT_REQUIRE(cells_per_leaf >= 1, "cells_per_leaf must be >= 1");
-  CT_REQUIRE(n_nodes && depth && nodes_out && bb_indices_out && bb_coords, "null pointer");
-  size_t need = 0;
-  carve(nullptr, n_elements, n_buckets, &need);
-  if (workspace_bytes < need) {
-    set_error("build workspace too small: %zu < %zu", workspace_bytes, need);
-    return CT_ERR_WORKSPACE;
-  }
-  hipStream_t st = as_stream(stream);
-  Work w = carve(static_cast<char*>(workspace), n_elements, n_buckets, &need);
-  const int n = (int)n_elements, nb = n_buckets, cpl = cells_per_leaf;
-  const unsigned gp = grid_for(n);
-  const int nblk = (n + kRankTile - 1) / kRankTile;
-
-  int A = (n > cpl) ? 1 : 0;
-  k_init<<<gp, kBlock, 0, st>>>(w.perm[0], w.seg, n, A, w.cnodes, w.act[0], w.counters);
-  CT_LAUNCH_CHECK();
-
-  std::vector<int> group_end = {1};  // creation-order id ranges, one per level
-  int cur = 0;
-  int32_t host_counters[4] = {1, 0, 0, 0};
-  int levels = 0;
-  while (A > 0) {
-    Slots& ca = w.act[cur];
-    Slots& na = w.act[cur ^ 1];
-    k_level_reset<<<grid_for((int64_t)A * nb), kBlock, 0, st>>>(A, nb, w.rmin, w.rmax, w.bmin, w.bmax,
-                                                                 w.counters);
-    CT_LAUNCH_CHECK();
-    k_range<<<gp, kBlock, 0, st>>>(n, w.seg, w.perm[0], ca.dim, bb_coords, w.rmin, w.rmax);
-    CT_LAUNCH_CHECK();
-    k_bucket<<<gp, kBlock, 0, st>>>(n, nb, w.seg, w.perm[0], ca.dim, bb_coords, w.rmin, w.rmax,
-                                    w.bid[0], w.counters);
-    CT_LAUNCH_CHECK();
-    k_rank_count<<<nblk, kBlock, 0, st>>>(n, nb, w.seg, w.bid[0], w.blockcnt);
-    CT_LAUNCH_CHECK();
-    k_rank_scan<<<1, kBlock, 0, st>>>(nblk, nb, w.blockcnt);
-    CT_LAUNCH_CHECK();
-    k_rank_write<<<nblk, kBlock, 0, st>>>(n, nb, w.seg, w.bid[0], w.blockcnt, ca.ptr, ca.size, w.rank,
-                                          w.sstart, w.send);
-    CT_LAUNCH_CHECK();
-    k_offsets<<<grid_for(A), kBlock, 0, st>>>(A, nb, w.sstart, w.send, w.boff);
-    CT_LAUNCH_CHECK();
-    k_scatter<<<gp, kBlock, 0, st>>>(n, nb, w.seg, w.perm[0], w.bid[0], w.rank, ca.ptr, w.sstart,
-                                     w.boff, w.perm[1], w.bid[1]);
-    CT_LAUNCH_CHECK();
-    k_bbounds<<<gp, kBlock, 0, st>>>(n, nb, w.seg, w.perm[1], w.bid[1], ca.dim, bb_coords, w.bmin,
-                                     w.bmax);
-    CT_LAUNCH_CHECK();
-    k_decide<<<grid_for(A), kBlock, 0, st>>>(A, nb, cpl, ca, na, w.rmin, w.rmax, w.sstart, w.send,
-                                             w.boff, w.bmin, w.bmax, w.cnodes, w.decision,
-                                             w.right_index, w.next_l, w.next_r, w.counters);
-    CT_LAUNCH_CHECK();
-    k_reseg<<<gp, kBlock, 0, st>>>(n, w.seg, w.decision, w.right_index, w.next_l, w.next_r);
-    CT_LAUNCH_CHECK();
-    std::swap(w.perm[0], w.perm[1]);
-    cur ^= 1;
-    CT_HIP(hipMemcpyAsync(host_counters, w.counters, sizeof(host_counters), hipMemcpyDeviceToHost, st));
-    CT_HIP(hipStreamSynchronize(st));
-    if (host_counters[2] != 0) {
-      set_error(host_counters[2] == 1
-                    ? "degenerate bucketing: a cell centroid falls outside every bucket"
-                    : "degenerate bucketing: no finite split cost");
-      return CT_ERR_DEGENERATE;
-    }
-    group_end.push_back(host_counters[0]);
-    A = host_counters[1];
-    // Children are strictly smaller than their parent and a node retries once, so the
-    // loop ends within 2 * n_elements levels; the guard only protects the host loop.
-    if (++levels > 2 * n + 2) {
-      set_error("tree build did not converge");
-      return CT_ERR_DEGENERATE;
-    }
-  }
-  const int total = host_counters[0];
-
-  // DFS renumbering.
-  for (int g = (int)group_end.size() - 1; g >= 0; --g) {
-    const int lo = (g == 0) ? 0 : group_end[g - 1], hi = group_end[g];
-    if (hi > lo) {
-      k_icount<<<grid_for(hi - lo), kBlock, 0, st>>>(lo, hi, w.cnodes, w.icount);
-      CT_LAUNCH_CHECK();
-    }
-  }
-  for (size_t g = 0; g < group_end.size(); ++g) {
-    const int lo = (g == 0) ? 0 : group_end[g - 1], hi = group_end[g];
-    if (hi > lo) {
-      k_dfs<<<grid_for(hi - lo), kBlock, 0, st>>>(lo, hi, w.cnodes, w.icount, w.drank, w.newidx);
-      CT_LAUNCH_CHECK();
-    }
-  }
-  k_emit<<<grid_for(total), kBlock, 0, st>>>(total, w.cnodes, w.drank, w.newidx, nodes_out);
-  CT_LAUNCH_CHECK();
-  k_copy_i32<<<gp, kBlock, 0, st>>>(n, w.perm[0], bb_indices_out);
-  CT_LAUNCH_CHECK();
-  *n_nodes = total;
-  *depth = host_counters[3];
+  CT_REQUIRE(n_nodes && depth && nodes_out, "null pointer");
+  ct_build_info info{};
+  int rc = ct_build_plan(bb_coords, n_elements, n_buckets, cells_per_leaf, 0, workspace, workspace_bytes,
+                         bb_indices_out, nullptr, nullptr, &info, stream);
+  if (rc) return rc;
+  rc = ct_build_emit(n_elements, n_buckets, workspace, workspace_bytes, &info, nodes_out, nullptr, stream);
+  if (rc) return rc;
+  *n_nodes = info.n_nodes;
+  *depth = info.depth;
   return CT_OK;
 }
 

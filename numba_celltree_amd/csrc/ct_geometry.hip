@@ -191,6 +191,14 @@ __global__ void k_stats_finish(const unsigned long long* __restrict__ keys, doub
   if (i < 5) out[i] = dval((i == 0 || i == 2) ? ~keys[i] : keys[i]);
 }
 
+int bbox_stat_keys(const double* bb, int64_t n, double* distances, unsigned long long* keys, hipStream_t st) {
+  int rc = fill<unsigned long long>(keys, 5, 0ull, st);
+  if (rc) return rc;
+  k_bbox_stats<<<reduce_grid(n), kBlock, 0, st>>>(bb, n, distances, keys);
+  CT_LAUNCH_CHECK();
+  return CT_OK;
+}
+
 }  // namespace ct
 
 using namespace ct;
@@ -238,10 +246,8 @@ int ct_bbox_stats(const double* bb_coords, int64_t n, double* distances, double*
   hipStream_t st = as_stream(stream);
   // out5 doubles as the key scratch: 5 keys are reduced in place, then decoded.
   unsigned long long* keys = reinterpret_cast<unsigned long long*>(out5);
-  int rc = fill<unsigned long long>(keys, 5, 0ull, st);
+  int rc = bbox_stat_keys(bb_coords, n, distances, keys, st);
   if (rc) return rc;
-  k_bbox_stats<<<reduce_grid(n), kBlock, 0, st>>>(bb_coords, n, distances, keys);
-  CT_LAUNCH_CHECK();
   k_stats_finish<<<1, 64, 0, st>>>(keys, out5);
   CT_LAUNCH_CHECK();
   return CT_OK;
