@@ -92,6 +92,20 @@ int ct_build_face_bboxes(const int32_t* faces, int64_t n_faces, int32_t n_max_ve
 int ct_build_edge_bboxes(const int32_t* edges, int64_t n_edges, const double* vertices,
                          double tol, double* out, void* stream);
 
+/* A caller's face rows (int32 or int64, index_bytes 4 or 8, 3 to 8 columns) made ready for the
+ * calls below in one pass: faces_out (n_faces, n_max_vert) int32 with fill_value as -1 and the rows
+ * counter-clockwise (as ct_counter_clockwise), bb_out their boxes (as ct_build_face_bboxes) and, when
+ * not null, the `distances` of ct_bbox_stats.  No index is trusted: one outside [0, n_vertices) (or
+ * a fill value among a row's first three) is replaced by 0 and shows in `checks`, 8 device words:
+ * the largest and smallest index and the smallest of the first three columns (ct_check_values turns
+ * a host copy into the three int64), then the keys ct_build_plan takes its bbox statistics from.  The
+ * caller has to look at the first three before it uses any result. */
+int ct_prepare_faces(const void* faces_in, int32_t index_bytes, int64_t n_faces,
+                     int32_t n_max_vert, int64_t fill_value, int64_t n_vertices,
+                     const double* vertices, int32_t* faces_out, double* bb_out, double* distances,
+                     uint64_t* checks, void* stream);
+int ct_check_values(const uint64_t* checks_host, int64_t* out3_host);
+
 /* celltree_base.py:20-48 bbox_tree + bbox_distances.  distances: (n, 3) dx, dy, dxy;
  * out5: device array of 5 doubles = xmin, xmax, ymin, ymax, max(dxy) (the argument of
  * default_tolerance, celltree_base.py:51-52). */
@@ -117,22 +131,23 @@ typedef struct ct_build_info {
   int32_t n_small;   /* for ct_build_emit */
   int32_t reserved;
   double stats[5];   /* bbox_tree and the largest diagonal, as ct_bbox_stats */
-  int64_t flags[3];  /* the caller's flags array, or zeros */
+  int64_t checks[3]; /* ct_check_values of the caller's checks, or zeros */
 } ct_build_info;
 
 /* creation.py:384-413 initialize (+ build, :233-381) in two calls, so that the caller can
  * allocate exactly what the tree needs in between.  ct_build_plan builds the tree in the
- * workspace, writes bb_indices_out (n_elements) and, when `distances` is not null, the (n, 3)
- * distances of ct_bbox_stats, and fills *info (HOST); it synchronizes the stream, once for all
- * but very unbalanced trees.  `want_boxes`: also the tight node boxes.  `flags` (may be NULL): 3
- * device int64 copied to info->flags, so that a caller's own check values arrive with the same
- * synchronization; info is complete when the result is CT_OK or CT_ERR_DEGENERATE.
+ * workspace, writes bb_indices_out (n_elements) and fills *info (HOST); it synchronizes the
+ * stream, once for all but very unbalanced trees.  `want_boxes`: also the tight node boxes.
+ * `checks`: those of ct_prepare_faces for these boxes, whose statistics are used and whose check
+ * values arrive in info with the same synchronization; without them (NULL) the statistics are
+ * formed here and, when `distances` is not null, the (n, 3) distances of ct_bbox_stats written.
+ * info is complete when the result is CT_OK or CT_ERR_DEGENERATE.
  * ct_build_emit (asynchronous) writes nodes_out[0 .. info->n_nodes) in the reference's DFS
  * numbering and, when node_boxes_out is not null (needs want_boxes), what ct_node_boxes writes. */
 int ct_build_plan(const double* bb_coords, int64_t n_elements, int32_t n_buckets,
                   int32_t cells_per_leaf, int32_t want_boxes, void* workspace,
                   size_t workspace_bytes, int32_t* bb_indices_out, double* distances,
-                  const int64_t* flags, ct_build_info* info, void* stream);
+                  const uint64_t* checks, ct_build_info* info, void* stream);
 int ct_build_emit(int64_t n_elements, int32_t n_buckets, void* workspace, size_t workspace_bytes,
                   const ct_build_info* info, ct_node* nodes_out, double* node_boxes_out,
                   void* stream);

@@ -93,15 +93,67 @@ def faces_to_dev(faces, n_vertices: int, allow_fill: bool = True) -> torch.Tenso
         first3 = allow_fill and f.ndim == 2 and f.shape[1] >= 3
         lo3 = f[:, :3].amin() if first3 else lo
         hi, lo, lo3 = (int(v) for v in torch.stack([hi, lo, lo3]).tolist())
-        if hi >= min(int(n_vertices), 2**31):
-            raise ValueError(f"element index {hi} is out of bounds for {int(n_vertices)} vertices")
-        if lo < (-1 if allow_fill else 0):
-            what = "[-1, n_vertices)" if allow_fill else "[0, n_vertices)"
-            raise ValueError(f"element indices must lie in {what}, found {lo}")
-        if first3 and lo3 < 0:
-            # polygon_length (geometry_utils.py:72-79) takes the first 3 entries as vertices
-            raise ValueError("every face needs at least 3 vertices (a fill value among its first 3 entries)")
+        check_indices(hi, lo, lo3 if first3 else 0, n_vertices, allow_fill)
     return f.to(device=device(), dtype=torch.int32).contiguous()
+
+
+def check_indices(hi: int, lo: int, lo3: int, n_vertices: int, allow_fill: bool = True) -> None:
+    """Raises unless the largest (hi), smallest (lo) and smallest first-three-columns (lo3) index
+    of an element array address ``n_vertices`` vertices."""
+    if hi >= min(int(n_vertices), 2**31):
+        raise ValueError(f"element index {hi} is out of bounds for {int(n_vertices)} vertices")
+    if lo < (-1 if allow_fill else 0):
+        what = "[-1, n_vertices)" if allow_fill else "[0, n_vertices)"
+        raise ValueError(f"element indices must lie in {what}, found {lo}")
+    if lo3 < 0:
+        # polygon_length (geometry_utils.py:72-79) takes the first 3 entries as vertices
+        raise ValueError("every face needs at least 3 vertices (a fill value among its first 3 entries)")
+
+
+class PreparedFaces:
+    """Device face rows made ready by ct_prepare_faces: ``faces`` (int32, counter-clockwise), ``bb``
+    (their boxes), ``distances`` (when asked for) and ``checks`` (8 device words; ``check`` raises what
+    ``faces_to_dev`` raises once they are on the host)."""
+
+    def __init__(self, faces, bb, distances, checks, n_vertices):
+        self.faces, self.bb, self.distances, self.checks, self.n_vertices = faces, bb, distances, checks, n_vertices
+
+    def check(self, words) -> None:
+        """``words``: the first three of ``checks`` as host integers (int64 bit patterns)."""
+        raw = (ctypes.c_uint64 * 3)(*[int(w) & 0xFFFFFFFFFFFFFFFF for w in words[:3]])
+        out = (ctypes.c_int64 * 3)()
+        _native.call("ct_check_values", raw, out)
+        check_indices(out[0], out[1], out[2], self.n_vertices)
+
+
+def prepare_faces(faces, fill_value, d_vertices: torch.Tensor, with_distances: bool, checks=None):
+    """The rows of a device index array in one pass (PreparedFaces; the index checks are the
+    caller's, after its next synchronization), or None where that pass does not apply: host
+    arrays, another device, no faces or vertices, fewer than 3 or more than 8 columns, a fill value
+    that is no integer.  ``checks``: 8 int64 to use for the check words."""
+    if not is_device_tensor(faces) or faces.device != device() or faces.ndim != 2:
+        return None
+    n, nmax = int(faces.shape[0]), int(faces.shape[1])
+    nv = int(d_vertices.shape[0])
+    if n == 0 or nv == 0 or not 3 <= nmax <= 8 or faces.is_complex():
+        return None
+    try:
+        fill = int(fill_value)
+    except (TypeError, ValueError, OverflowError):
+        return None
+    if fill != fill_value or not -(2**63) <= fill < 2**63:
+        return None
+    if faces.dtype not in (torch.int32, torch.int64):
+        faces = faces.to(torch.int64)
+    faces = faces.contiguous()
+    out = empty((n, nmax), torch.int32)
+    bb = empty((n, 4), torch.float64)
+    distances = empty((n, 3), torch.float64) if with_distances else None
+    if checks is None:
+        checks = empty(8, torch.int64)
+    _native.call("ct_prepare_faces", ptr(faces), faces.element_size(), n, nmax, fill, nv, ptr(d_vertices), ptr(out),
+                 ptr(bb), ptr(distances), ptr(checks), stream())
+    return PreparedFaces(out, bb, distances, checks, nv)
 
 
 def index_to_dev(x, n: int, allow_missing: bool = False) -> torch.Tensor:
@@ -118,11 +170,12 @@ def empty(shape, dtype) -> torch.Tensor:
     return torch.empty(shape, dtype=dtype, device=device())
 
 
-def exclusive_scan(counts: torch.Tensor, total: bool = True):
+def exclusive_scan(counts: torch.Tensor, total: bool = True, offsets=None):
     """Offsets (n + 1, int64, device) of ``counts`` and the total (host int: synchronizes;
-    None with ``total=False``)."""
+    None with ``total=False``).  ``offsets``: n + 1 or more int64 to write them to."""
     n = counts.numel()
-    offsets = empty(n + 1, torch.int64)
+    if offsets is None:
+        offsets = empty(n + 1, torch.int64)
     ws = empty(int(_native.lib().ct_scan_workspace_bytes(n)), torch.uint8)
     _native.call("ct_exclusive_scan", ptr(counts), n, ptr(offsets), ptr(ws), ws.numel(), stream())
     return offsets, (int(offsets[n].item()) if total else None)

@@ -125,7 +125,7 @@ class CtBuildInfo(ctypes.Structure):
         ("n_small", ctypes.c_int32),
         ("reserved", ctypes.c_int32),
         ("stats", ctypes.c_double * 5),
-        ("flags", ctypes.c_int64 * 3),
+        ("checks", ctypes.c_int64 * 3),
     ]
 
 
@@ -150,6 +150,8 @@ SIGNATURES = {
     "ct_counter_clockwise": (ctypes.c_int, [_P, _P, _I64, _I32, _P]),
     "ct_build_face_bboxes": (ctypes.c_int, [_P, _I64, _I32, _P, _P, _P]),
     "ct_build_edge_bboxes": (ctypes.c_int, [_P, _I64, _P, _F64, _P, _P]),
+    "ct_prepare_faces": (ctypes.c_int, [_P, _I32, _I64, _I32, _I64, _I64, _P, _P, _P, _P, _P, _P]),
+    "ct_check_values": (ctypes.c_int, [_P, _P]),
     "ct_bbox_stats": (ctypes.c_int, [_P, _I64, _P, _P, _P]),
     "ct_vertex_extent": (ctypes.c_int, [_P, _I64, _P, _P]),
     "ct_max_nodes": (_I64, [_I64]),

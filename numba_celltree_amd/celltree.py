@@ -37,6 +37,11 @@ class CellTree2d(CellTree2dBase):
         if cells_per_leaf < 1:
             raise ValueError("cells_per_leaf must be >= 1")
         vertices = cast_vertices(vertices, copy=True)
+        d_vertices = D.to_dev(vertices, torch.float64) if D.is_device_tensor(faces) else None
+        prep = None if d_vertices is None else D.prepare_faces(faces, fill_value, d_vertices, with_distances=True)
+        if prep is not None:
+            self._build_tree(d_vertices, prep.faces, prep.bb, n_buckets, cells_per_leaf, prep)
+            return
         faces = cast_faces(faces, fill_value)
         d_vertices = D.to_dev(vertices, torch.float64)
         d_faces = D.faces_to_dev(faces, d_vertices.shape[0])
@@ -86,11 +91,15 @@ class CellTree2d(CellTree2dBase):
             _native.call("ct_locate_points", self.tree_ref, D.ptr(pts), n, tolerance, D.ptr(out), D.stream())
         return out
 
-    def _locate_boxes_dev(self, d_boxes: torch.Tensor):
+    def _locate_boxes_dev(self, d_boxes: torch.Tensor, prep=None):
+        """``prep``: the faces (D.PreparedFaces) whose boxes these are; their index checks are made
+        here, with the first value read back."""
         n = int(d_boxes.shape[0])
         st = D.stream()
         order, srt = self._order(1, d_boxes)
-        split = self._split(1, d_boxes, order)
+        split = self._split(1, d_boxes, order, prep)
+        if split is None and prep is not None:
+            prep.check(prep.checks[:3].tolist())
         if split is not None:
             subs, part_offsets, m = split
             counts = D.empty(max(m, 1), torch.int64)
@@ -157,10 +166,24 @@ class CellTree2d(CellTree2dBase):
         _native.call("ct_build_face_bboxes", D.ptr(d_faces), n, nmax, D.ptr(d_vertices), D.ptr(bb), st)
         return bb
 
-    def _face_pairs(self, d_vertices, d_faces, with_area: bool):
+    def _faces_in(self, vertices, faces, fill_value: int):
+        """(vertices, faces, prepared faces or None) of a face query on the device; ``None``: the
+        faces are checked but neither reordered nor boxed yet."""
+        d_vertices = D.to_dev(cast_vertices(vertices), torch.float64)
+        if D.is_device_tensor(faces) and faces.ndim == 2:
+            # behind the part offsets of the query split (_split), read back together
+            n = int(faces.shape[0])
+            row = D.empty(n + 9, torch.int64)
+            prep = D.prepare_faces(faces, fill_value, d_vertices, with_distances=False, checks=row[n + 1:])
+            if prep is not None:
+                prep.part_offsets = row
+                return d_vertices, prep.faces, prep
+        return d_vertices, D.faces_to_dev(cast_faces(faces, fill_value), d_vertices.shape[0]), None
+
+    def _face_pairs(self, d_vertices, d_faces, with_area: bool, prep=None):
         """locate_boxes on the faces' bboxes, then the fused SAT (+ clip area) pair stage."""
-        bb = self._prepare_faces(d_vertices, d_faces)
-        ii, jj = self._locate_boxes_dev(bb)
+        bb = self._prepare_faces(d_vertices, d_faces) if prep is None else prep.bb
+        ii, jj = self._locate_boxes_dev(bb, prep)
         n = int(ii.numel())
         area = D.empty(n, torch.float64) if with_area else None
         keep = D.empty(n, torch.int64)
@@ -189,9 +212,8 @@ class CellTree2d(CellTree2dBase):
     def intersect_faces(self, vertices, faces, fill_value: int) -> Tuple:
         """Face pairs with overlap area > 0, and the area (celltree.py:228-269)."""
         io = D.Io(vertices, faces)
-        d_vertices = D.to_dev(cast_vertices(vertices), torch.float64)
-        d_faces = D.faces_to_dev(cast_faces(faces, fill_value), d_vertices.shape[0])
-        i, j, a = self._face_pairs(d_vertices, d_faces, with_area=True)
+        d_vertices, d_faces, prep = self._faces_in(vertices, faces, fill_value)
+        i, j, a = self._face_pairs(d_vertices, d_faces, True, prep)
         return io.out(i), io.out(j), io.out(a)
 
     def intersect_edges(self, edge_coords) -> Tuple:

@@ -59,7 +59,9 @@ class CellTree2dBase:
 
     # ------------------------------------------------------------------ build
     def _build_tree(self, vertices: torch.Tensor, elements: torch.Tensor, bb_coords: torch.Tensor,
-                    n_buckets: int, cells_per_leaf: int) -> None:
+                    n_buckets: int, cells_per_leaf: int, prep=None) -> None:
+        """``prep``: the elements as D.PreparedFaces, whose boxes bb_coords are; their index checks
+        are made here, with the build's own readback."""
         n = int(elements.shape[0])
         if n == 0:
             raise ValueError("a cell tree needs at least one element")
@@ -67,13 +69,16 @@ class CellTree2dBase:
         st = D.stream()
         ws = D.empty(int(L.ct_build_workspace_bytes(n, n_buckets)), torch.uint8)
         bb_indices = D.empty(n, torch.int32)
-        distances = D.empty((n, 3), torch.float64)
+        distances = D.empty((n, 3), torch.float64) if prep is None else prep.distances
         want_boxes = int(elements.shape[1]) >= 3
         info = _native.CtBuildInfo()
-        _native.call(
-            "ct_build_plan", D.ptr(bb_coords), n, n_buckets, cells_per_leaf, int(want_boxes), D.ptr(ws), ws.numel(),
-            D.ptr(bb_indices), D.ptr(distances), None, ctypes.byref(info), st,
+        rc = L.ct_build_plan(
+            D.ptr(bb_coords), n, n_buckets, cells_per_leaf, int(want_boxes), D.ptr(ws), ws.numel(), D.ptr(bb_indices),
+            D.ptr(distances), D.ptr(None if prep is None else prep.checks), ctypes.byref(info), st,
         )
+        if prep is not None and rc in (_native.CT_OK, _native.CT_ERR_DEGENERATE):
+            D.check_indices(*info.checks, prep.n_vertices)
+        _native.check(rc, "ct_build_plan")
         nodes_raw = D.empty(32 * info.n_nodes, torch.uint8)
         node_boxes = D.empty((info.n_nodes + 1, 4), torch.float64) if want_boxes else None
         _native.call("ct_build_emit", n, n_buckets, D.ptr(ws), ws.numel(), ctypes.byref(info), D.ptr(nodes_raw),
@@ -430,7 +435,7 @@ class CellTree2dBase:
     EDGE_SPLIT_LEAF_CELLS = 64
     SPLIT_MAX_PARTS = 16
 
-    def _split(self, kind: int, queries: torch.Tensor, order):
+    def _split(self, kind: int, queries: torch.Tensor, order, prep=None):
         """(subqueries (m, 2) int32, part offsets (n + 1), m) for kind 1 boxes, 2 segment-face,
         3 segment-edge, or None when the batch is not split.  Batches too small to be ordered
         (order None: queries in their own order) are split too: with few lanes, one long walk
@@ -445,7 +450,12 @@ class CellTree2dBase:
         parts = D.empty(n, torch.int64)
         keep = D.empty(n * int(self.SPLIT_MAX_PARTS), torch.int32)  # frontiers, for the write call
         _native.call("ct_split_queries", *args, D.ptr(parts), None, None, D.ptr(keep), st)
-        part_offsets, m = D.exclusive_scan(parts)
+        if prep is None:
+            part_offsets, m = D.exclusive_scan(parts)
+        else:
+            part_offsets, _ = D.exclusive_scan(parts, total=False, offsets=prep.part_offsets)
+            m, *words = part_offsets[n: n + 4].tolist()
+            prep.check(words)
         subs = D.empty((max(m, 1), 2), torch.int32)
         _native.call("ct_split_queries", *args, None, D.ptr(part_offsets), D.ptr(subs), D.ptr(keep), st)
         return subs, part_offsets, m

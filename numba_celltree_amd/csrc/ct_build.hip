@@ -87,8 +87,8 @@ struct Header {
   int32_t tiles[2];
   int32_t n_nodes;    // of the whole tree (k_top)
   int32_t pad[3];
+  Key checks[3];      // of ct_prepare_faces, passed through
   Key stats[5];       // as bbox_stat_keys leaves them: ~min x, max x, ~min y, max y, max diagonal
-  int64_t flags[3];   // the caller's check values, passed through
 };
 
 struct Work {
@@ -254,8 +254,9 @@ __device__ __forceinline__ Split decide(int nb, int size, int att, double range_
 
 // ------------------------------------------------------------------- large nodes
 // The root: a leaf (n <= cells_per_leaf), a subtree of k_small (n <= T) or the first large node.
-__global__ void __launch_bounds__(kBlock) k_init(int n, int nb, int cells_per_leaf, int T, Work w,
-                                                 int32_t* __restrict__ out) {
+// given: the caller's 3 check values and 5 statistics, or null (the statistics are in the header).
+__global__ void __launch_bounds__(kBlock) k_init(int n, int cells_per_leaf, int T, const Key* __restrict__ given,
+                                                 Work w, int32_t* __restrict__ out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) {
     w.perm[0][i] = i;
@@ -275,6 +276,9 @@ __global__ void __launch_bounds__(kBlock) k_init(int n, int nb, int cells_per_le
     s.depth[0] = 0;
     s.tile0[0] = 0;
     Header& h = *w.head;
+    for (int k = 0; k < 3; ++k) h.checks[k] = given ? given[k] : 0;
+    if (given)
+      for (int k = 0; k < 5; ++k) h.stats[k] = given[3 + k];
     for (int k = 0; k < 4; ++k) s.range[k] = (k & 1) ? h.stats[k] : ~h.stats[k];
     w.small.id[0] = 0;
     w.small.ptr[0] = 0;
@@ -852,8 +856,7 @@ __global__ void __launch_bounds__(THREADS) k_small(int nb, int cells_per_leaf, i
 constexpr int kTopBlock = 1024;
 
 __global__ void __launch_bounds__(kTopBlock) k_top(int levels, int want_boxes, const double* __restrict__ bb, Work w,
-                                                   const int32_t* __restrict__ cells,
-                                                   const int64_t* __restrict__ flags) {
+                                                   const int32_t* __restrict__ cells) {
   const int tid = threadIdx.x, M = w.head->next_id;
   ct_node* cn = w.cnodes;
   // leaves: one wavefront each
@@ -905,7 +908,6 @@ __global__ void __launch_bounds__(kTopBlock) k_top(int levels, int want_boxes, c
     __syncthreads();
   }
   if (tid == 0) w.head->n_nodes = 1 + 2 * w.icount[0];
-  if (tid < 3) w.head->flags[tid] = flags ? flags[tid] : 0;
 }
 
 // Nodes to their reference indices: workgroups below n_small copy a subtree each (its nodes are
@@ -969,6 +971,12 @@ using namespace ct;
 
 extern "C" {
 
+int ct_check_values(const uint64_t* checks_host, int64_t* out3_host) {
+  CT_REQUIRE(checks_host && out3_host, "null pointer");
+  for (int k = 0; k < 3; ++k) out3_host[k] = (int64_t)((k ? ~checks_host[k] : checks_host[k]) ^ 0x8000000000000000ull);
+  return CT_OK;
+}
+
 int64_t ct_max_nodes(int64_t n_elements) {  // creation.py:216-230
   int64_t n_nodes = n_elements;
   int64_t nodes = (n_elements + 1) / 2;
@@ -988,7 +996,7 @@ size_t ct_build_workspace_bytes(int64_t n_elements, int32_t n_buckets) {
 
 int ct_build_plan(const double* bb_coords, int64_t n_elements, int32_t n_buckets, int32_t cells_per_leaf,
                   int32_t want_boxes, void* workspace, size_t workspace_bytes, int32_t* bb_indices_out,
-                  double* distances, const int64_t* flags, ct_build_info* info, void* stream) {
+                  double* distances, const uint64_t* checks, ct_build_info* info, void* stream) {
   int rc = check_build(n_elements, n_buckets, cells_per_leaf, workspace_bytes);
   if (rc) return rc;
   CT_REQUIRE(workspace && bb_indices_out && bb_coords && info, "null pointer");
@@ -997,9 +1005,11 @@ int ct_build_plan(const double* bb_coords, int64_t n_elements, int32_t n_buckets
   const Work w = carve(static_cast<char*>(workspace), n_elements, n_buckets, &need);
   const int n = (int)n_elements, nb = n_buckets, cpl = cells_per_leaf, T = small_cells(nb);
 
-  rc = bbox_stat_keys(bb_coords, n, distances, w.head->stats, st);
-  if (rc) return rc;
-  k_init<<<grid_for(n), kBlock, 0, st>>>(n, nb, cpl, T, w, bb_indices_out);
+  if (checks == nullptr) {
+    rc = bbox_stat_keys(bb_coords, n, distances, w.head->stats, st);
+    if (rc) return rc;
+  }
+  k_init<<<grid_for(n), kBlock, 0, st>>>(n, cpl, T, reinterpret_cast<const Key*>(checks), w, bb_indices_out);
   CT_LAUNCH_CHECK();
 
   Header h{};
@@ -1025,7 +1035,7 @@ int ct_build_plan(const double* bb_coords, int64_t n_elements, int32_t n_buckets
     const unsigned small_grid = (unsigned)std::min((int64_t)2048, (int64_t)n / 2 + 1);
     rc = launch_small(nb, cpl, done_small, want_boxes, bb_coords, w, bb_indices_out, small_grid, st);
     if (rc) return rc;
-    k_top<<<1, kTopBlock, 0, st>>>(levels, want_boxes, bb_coords, w, bb_indices_out, flags);
+    k_top<<<1, kTopBlock, 0, st>>>(levels, want_boxes, bb_coords, w, bb_indices_out);
     CT_LAUNCH_CHECK();
     CT_HIP(hipMemcpyAsync(&h, w.head, sizeof(h), hipMemcpyDeviceToHost, st));
     CT_HIP(hipStreamSynchronize(st));
@@ -1046,7 +1056,9 @@ int ct_build_plan(const double* bb_coords, int64_t n_elements, int32_t n_buckets
   info->n_small = h.n_small;
   info->reserved = 0;
   for (int k = 0; k < 5; ++k) info->stats[k] = dval((k == 0 || k == 2) ? ~h.stats[k] : h.stats[k]);
-  for (int k = 0; k < 3; ++k) info->flags[k] = h.flags[k];
+  ct_check_values(reinterpret_cast<const uint64_t*>(h.checks), info->checks);
+  if (checks == nullptr)
+    for (int64_t& c : info->checks) c = 0;
   if (h.err != 0) {
     set_error(h.err == 1 ? "degenerate bucketing: a cell centroid falls outside every bucket"
                          : "degenerate bucketing: no finite split cost");

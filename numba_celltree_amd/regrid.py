@@ -22,7 +22,6 @@ import torch
 
 from numba_celltree_amd import _device as D
 from numba_celltree_amd import _native
-from numba_celltree_amd.cast import cast_faces, cast_vertices
 
 
 def _offsets(index: torch.Tensor, n: int) -> torch.Tensor:
@@ -48,13 +47,12 @@ class RegridTopology:
 
     def __init__(self, tree, tgt_vertices, tgt_faces, fill_value: int = -1):
         self.tree = tree
-        d_tv = D.to_dev(cast_vertices(tgt_vertices), torch.float64)
-        d_tf = D.faces_to_dev(cast_faces(tgt_faces, fill_value), d_tv.shape[0])
+        d_tv, d_tf, prep = tree._faces_in(tgt_vertices, tgt_faces, fill_value)
         if int(d_tf.shape[1]) > 8 or int(tree.d_elements.shape[1]) > 8:
             raise ValueError("regridding supports faces of at most 8 vertices")
         # intersect_faces reorders the target rows counter-clockwise in place (d_tf) and
         # returns the pairs grouped by target in ascending order.
-        tt, ss, _ = tree._face_pairs(d_tv, d_tf, with_area=True)
+        tt, ss, _ = tree._face_pairs(d_tv, d_tf, True, prep)
         self.tgt_vertices = d_tv
         self.tgt_faces = d_tf
         self.src_faces = tree.d_elements
