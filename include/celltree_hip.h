@@ -263,10 +263,11 @@ int ct_locate_points_on_edge(const ct_tree* tree, const double* points, int64_t 
                              int64_t* out, void* stream);
 
 /* Scheduling helper, no reference counterpart: a processing order for n queries (kind 0
- * points (n, 2), 1 boxes (n, 4), 2 segments (n, 2, 2)) from a bucket sort on a 20-bit key:
- * points by the Morton key of a 1024 x 1024 grid over `bbox` (HOST array of 4); boxes and
- * segments by a work class (log2 of their bbox area relative to `bbox`) above the Morton key
- * of their centre.  The order is grouped by the top 8 key bits and sorted by the full key
+ * points (n, 2), 1 boxes (n, 4), 2 segments (n, 2, 2), for one lane per query; 3 boxes, 4
+ * segments, for ct_gather_count) from a bucket sort on a 20-bit key: points, kinds 3 and 4 (by
+ * their centre) by the Morton key of a 1024 x 1024 grid over `bbox` (HOST array of 4); kinds 1 and
+ * 2 by a work class (log2 of their bbox area relative to `bbox`) above a 16-bit Morton key of
+ * their centre.  The order is grouped by the top 8 key bits and sorted by the full key
  * within chunks of 32768 queries of one group (a group larger than that is a sequence of
  * such sorted chunks).  Passing the order to a count / write pass gives each wavefront
  * neighbouring queries of similar cost; results are unchanged by it.  `sorted` (may be NULL)
@@ -389,6 +390,33 @@ int ct_locate_edges_write_sub(const ct_tree* tree, const double* segments, const
 int ct_sort_staged_rows(const int64_t* offsets, const int64_t* query_start, const int32_t* rows_query,
                         const int32_t* rows_cell, const double* rows_xy, const double* rows_t, int64_t n_rows,
                         int64_t* ii, int64_t* jj, double* xy, void* stream);
+
+/* Box and segment queries by wavefronts, a few queries each (kind 1 boxes, 2 segment-face, 3
+ * segment-edge; trees of depth <= CT_MAX_DEPTH), without subqueries.  ct_gather_count writes
+ * counts[q] and starts[q] and keeps the rows in the caller's pool of pool_rows entries (pool_cell;
+ * segments also pool_xy, 4 doubles each, and pool_src); ct_gather_pool_rows suggests a size.
+ * starts[q] < 0: q is left to the caller (more rows than a wavefront's lists hold, or no room in the
+ * pool), counts[q] = 0.  tail: ct_gather_tail_words() int64 of working words; tail[0] = the number of
+ * queries left.  visit_cells (boxes; ct_visit_cells): (n_elements) the cells in the order in which a
+ * walk that enters every node meets them.  After an exclusive scan of the counts (with those of the
+ * queries left filled in) into offsets (n + 1), ct_gather_rows writes the rows kept at their
+ * offsets: boxes (ii, jj) in DFS order within a query, segments (ii, jj, xy) by t
+ * (geometry_utils.py:564-574); ct_place_rows writes those of the queries left: row r of sub-query
+ * s = sub_ii[r] (query idx[s]) to offsets[idx[s]] + r - sub_offsets[s]. */
+int64_t ct_gather_tail_words(void);
+int64_t ct_gather_pool_rows(int32_t kind, int64_t n);
+int ct_visit_cells(const ct_tree* tree, int32_t* out, void* stream);
+int ct_gather_count(const ct_tree* tree, int32_t kind, const double* queries, int64_t n,
+                    const int32_t* order, const int32_t* visit_cells, int64_t pool_rows,
+                    int32_t* pool_cell, double* pool_xy, int32_t* pool_src, int64_t* counts,
+                    int64_t* starts, int64_t* tail, void* stream);
+int ct_gather_rows(int32_t kind, int64_t n, const int64_t* offsets, const int64_t* starts,
+                   const int32_t* pool_cell, const double* pool_xy, const int32_t* pool_src,
+                   int64_t* ii, int64_t* jj, double* xy, void* stream);
+int ct_place_rows(int64_t rows, const int64_t* idx, const int64_t* sub_offsets,
+                  const int64_t* offsets, const int64_t* sub_ii, const int64_t* sub_jj,
+                  const double* sub_xy, int64_t* ii, int64_t* jj, double* xy, void* stream);
+
 
 /* geometry_utils.py:564-574 sort_intersections_by_edge on grouped output (ii ascending, the
  * rows of segment s in [offsets[s], offsets[s+1])): writes jj and xy (n_rows, 2, 2) stably

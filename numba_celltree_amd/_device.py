@@ -170,6 +170,12 @@ def empty(shape, dtype) -> torch.Tensor:
     return torch.empty(shape, dtype=dtype, device=device())
 
 
+def gather_row(n: int) -> torch.Tensor:
+    """The int64 words of a ct_gather_* call on n queries: n + 1 offsets, 8 check words
+    (PreparedFaces), the working words."""
+    return empty(n + 9 + int(_native.lib().ct_gather_tail_words()), torch.int64)
+
+
 def exclusive_scan(counts: torch.Tensor, total: bool = True, offsets=None):
     """Offsets (n + 1, int64, device) of ``counts`` and the total (host int: synchronizes;
     None with ``total=False``).  ``offsets``: n + 1 or more int64 to write them to."""

@@ -184,6 +184,12 @@ SIGNATURES = {
                                                  _P]),
     "ct_subquery_spans": (ctypes.c_int, [_P, _I64, _P, _P, _P, _P, _P]),
     "ct_sort_staged_rows": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _I64, _P, _P, _P, _P]),
+    "ct_gather_tail_words": (_I64, []),
+    "ct_gather_pool_rows": (_I64, [_I32, _I64]),
+    "ct_visit_cells": (ctypes.c_int, [_TP, _P, _P]),
+    "ct_gather_count": (ctypes.c_int, [_TP, _I32, _P, _I64, _P, _P, _I64, _P, _P, _P, _P, _P, _P, _P]),
+    "ct_gather_rows": (ctypes.c_int, [_I32, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
+    "ct_place_rows": (ctypes.c_int, [_I64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "ct_locate_points_ordered_noalloc": (ctypes.c_int, [_TP, _P, _I64, _F64, _P, _P]),
     "ct_locate_points_on_edge": (ctypes.c_int, [_TP, _P, _I64, _F64, _P, _P]),
     "ct_order_workspace_bytes": (_SZ, [_I64]),

@@ -96,22 +96,11 @@ class CellTree2d(CellTree2dBase):
         here, with the first value read back."""
         n = int(d_boxes.shape[0])
         st = D.stream()
+        if self._gathers(n):
+            return self._gather(1, d_boxes, self._order(3, d_boxes)[0], prep)
         order, srt = self._order(1, d_boxes)
-        split = self._split(1, d_boxes, order, prep)
-        if split is None and prep is not None:
+        if prep is not None:
             prep.check(prep.checks[:3].tolist())
-        if split is not None:
-            subs, part_offsets, m = split
-            counts = D.empty(max(m, 1), torch.int64)
-            hits, slots = self._hit_record(m, self.BOX_HIT_SLOTS, self.BOX_HIT_BUDGET)
-            _native.call("ct_locate_boxes_count_sub", self.tree_ref, D.ptr(d_boxes), D.ptr(subs), m, D.ptr(counts),
-                         D.ptr(hits), slots, st)
-            offsets, total = self._sub_offsets(order, n, part_offsets, counts)
-            ii = D.empty(total, torch.int64)
-            jj = D.empty(total, torch.int64)
-            _native.call("ct_locate_boxes_write_sub", self.tree_ref, D.ptr(d_boxes), D.ptr(subs), m, D.ptr(offsets),
-                         D.ptr(counts), D.ptr(hits), slots, D.ptr(ii), D.ptr(jj), st)
-            return ii, jj
         counts = D.empty(n, torch.int64)
         hits, slots = self._hit_record(n, self.BOX_HIT_SLOTS, self.BOX_HIT_BUDGET)
         _native.call("ct_locate_boxes_count_rec", self.tree_ref, D.ptr(d_boxes), n, D.ptr(order), D.ptr(srt),
@@ -171,12 +160,12 @@ class CellTree2d(CellTree2dBase):
         faces are checked but neither reordered nor boxed yet."""
         d_vertices = D.to_dev(cast_vertices(vertices), torch.float64)
         if D.is_device_tensor(faces) and faces.ndim == 2:
-            # behind the part offsets of the query split (_split), read back together
+            # the check words lie behind the box query's offsets (_gather), read back together
             n = int(faces.shape[0])
-            row = D.empty(n + 9, torch.int64)
-            prep = D.prepare_faces(faces, fill_value, d_vertices, with_distances=False, checks=row[n + 1:])
+            row = D.gather_row(n)
+            prep = D.prepare_faces(faces, fill_value, d_vertices, with_distances=False, checks=row[n + 1: n + 9])
             if prep is not None:
-                prep.part_offsets = row
+                prep.row = row
                 return d_vertices, prep.faces, prep
         return d_vertices, D.faces_to_dev(cast_faces(faces, fill_value), d_vertices.shape[0]), None
 

@@ -146,6 +146,11 @@ class CellTree2dBase:
             self.d_leaf_bb = D.empty((n, 4), torch.float64)
             _native.call("ct_pack_leaf_bboxes", self.tree_ref, D.ptr(self.d_leaf_bb), st)
             t.leaf_bb = self.d_leaf_bb.data_ptr()
+        self.d_visit_cells = None
+        if nmax >= 3:
+            # The cells in visit order: box queries turn visit numbers into cells.
+            self.d_visit_cells = D.empty(n, torch.int32)
+            _native.call("ct_visit_cells", self.tree_ref, D.ptr(self.d_visit_cells), st)
         t.parents = None
         self.d_parents = None
         if self.depth > _native.CT_MAX_DEPTH:
@@ -375,11 +380,14 @@ class CellTree2dBase:
         _native.call(fn, self.tree_ref, D.ptr(pts), n, float(tolerance), D.ptr(out), D.stream())
         return io.out(out)
 
-    # Hit cells the count pass records per segment (slot-major, so only slots in use are
-    # touched); segments with at most that many hits are written from the record instead of
-    # a second tree walk.  The long segments carry most of the rows, so the record pays off
-    # only when it covers them: up to EDGE_HIT_SLOTS slots within EDGE_HIT_BUDGET int32
-    # entries (1 GiB); below 4 slots the write pass walks the tree again.
+    # Rows of box and segment batches.  Wavefront walks (_gather) keep them in a pool of at most
+    # EDGE_HIT_BUDGET (40 bytes each) or BOX_HIT_BUDGET rows (4 bytes).  Subqueries and whole walks
+    # record hit cells per query in the count pass (slot-major, so only slots in use are touched),
+    # up to EDGE_HIT_SLOTS or BOX_HIT_SLOTS (wide boxes have hundreds of hits) within the same
+    # budgets as int32 entries; queries with at most that many hits are written from the record
+    # instead of a second tree walk, and below 4 slots the write pass walks the tree again.  All are
+    # class defaults; setting them on a tree instance changes that tree only (results never
+    # depend on them).
     EDGE_HIT_SLOTS = 256
     EDGE_HIT_BUDGET = 1 << 28
 
@@ -389,10 +397,6 @@ class CellTree2dBase:
     EDGE_XY_SLOTS = 32
     EDGE_XY_BUDGET = 1 << 31
 
-    # Box queries: a box's hits are its output rows, and wide boxes have hundreds (up to ~900
-    # for boxes of 20 cell widths on a million-cell mesh), so the record is larger: up to BOX_HIT_SLOTS slots within BOX_HIT_BUDGET int32
-    # entries (4 GiB).  All four are class defaults; setting them on a tree instance changes
-    # that tree only (results never depend on them).
     BOX_HIT_SLOTS = 1024
     BOX_HIT_BUDGET = 1 << 30
 
@@ -425,7 +429,7 @@ class CellTree2dBase:
                 xs //= 2
         return None, 0
 
-    # Work splitting of the largest box and segment queries (ct_split_queries): a query expected
+    # Work splitting of the queries a wavefront walk leaves over (ct_split_queries): a query expected
     # to meet more than SPLIT_MIN_CELLS cells is cut into at most SPLIT_MAX_PARTS subqueries by
     # subtree, expanding subtrees of more than SPLIT_LEAF_CELLS (boxes) or EDGE_SPLIT_LEAF_CELLS
     # (segments) cells; results are identical.  Segments take larger leaves: fewer subqueries
@@ -435,7 +439,7 @@ class CellTree2dBase:
     EDGE_SPLIT_LEAF_CELLS = 64
     SPLIT_MAX_PARTS = 16
 
-    def _split(self, kind: int, queries: torch.Tensor, order, prep=None):
+    def _split(self, kind: int, queries: torch.Tensor, order):
         """(subqueries (m, 2) int32, part offsets (n + 1), m) for kind 1 boxes, 2 segment-face,
         3 segment-edge, or None when the batch is not split.  Batches too small to be ordered
         (order None: queries in their own order) are split too: with few lanes, one long walk
@@ -450,15 +454,116 @@ class CellTree2dBase:
         parts = D.empty(n, torch.int64)
         keep = D.empty(n * int(self.SPLIT_MAX_PARTS), torch.int32)  # frontiers, for the write call
         _native.call("ct_split_queries", *args, D.ptr(parts), None, None, D.ptr(keep), st)
-        if prep is None:
-            part_offsets, m = D.exclusive_scan(parts)
-        else:
-            part_offsets, _ = D.exclusive_scan(parts, total=False, offsets=prep.part_offsets)
-            m, *words = part_offsets[n: n + 4].tolist()
-            prep.check(words)
+        part_offsets, m = D.exclusive_scan(parts)
         subs = D.empty((max(m, 1), 2), torch.int32)
         _native.call("ct_split_queries", *args, None, D.ptr(part_offsets), D.ptr(subs), D.ptr(keep), st)
         return subs, part_offsets, m
+
+    def _gathers(self, n: int) -> bool:
+        """Whether a batch of n box or segment queries goes through ct_gather_*: every batch on a
+        tree the stack walks take and 32-bit offsets address, unless splitting is turned off
+        (SPLIT_MAX_PARTS <= 1: whole walks)."""
+        return (n > 0 and self.depth <= _native.CT_MAX_DEPTH and int(self.SPLIT_MAX_PARTS) > 1
+                and max(self.n_nodes, int(self.d_elements.shape[0])) < self.GATHER_MAX_RECORDS)
+
+    GATHER_MAX_RECORDS = 1 << 26
+
+    @staticmethod
+    def _pool(rows: int, widths):
+        """(rows, arrays): a row pool of int32 / float64 (rows, width) arrays; fewer rows (down to
+        none) when the device cannot hold it, so memory pressure costs a second walk, not the call."""
+        rows = min(int(rows), 2**31 - 1)
+        while rows > 0:
+            try:
+                return rows, [D.empty((rows, w), dtype) for dtype, w in widths]
+            except torch.cuda.OutOfMemoryError:
+                torch.cuda.empty_cache()
+                rows //= 2
+        return 0, [None for _ in widths]
+
+    def _gather(self, kind: int, queries: torch.Tensor, order, prep=None):
+        """Rows of a box (kind 1), segment-face (2) or segment-edge (3) batch: (ii, jj) or
+        (ii, jj, xy).  One readback: the row total, the queries left over, and the index checks of
+        ``prep``."""
+        n = int(queries.shape[0])
+        st = D.stream()
+        L = _native.lib()
+        rows = int(L.ct_gather_pool_rows(kind, n))
+        if kind == 1:
+            rows, (cell,) = self._pool(min(rows, int(self.BOX_HIT_BUDGET)), [(torch.int32, 1)])
+            pxy = src = None
+        else:
+            rows, (cell, pxy, src) = self._pool(min(rows, int(self.EDGE_HIT_BUDGET)),
+                                                [(torch.int32, 1), (torch.float64, 4), (torch.int32, 1)])
+        pool = (D.ptr(cell), D.ptr(pxy), D.ptr(src))
+        counts = D.empty(n, torch.int64)
+        starts = D.empty(n, torch.int64)
+        row = D.gather_row(n) if prep is None else prep.row  # offsets, check words, working words
+        _native.call("ct_gather_count", self.tree_ref, kind, D.ptr(queries), n, D.ptr(order),
+                     D.ptr(self.d_visit_cells), rows, *pool, D.ptr(counts), D.ptr(starts), D.ptr(row[n + 9:]), st)
+        D.exclusive_scan(counts, total=False, offsets=row)
+        total, *words, left = row[n: n + 10].tolist()
+        if prep is not None:
+            prep.check(words)
+        if left:
+            # Queries with more rows than a wavefront's lists hold, as subqueries; their counts join.
+            idx = torch.nonzero(starts < 0)[:, 0]
+            big = queries[idx].contiguous()
+            sub = self._split_rows(kind, big, self._order(1 if kind == 1 else 2, big)[0])
+            counts[idx] = torch.diff(sub[0])
+            _, total = D.exclusive_scan(counts, offsets=row)
+        ii = D.empty(total, torch.int64)
+        jj = D.empty(total, torch.int64)
+        xy = None if kind == 1 else D.empty((total, 2, 2), torch.float64)
+        _native.call("ct_gather_rows", kind, n, D.ptr(row), D.ptr(starts), *pool, D.ptr(ii), D.ptr(jj), D.ptr(xy), st)
+        if left:
+            _native.call("ct_place_rows", int(sub[1].numel()), D.ptr(idx), D.ptr(sub[0]), D.ptr(row), D.ptr(sub[1]),
+                         D.ptr(sub[2]), D.ptr(sub[3]), D.ptr(ii), D.ptr(jj), D.ptr(xy), st)
+        return (ii, jj) if kind == 1 else (ii, jj, xy)
+
+    def _split_rows(self, kind: int, queries: torch.Tensor, order):
+        """(offsets, ii, jj, xy or None) of a batch through subqueries by subtree (ct_split_queries):
+        the queries with too many rows for one wavefront."""
+        n = int(queries.shape[0])
+        st = D.stream()
+        subs, part_offsets, m = self._split(kind, queries, order)
+        counts = D.empty(max(m, 1), torch.int64)
+        if kind == 1:
+            hits, slots = self._hit_record(m, self.BOX_HIT_SLOTS, self.BOX_HIT_BUDGET)
+            _native.call("ct_locate_boxes_count_sub", self.tree_ref, D.ptr(queries), D.ptr(subs), m, D.ptr(counts),
+                         D.ptr(hits), slots, st)
+            offsets, total = self._sub_offsets(order, n, part_offsets, counts)
+            ii = D.empty(total, torch.int64)
+            jj = D.empty(total, torch.int64)
+            _native.call("ct_locate_boxes_write_sub", self.tree_ref, D.ptr(queries), D.ptr(subs), m, D.ptr(offsets),
+                         D.ptr(counts), D.ptr(hits), slots, D.ptr(ii), D.ptr(jj), st)
+            return offsets, ii, jj, None
+        edges = 1 if kind == 2 else 0  # the C ABI's kind of a segment query
+        hits, slots = self._hit_record(m, self.EDGE_HIT_SLOTS, self.EDGE_HIT_BUDGET)
+        hit_xy, xy_slots = (None, 0) if hits is None else self._xy_record(m, slots, self.EDGE_XY_SLOTS,
+                                                                          self.EDGE_XY_BUDGET)
+        _native.call("ct_locate_edges_count_sub", self.tree_ref, D.ptr(queries), D.ptr(subs), m, edges,
+                     D.ptr(counts), D.ptr(hits), slots, D.ptr(hit_xy), xy_slots, st)
+        # staging rows in processing order, then the per-segment sort into the output rows
+        sub_offsets, total = D.exclusive_scan(counts[:m])
+        per_query = D.empty(n, torch.int64)
+        query_start = D.empty(n, torch.int64)
+        _native.call("ct_subquery_spans", D.ptr(order), n, D.ptr(part_offsets), D.ptr(sub_offsets),
+                     D.ptr(per_query), D.ptr(query_start), st)
+        offsets, _ = D.exclusive_scan(per_query, total=False)
+        rows_query = D.empty(total, torch.int32)
+        rows_cell = D.empty(total, torch.int32)
+        rows_xy = D.empty((total, 4), torch.float64)
+        rows_t = D.empty(total, torch.float64)
+        _native.call("ct_locate_edges_write_sub", self.tree_ref, D.ptr(queries), D.ptr(subs), m, edges,
+                     D.ptr(sub_offsets), D.ptr(hits), slots, D.ptr(hit_xy), xy_slots, D.ptr(rows_query),
+                     D.ptr(rows_cell), D.ptr(rows_xy), D.ptr(rows_t), st)
+        ii = D.empty(total, torch.int64)
+        jj = D.empty(total, torch.int64)
+        xy = D.empty((total, 2, 2), torch.float64)
+        _native.call("ct_sort_staged_rows", D.ptr(offsets), D.ptr(query_start), D.ptr(rows_query),
+                     D.ptr(rows_cell), D.ptr(rows_xy), D.ptr(rows_t), total, D.ptr(ii), D.ptr(jj), D.ptr(xy), st)
+        return offsets, ii, jj, xy
 
     def _sub_offsets(self, order, n: int, part_offsets, counts):
         """Turns per-subquery counts into prefixes within each query; returns the query offsets
@@ -482,36 +587,9 @@ class CellTree2dBase:
         tensors)."""
         n = int(edge_coords.shape[0])
         st = D.stream()
+        if self._gathers(n):
+            return self._gather(2 if kind == 1 else 3, edge_coords, self._order(4, edge_coords)[0])
         order, srt = self._order(2, edge_coords)
-        split = self._split(2 if kind == 1 else 3, edge_coords, order)
-        if split is not None:
-            subs, part_offsets, m = split
-            counts = D.empty(max(m, 1), torch.int64)
-            hits, slots = self._hit_record(m, self.EDGE_HIT_SLOTS, self.EDGE_HIT_BUDGET)
-            hit_xy, xy_slots = (None, 0) if hits is None else self._xy_record(m, slots, self.EDGE_XY_SLOTS,
-                                                                              self.EDGE_XY_BUDGET)
-            _native.call("ct_locate_edges_count_sub", self.tree_ref, D.ptr(edge_coords), D.ptr(subs), m, kind,
-                         D.ptr(counts), D.ptr(hits), slots, D.ptr(hit_xy), xy_slots, st)
-            # staging rows in processing order, then the per-segment sort into the output rows
-            sub_offsets, total = D.exclusive_scan(counts[:m])
-            per_query = D.empty(n, torch.int64)
-            query_start = D.empty(n, torch.int64)
-            _native.call("ct_subquery_spans", D.ptr(order), n, D.ptr(part_offsets), D.ptr(sub_offsets),
-                         D.ptr(per_query), D.ptr(query_start), st)
-            offsets, _ = D.exclusive_scan(per_query, total=False)
-            rows_query = D.empty(total, torch.int32)
-            rows_cell = D.empty(total, torch.int32)
-            rows_xy = D.empty((total, 4), torch.float64)
-            rows_t = D.empty(total, torch.float64)
-            _native.call("ct_locate_edges_write_sub", self.tree_ref, D.ptr(edge_coords), D.ptr(subs), m, kind,
-                         D.ptr(sub_offsets), D.ptr(hits), slots, D.ptr(hit_xy), xy_slots, D.ptr(rows_query),
-                         D.ptr(rows_cell), D.ptr(rows_xy), D.ptr(rows_t), st)
-            ii = D.empty(total, torch.int64)
-            jj = D.empty(total, torch.int64)
-            xy = D.empty((total, 2, 2), torch.float64)
-            _native.call("ct_sort_staged_rows", D.ptr(offsets), D.ptr(query_start), D.ptr(rows_query),
-                         D.ptr(rows_cell), D.ptr(rows_xy), D.ptr(rows_t), total, D.ptr(ii), D.ptr(jj), D.ptr(xy), st)
-            return ii, jj, xy
         counts = D.empty(n, torch.int64)
         hits, slots = self._hit_record(n, self.EDGE_HIT_SLOTS, self.EDGE_HIT_BUDGET)
         _native.call(

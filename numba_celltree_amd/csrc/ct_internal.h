@@ -261,20 +261,14 @@ __device__ __forceinline__ bool cohen_sutherland(P2 a, P2 b, const Box& box, P2*
   for (int iter = 0; (k1 | k2) != 0; ++iter) {
     if ((k1 & k2) != 0 || iter >= 64) return false;
     const int opt = k1 ? k1 : k2;
-    double x, y;
-    if (opt & 8) {
-      x = a.x + dx * (box.ymax - a.y) / dy;
-      y = box.ymax;
-    } else if (opt & 4) {
-      x = a.x + dx * (box.ymin - a.y) / dy;
-      y = box.ymin;
-    } else if (opt & 2) {
-      y = a.y + dy * (box.xmax - a.x) / dx;
-      x = box.xmax;
-    } else {
-      y = a.y + dy * (box.xmin - a.x) / dx;
-      x = box.xmin;
-    }
+    // x = a.x + dx * (bound - a.y) / dy at a y bound, y = a.y + dy * (bound - a.x) / dx at an x bound:
+    // one expression on selected operands, so that lanes at different bounds share its division.
+    const bool at_y = (opt & 12) != 0;
+    const double bound = at_y ? ((opt & 8) ? box.ymax : box.ymin) : ((opt & 2) ? box.xmax : box.xmin);
+    const double u = at_y ? a.x : a.y, du = at_y ? dx : dy;
+    const double v = at_y ? a.y : a.x, dv = at_y ? dy : dx;
+    const double w = u + du * (bound - v) / dv;
+    const double x = at_y ? w : bound, y = at_y ? bound : w;
     if (opt == k1) {
       a = {x, y};
       k1 = cs_code(a, box);
@@ -342,14 +336,12 @@ __device__ __forceinline__ bool cb_collinear(P2 a, P2 b, P2 v0, P2 v1, P2* c, P2
   return true;
 }
 
-// cyrus_beck.py:142-241 cyrus_beck_line_polygon_clip (polygon CCW).
+// cyrus_beck.py:142-241 cyrus_beck_line_polygon_clip (polygon CCW), with the two end points' place
+// already known.
 template <int MAXV>
-__device__ __forceinline__ bool cyrus_beck(P2 a, P2 b, const P2 (&poly)[MAXV], int len, double tol,
-                                           P2* c, P2* d) {
+__device__ __forceinline__ bool cyrus_beck_in(P2 a, P2 b, bool a_in, bool b_in, const P2 (&poly)[MAXV], int len, P2* c,
+                                              P2* d) {
   const double sx = b.x - a.x, sy = b.y - a.y;
-  if (sx == 0 && sy == 0) return false;
-  const bool a_in = point_in_poly_or_edge<MAXV>(a, poly, len, tol);
-  const bool b_in = point_in_poly_or_edge<MAXV>(b, poly, len, tol);
   if (a_in && b_in) {
     *c = a;
     *d = b;
@@ -421,6 +413,15 @@ __device__ __forceinline__ bool cyrus_beck(P2 a, P2 b, const P2 (&poly)[MAXV], i
     return true;
   }
   return false;
+}
+
+template <int MAXV>
+__device__ __forceinline__ bool cyrus_beck(P2 a, P2 b, const P2 (&poly)[MAXV], int len, double tol,
+                                           P2* c, P2* d) {
+  if (b.x - a.x == 0 && b.y - a.y == 0) return false;
+  const bool a_in = point_in_poly_or_edge<MAXV>(a, poly, len, tol);
+  const bool b_in = point_in_poly_or_edge<MAXV>(b, poly, len, tol);
+  return cyrus_beck_in<MAXV>(a, b, a_in, b_in, poly, len, c, d);
 }
 
 // ---------------------------------------------------------- segment x segment

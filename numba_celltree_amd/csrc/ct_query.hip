@@ -86,7 +86,7 @@ __device__ __forceinline__ unsigned order_key(int kind, const double* __restrict
   }
   const double4 d = reinterpret_cast<const double4*>(q)[i];
   double cx, cy, w, h;
-  if (kind == 1) {  // (xmin, xmax, ymin, ymax)
+  if (kind == 1 || kind == 3) {  // (xmin, xmax, ymin, ymax)
     cx = 0.5 * (d.x + d.y);
     cy = 0.5 * (d.z + d.w);
     w = d.y - d.x;
@@ -96,6 +96,10 @@ __device__ __forceinline__ unsigned order_key(int kind, const double* __restrict
     cy = 0.5 * (d.y + d.w);
     w = fabs(d.z - d.x);
     h = fabs(d.w - d.y);
+  }
+  if (kind >= 3) {
+    return spread_bits(grid_coord(cx, g.bb.xmin, g.sx, 1024.0)) |
+           (spread_bits(grid_coord(cy, g.bb.ymin, g.sy, 1024.0)) << 1);
   }
   // Work proxy relative to the tree bbox: a box's area (its hits grow with it); a segment's
   // squared length (its walk grows with its length; its bbox area is 0 when axis-parallel).
@@ -1056,7 +1060,7 @@ size_t ct_order_workspace_bytes(int64_t n) {
 
 int ct_query_order(int32_t kind, const double* queries, int64_t n, const double* bbox, void* workspace,
                    size_t workspace_bytes, int32_t* order, double* sorted, void* stream) {
-  CT_REQUIRE(kind >= 0 && kind <= 2 && n >= 0 && n < ((int64_t)1 << 31) && bbox && order,
+  CT_REQUIRE(kind >= 0 && kind <= 4 && n >= 0 && n < ((int64_t)1 << 31) && bbox && order,
              "bad arguments");
   if (n == 0) return CT_OK;
   size_t need = 0;

@@ -302,7 +302,22 @@ __device__ __forceinline__ bool edge_face_clip_row(const TreeView& t, int k, int
     ymax = pmax(ymax, poly[i].y);
   }
   const double tol = pmax(kMinTolerance, kToleranceFactor * pmax(xmax - xmin, ymax - ymin));
-  return cyrus_beck<MAXV>(a, b, poly, len, tol, cc, dd);
+  if (b.x - a.x == 0 && b.y - a.y == 0) return false;
+  // An end point outside the row's box by more than the tolerance and the rounding of its test is
+  // in neither sense inside: no edge is within tol of it, and it sees an even number of edges beside
+  // it (all or none of them left of it).  Most cells of a segment hold neither end, so the lanes
+  // test one point each, and a second round runs only where a lane needs both.
+  const double m = 4.0 * tol + 1e-13 * pmax(pmax(fabs(xmin), fabs(xmax)), pmax(fabs(ymin), fabs(ymax)));
+  auto near = [&](P2 p) { return !(p.x < xmin - m || p.x > xmax + m || p.y < ymin - m || p.y > ymax + m); };
+  const bool near_a = near(a), near_b = near(b);
+  bool a_in = false, b_in = false;
+  if (near_a || near_b) {
+    const bool in = point_in_cell<MAXV>(near_a ? a : b, poly, tol);
+    if (near_a) a_in = in;
+    else b_in = in;
+    if (near_a && near_b) b_in = point_in_cell<MAXV>(b, poly, tol);
+  }
+  return cyrus_beck_in<MAXV>(a, b, a_in, b_in, poly, len, cc, dd);
 }
 
 template <int MAXV>
