@@ -417,7 +417,6 @@ int ct_place_rows(int64_t rows, const int64_t* idx, const int64_t* sub_offsets,
                   const int64_t* offsets, const int64_t* sub_ii, const int64_t* sub_jj,
                   const double* sub_xy, int64_t* ii, int64_t* jj, double* xy, void* stream);
 
-
 /* geometry_utils.py:564-574 sort_intersections_by_edge on grouped output (ii ascending, the
  * rows of segment s in [offsets[s], offsets[s+1])): writes jj and xy (n_rows, 2, 2) stably
  * sorted within each segment by t = (xy[:,0] - a) . (b - a), NaN last, into jj_out / xy_out
@@ -649,6 +648,24 @@ int ct_batch_edges_write_rec(const ct_batch* batch, const double* segments, int6
 int ct_batch_sort_intersections(const double* segments, int64_t n_segments, const int64_t* offsets,
                                 const int64_t* ii, const int64_t* jj, const double* xy, int64_t capacity,
                                 int32_t n_workgroups, int64_t* jj_out, double* xy_out, void* stream);
+
+/* intersect_edges for every tree's segments by wavefront walks (as ct_gather_count), in two calls with
+ * no host synchronization between them, so the sequence can be captured.  `tile`: the largest
+ * tile's queries, a multiple of 64.  ct_batch_gather_edges writes counts[q] and starts[q], and keeps
+ * the rows in the pool of pool_rows entries (0, or a tree of 2^26 nodes or cells or more in the batch:
+ * pass 0 then; every query is walked by one lane); tail: ct_gather_tail_words() int64 of working
+ * words.  After ct_exclusive_scan(counts) into offsets, ct_batch_gather_rows writes the rows of every
+ * query that ends within `capacity`, in the order ct_batch_sort_intersections gives, to (ii, jj,
+ * xy); jj_left, xy_left (capacity): working space for the rows of queries with starts[q] < 0, sorted by
+ * n_workgroups workgroups. */
+int ct_batch_gather_edges(const ct_batch* batch, const double* segments, int64_t n_queries, int32_t tile,
+                          int64_t pool_rows, int32_t* pool_cell, double* pool_xy, int32_t* pool_src,
+                          int64_t* counts, int64_t* starts, int64_t* tail, void* stream);
+int ct_batch_gather_rows(const ct_batch* batch, const double* segments, int64_t n_queries,
+                         const int64_t* offsets, const int64_t* starts, const int64_t* tail,
+                         const int32_t* pool_cell, const double* pool_xy, const int32_t* pool_src,
+                         int64_t capacity, int32_t n_workgroups, int64_t* ii, int64_t* jj_left, double* xy_left,
+                         int64_t* jj, double* xy, void* stream);
 
 #ifdef __cplusplus
 }

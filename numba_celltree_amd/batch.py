@@ -10,8 +10,8 @@ rows (ii = concatenated segment index, jj = cell of that segment's tree, xy) in 
 reference's per-segment order, tree after tree, with ``row_offsets`` marking each tree's
 rows.
 
-``BatchGraph`` captures a whole batch step (points, then segments: count, scan, write,
-sort) in a HIP graph through ``torch.cuda.CUDAGraph``; a replay is one host call.  The
+``BatchGraph`` captures a whole batch step (points, then segments: walks, scan, rows) in a
+HIP graph through ``torch.cuda.CUDAGraph``; a replay is one host call.  The
 launch shape (workgroup size, workgroups per CU, tile size, stack class, queue count) is a
 ``BatchConfig``; ``autotune`` times candidates on the actual batch and keeps the fastest.
 """
@@ -89,6 +89,8 @@ class TreeBatch:
         self.depths = np.array([int(t.depth) for t in trees])
         self.n_cells = np.array([int(t.d_elements.shape[0]) for t in trees])
         self.n_cu = _cu_count()
+        # trees the wavefront walks take (the others' segments are walked by one lane each)
+        self.gathers = all(max(int(t.n_nodes), int(t.d_elements.shape[0])) < t.GATHER_MAX_RECORDS for t in trees)
 
     # --------------------------------------------------------------- planning
     def plan(self, counts: Sequence[int], config: BatchConfig, weight: float = 1.0) -> "BatchPlan":
@@ -239,28 +241,41 @@ def concat_queries(sets: Sequence, width: int) -> Tuple[torch.Tensor, np.ndarray
     return cat, counts
 
 
-# Hit record of the batched segment passes (as CellTree2d.EDGE_HIT_SLOTS / EDGE_HIT_BUDGET):
-# up to EDGE_HIT_SLOTS recorded cells per segment within EDGE_HIT_BUDGET int32 entries.  A
-# batch is one large call, so the budget is 8 GiB (2.8% of a 288 GB device; slot-major, so
-# only slots in use are written): 256 slots for 7.5M segments.  With 35 slots (1 GiB) the
-# long segments, which carry most rows, still walked twice and the record did not pay.
+# Row pool of the batched segment walks: at most EDGE_HIT_SLOTS rows per segment on average and
+# EDGE_HIT_BUDGET int32 words (8 GiB, 2.8% of a 288 GB device; a row takes 10).  Segments that find it
+# used up are walked by one lane each.
 EDGE_HIT_SLOTS = 256
 EDGE_HIT_BUDGET = 1 << 31
+POOL_WAVES = 4096  # wavefronts of a walk, each taking up to POOL_CHUNK rows at a time
+POOL_CHUNK = 2048
+POOL_GUESS = 64    # rows per segment where their number is not known yet
 
 
 class EdgeBuffers:
-    """Device buffers of a batched segment pass with room for `capacity` rows, and the
-    count pass's hit record (None below 4 slots per segment)."""
+    """Device buffers of a batched segment pass with room for `capacity` rows, and its row pool for
+    about `expected` rows (default: `capacity`; record=False: no pool)."""
 
-    def __init__(self, n_queries: int, capacity: int, record: bool = True):
-        self.hits, self.slots = None, 0
-        if record and n_queries:
-            # Fewer slots (down to none) when the device cannot hold the full record.
-            self.hits, self.slots = CellTree2dBase._hit_record(n_queries, EDGE_HIT_SLOTS, EDGE_HIT_BUDGET)
-        self.capacity = int(capacity)
+    def __init__(self, n_queries: int, capacity: int, record: bool = True, expected: Optional[int] = None):
+        self.n_queries = n_queries
         self.counts = D.empty(n_queries, torch.int64)
+        self.starts = D.empty(n_queries, torch.int64)
         self.offsets = D.empty(n_queries + 1, torch.int64)
         self.scan_ws = D.empty(int(_native.lib().ct_scan_workspace_bytes(n_queries)), torch.uint8)
+        self.tail = D.empty(int(_native.lib().ct_gather_tail_words()), torch.int64)
+        expected = int(capacity) if expected is None else int(expected)
+        rows = 0
+        if record and n_queries:
+            # a quarter more, since a wavefront drops the end of a chunk that is too short for its
+            # next segments; and a chunk at hand per wavefront
+            rows = expected + expected // 4 + POOL_CHUNK * min(POOL_WAVES, n_queries)
+            rows = min(rows, n_queries * int(EDGE_HIT_SLOTS), int(EDGE_HIT_BUDGET) // 10)
+        self.pool_rows, self.pool = CellTree2dBase._pool(
+            rows, [(torch.int32, 1), (torch.float64, 4), (torch.int32, 1)])
+        self.room(capacity)
+
+    def room(self, capacity: int) -> None:
+        """Output arrays for `capacity` rows."""
+        self.capacity = int(capacity)
         self.ii = D.empty(self.capacity, torch.int64)
         self.jj = D.empty(self.capacity, torch.int64)
         self.xy = D.empty((self.capacity, 2, 2), torch.float64)
@@ -268,17 +283,31 @@ class EdgeBuffers:
         self.xy_sorted = D.empty((self.capacity, 2, 2), torch.float64)
 
 
-def run_edges(plan: BatchPlan, segments: torch.Tensor, buf: EdgeBuffers, sort_workgroups: int) -> None:
-    """count -> scan -> write -> per-segment sort, all enqueued (no host synchronization)."""
+def gather_edges(plan: BatchPlan, segments: torch.Tensor, buf: EdgeBuffers) -> None:
+    """Walks and the scan of the counts (offsets[-1]: the rows), enqueued."""
     n = plan.n_queries
     st = D.stream()
-    plan.edges_count(segments, buf.counts, buf.hits, buf.slots)
+    _check(segments, (n, 2, 2), torch.float64)
+    if not plan.batch.gathers:
+        buf.pool_rows = 0
+    _native.call("ct_batch_gather_edges", plan.ref, D.ptr(segments), n, int(plan.config.tile), buf.pool_rows,
+                 *(D.ptr(a) for a in buf.pool), D.ptr(buf.counts), D.ptr(buf.starts), D.ptr(buf.tail), st)
     _native.call("ct_exclusive_scan", D.ptr(buf.counts), n, D.ptr(buf.offsets), D.ptr(buf.scan_ws),
                  buf.scan_ws.numel(), st)
-    plan.edges_write(segments, buf.offsets, buf.capacity, buf.ii, buf.jj, buf.xy, buf.hits, buf.slots)
-    _native.call("ct_batch_sort_intersections", D.ptr(segments), n, D.ptr(buf.offsets), D.ptr(buf.ii),
-                 D.ptr(buf.jj), D.ptr(buf.xy), buf.capacity, int(sort_workgroups), D.ptr(buf.jj_sorted),
-                 D.ptr(buf.xy_sorted), st)
+
+
+def gather_rows(plan: BatchPlan, segments: torch.Tensor, buf: EdgeBuffers, sort_workgroups: int) -> None:
+    """The rows of gather_edges within the buffers' capacity, enqueued."""
+    _native.call("ct_batch_gather_rows", plan.ref, D.ptr(segments), plan.n_queries, D.ptr(buf.offsets),
+                 D.ptr(buf.starts), D.ptr(buf.tail), *(D.ptr(a) for a in buf.pool), buf.capacity,
+                 int(sort_workgroups), D.ptr(buf.ii), D.ptr(buf.jj), D.ptr(buf.xy), D.ptr(buf.jj_sorted),
+                 D.ptr(buf.xy_sorted), D.stream())
+
+
+def run_edges(plan: BatchPlan, segments: torch.Tensor, buf: EdgeBuffers, sort_workgroups: int) -> None:
+    """walks -> scan -> rows, all enqueued (no host synchronization)."""
+    gather_edges(plan, segments, buf)
+    gather_rows(plan, segments, buf, sort_workgroups)
 
 
 class BatchResult:
@@ -328,10 +357,8 @@ class BatchGraph:
         self.buf = None
         if self.eplan is not None:
             if capacity is None:
-                probe = EdgeBuffers(self.eplan.n_queries, 0, record=False)
-                self.eplan.edges_count(segments, probe.counts)
-                _native.call("ct_exclusive_scan", D.ptr(probe.counts), self.eplan.n_queries, D.ptr(probe.offsets),
-                             D.ptr(probe.scan_ws), probe.scan_ws.numel(), D.stream())
+                probe = EdgeBuffers(self.eplan.n_queries, 0, expected=POOL_GUESS * self.eplan.n_queries)
+                gather_edges(self.eplan, segments, probe)
                 capacity = int(probe.offsets[-1].item())
                 del probe
             self.buf = EdgeBuffers(self.eplan.n_queries, capacity)
@@ -393,13 +420,10 @@ def intersect_edges(batch: TreeBatch, segment_sets: Sequence, config: BatchConfi
     segs = segs.reshape(-1, 2, 2)
     plan = batch.plan(counts, config)
     n = plan.n_queries
-    probe = EdgeBuffers(n, 0, record=False)
-    plan.edges_count(segs, probe.counts)
-    _native.call("ct_exclusive_scan", D.ptr(probe.counts), n, D.ptr(probe.offsets), D.ptr(probe.scan_ws),
-                 probe.scan_ws.numel(), D.stream())
-    total = int(probe.offsets[-1].item())
-    buf = EdgeBuffers(n, total)
-    run_edges(plan, segs, buf, 4 * batch.n_cu)
+    buf = EdgeBuffers(n, 0, expected=POOL_GUESS * n)
+    gather_edges(plan, segs, buf)
+    buf.room(int(buf.offsets[-1].item()))
+    gather_rows(plan, segs, buf, 4 * batch.n_cu)
     res = BatchResult(None, plan, None, buf.ii, buf.jj_sorted, buf.xy_sorted, buf.offsets)
     ro = res.row_offsets()
     return [res.edges_of(m, ro) for m in range(batch.n_trees)]
@@ -421,8 +445,8 @@ _TUNED: Dict[Tuple, BatchConfig] = {}
 def autotune(batch: TreeBatch, kind: str, queries: torch.Tensor, counts: Sequence[int],
              candidates: Optional[Sequence[BatchConfig]] = None, reps: int = 3,
              cache_path: Optional[str] = None) -> Tuple[BatchConfig, List[Tuple[BatchConfig, float]]]:
-    """Time every candidate config on this batch (kind "points" or "edges": the count pass,
-    the dominant kernel) and return the fastest, with all (config, ms) timings.  Results are
+    """Time every candidate config on this batch (kind "points" or "edges": the one-lane count pass;
+    wavefront walks take only the tiles and queues of a config) and return the fastest, with all (config, ms) timings.  Results are
     kept per (kind, tree count, query count, depth, vertex class), in memory and, with
     `cache_path`, in a JSON file."""
     if kind not in ("points", "edges"):

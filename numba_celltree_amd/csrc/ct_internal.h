@@ -471,4 +471,10 @@ __device__ __forceinline__ bool lines_intersect(P2 a, P2 b, P2 p, P2 q, P2* out)
   return false;
 }
 
+// ct_gather.hip: rows of the queries with starts >= 0 from a row pool to their offsets, those of
+// queries that end past `capacity` left out.
+int launch_pool_rows(bool segments, int64_t n, const int64_t* offsets, const int64_t* starts, const int32_t* pool_cell,
+                     const double* pool_xy, const int32_t* pool_src, int64_t capacity, int64_t* ii, int64_t* jj,
+                     double* xy, hipStream_t st);
+
 }  // namespace ct

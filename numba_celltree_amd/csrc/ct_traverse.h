@@ -592,11 +592,12 @@ constexpr int kRankHalo = 256;
 constexpr int kRankWindow = kRankTile + 2 * kRankHalo;
 
 // Every lane of the workgroup calls this with the same r0 (it synchronises the workgroup);
-// tw holds kRankWindow doubles of LDS.
+// tw holds kRankWindow doubles of LDS.  With `starts`: only the rows of segments with starts < 0.
 __device__ __forceinline__ void sort_tile(const double* __restrict__ segs, const int64_t* __restrict__ offsets,
                                           const int64_t* __restrict__ ii, const int64_t* __restrict__ jj_in,
                                           const double* __restrict__ xy_in, int64_t n_rows, int64_t r0,
-                                          int64_t* __restrict__ jj_out, double* __restrict__ xy_out, double* tw) {
+                                          int64_t* __restrict__ jj_out, double* __restrict__ xy_out, double* tw,
+                                          const int64_t* __restrict__ starts = nullptr) {
   const double4* __restrict__ s4v = reinterpret_cast<const double4*>(segs);
   const double2* __restrict__ xy2 = reinterpret_cast<const double2*>(xy_in);
   const int64_t w0 = r0 > kRankHalo ? r0 - kRankHalo : 0;
@@ -607,6 +608,7 @@ __device__ __forceinline__ void sort_tile(const double* __restrict__ segs, const
     const int64_t r = r0 + k;
     if (r >= n_rows) break;
     const int64_t s = ii[r];
+    if (starts != nullptr && starts[s] >= 0) continue;
     const int64_t lo = offsets[s], hi = offsets[s + 1];
     const double t = tw[r - w0];
     int64_t rank = lo;

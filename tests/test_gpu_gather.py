@@ -67,3 +67,34 @@ def test_rows_of_whole_walks(kind, per_leaf, n, budget):
             assert np.array_equal(g, w, equal_nan=g.dtype.kind == "f")
         ref = getattr(oracle, name)(q)
         assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1])
+
+
+@pytest.mark.parametrize("tile, slots", [(64, 256), (1024, 256), (256, 8), (256, 0)])
+def test_batched_rows_of_single_calls(monkeypatch, tile, slots):
+    """A captured batch of segments, some of more rows than a wavefront's lists hold, and pools that
+    suffice, run out or are absent: the rows of every tree's own call, on every replay."""
+    import torch
+
+    import numba_celltree_amd as M
+    from numba_celltree_amd import batch as B
+
+    monkeypatch.setattr(B, "EDGE_HIT_SLOTS", slots)
+    meshes = [mesh("mixed"), S.jittered_grid(200, L, 0.2, 0.5, 9), mesh("hexagons"), mesh("ties")]
+    trees = [M.CellTree2d(torch.from_numpy(v).cuda(), torch.from_numpy(f).cuda(), -1) for v, f in meshes]
+    sets = [queries(n, 11 * n)[1] for n in (1, 700, 5000, 130)]
+    sets[1][5] = [[-1.0, -1.0], [L + 1.0, L + 0.5]]  # crosses some 600 cells
+    tb = B.TreeBatch(trees)
+    segs, counts = B.concat_queries(sets, 4)
+    graph = B.BatchGraph(tb, segments=segs.reshape(-1, 2, 2), segment_counts=counts,
+                         edges_config=B.BatchConfig(tile=tile))
+    want = [t.intersect_edges(torch.from_numpy(s).cuda()) for t, s in zip(trees, sets)]
+    assert max(int(torch.bincount(w[0]).max()) for w in want) > 320
+    for replay in range(3):
+        print(tile, slots, replay, flush=True)
+        graph.buf.jj_sorted.fill_(-7)
+        graph.replay()
+        res = graph.result()
+        for m, w in enumerate(want):
+            got = res.edges_of(m)
+            assert torch.equal(got[0], w[0]) and torch.equal(got[1], w[1])
+            assert torch.equal(got[2].view(torch.int64), w[2].view(torch.int64))
