@@ -468,7 +468,7 @@ def main() -> int:
     from numba_celltree_amd import _device as D
 
     tol = tree._default_tolerance()
-    ordered = tree.ORDERED_MIN is not None and args.points >= tree.ORDERED_MIN
+    ordered = tree.orders_points(args.points)
 
     def step(ev=None):
         # One locate_points call, split so the traversal kernel can be timed on its own:

@@ -62,9 +62,18 @@ class CellTree2d(CellTree2dBase):
         return self._elements_host()
 
     # ----------------------------------------------------------------- queries
-    # Point batches at least this large are processed in Morton order (ct_query_order, then
-    # ct_locate_points_in_order): neighbouring lanes then share their root-to-leaf paths.
-    ORDERED_MIN = 1 << 18
+    # Point batches at least this large, of a tree whose face rows and they multiply to at least
+    # ORDERED_WORK, are processed in Morton order (ct_query_order, then ct_locate_points_in_order):
+    # neighbouring lanes then share their root-to-leaf paths.  The sort takes 45 us and 7 ns per 1000
+    # points; what it saves grows with the points and with what of the tree does not fit the L2s.  In
+    # order / as they come, microseconds: 20,000 triangles, 2.6e5 points 79 / 33, 4e6 333 / 266;
+    # 200,000 cells, 1e6 146 / 125, 4e6 359 / 414; a million cells, 2.6e5 96 / 61, 1e6 155 / 173,
+    # 4e6 384 / 627.
+    ORDERED_MIN = 3 << 18
+    ORDERED_WORK = 1 << 40
+    # Points whose gradients go to the vertices are put in order from this size on: it also lets the
+    # backward add a face's points before it adds them to memory (1e6 points: 79 instead of 258 us).
+    ORDERED_GRAD_MIN = 1 << 18
 
     def locate_points(self, points, tolerance: Optional[float] = None):
         """Index of the face containing each point, -1 outside (celltree.py:99-128)."""
@@ -75,15 +84,24 @@ class CellTree2d(CellTree2dBase):
         out = self._locate_points_dev(pts, float(tolerance))
         return io.out(out)
 
+    def orders_points(self, n: int) -> bool:
+        """Whether a batch of n points is located in Morton order."""
+        return (self.ORDERED_MIN is not None and n >= self.ORDERED_MIN
+                and n * int(self.d_elements.numel()) >= self.ORDERED_WORK)
+
+    def _point_order(self, pts: torch.Tensor):
+        """The Morton order of a point batch.  The order alone: writing the points in sorted order
+        costs more in the sort (0.3 -> 0.8 ms at 1e7 points) than the contiguous read saves in the
+        traversal."""
+        return D.query_order(0, pts, self._bbox)
+
     def _locate_points_dev(self, pts: torch.Tensor, tolerance: float, order=None, sorted_pts=None) -> torch.Tensor:
         """``order`` / ``sorted_pts``: a processing order from ``D.query_order`` and, optionally,
         the points in that order (then read contiguously)."""
         n = int(pts.shape[0])
         out = D.empty(n, torch.int64)
-        if order is None and self.ORDERED_MIN is not None and n >= self.ORDERED_MIN:
-            # The order alone: writing the points in sorted order costs more in the sort
-            # (0.3 -> 0.8 ms at 1e7 points) than the contiguous read saves in the traversal.
-            order = D.query_order(0, pts, self._bbox)
+        if order is None and self.orders_points(n):
+            order = self._point_order(pts)
         if order is not None:
             _native.call("ct_locate_points_in_order", self.tree_ref, D.ptr(pts), n, D.ptr(order), D.ptr(sorted_pts),
                          tolerance, D.ptr(out), D.stream())
@@ -97,7 +115,7 @@ class CellTree2d(CellTree2dBase):
         n = int(d_boxes.shape[0])
         st = D.stream()
         if self._gathers(n):
-            return self._gather(1, d_boxes, self._order(3, d_boxes)[0], prep)
+            return self._gather(1, d_boxes, self._gather_order(3, d_boxes), prep)
         order, srt = self._order(1, d_boxes)
         if prep is not None:
             prep.check(prep.checks[:3].tolist())

@@ -43,9 +43,16 @@ def default_tolerance(bb_diagonal) -> float:  # celltree_base.py:51-52
 
 
 class CellTree2dBase:
-    # Box and segment batches at least this large are processed in the order of
-    # ct_query_order (similar work per wavefront); results do not depend on it.
+    # Box and segment batches at least this large are processed in the order of ct_query_order
+    # (similar work per wavefront) by subqueries and whole walks; results do not depend on it.
     ORDER_MIN = 4096
+    # Wavefront walks gain less from an order (Morton): their lanes work together as they are, and only
+    # the tree's part in the L2s differs.  From these sizes on it pays for its 45 us and the queries'
+    # scattered loads: in order / as they come, microseconds: boxes, 200,000 cells, 3.2e4 212 / 186,
+    # 2.6e5 426 / 448, 6e5 764 / 860; 50,000 cells, 2.6e5 338 / 310, 6e5 579 / 564; segments, 200,000
+    # cells, 1e5 435 / 407, 2.6e5 790 / 812, 6e5 1510 / 1606; a million cells, 6e5 1671 / 1832.
+    GATHER_ORDER_MIN = 1 << 18
+    GATHER_ORDER_CELLS = 1 << 17
     # Whether ordered box / segment passes also read their queries from a sorted copy.
     SORTED_QUERIES = False
 
@@ -56,6 +63,12 @@ class CellTree2dBase:
         if self.SORTED_QUERIES:
             return D.query_order(kind, queries, self._bbox, with_sorted=True)
         return D.query_order(kind, queries, self._bbox), None
+
+    def _gather_order(self, kind: int, queries: torch.Tensor):
+        if (int(queries.shape[0]) < self.GATHER_ORDER_MIN
+                or int(self.d_elements.shape[0]) < self.GATHER_ORDER_CELLS):
+            return None
+        return D.query_order(kind, queries, self._bbox)
 
     # ------------------------------------------------------------------ build
     def _build_tree(self, vertices: torch.Tensor, elements: torch.Tensor, bb_coords: torch.Tensor,
@@ -516,7 +529,7 @@ class CellTree2dBase:
         jj = D.empty(total, torch.int64)
         xy = None if kind == 1 else D.empty((total, 2, 2), torch.float64)
         _native.call("ct_gather_rows", kind, n, D.ptr(row), D.ptr(starts), *pool, D.ptr(ii), D.ptr(jj), D.ptr(xy), st)
-        if left:
+        if left and int(sub[1].numel()):
             _native.call("ct_place_rows", int(sub[1].numel()), D.ptr(idx), D.ptr(sub[0]), D.ptr(row), D.ptr(sub[1]),
                          D.ptr(sub[2]), D.ptr(sub[3]), D.ptr(ii), D.ptr(jj), D.ptr(xy), st)
         return (ii, jj) if kind == 1 else (ii, jj, xy)
@@ -551,6 +564,11 @@ class CellTree2dBase:
         _native.call("ct_subquery_spans", D.ptr(order), n, D.ptr(part_offsets), D.ptr(sub_offsets),
                      D.ptr(per_query), D.ptr(query_start), st)
         offsets, _ = D.exclusive_scan(per_query, total=False)
+        ii = D.empty(total, torch.int64)
+        jj = D.empty(total, torch.int64)
+        xy = D.empty((total, 2, 2), torch.float64)
+        if total == 0:
+            return offsets, ii, jj, xy
         rows_query = D.empty(total, torch.int32)
         rows_cell = D.empty(total, torch.int32)
         rows_xy = D.empty((total, 4), torch.float64)
@@ -558,9 +576,6 @@ class CellTree2dBase:
         _native.call("ct_locate_edges_write_sub", self.tree_ref, D.ptr(queries), D.ptr(subs), m, edges,
                      D.ptr(sub_offsets), D.ptr(hits), slots, D.ptr(hit_xy), xy_slots, D.ptr(rows_query),
                      D.ptr(rows_cell), D.ptr(rows_xy), D.ptr(rows_t), st)
-        ii = D.empty(total, torch.int64)
-        jj = D.empty(total, torch.int64)
-        xy = D.empty((total, 2, 2), torch.float64)
         _native.call("ct_sort_staged_rows", D.ptr(offsets), D.ptr(query_start), D.ptr(rows_query),
                      D.ptr(rows_cell), D.ptr(rows_xy), D.ptr(rows_t), total, D.ptr(ii), D.ptr(jj), D.ptr(xy), st)
         return offsets, ii, jj, xy
@@ -588,7 +603,7 @@ class CellTree2dBase:
         n = int(edge_coords.shape[0])
         st = D.stream()
         if self._gathers(n):
-            return self._gather(2 if kind == 1 else 3, edge_coords, self._order(4, edge_coords)[0])
+            return self._gather(2 if kind == 1 else 3, edge_coords, self._gather_order(4, edge_coords))
         order, srt = self._order(2, edge_coords)
         counts = D.empty(n, torch.int64)
         hits, slots = self._hit_record(n, self.EDGE_HIT_SLOTS, self.EDGE_HIT_BUDGET)

@@ -38,8 +38,9 @@ constexpr uint32_t kIndexMask = (1u << kOwnerShift) - 1u;
 constexpr int64_t kMaxRecords = (int64_t)1 << 26;
 
 // LDS list lengths.  The stack: a step of P entries needs room for P more; P shrinks as the stack
-// fills, and depth + 1 places always remain for a single entry's way down (kStack + depth + 1 in all).
-constexpr int kStack = 512;
+// fills, and depth + 1 places always remain for a single entry's way down (kStack + depth + 1 in all;
+// 512 instead of 320 costs boxes two wavefronts a CU, 1.28 instead of 1.22 ms, and 256 nothing).
+constexpr int kStack = 320;
 constexpr int kCells = 192;  // 63 left over + 2 per lane
 constexpr int kCands = 128;  // 63 left over + 64
 // Hits a wavefront holds, and the expected hits of the queries it walks together: fewer and the steps
@@ -47,8 +48,12 @@ constexpr int kCands = 128;  // 63 left over + 64
 // flight or groups overflow and are walked again one by one.  Measured, 1e6 queries, milliseconds:
 // boxes 768/384 1.27, 768/480 1.22, 768/576 1.27, 512/384 1.91, 640/640 1.59;
 // segments 256/160 2.67, 256/224 2.55, 320/280 2.50, 384/336 2.65, 512/448 2.77.
-constexpr int kBoxHits = 768, kBoxGroup = 480;
+// A box walked alone may have kBoxHits: boxes of 20 cell widths have 900 (8e3 of them on 20,000
+// triangles: 0.16 ms, and 0.60 with 768, most of it for the few then left to the subqueries).
+constexpr int kBoxHits = 1024, kBoxGroupHits = 768, kBoxGroup = 480;
 constexpr int kSegHits = 320, kSegGroup = 280;
+// Expected hits beyond which a query is left without a walk that would most likely be in vain.
+constexpr int kLeaveTimes = 2;
 
 // Counters for pool allocation, each on its own 128-byte line: one counter for all wavefronts
 // would serialize them (about 11 ns per atomic on one address).
@@ -308,6 +313,7 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
   // Each lane one query: down from the root while a single child is viable.
   int64_t q = 0;
   int start = -1, weight = 0;
+  bool big = false;
   if (lane < nq) {
     q = query_index(order, i0 + lane);
     QueryRec<KIND> rec;
@@ -335,8 +341,9 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
     }
     if (in) {
       weight = expected<KIND>(rec, p.cell);
-      start = 0;
-      while (true) {
+      big = weight > kLeaveTimes * kHits;
+      start = big ? -1 : 0;
+      while (start >= 0) {
         const NodeLd nd = ld_node(t.nodes, start);
         if (nd.child == -1) break;
         bool left, right;
@@ -374,7 +381,7 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
     if (mine && start >= 0)
       stack[below(alive)] = (uint32_t)lane << kOwnerShift | (uint32_t)start;
     // Hits this group may have: the lists' length, and the pool rows at hand (segments).
-    int room = kHits;
+    int room = KIND == kBoxes && g1 - g0 > 1 ? kBoxGroupHits : kHits;
     if (KIND != kBoxes && alive) {
       const int want = g1 - g0 == 1 ? kHits : min(kHits, 2 * wsum + 32);
       if (rows.end - rows.at < want) rows.refill(pool, tail);
@@ -563,7 +570,7 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
         if (!left_over) {
           if (g1 - g0 > 1) {
             if (nhit <= 256) group_by_owner<4, false>(hits, nullptr, nullptr, nhit, lane, first, cnt);
-            else group_by_owner<kBoxHits / 64, false>(hits, nullptr, nullptr, nhit, lane, first, cnt);
+            else group_by_owner<kBoxGroupHits / 64, false>(hits, nullptr, nullptr, nhit, lane, first, cnt);
           }
           // as many owners at a time as 64 words hold, or one larger owner
           for (int o = g0; o < g1;) {
@@ -603,7 +610,7 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
       }
     }
     if (mine) {
-      const bool leave = left_over && (over ? start >= 0 : c_own > 0);
+      const bool leave = big || (left_over && (over ? start >= 0 : c_own > 0));
       counts[q] = leave ? 0 : c_own;
       starts[q] = leave ? -1 : at + my_first;
       if (leave) atomicAdd(reinterpret_cast<unsigned long long*>(tail), 1ull);

@@ -53,6 +53,8 @@ def test_rows_of_whole_walks(kind, per_leaf, n, budget):
         tree, oracle = M.EdgeCellTree2d(v, e, 4, per_leaf), R.OracleEdgeCellTree2d(v, e, 4, per_leaf)
     else:
         tree, oracle = M.CellTree2d(v, f, -1, 4, per_leaf), R.OracleCellTree2d(v, f, -1, 4, per_leaf)
+    if n > 5000:
+        tree.GATHER_ORDER_MIN = tree.GATHER_ORDER_CELLS = 0
     boxes, seg = queries(n, 7 * n + per_leaf)
     calls = [("intersect_edges", seg)] + ([] if kind == "edges" else [("locate_boxes", boxes)])
     for name, q in calls:
