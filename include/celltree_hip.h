@@ -585,6 +585,19 @@ int ct_barycentric_wachspress_backward(const double* points, const int64_t* face
                                        const int32_t* faces, int32_t n_max_vert, const double* vertices, double tol,
                                        const double* g_weights, double* g_points, double* g_vertices, void* stream);
 
+/* The two with the points' processing order from ct_query_order kind 0 (NULL: none): a face's
+ * points then lie together and are summed before they are added to the vertices. */
+int ct_barycentric_triangle_backward_ordered(const double* points, const int64_t* face_indices,
+                                             const int32_t* order, int64_t n, const int32_t* faces,
+                                             int32_t n_max_vert, const double* vertices,
+                                             const double* g_weights, double* g_points,
+                                             double* g_vertices, void* stream);
+int ct_barycentric_wachspress_backward_ordered(const double* points, const int64_t* face_indices,
+                                               const int32_t* order, int64_t n, const int32_t* faces,
+                                               int32_t n_max_vert, const double* vertices, double tol,
+                                               const double* g_weights, double* g_points,
+                                               double* g_vertices, void* stream);
+
 /* ------------------------------------------------------------------ batched trees */
 /* No reference counterpart: many trees and their query sets in one persistent launch,
  * replacing a loop of per-mesh calls (celltree.py:216-239 locate_points, celltree.py:294-303

@@ -22,11 +22,12 @@ class BarycentricFunction(torch.autograd.Function):
     """Weights of points (n, 2) in faces face_index (n,) of a mesh (vertices (n_vertices, 2),
     faces (n_faces, k) int32), all on the current GPU; points and vertices float64.
     ``wachspress``: Wachspress weights (n, k) for k >= 3 (k <= 16 for the adjoint), else
-    triangle weights (n, 3) of the first three vertices.  ``barycentric_weights`` converts and
-    checks its inputs."""
+    triangle weights (n, 3) of the first three vertices.  ``order``: the points' processing order
+    (D.query_order kind 0; the backward sums a face's points with it), or None.
+    ``barycentric_weights`` converts and checks its inputs."""
 
     @staticmethod
-    def forward(ctx, points, vertices, faces, face_index, tolerance: float, wachspress: bool = False):
+    def forward(ctx, points, vertices, faces, face_index, tolerance: float, wachspress: bool = False, order=None):
         _require("points", points, (None, 2))
         _require("vertices", vertices, (None, 2))
         if faces.dtype != torch.int32 or faces.ndim != 2 or int(faces.shape[1]) < 3 or not faces.is_cuda:
@@ -40,26 +41,26 @@ class BarycentricFunction(torch.autograd.Function):
         fn = "ct_barycentric_wachspress_weights" if wachspress else "ct_barycentric_triangle_weights"
         _native.call(fn, D.ptr(points), D.ptr(face_index), n, D.ptr(faces), k, D.ptr(vertices), float(tolerance),
                      D.ptr(w), D.stream())
-        ctx.save_for_backward(points, vertices, faces, face_index)
+        ctx.save_for_backward(points, vertices, faces, face_index, order)
         ctx.tolerance = float(tolerance)
         ctx.wachspress = bool(wachspress)
         return w
 
     @staticmethod
     def backward(ctx, gw):
-        points, vertices, faces, face_index = ctx.saved_tensors
+        points, vertices, faces, face_index, order = ctx.saved_tensors
         n = int(points.shape[0])
         gp = D.empty((n, 2), torch.float64) if ctx.needs_input_grad[0] else None
         gv = torch.zeros_like(vertices) if ctx.needs_input_grad[1] else None
         gw = gw.to(torch.float64).contiguous()
         if ctx.wachspress:
-            _native.call("ct_barycentric_wachspress_backward", D.ptr(points), D.ptr(face_index), n, D.ptr(faces),
-                         int(faces.shape[1]), D.ptr(vertices), ctx.tolerance, D.ptr(gw), D.ptr(gp), D.ptr(gv),
+            _native.call("ct_barycentric_wachspress_backward_ordered", D.ptr(points), D.ptr(face_index), D.ptr(order), n,
+                         D.ptr(faces), int(faces.shape[1]), D.ptr(vertices), ctx.tolerance, D.ptr(gw), D.ptr(gp), D.ptr(gv),
                          D.stream())
         else:
-            _native.call("ct_barycentric_triangle_backward", D.ptr(points), D.ptr(face_index), n, D.ptr(faces),
-                         int(faces.shape[1]), D.ptr(vertices), D.ptr(gw), D.ptr(gp), D.ptr(gv), D.stream())
-        return gp, gv, None, None, None, None
+            _native.call("ct_barycentric_triangle_backward_ordered", D.ptr(points), D.ptr(face_index), D.ptr(order), n,
+                         D.ptr(faces), int(faces.shape[1]), D.ptr(vertices), D.ptr(gw), D.ptr(gp), D.ptr(gv), D.stream())
+        return gp, gv, None, None, None, None, None
 
 
 def barycentric_weights(tree, points: torch.Tensor, vertices: Optional[torch.Tensor] = None,
@@ -78,6 +79,11 @@ def barycentric_weights(tree, points: torch.Tensor, vertices: Optional[torch.Ten
     points, vertices = (_as_f64(x) for x in (points, vertices))
     _require("points", points, (None, 2))
     _require("vertices", vertices, (int(tree.d_vertices.shape[0]), 2))
-    face = tree._locate_points_dev(points.detach().contiguous(), float(tolerance))
-    w = BarycentricFunction.apply(points, vertices, tree.d_elements, face, float(tolerance), k > 3)
+    at = points.detach().contiguous()
+    n = int(at.shape[0])
+    order = None
+    if tree.orders_points(n) or (vertices.requires_grad and n >= tree.ORDERED_GRAD_MIN):
+        order = tree._point_order(at)
+    face = tree._locate_points_dev(at, float(tolerance), order)
+    w = BarycentricFunction.apply(points, vertices, tree.d_elements, face, float(tolerance), k > 3, order)
     return face, w

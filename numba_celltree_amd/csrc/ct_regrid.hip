@@ -641,61 +641,140 @@ __global__ void __launch_bounds__(kBlock) k_apply_t(const int64_t* __restrict__ 
   gF[i] = acc;
 }
 
+// Vertex gradients of the barycentric adjoints.  Points are many times the faces where the weights are
+// trained, and an atomic add to memory shared by eight L2s runs at about 23 per nanosecond for the
+// whole device: one per point and coordinate bounds the kernel (1e6 points on 20,000 triangles:
+// 258 us).  With the points in a spatial order (ct_query_order kind 0) a
+// wavefront's 64 points lie in a few faces, and the lanes of a face sum first: 79 us, what the
+// points' scattered rows take (1e6 triangles, about a point each: the whole pass 486 -> 392 us).
+
+// Sums P = 2^k values over the wavefront: lane l gets the sum of value folded(l) of P.  Every step
+// trades half of the values for the lane's partner's other half, so P - 1 + (6 - k) shuffles.
+template <int P>
+__device__ __forceinline__ double wave_fold(double (&v)[P], int lane) {
+  int step = 1;
+#pragma unroll
+  for (int h = P / 2; h > 0; h >>= 1, step <<= 1) {
+    const bool high = (lane & step) != 0;
+#pragma unroll
+    for (int j = 0; j < h; ++j) {
+      const double mine = high ? v[j + h] : v[j], other = high ? v[j] : v[j + h];
+      v[j] = mine + __shfl_xor(other, step, 64);
+    }
+  }
+  double r = v[0];
+  for (; step < 64; step <<= 1) r += __shfl_xor(r, step, 64);
+  return r;
+}
+
+template <int P>
+__device__ __forceinline__ int folded(int lane) {
+  int c = 0, step = 1;
+#pragma unroll
+  for (int h = P / 2; h > 0; h >>= 1, step <<= 1) c += (lane & step) ? h : 0;
+  return c;
+}
+
+// g_vtx[vid[k]] += g[k], k < len, for the lanes with a face (f >= 0); every lane of the wavefront
+// calls this.  A face of more than two lanes is summed first (ordered points; two lanes' adds cost
+// about what the shuffles do).
+template <int NV>
+__device__ __forceinline__ void add_to_vertices(bool ordered, int f, int len, const int (&vid)[NV], const P2 (&g)[NV],
+                                                double* __restrict__ g_vtx) {
+  constexpr int P = NV <= 1 ? 2 : NV <= 2 ? 4 : NV <= 4 ? 8 : NV <= 8 ? 16 : 32;
+  const int lane = lane_id();
+  bool direct = f >= 0;
+  if (ordered) {
+    uint64_t todo = __ballot(f >= 0);
+    while (todo) {
+      const int lead = __ffsll((unsigned long long)todo) - 1;
+      const int face = __builtin_amdgcn_readlane(f, lead);
+      const uint64_t same = __ballot(f == face);
+      todo &= ~same;
+      if (__popcll(same) <= 2) continue;
+      double v[P];
+#pragma unroll
+      for (int k = 0; k < P / 2; ++k) {
+        const bool in = f == face && k < NV && (k < NV ? k < len : false);
+        v[2 * k] = in ? g[k < NV ? k : 0].x : 0.0;
+        v[2 * k + 1] = in ? g[k < NV ? k : 0].y : 0.0;
+      }
+      const double sum = wave_fold<P>(v, lane);
+      const int c = folded<P>(lane);
+      int to = 0;
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        const int id = __builtin_amdgcn_readlane(vid[k], lead);
+        if (c >> 1 == k) to = id;
+      }
+      if (lane < P && (c >> 1) < __builtin_amdgcn_readlane(len, lead)) atomicAdd(g_vtx + 2 * (int64_t)to + (c & 1), sum);
+      if (f == face) direct = false;
+    }
+  }
+  if (direct) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      if (k < len) {
+        atomicAdd(g_vtx + 2 * (int64_t)vid[k], g[k].x);
+        atomicAdd(g_vtx + 2 * (int64_t)vid[k] + 1, g[k].y);
+      }
+  }
+}
+
 // Adjoint of barycentric_triangle.py:28-43 compute_weights (face held fixed):
 //   ab = b - a, ac = c - a, ap = p - a; Aa = |ab x ap|, Ac = |ac x ap|, A = |ab x ac|
 //   w = Aa / A (as (1/A) * Aa), v = Ac / A, u = 1 - v - w.
 __global__ void __launch_bounds__(kBlock) k_bary_tri_backward(const double* __restrict__ pts,
-                                                              const int64_t* __restrict__ face, int64_t n,
+                                                              const int64_t* __restrict__ face,
+                                                              const int32_t* __restrict__ order, int64_t n,
                                                               const int32_t* __restrict__ faces, int nmax,
                                                               const double* __restrict__ vtx,
                                                               const double* __restrict__ gw,
                                                               double* __restrict__ g_pts,
                                                               double* __restrict__ g_vtx) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int64_t f = face[i];
-  if (f < 0) {
-    if (g_pts) {
-      g_pts[2 * i] = 0.0;
-      g_pts[2 * i + 1] = 0.0;
-    }
-    return;
+  const int64_t at = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  int64_t i = 0, f = -1;
+  if (at < n) {
+    i = order ? order[at] : at;
+    f = face[i];
   }
-  const int32_t* row = faces + f * nmax;
-  const int ia = row[0], ib = row[1], ic = row[2];
-  const P2 a = ld_vertex(vtx, ia), b = ld_vertex(vtx, ib), c = ld_vertex(vtx, ic);
-  const P2 p = {pts[2 * i], pts[2 * i + 1]};
-  const double abx = b.x - a.x, aby = b.y - a.y;
-  const double acx = c.x - a.x, acy = c.y - a.y;
-  const double apx = p.x - a.x, apy = p.y - a.y;
-  const double cAa = abx * apy - aby * apx;
-  const double cAc = acx * apy - acy * apx;
-  const double cA = abx * acy - aby * acx;
-  const double Aa = fabs(cAa), Ac = fabs(cAc), A = fabs(cA);
-  const double inv = 1.0 / A;
-  const double gu = gw[3 * i], gv = gw[3 * i + 1], gww = gw[3 * i + 2];
-  const double gv_t = gv - gu, gw_t = gww - gu;  // u = 1 - v - w
-  const double g_inv = gw_t * Aa + gv_t * Ac;
-  const double gAa = gw_t * inv, gAc = gv_t * inv;
-  const double gA = -g_inv * inv * inv;
-  auto sgn = [](double x) { return x > 0 ? 1.0 : (x < 0 ? -1.0 : 0.0); };
-  const double g1 = gAa * sgn(cAa), g2 = gAc * sgn(cAc), g3 = gA * sgn(cA);
-  // cross(u, v) = u.x v.y - u.y v.x: d/du = (v.y, -v.x), d/dv = (-u.y, u.x)
-  double gabx = g1 * apy + g3 * acy, gaby = -g1 * apx - g3 * acx;
-  double gacx = g2 * apy - g3 * aby, gacy = -g2 * apx + g3 * abx;
-  double gapx = -g1 * aby - g2 * acy, gapy = g1 * abx + g2 * acx;
-  if (g_pts) {
+  int vid[3] = {0, 0, 0};
+  P2 g[3] = {};
+  double gapx = 0.0, gapy = 0.0;
+  if (f >= 0) {
+    const int32_t* row = faces + f * nmax;
+    vid[0] = row[0];
+    vid[1] = row[1];
+    vid[2] = row[2];
+    const P2 a = ld_vertex(vtx, vid[0]), b = ld_vertex(vtx, vid[1]), c = ld_vertex(vtx, vid[2]);
+    const P2 p = {pts[2 * i], pts[2 * i + 1]};
+    const double abx = b.x - a.x, aby = b.y - a.y;
+    const double acx = c.x - a.x, acy = c.y - a.y;
+    const double apx = p.x - a.x, apy = p.y - a.y;
+    const double cAa = abx * apy - aby * apx;
+    const double cAc = acx * apy - acy * apx;
+    const double cA = abx * acy - aby * acx;
+    const double Aa = fabs(cAa), Ac = fabs(cAc), A = fabs(cA);
+    const double inv = 1.0 / A;
+    const double gu = gw[3 * i], gv = gw[3 * i + 1], gww = gw[3 * i + 2];
+    const double gv_t = gv - gu, gw_t = gww - gu;  // u = 1 - v - w
+    const double g_inv = gw_t * Aa + gv_t * Ac;
+    const double gAa = gw_t * inv, gAc = gv_t * inv;
+    const double gA = -g_inv * inv * inv;
+    auto sgn = [](double x) { return x > 0 ? 1.0 : (x < 0 ? -1.0 : 0.0); };
+    const double g1 = gAa * sgn(cAa), g2 = gAc * sgn(cAc), g3 = gA * sgn(cA);
+    // cross(u, v) = u.x v.y - u.y v.x: d/du = (v.y, -v.x), d/dv = (-u.y, u.x)
+    g[1] = {g1 * apy + g3 * acy, -g1 * apx - g3 * acx};
+    g[2] = {g2 * apy - g3 * aby, -g2 * apx + g3 * abx};
+    gapx = -g1 * aby - g2 * acy;
+    gapy = g1 * abx + g2 * acx;
+    g[0] = {-(g[1].x + g[2].x + gapx), -(g[1].y + g[2].y + gapy)};
+  }
+  if (g_pts && at < n) {
     g_pts[2 * i] = gapx;
     g_pts[2 * i + 1] = gapy;
   }
-  if (g_vtx) {
-    atomicAdd(g_vtx + 2 * ib, gabx);
-    atomicAdd(g_vtx + 2 * ib + 1, gaby);
-    atomicAdd(g_vtx + 2 * ic, gacx);
-    atomicAdd(g_vtx + 2 * ic + 1, gacy);
-    atomicAdd(g_vtx + 2 * ia, -(gabx + gacx + gapx));
-    atomicAdd(g_vtx + 2 * ia + 1, -(gaby + gacy + gapy));
-  }
+  if (g_vtx) add_to_vertices<3>(order != nullptr, (int)f, 3, vid, g, g_vtx);
 }
 
 // Adjoint of barycentric_wachspress.py:38-85 compute_weights (face and branch held fixed).
@@ -707,31 +786,20 @@ __global__ void __launch_bounds__(kBlock) k_bary_tri_backward(const double* __re
 // The forward quantities are recomputed with the forward's own expressions, so the branch
 // (interior or which edge) is the one the forward took.  Vertex gradients are added with
 // atomics (a vertex is shared by many faces).
+//
+// The adjoint of one point p in face f for dL/dlambda g: the vertex gradients (gv, of the vertices vid)
+// and the point's (gp); returns the face's number of vertices.
 template <int MAXV>
-__global__ void __launch_bounds__(kBlock) k_bary_wachspress_backward(
-    const double* __restrict__ pts, const int64_t* __restrict__ face, int64_t n, const int32_t* __restrict__ faces,
-    int nmax, const double* __restrict__ vtx, double tol, const double* __restrict__ gw, double* __restrict__ g_pts,
-    double* __restrict__ g_vtx) {
-  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n) return;
-  const int64_t f = face[q];
-  if (f < 0) {
-    if (g_pts) {
-      g_pts[2 * q] = 0.0;
-      g_pts[2 * q + 1] = 0.0;
-    }
-    return;
-  }
+__device__ __forceinline__ int wachspress_adjoint(P2 p, int64_t f, const int32_t* __restrict__ faces, int nmax,
+                                                  const double* __restrict__ vtx, double tol,
+                                                  const double* __restrict__ g, int (&vid)[MAXV], P2 (&gv)[MAXV],
+                                                  P2* gp) {
   P2 poly[MAXV];
-  int vid[MAXV];
   const int len = load_face_idx<MAXV>(faces, nmax, f, vtx, poly, vid);
-  const P2 p = {pts[2 * q], pts[2 * q + 1]};
-  const double* g = gw + q * nmax;
   P2 last = poly[0];
 #pragma unroll
   for (int k = 0; k < MAXV; ++k)
     if (k == len - 1) last = poly[k];
-  P2 gv[MAXV];
 #pragma unroll
   for (int k = 0; k < MAXV; ++k) gv[k] = P2{0.0, 0.0};
   P2 gv_last = {0.0, 0.0};  // added to vertex len - 1 at the end
@@ -876,24 +944,40 @@ __global__ void __launch_bounds__(kBlock) k_bary_wachspress_backward(
       }
     }
   }
-  if (g_pts) {
-    g_pts[2 * q] = gpx;
-    g_pts[2 * q + 1] = gpy;
-  }
-  if (g_vtx) {
 #pragma unroll
-    for (int k = 0; k < MAXV; ++k) {
-      if (k < len) {
-        double gx = gv[k].x, gy = gv[k].y;
-        if (k == len - 1) {
-          gx += gv_last.x;
-          gy += gv_last.y;
-        }
-        atomicAdd(g_vtx + 2 * vid[k], gx);
-        atomicAdd(g_vtx + 2 * vid[k] + 1, gy);
-      }
+  for (int k = 0; k < MAXV; ++k) {
+    if (k == len - 1) {
+      gv[k].x += gv_last.x;
+      gv[k].y += gv_last.y;
     }
   }
+  *gp = {gpx, gpy};
+  return len;
+}
+
+template <int MAXV>
+__global__ void __launch_bounds__(kBlock) k_bary_wachspress_backward(
+    const double* __restrict__ pts, const int64_t* __restrict__ face, const int32_t* __restrict__ order, int64_t n,
+    const int32_t* __restrict__ faces, int nmax, const double* __restrict__ vtx, double tol,
+    const double* __restrict__ gw, double* __restrict__ g_pts, double* __restrict__ g_vtx) {
+  const int64_t at = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  int64_t q = 0, f = -1;
+  if (at < n) {
+    q = order ? order[at] : at;
+    f = face[q];
+  }
+  int vid[MAXV];
+  P2 gv[MAXV], gp = {0.0, 0.0};
+#pragma unroll
+  for (int k = 0; k < MAXV; ++k) vid[k] = 0;
+  int len = 0;
+  if (f >= 0)
+    len = wachspress_adjoint<MAXV>({pts[2 * q], pts[2 * q + 1]}, f, faces, nmax, vtx, tol, gw + q * nmax, vid, gv, &gp);
+  if (g_pts && at < n) {
+    g_pts[2 * q] = gp.x;
+    g_pts[2 * q + 1] = gp.y;
+  }
+  if (g_vtx) add_to_vertices<MAXV>(order != nullptr, (int)f, len, vid, gv, g_vtx);
 }
 
 inline int vclass(int nmax) { return nmax <= 4 ? 4 : nmax <= 8 ? 8 : 16; }
@@ -976,19 +1060,26 @@ int ct_regrid_apply_transpose(const int64_t* src_offsets, const int64_t* perm, c
   return launch_apply_t(src_offsets, perm, src_tgt, area, tgt_area, gy, n_fields, n_src, gF, as_stream(stream));
 }
 
-int ct_barycentric_triangle_backward(const double* points, const int64_t* face_indices, int64_t n,
+int ct_barycentric_triangle_backward_ordered(const double* points, const int64_t* face_indices, const int32_t* order, int64_t n,
                                      const int32_t* faces, int32_t n_max_vert, const double* vertices,
                                      const double* g_weights, double* g_points, double* g_vertices,
                                      void* stream) {
   CT_REQUIRE(n >= 0 && n_max_vert >= 3, "bad sizes");
   if (n == 0) return CT_OK;
-  k_bary_tri_backward<<<grid_for(n), kBlock, 0, as_stream(stream)>>>(points, face_indices, n, faces, n_max_vert,
+  k_bary_tri_backward<<<grid_for(n), kBlock, 0, as_stream(stream)>>>(points, face_indices, order, n, faces, n_max_vert,
                                                                      vertices, g_weights, g_points, g_vertices);
   CT_LAUNCH_CHECK();
   return CT_OK;
 }
 
-int ct_barycentric_wachspress_backward(const double* points, const int64_t* face_indices, int64_t n,
+int ct_barycentric_triangle_backward(const double* points, const int64_t* face_indices, int64_t n, const int32_t* faces,
+                                     int32_t n_max_vert, const double* vertices, const double* g_weights,
+                                     double* g_points, double* g_vertices, void* stream) {
+  return ct_barycentric_triangle_backward_ordered(points, face_indices, nullptr, n, faces, n_max_vert, vertices, g_weights,
+                                            g_points, g_vertices, stream);
+}
+
+int ct_barycentric_wachspress_backward_ordered(const double* points, const int64_t* face_indices, const int32_t* order, int64_t n,
                                        const int32_t* faces, int32_t n_max_vert, const double* vertices, double tol,
                                        const double* g_weights, double* g_points, double* g_vertices, void* stream) {
   CT_REQUIRE(n >= 0 && n_max_vert >= 3 && n_max_vert <= 16, "n_max_vert must be in [3, 16]");
@@ -996,16 +1087,23 @@ int ct_barycentric_wachspress_backward(const double* points, const int64_t* face
   const unsigned g = grid_for(n);
   hipStream_t st = as_stream(stream);
   if (n_max_vert <= 4)
-    k_bary_wachspress_backward<4><<<g, kBlock, 0, st>>>(points, face_indices, n, faces, n_max_vert, vertices, tol,
+    k_bary_wachspress_backward<4><<<g, kBlock, 0, st>>>(points, face_indices, order, n, faces, n_max_vert, vertices, tol,
                                                         g_weights, g_points, g_vertices);
   else if (n_max_vert <= 8)
-    k_bary_wachspress_backward<8><<<g, kBlock, 0, st>>>(points, face_indices, n, faces, n_max_vert, vertices, tol,
+    k_bary_wachspress_backward<8><<<g, kBlock, 0, st>>>(points, face_indices, order, n, faces, n_max_vert, vertices, tol,
                                                         g_weights, g_points, g_vertices);
   else
-    k_bary_wachspress_backward<16><<<g, kBlock, 0, st>>>(points, face_indices, n, faces, n_max_vert, vertices, tol,
+    k_bary_wachspress_backward<16><<<g, kBlock, 0, st>>>(points, face_indices, order, n, faces, n_max_vert, vertices, tol,
                                                          g_weights, g_points, g_vertices);
   CT_LAUNCH_CHECK();
   return CT_OK;
+}
+
+int ct_barycentric_wachspress_backward(const double* points, const int64_t* face_indices, int64_t n, const int32_t* faces,
+                                     int32_t n_max_vert, const double* vertices, double tol, const double* g_weights,
+                                     double* g_points, double* g_vertices, void* stream) {
+  return ct_barycentric_wachspress_backward_ordered(points, face_indices, nullptr, n, faces, n_max_vert, vertices, tol, g_weights,
+                                            g_points, g_vertices, stream);
 }
 
 int ct_regrid_rest_targets(const ct_regrid_topology* topo, int64_t* rest_targets, int64_t* n_out, void* stream) {
