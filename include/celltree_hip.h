@@ -550,6 +550,19 @@ typedef struct ct_regrid_topology {
   int64_t n_rest_targets;
 } ct_regrid_topology;
 
+/* The arrays of a topology that follow from its pairs (tt, ss: in target order) and faces, on the
+ * device: tgt_offsets (n_tgt + 1), src_offsets (n_src + 1), perm_by_src (n_pairs; the pairs of a source
+ * ascending), src_tgt = tt[perm_by_src], the corners face * n_max + slot of every vertex ascending
+ * (offsets n_vertices + 1; corners with room for n * n_max) and rest_targets (room for n_tgt, in no
+ * order).  info (device, 3): the rest targets, the target and the source corners.  Fewer than
+ * 2^32 - 1 pairs and corners together.  No synchronization. */
+size_t ct_regrid_lists_workspace_bytes(const ct_regrid_topology* topo);
+int ct_regrid_lists(const ct_regrid_topology* topo, void* workspace, size_t workspace_bytes,
+                    int64_t* tgt_offsets, int64_t* src_offsets, int64_t* perm_by_src, int64_t* src_tgt,
+                    int64_t* tgt_vertex_offsets, int64_t* tgt_vertex_corners,
+                    int64_t* src_vertex_offsets, int64_t* src_vertex_corners, int64_t* rest_targets,
+                    int64_t* info, void* stream);
+
 /* Fills rest_targets (device, capacity n_tgt) with the targets the vertex backward's pair pass
  * leaves to its per-target pass -- those without pairs and those whose pairs cross a block of
  * the pair pass -- and *n_out (HOST) with their count.  Depends on the topology only, so it

@@ -221,6 +221,8 @@ SIGNATURES = {
     "ct_regrid_apply": (ctypes.c_int, [_P, _P, _P, _P, _P, _I32, _I64, _P, _P]),
     "ct_regrid_apply_transpose": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _I32, _I64, _P, _P]),
     "ct_barycentric_triangle_backward": (ctypes.c_int, [_P, _P, _I64, _P, _I32, _P, _P, _P, _P, _P]),
+    "ct_regrid_lists_workspace_bytes": (_SZ, [_RP]),
+    "ct_regrid_lists": (ctypes.c_int, [_RP, _P, _SZ, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "ct_regrid_rest_targets": (ctypes.c_int, [_RP, _P, _P, _P]),
     "ct_regrid_backward_workspace_bytes": (_SZ, [_RP]),
     "ct_regrid_vertex_backward": (ctypes.c_int, [_RP, _P, _P, _P, _P, _P, _P, _I32, _P, _SZ, _P, _P, _P]),

@@ -179,36 +179,6 @@ __device__ __forceinline__ T ld_rec(const void* __restrict__ base, uint32_t x, u
   return *reinterpret_cast<const T*>(static_cast<const char*>(base) + (x * 32u + half * 16u));
 }
 
-// Ascending bitonic sort of 64 * R words, word r * 64 + lane in v[r] of the lane.
-template <int R>
-__device__ __forceinline__ void wave_sort(uint32_t (&v)[R], int lane) {
-#pragma unroll
-  for (int k = 2; k <= 64 * R; k <<= 1) {
-#pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      if (j >= 64) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const int p = r ^ (j >> 6);
-          if (p > r) {
-            const bool up = ((r << 6) & k) == 0;
-            const uint32_t a = v[r], b = v[p];
-            v[r] = up ? min(a, b) : max(a, b);
-            v[p] = up ? max(a, b) : min(a, b);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const uint32_t o = __shfl_xor(v[r], j, 64);
-          const bool low = ((((r << 6) | lane) & k) == 0) == ((lane & j) == 0);  // this lane keeps the smaller
-          v[r] = (o < v[r]) == low ? o : v[r];
-        }
-      }
-    }
-  }
-}
-
 // The cells of the visit numbers in list[0, m), m <= 64 * R, in ascending order, to out.
 template <int R>
 __device__ __forceinline__ void sorted_cells(const uint32_t* list, int m, int lane,

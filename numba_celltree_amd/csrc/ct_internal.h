@@ -471,6 +471,12 @@ __device__ __forceinline__ bool lines_intersect(P2 a, P2 b, P2 p, P2 q, P2* out)
   return false;
 }
 
+// True when target pairs [begin, end) all fall in one block of kBlock consecutive pairs, the
+// pairs of one k_pair_backward workgroup.
+__host__ __device__ __forceinline__ bool whole_in_block(int64_t begin, int64_t end) {
+  return end > begin && begin / kBlock == (end - 1) / kBlock;
+}
+
 // ct_gather.hip: rows of the queries with starts >= 0 from a row pool to their offsets, those of
 // queries that end past `capacity` left out.
 int launch_pool_rows(bool segments, int64_t n, const int64_t* offsets, const int64_t* starts, const int32_t* pool_cell,

@@ -61,6 +61,36 @@ __device__ __forceinline__ void wave_run_minmax(int key, unsigned long long lo,
   }
 }
 
+// Ascending bitonic sort of 64 * R words, word r * 64 + lane in v[r] of the lane.
+template <int R>
+__device__ __forceinline__ void wave_sort(uint32_t (&v)[R], int lane) {
+#pragma unroll
+  for (int k = 2; k <= 64 * R; k <<= 1) {
+#pragma unroll
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      if (j >= 64) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const int p = r ^ (j >> 6);
+          if (p > r) {
+            const bool up = ((r << 6) & k) == 0;
+            const uint32_t a = v[r], b = v[p];
+            v[r] = up ? min(a, b) : max(a, b);
+            v[p] = up ? max(a, b) : min(a, b);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const uint32_t o = __shfl_xor(v[r], j, 64);
+          const bool low = ((((r << 6) | lane) & k) == 0) == ((lane & j) == 0);  // this lane keeps the smaller
+          v[r] = (o < v[r]) == low ? o : v[r];
+        }
+      }
+    }
+  }
+}
+
 template <typename T>
 __global__ void k_fill(T* __restrict__ p, int64_t n, T value) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;

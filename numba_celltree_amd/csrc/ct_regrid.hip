@@ -277,12 +277,6 @@ __device__ __forceinline__ void overlap_area_gradient(const P2 (&a)[MA], int la,
 //                           (both meshes in one launch)
 // Corner rows have one P2 per face slot (stride n_max of that mesh).
 
-// True when target pairs [begin, end) all fall in one block of kBlock consecutive pairs, the
-// pairs of one k_pair_backward workgroup.
-__host__ __device__ __forceinline__ bool whole_in_block(int64_t begin, int64_t end) {
-  return end > begin && begin / kBlock == (end - 1) / kBlock;
-}
-
 // TC[t] slot `slot` = (sum over the target's pairs of `row(k)`, in pair order) plus the
 // target-area term of that slot, as k_target_corners sums it.
 template <int MAXV, typename Row>

@@ -17,29 +17,10 @@ import dataclasses
 import weakref
 from typing import Optional, Tuple
 
-import numpy as np
 import torch
 
 from numba_celltree_amd import _device as D
 from numba_celltree_amd import _native
-
-
-def _offsets(index: torch.Tensor, n: int) -> torch.Tensor:
-    counts = torch.bincount(index, minlength=n).to(torch.int64) if index.numel() else torch.zeros(
-        n, dtype=torch.int64, device=index.device)
-    offsets, _ = D.exclusive_scan(counts)
-    return offsets
-
-
-def _vertex_corners(faces: torch.Tensor, n_vertices: int):
-    """(offsets (n_vertices + 1), corners): the corners face * n_max + slot of every vertex,
-    ascending (a stable sort of the corners by vertex)."""
-    flat = faces.reshape(-1).to(torch.int64)
-    ids = torch.arange(flat.numel(), dtype=torch.int64, device=flat.device)
-    valid = flat >= 0
-    v = flat[valid]
-    order = torch.argsort(v, stable=True)
-    return _offsets(v, n_vertices), ids[valid][order].contiguous()
 
 
 class RegridTopology:
@@ -61,28 +42,35 @@ class RegridTopology:
         self.tt = tt
         self.ss = ss
         self.n_pairs = int(tt.numel())
-        self.tgt_offsets = _offsets(tt, self.n_tgt)
-        self.perm_by_src = torch.argsort(ss, stable=True)
-        self.src_tgt = tt[self.perm_by_src].contiguous()
-        self.src_offsets = _offsets(ss, self.n_src)
         self.n_tgt_vertices = int(d_tv.shape[0])
         self.n_src_vertices = int(tree.d_vertices.shape[0])
-        self.tgt_vertex_offsets, self.tgt_vertex_corners = _vertex_corners(d_tf, self.n_tgt_vertices)
-        self.src_vertex_offsets, self.src_vertex_corners = _vertex_corners(self.src_faces, self.n_src_vertices)
         s = _native.CtRegridTopology()
-        for name in ("tgt_faces", "src_faces", "tt", "ss", "tgt_offsets", "src_offsets", "perm_by_src",
-                     "tgt_vertex_offsets", "tgt_vertex_corners", "src_vertex_offsets", "src_vertex_corners"):
+        for name in ("tgt_faces", "src_faces", "tt", "ss"):
             setattr(s, name, getattr(self, name).data_ptr())
         s.n_pairs, s.n_tgt, s.n_src = self.n_pairs, self.n_tgt, self.n_src
         s.n_tgt_vertices, s.n_src_vertices = self.n_tgt_vertices, self.n_src_vertices
         s.n_max_t, s.n_max_s = int(d_tf.shape[1]), int(self.src_faces.shape[1])
-        # the targets the vertex backward's pair pass leaves to its per-target pass
-        rest = D.empty(max(self.n_tgt, 1), torch.int64)
-        n_rest = ctypes.c_int64(0)
-        _native.call("ct_regrid_rest_targets", ctypes.byref(s), D.ptr(rest), ctypes.byref(n_rest), D.stream())
-        self.rest_targets = rest  # the first n_rest_targets entries
-        s.rest_targets = rest.data_ptr()
-        s.n_rest_targets = n_rest.value
+        # the lists the forward and the adjoints gather through; the lengths of the last three (the
+        # targets the vertex backward's pair pass leaves to its per-target pass) come to the host
+        ref = ctypes.byref(s)
+        ws = D.empty(int(_native.lib().ct_regrid_lists_workspace_bytes(ref)), torch.uint8)
+        sizes = {"tgt_offsets": self.n_tgt + 1, "src_offsets": self.n_src + 1, "perm_by_src": self.n_pairs,
+                 "src_tgt": self.n_pairs, "tgt_vertex_offsets": self.n_tgt_vertices + 1,
+                 "tgt_vertex_corners": self.n_tgt * s.n_max_t, "src_vertex_offsets": self.n_src_vertices + 1,
+                 "src_vertex_corners": self.n_src * s.n_max_s, "rest_targets": max(self.n_tgt, 1)}
+        lists = {name: D.empty(n, torch.int64) for name, n in sizes.items()}
+        info = D.empty(3, torch.int64)
+        _native.call("ct_regrid_lists", ref, D.ptr(ws), ws.numel(), *(D.ptr(a) for a in lists.values()), D.ptr(info),
+                     D.stream())
+        n_rest, n_tgt_corners, n_src_corners = info.tolist()
+        for name, a in lists.items():
+            if name != "src_tgt":
+                setattr(s, name, a.data_ptr())
+        for name, n in (("tgt_vertex_corners", n_tgt_corners), ("src_vertex_corners", n_src_corners),
+                        ("rest_targets", n_rest)):
+            lists[name] = lists[name][:n]
+        vars(self).update(lists)
+        s.n_rest_targets = n_rest
         self._struct = s
         self._area_cache = None
 
