@@ -473,6 +473,20 @@ int ct_compact_pairs(const int64_t* ii, const int64_t* jj, const double* area,
                      const int64_t* keep, const int64_t* offsets, int64_t n, int64_t* ii_out,
                      int64_t* jj_out, double* area_out, void* stream);
 
+/* The pair stages and the compaction with a bit per pair instead of an int64: masks ((n + 63) / 64;
+ * bit k % 64 of word k / 64), counts (as many: the kept pairs of every word), and offsets =
+ * ct_exclusive_scan of the counts. */
+int ct_face_pairs_masks(const double* vertices_a, const int32_t* faces_a, int32_t n_max_a,
+                        const double* vertices_b, const int32_t* faces_b, int32_t n_max_b,
+                        const int64_t* ii, const int64_t* jj, int64_t n, int32_t with_area,
+                        double* area, int64_t* masks, int64_t* counts, void* stream);
+int ct_box_pairs_masks(const double* bbox_coords, const double* vertices, const int32_t* faces,
+                       int32_t n_max_vert, const int64_t* ii, const int64_t* jj, int64_t n,
+                       double* area, int64_t* masks, int64_t* counts, void* stream);
+int ct_compact_masks(const int64_t* ii, const int64_t* jj, const double* area, const int64_t* masks,
+                     const int64_t* offsets, int64_t n, int64_t* ii_out, int64_t* jj_out,
+                     double* area_out, void* stream);
+
 /* ----------------------------------------------------------------- barycentric */
 
 /* barycentric_triangle.py:46-64 -> out (n, 3). */

@@ -213,6 +213,9 @@ SIGNATURES = {
     "ct_face_pairs": (ctypes.c_int, [_P, _P, _I32, _P, _P, _I32, _P, _P, _I64, _I32, _P, _P, _P]),
     "ct_box_pairs": (ctypes.c_int, [_P, _P, _P, _I32, _P, _P, _I64, _P, _P, _P]),
     "ct_compact_pairs": (ctypes.c_int, [_P, _P, _P, _P, _P, _I64, _P, _P, _P, _P]),
+    "ct_face_pairs_masks": (ctypes.c_int, [_P, _P, _I32, _P, _P, _I32, _P, _P, _I64, _I32, _P, _P, _P, _P]),
+    "ct_box_pairs_masks": (ctypes.c_int, [_P, _P, _P, _I32, _P, _P, _I64, _P, _P, _P, _P]),
+    "ct_compact_masks": (ctypes.c_int, [_P, _P, _P, _P, _P, _I64, _P, _P, _P, _P]),
     "ct_barycentric_triangle_weights": (ctypes.c_int, [_P, _P, _I64, _P, _I32, _P, _F64, _P, _P]),
     "ct_barycentric_wachspress_weights": (ctypes.c_int, [_P, _P, _I64, _P, _I32, _P, _F64, _P, _P]),
     "ct_compute_barycentric_weights": (ctypes.c_int, [_TP, _P, _I64, _F64, _P, _P, _P]),

@@ -139,13 +139,19 @@ class CellTree2d(CellTree2dBase):
         ii, jj = self._locate_boxes_dev(d_boxes)
         return io.out(ii), io.out(jj)
 
-    def _compact(self, ii, jj, area, keep):
-        offsets, total = D.exclusive_scan(keep)
+    @staticmethod
+    def _kept(n: int):
+        """(masks, counts) of a pair stage."""
+        return D.empty((n + 63) // 64, torch.int64), D.empty((n + 63) // 64, torch.int64)
+
+    def _compact(self, ii, jj, area, kept):
+        masks, counts = kept
+        offsets, total = D.exclusive_scan(counts)
         io_ = D.empty(total, torch.int64)
         jo = D.empty(total, torch.int64)
         ao = D.empty(total, torch.float64) if area is not None else None
         _native.call(
-            "ct_compact_pairs", D.ptr(ii), D.ptr(jj), D.ptr(area), D.ptr(keep), D.ptr(offsets),
+            "ct_compact_masks", D.ptr(ii), D.ptr(jj), D.ptr(area), D.ptr(masks), D.ptr(offsets),
             int(ii.numel()), D.ptr(io_), D.ptr(jo), D.ptr(ao), D.stream(),
         )
         return io_, jo, ao
@@ -157,12 +163,12 @@ class CellTree2d(CellTree2dBase):
         ii, jj = self._locate_boxes_dev(d_boxes)
         n = int(ii.numel())
         area = D.empty(n, torch.float64)
-        keep = D.empty(n, torch.int64)
+        kept = self._kept(n)
         _native.call(
-            "ct_box_pairs", D.ptr(d_boxes), D.ptr(self.d_vertices), D.ptr(self.d_elements),
-            int(self.d_elements.shape[1]), D.ptr(ii), D.ptr(jj), n, D.ptr(area), D.ptr(keep), D.stream(),
+            "ct_box_pairs_masks", D.ptr(d_boxes), D.ptr(self.d_vertices), D.ptr(self.d_elements),
+            int(self.d_elements.shape[1]), D.ptr(ii), D.ptr(jj), n, D.ptr(area), *(D.ptr(t) for t in kept), D.stream(),
         )
-        i, j, a = self._compact(ii, jj, area, keep)
+        i, j, a = self._compact(ii, jj, area, kept)
         return io.out(i), io.out(j), io.out(a)
 
     def _prepare_faces(self, d_vertices: torch.Tensor, d_faces: torch.Tensor) -> torch.Tensor:
@@ -193,13 +199,13 @@ class CellTree2d(CellTree2dBase):
         ii, jj = self._locate_boxes_dev(bb, prep)
         n = int(ii.numel())
         area = D.empty(n, torch.float64) if with_area else None
-        keep = D.empty(n, torch.int64)
+        kept = self._kept(n)
         _native.call(
-            "ct_face_pairs", D.ptr(d_vertices), D.ptr(d_faces), int(d_faces.shape[1]),
+            "ct_face_pairs_masks", D.ptr(d_vertices), D.ptr(d_faces), int(d_faces.shape[1]),
             D.ptr(self.d_vertices), D.ptr(self.d_elements), int(self.d_elements.shape[1]),
-            D.ptr(ii), D.ptr(jj), n, int(with_area), D.ptr(area), D.ptr(keep), D.stream(),
+            D.ptr(ii), D.ptr(jj), n, int(with_area), D.ptr(area), *(D.ptr(t) for t in kept), D.stream(),
         )
-        return self._compact(ii, jj, area, keep)
+        return self._compact(ii, jj, area, kept)
 
     def locate_faces(self, vertices, faces) -> Tuple:
         """Face pairs that intersect or touch (SAT), celltree.py:186-226.

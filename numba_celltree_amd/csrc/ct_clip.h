@@ -153,12 +153,26 @@ __device__ __forceinline__ int sh_run(const P2 (&subj)[MA], int ls, const P2 (&c
   return len;
 }
 
+template <int CAP>
+__device__ __forceinline__ P2 mean_vertex(const P2 (&poly)[CAP], int len) {
+  P2 sum = {0.0, 0.0};
+#pragma unroll
+  for (int i = 0; i < CAP; ++i)
+    if (i < len) {
+      sum.x += poly[i].x;
+      sum.y += poly[i].y;
+    }
+  const double w = 1.0 / (double)len;
+  return {sum.x * w, sum.y * w};
+}
+
 // The same clip with plain runtime indexing (scratch memory), for the large vertex classes
 // (CAP > 16), where most of a clip row would sit past its LDS slots anyway and the unrolled
 // loops would run to 32+ slots; faces of more than 8 vertices are rare.  Same operations in
 // the same order as sh_stage.
 template <int MA, int MB>
-__device__ __forceinline__ double clip_area_indexed(const P2 (&subj)[MA], int ls, const P2 (&clip)[MB], int lc) {
+__device__ __forceinline__ double clip_area_indexed(const P2 (&subj)[MA], int ls, const P2 (&clip)[MB], int lc,
+                                                    P2* centre) {
   constexpr int CAP = MA + MB;
   P2 outp[CAP], inp[CAP];
   for (int i = 0; i < CAP; ++i) outp[i] = (i < MA) ? subj[i < MA ? i : 0] : P2{0.0, 0.0};
@@ -205,12 +219,13 @@ __device__ __forceinline__ double clip_area_indexed(const P2 (&subj)[MA], int ls
     }
     r = s;
   }
+  if (centre != nullptr) *centre = mean_vertex<CAP>(outp, n_out);
   return polygon_area<CAP>(outp, n_out);
 }
 
 // sutherland_hodgman.py:84-148 polygon_polygon_clip_area.  `row` is the lane's clip row of
 // clip_row_cap<MA, MB>() slots (CT_CLIP_ROWS); the indexed path for the large classes does
-// not use it.
+// not use it.  centre (may be null): the mean of the clipped polygon's vertices, when it has an area.
 template <int MA, int MB>
 constexpr int clip_row_cap() {
   return MA + MB > 16 ? 1 : MA + MB;
@@ -218,15 +233,17 @@ constexpr int clip_row_cap() {
 
 template <int MA, int MB, class Row>
 __device__ __forceinline__ double clip_area(const P2 (&subj)[MA], int ls, const P2 (&clip)[MB], int lc,
-                                            const Row& row) {
+                                            const Row& row, P2* centre = nullptr) {
   constexpr int CAP = MA + MB;
   if constexpr (CAP > 16) {
-    return clip_area_indexed<MA, MB>(subj, ls, clip, lc);
+    return clip_area_indexed<MA, MB>(subj, ls, clip, lc, centre);
   } else {
     static_assert(Row::kLds + Row::kExtra == CAP, "clip row of the wrong capacity");
     P2 poly[CAP];
     const int len = sh_run<MA, MB, CAP>(subj, ls, clip, lc, lc, row, poly);
-    return (len < 3) ? 0.0 : polygon_area<CAP>(poly, len);
+    if (len < 3) return 0.0;
+    if (centre != nullptr) *centre = mean_vertex<CAP>(poly, len);
+    return polygon_area<CAP>(poly, len);
   }
 }
 
