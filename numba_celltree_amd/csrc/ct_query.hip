@@ -46,6 +46,137 @@ __global__ void __launch_bounds__(kBlock) k_locate_points(TreeView t, const doub
   __builtin_nontemporal_store((int64_t)locate_one<MAXV, STACK, ON_EDGE, LEAF>(t, p, tol, stack), out + q);
 }
 
+// ----------------------------------------------------------------- small point batches
+// A batch that cannot fill the device takes as long as its longest walk: a chain of up to 50 dependent
+// loads (20,000 triangles), while the 64 lanes of a wavefront wait for each other at every leaf.  Here
+// a wavefront has few points and explores their walks in all directions at once: a lane holds a node,
+// and where both children are viable an idle lane takes the second; the chain is the tree's depth
+// below the start node (15), then every cell of the leaves is tested at once.  What the reference
+// returns is the first hit of a depth-first walk (query.py:62-107): a lane carries the choices that
+// lead to its node, a bit where both children were viable (0: the one the walk enters first), and the
+// first hit is the least in (choices, position in the leaf).  Points with more choices than the key has
+// bits or more nodes at once than there are lanes walk as in k_locate_points.
+//
+// Microseconds, k_locate_points / here: 20,000 triangles, 1e3 points 19.5 / 8.2, 6e4 21.1 / 12.5; a million
+// cells, 1e3 19.6 / 9.8, 2e4 27.9 / 18.0, 6e4 38.1 / 22.4.  A walk of every viable node costs more loads
+// in all, so from some 1.3e5 points on (42.5 / 38.9 on a million cells, 17.1 / 18.0 on 2,000) the
+// one-lane walk is the better one (2.6e5: 60.2 / 65.2).  16 points a wavefront (8: 6e4 points 29.0), fewer
+// while 4096 wavefronts suffice; entries in an LDS stack instead of the lanes' registers: 1e3 points
+// 15.9; one point a wavefront in the old walk: 13.2.
+constexpr int kTeamMaxPoints = 16, kTeamKeyBits = 32;
+constexpr int64_t kTeamMax = 1 << 17, kTeamWaves = 4096;
+
+struct TeamEntry {
+  P2 p;
+  int at;         // node, or position in bb_indices
+  uint32_t key;   // choices, from the highest bit
+  uint32_t info;  // point | choices made << 8
+};
+
+template <int MAXV, int STACK, bool ON_EDGE, int LEAF>
+__global__ void __launch_bounds__(64) k_locate_team(TreeView t, const double* __restrict__ pts, QueryOrder ord, int64_t n,
+                                                    int per_wave, double tol, int64_t* __restrict__ out) {
+  __shared__ TeamEntry spare[64];
+  __shared__ unsigned long long best[kTeamMaxPoints];
+  __shared__ int64_t slot_of[kTeamMaxPoints];
+  __shared__ int alone[kTeamMaxPoints];
+  const int lane = threadIdx.x;
+  const uint64_t lower = (1ull << lane) - 1;
+  const int64_t i0 = (int64_t)blockIdx.x * per_wave;
+  const int m = (int)min((int64_t)per_wave, n - i0);
+  TeamEntry e{};
+  e.at = -1;
+  if (lane < m) {
+    const int64_t q = ord.order ? (int64_t)ord.order[i0 + lane] : i0 + lane;
+    e.p = ld_point(pts, q);
+    e.at = start_node(t, e.p);
+    e.info = (uint32_t)lane;
+    slot_of[lane] = q;
+    best[lane] = ~0ull;
+    alone[lane] = 0;
+  }
+  const TeamEntry own = e;
+  int ptr = 0, size = 0;  // a leaf's cells, once the lane stands on one
+  // Entries of the lanes `give` to idle lanes, as far as these go; true: this lane took one.
+  auto hand_over = [&](bool give, bool busy, const TeamEntry& x, bool* given) {
+    const uint64_t mg = __ballot(give), idle = ~__ballot(busy);
+    const int rank = __popcll(mg & lower);
+    *given = give && rank < __popcll(idle);
+    __syncthreads();  // one wavefront: orders LDS accesses
+    if (*given) spare[rank] = x;
+    __syncthreads();
+    const int r = __popcll(idle & lower);
+    const bool take = !busy && r < __popcll(mg);
+    if (take) e = spare[r];
+    return take;
+  };
+  while (__ballot(e.at >= 0)) {
+    bool second = false;
+    TeamEntry far = e;
+    if (e.at >= 0) {
+      const NodeLd nd = ld_node(t.nodes, e.at);
+      e.at = -1;
+      if (nd.child == -1) {
+        ptr = nd.ptr;
+        size = nd.size;
+      } else {
+        const double v = nd.dim ? e.p.y : e.p.x;
+        const bool left = v <= nd.Lmax, right = v >= nd.Rmin;
+        if (left || right) e.at = nd.child + (left ? 0 : 1);
+        if (left && right) {  // query.py:93-101
+          const bool right_first = (nd.Lmax - v) < (v - nd.Rmin);
+          const uint32_t choices = e.info >> 8;
+          e.at = nd.child + (right_first ? 1 : 0);
+          e.info += 1u << 8;
+          far = e;
+          far.at = nd.child + (right_first ? 0 : 1);
+          far.key |= 0x80000000u >> (choices & 31u);
+          second = true;
+          if (choices >= kTeamKeyBits) alone[e.info & 0xffu] = 1;
+        }
+      }
+    }
+    if (__ballot(second)) {
+      bool given;
+      hand_over(second, e.at >= 0 || size > 0, far, &given);
+      if (second && !given) alone[e.info & 0xffu] = 1;
+    }
+  }
+  // the second cells of the leaves to idle lanes, the others one after the other
+  bool gave = false;
+  if (__ballot(size > 1)) {
+    TeamEntry x = e;
+    x.at = ptr + 1;
+    if (hand_over(size > 1, size > 0, x, &gave)) {
+      ptr = e.at;
+      size = 1;
+    }
+  }
+  unsigned long long word = ~0ull;
+  int cell = -1;
+  for (int j = 0; __ballot(j < size); ++j) {
+    if (j >= size || (j == 1 && gave) || cell >= 0) continue;
+    NodeLd one{};
+    one.ptr = ptr + j;
+    one.size = 1;
+    if (leaf_hit<MAXV, STACK, ON_EDGE, LEAF>(t, e.p, tol, one, &cell))
+      word = (unsigned long long)e.key << 32 | (unsigned)(ptr + j);
+  }
+  const int who = (int)(e.info & 0xffu);
+  __syncthreads();
+  if (cell >= 0) atomicMin(&best[who], word);
+  __syncthreads();
+  if (cell >= 0 && best[who] == word && !alone[who]) out[slot_of[who]] = cell;
+  if (lane < m) {
+    if (alone[lane]) {
+      CT_LANE_STACK(STACK, walk);
+      out[slot_of[lane]] = locate_one<MAXV, STACK, ON_EDGE, LEAF>(t, own.p, tol, walk);
+    } else if (best[lane] == ~0ull) {
+      out[slot_of[lane]] = -1;
+    }
+  }
+}
+
 // ----------------------------------------------------------------- query ordering
 // Sort of the queries by a 20-bit key.  Points: the Morton key of a 1024 x 1024 grid over
 // the tree bbox.  Boxes and segments: a 4-bit work class (log2 of the query's bbox area
@@ -844,7 +975,13 @@ struct LocateLaunch {
   hipStream_t st;
   template <int S>
   int run() {
-    k_locate_points<MAXV, S, ON_EDGE, LEAF><<<grid_xcd(n), kBlock, 0, st>>>(t, pts, order, n, tol, out);
+    if (n <= kTeamMax) {
+      const int per_wave = (int)std::min((int64_t)kTeamMaxPoints, std::max((int64_t)1, (n + kTeamWaves - 1) / kTeamWaves));
+      k_locate_team<MAXV, S, ON_EDGE, LEAF><<<(unsigned)((n + per_wave - 1) / per_wave), 64, 0, st>>>(t, pts, order, n,
+                                                                                               per_wave, tol, out);
+    } else {
+      k_locate_points<MAXV, S, ON_EDGE, LEAF><<<grid_xcd(n), kBlock, 0, st>>>(t, pts, order, n, tol, out);
+    }
     CT_LAUNCH_CHECK();
     return CT_OK;
   }
