@@ -16,7 +16,8 @@ from numba_celltree_amd.constants import NodeDType
 
 
 def device() -> torch.device:
-    if not torch.cuda.is_available():
+    # Every array of a call asks for this: is_available() counts the devices anew each time.
+    if not torch.cuda.is_initialized() and not torch.cuda.is_available():
         raise RuntimeError(
             "numba_celltree_amd computes on a ROCm GPU only, and none is visible "
             "(torch.cuda.is_available() is False)"
@@ -24,12 +25,13 @@ def device() -> torch.device:
     return torch.device("cuda", torch.cuda.current_device())
 
 
-def stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+def stream() -> int:
+    """The current stream's handle (without torch.cuda.current_stream()'s Stream object)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
-def ptr(t) -> ctypes.c_void_p:
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+def ptr(t) -> int:
+    return 0 if t is None else t.data_ptr()
 
 
 def is_device_tensor(x) -> bool:
@@ -67,7 +69,7 @@ def to_dev(x, dtype: torch.dtype) -> torch.Tensor:
     """
     dev = device()
     if isinstance(x, torch.Tensor):
-        t = x.to(device=dev, dtype=dtype).contiguous()
+        t = (x if x.dtype == dtype and x.device == dev else x.to(device=dev, dtype=dtype)).contiguous()
     else:
         t = host_tensor(np.asarray(x)).to(device=dev, dtype=dtype).contiguous()
     if t.data_ptr() % 32:
