@@ -227,6 +227,11 @@ int ct_node_boxes(const ct_tree* tree, int32_t* scratch, double* out, void* stre
  * or without it.  Requires 1 <= n <= 4096. */
 int ct_start_grid(const ct_tree* tree, int32_t n, int32_t* out, void* stream);
 
+/* ct_pack_leaf_coords, ct_pack_leaf_bboxes, ct_visit_cells and ct_start_grid in one launch; NULL
+ * arrays are left out. */
+int ct_tree_layouts(const ct_tree* tree, double* leaf_coords, double* leaf_bb, int32_t* visit_cells,
+                    int32_t grid_n, int32_t* grid, void* stream);
+
 size_t ct_locate_workspace_bytes(int64_t n);
 
 /* query.py:110-117 locate_points, same results as ct_locate_points: the queries are first

@@ -188,6 +188,7 @@ SIGNATURES = {
     "ct_sort_staged_rows": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _I64, _P, _P, _P, _P]),
     "ct_gather_tail_words": (_I64, []),
     "ct_gather_pool_rows": (_I64, [_I32, _I64]),
+    "ct_tree_layouts": (ctypes.c_int, [_TP, _P, _P, _P, _I32, _P, _P]),
     "ct_visit_cells": (ctypes.c_int, [_TP, _P, _P]),
     "ct_gather_count": (ctypes.c_int, [_TP, _I32, _P, _I64, _P, _P, _I64, _P, _P, _P, _P, _P, _P, _P]),
     "ct_gather_rows": (ctypes.c_int, [_I32, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P]),

@@ -146,24 +146,23 @@ class CellTree2dBase:
         self._ctree = t
         self._host = {}
         nmax = int(elements.shape[1])
-        self.d_leaf_coords = None
-        if 3 <= nmax <= 8:
-            # Leaf-ordered vertex copy: a leaf's cells become one contiguous read.
-            self.d_leaf_coords = D.empty((n, nmax, 2), torch.float64)
-            _native.call("ct_pack_leaf_coords", self.tree_ref, D.ptr(self.d_leaf_coords), st)
-            t.leaf_coords = self.d_leaf_coords.data_ptr()
-        t.leaf_bb = None
-        self.d_leaf_bb = None
-        if LEAF_BBOXES and n > 0:
-            # Leaf-ordered cell boxes: box and segment queries read a leaf's boxes directly.
-            self.d_leaf_bb = D.empty((n, 4), torch.float64)
-            _native.call("ct_pack_leaf_bboxes", self.tree_ref, D.ptr(self.d_leaf_bb), st)
-            t.leaf_bb = self.d_leaf_bb.data_ptr()
-        self.d_visit_cells = None
-        if nmax >= 3:
-            # The cells in visit order: box queries turn visit numbers into cells.
-            self.d_visit_cells = D.empty(n, torch.int32)
-            _native.call("ct_visit_cells", self.tree_ref, D.ptr(self.d_visit_cells), st)
+        # Leaf-ordered vertices: a leaf's cells become one contiguous read.
+        self.d_leaf_coords = D.empty((n, nmax, 2), torch.float64) if 3 <= nmax <= 8 else None
+        # Leaf-ordered cell boxes: box and segment queries read a leaf's boxes directly.
+        self.d_leaf_bb = D.empty((n, 4), torch.float64) if LEAF_BBOXES and n > 0 else None
+        # The cells in visit order: box queries turn visit numbers into cells.
+        self.d_visit_cells = D.empty(n, torch.int32) if nmax >= 3 else None
+        # Per grid cell, the node where every point walk through it starts.
+        g = start_grid_size(self.n_nodes)
+        self.d_start_grid = D.empty((g, g), torch.int32) if g else None
+        t.leaf_bb = t.start_grid = None
+        t.start_grid_n = 0
+        _native.call("ct_tree_layouts", self.tree_ref, D.ptr(self.d_leaf_coords), D.ptr(self.d_leaf_bb),
+                     D.ptr(self.d_visit_cells), g, D.ptr(self.d_start_grid), st)
+        t.leaf_coords = D.ptr(self.d_leaf_coords) or None
+        t.leaf_bb = D.ptr(self.d_leaf_bb) or None
+        t.start_grid = D.ptr(self.d_start_grid) or None
+        t.start_grid_n = g
         t.parents = None
         self.d_parents = None
         if self.depth > _native.CT_MAX_DEPTH:
@@ -171,16 +170,6 @@ class CellTree2dBase:
             self.d_parents = D.empty(self.n_nodes, torch.int32)
             _native.call("ct_node_parents", self.tree_ref, D.ptr(self.d_parents), st)
             t.parents = self.d_parents.data_ptr()
-        t.start_grid = None
-        t.start_grid_n = 0
-        self.d_start_grid = None
-        g = start_grid_size(self.n_nodes)
-        if g:
-            # Per grid cell, the node where every point walk through it starts.
-            self.d_start_grid = D.empty((g, g), torch.int32)
-            _native.call("ct_start_grid", self.tree_ref, g, D.ptr(self.d_start_grid), st)
-            t.start_grid = self.d_start_grid.data_ptr()
-            t.start_grid_n = g
         t.node_boxes = None
         self.d_node_boxes = None
         if nmax >= 3:

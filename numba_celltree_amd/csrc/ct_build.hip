@@ -21,7 +21,7 @@
 // anything back (an idle level costs three empty launches), and synchronizes once.  With a
 // sequence of 11 kernels and a host synchronization for each of the 22 levels, and the node boxes
 // in one launch a level, the constructor took 5.78 ms for 999,941 cells and 1.67 ms for 20,000;
-// now 1.42 and 0.43 ms.
+// now 1.14 and 0.31 ms.
 //
 // The stable partition is the order sort_bbox_indices (:54-151) produces with its repeated
 // stable_partition.  Per node as in the reference: special case (:312-320), empty-bucket merge
@@ -79,12 +79,16 @@ struct Smalls {  // roots of the subtrees k_small builds
 
 // Read back by the host in one transfer.
 struct Header {
+  // counters that k_node_decide raises together: one 64-bit atomic instead of several on the few
+  // addresses that all nodes of a level meet at (11 ns each)
   int32_t next_id;    // nodes created by the large-node stage (and the root)
+  int32_t n_small;
+  struct {
+    int32_t active;   // large nodes
+    int32_t tiles;    // and their tiles
+  } level[2];         // per level parity
   int32_t err;        // 1: a centroid in no bucket, 2: no finite split cost
   int32_t depth;
-  int32_t n_small;
-  int32_t active[2];  // large nodes per level parity
-  int32_t tiles[2];
   int32_t n_nodes;    // of the whole tree (k_top)
   int32_t pad[3];
   Key checks[3];      // of ct_prepare_faces, passed through
@@ -289,10 +293,10 @@ __global__ void __launch_bounds__(kBlock) k_init(int n, int cells_per_leaf, int 
     h.err = 0;
     h.depth = 0;
     h.n_small = small ? 1 : 0;
-    h.active[0] = large ? 1 : 0;
-    h.active[1] = 0;
-    h.tiles[0] = large ? tiles : 0;
-    h.tiles[1] = 0;
+    h.level[0].active = large ? 1 : 0;
+    h.level[1].active = 0;
+    h.level[0].tiles = large ? tiles : 0;
+    h.level[1].tiles = 0;
     h.n_nodes = 0;
     w.group_end[0] = 1;
   }
@@ -307,11 +311,11 @@ __global__ void __launch_bounds__(kBlock) k_tile_count(int nb, int level, int pa
   Header* h = w.head;
   const int t = blockIdx.x;
   if (t == 0 && threadIdx.x == 0) {  // k_node_decide of this level fills the next level's lists
-    h->active[par ^ 1] = 0;
-    h->tiles[par ^ 1] = 0;
+    h->level[par ^ 1].active = 0;
+    h->level[par ^ 1].tiles = 0;
     w.group_end[level] = h->next_id;
   }
-  if (t >= h->tiles[par]) return;
+  if (t >= h->level[par].tiles) return;
   const Slots& cur = w.act[par];
   const int s = cur.map[t];
   const int d = cur.dim[s];
@@ -361,12 +365,13 @@ __global__ void __launch_bounds__(kDecideBlock) k_node_decide(int nb, int cells_
   __shared__ int next_slot[2], next_tile[2], next_tiles[2];
   Header* h = w.head;
   const int s = blockIdx.x;
-  if (s >= h->active[par]) return;
+  if (s >= h->level[par].active) return;
   const Slots& cur = w.act[par];
   const Slots& nxt = w.act[par ^ 1];
   const int X = cur.id[s], ptr = cur.ptr[s], size = cur.size[s], dim = cur.dim[s];
   const int att = cur.att[s], depth = cur.depth[s], tile0 = cur.tile0[s];
-  const int ntiles = (size + kTile - 1) / kTile;
+  auto tiles_of = [](int cells) { return (cells + kTile - 1) / kTile; };
+  const int ntiles = tiles_of(size);
   const int tid = threadIdx.x;
   for (int k = tid; k < 4 * nb; k += kDecideBlock) bnd[k] = (k & 1) ? 0ull : ~0ull;
   __syncthreads();
@@ -418,10 +423,7 @@ __global__ void __launch_bounds__(kDecideBlock) k_node_decide(int nb, int cells_
         nb, size, att, range_Rmin, range_Lmax, [&](int b) { return cnt[b]; },
         [&](int b) { return dval(bnd[4 * b + 2 * dim]); }, [&](int b) { return dval(bnd[4 * b + 2 * dim + 1]); });
     const int ndim = dim ? 0 : 1;
-    auto push_large = [&](int which, int id, int cptr, int csize, int catt, int cdepth, const Key (&r)[4]) {
-      const int ns = atomicAdd(&h->active[par ^ 1], 1);
-      const int nt = (csize + kTile - 1) / kTile;
-      const int t0 = atomicAdd(&h->tiles[par ^ 1], nt);
+    auto push_large = [&](int which, int ns, int t0, int id, int cptr, int csize, int catt, int cdepth, const Key (&r)[4]) {
       nxt.id[ns] = id;
       nxt.ptr[ns] = cptr;
       nxt.size[ns] = csize;
@@ -432,25 +434,45 @@ __global__ void __launch_bounds__(kDecideBlock) k_node_decide(int nb, int cells_
       for (int k = 0; k < 4; ++k) nxt.range[4 * ns + k] = r[k];
       next_slot[which] = ns;
       next_tile[which] = t0;
-      next_tiles[which] = nt;
+      next_tiles[which] = tiles_of(csize);
     };
+    // two counters that lie together, the first in the low half
+    auto raise = [](int32_t* first, int a, int b) {
+      return atomicAdd(reinterpret_cast<Key*>(first), (Key)(unsigned)a | (Key)(unsigned)b << 32);
+    };
+    int32_t* const level = &h->level[par ^ 1].active;
     if (sp.bad_cost) h->err = 2;
     if (sp.decision == kRetry) {
       w.cnodes[X].dim = ndim;
       const Key r[4] = {range[0], range[1], range[2], range[3]};
-      push_large(0, X, ptr, size, 1, depth, r);
+      const Key at = raise(level, 1, ntiles);
+      push_large(0, (int)(unsigned)at, (int)(at >> 32), X, ptr, size, 1, depth, r);
     } else if (sp.decision == kSplit) {
-      const int c = atomicAdd(&h->next_id, 2);
+      const int csizes[2] = {sp.left, size - sp.left};
+      int smalls = 0, larges = 0, tiles = 0;
+      for (int side = 0; side < 2; ++side) {
+        if (csizes[side] <= cells_per_leaf) continue;
+        if (csizes[side] <= T) {
+          ++smalls;
+        } else {
+          ++larges;
+          tiles += tiles_of(csizes[side]);
+        }
+      }
+      const Key ids = raise(&h->next_id, 2, smalls);
+      Key at = larges ? raise(level, larges, tiles) : 0;
+      const int c = (int)(unsigned)ids;
+      int small = (int)(ids >> 32);
       w.cnodes[X].Lmax = sp.Lmax;
       w.cnodes[X].Rmin = sp.Rmin;
       w.cnodes[X].child = c;
-      atomicMax(&h->depth, depth + 1);
+      if (h->depth < depth + 1) atomicMax(&h->depth, depth + 1);
       for (int side = 0; side < 2; ++side) {
-        const int id = c + side, cptr = side ? ptr + sp.left : ptr, csize = side ? size - sp.left : sp.left;
+        const int id = c + side, cptr = side ? ptr + sp.left : ptr, csize = csizes[side];
         w.cnodes[id] = ct_node{-1.0, -1.0, -1, cptr, csize, ndim};  // creation.py:27-29
         if (csize <= cells_per_leaf) continue;
         if (csize <= T) {
-          const int k = atomicAdd(&h->n_small, 1);
+          const int k = small++;
           w.small.id[k] = id;
           w.small.ptr[k] = cptr;
           w.small.size[k] = csize;
@@ -464,7 +486,8 @@ __global__ void __launch_bounds__(kDecideBlock) k_node_decide(int nb, int cells_
             const Key x = bnd[4 * b + k];  // the neutral key for an empty bucket
             r[k] = (k & 1) ? (x > r[k] ? x : r[k]) : (x < r[k] ? x : r[k]);
           }
-        push_large(side, id, cptr, csize, 0, depth + 1, r);
+        push_large(side, (int)(unsigned)at, (int)(at >> 32), id, cptr, csize, 0, depth + 1, r);
+        at += (Key)1 | (Key)(unsigned)tiles_of(csize) << 32;
       }
     }
   }
@@ -483,7 +506,7 @@ __device__ __forceinline__ int packed(Key w, int b) { return (int)((w >> (16 * (
 __global__ void __launch_bounds__(kBlock) k_tile_scatter(int nb, int par, Work w, int32_t* __restrict__ out) {
   __shared__ Key lds[kBlock / 64];
   const int t = blockIdx.x;
-  if (t >= w.head->tiles[par]) return;
+  if (t >= w.head->level[par].tiles) return;
   const Slots& cur = w.act[par];
   const int s = cur.map[t];
   const int begin = (t - cur.tile0[s]) * kTile;
@@ -859,23 +882,27 @@ __global__ void __launch_bounds__(kTopBlock) k_top(int levels, int want_boxes, c
                                                    const int32_t* __restrict__ cells) {
   const int tid = threadIdx.x, M = w.head->next_id;
   ct_node* cn = w.cnodes;
-  // leaves: one wavefront each
-  for (int x = tid >> 6; x < M; x += kTopBlock / 64) {
-    const ct_node nd = cn[x];
-    if (nd.child != -1) continue;
-    double4 u = empty_box();
-    if (want_boxes) {
-      for (int k = nd.ptr + lane_id(); k < nd.ptr + nd.size; k += 64) u = box_union(u, ld_box4(bb, cells[k]));
+  // Leaves, found 64 nodes at a time (a node at a time, 3000 nodes of 999,941 cells took 50 of the
+  // kernel's 61 us), then a wavefront each.
+  for (int x0 = tid & ~63; x0 < M; x0 += kTopBlock) {
+    const int mine = x0 + lane_id();
+    for (uint64_t todo = __ballot(mine < M && cn[mine < M ? mine : 0].child == -1); todo; todo &= todo - 1) {
+      const int x = x0 + __ffsll((unsigned long long)todo) - 1;
+      const ct_node nd = cn[x];
+      double4 u = empty_box();
+      if (want_boxes) {
+        for (int k = nd.ptr + lane_id(); k < nd.ptr + nd.size; k += 64) u = box_union(u, ld_box4(bb, cells[k]));
 #pragma unroll
-      for (int d = 32; d >= 1; d >>= 1) {
-        const double4 v = make_double4(__shfl_xor(u.x, d, 64), __shfl_xor(u.y, d, 64), __shfl_xor(u.z, d, 64),
-                                       __shfl_xor(u.w, d, 64));
-        u = box_union(u, v);
+        for (int d = 32; d >= 1; d >>= 1) {
+          const double4 v = make_double4(__shfl_xor(u.x, d, 64), __shfl_xor(u.y, d, 64), __shfl_xor(u.z, d, 64),
+                                         __shfl_xor(u.w, d, 64));
+          u = box_union(u, v);
+        }
       }
-    }
-    if (lane_id() == 0) {
-      w.icount[x] = 0;
-      if (want_boxes) w.tbox[x] = u;
+      if (lane_id() == 0) {
+        w.icount[x] = 0;
+        if (want_boxes) w.tbox[x] = u;
+      }
     }
   }
   __syncthreads();
@@ -940,9 +967,16 @@ __global__ void __launch_bounds__(kBlock) k_emit(int n_small, int n_top, Work w,
   if (boxes) boxes[w.newidx[x] + 1] = w.tbox[x];
 }
 
-int launch_small(int nb, int cells_per_leaf, int first, int want_boxes, const double* bb, const Work& w, int32_t* out,
-                 unsigned grid, hipStream_t st) {
-  if (nb <= 4) k_small<4, 1024, 512><<<grid, 512, 0, st>>>(nb, cells_per_leaf, first, want_boxes, bb, w, out);
+// A lane per cell while there are no more subtrees than CUs (about 2 n / T of them), two cells per lane
+// and two workgroups a CU above: 20,000 cells 315 instead of 344 us, 999,941 cells 1283 against 1136.
+constexpr int64_t kWideCells = 128 * 1024;
+
+int launch_small(int64_t n, int nb, int cells_per_leaf, int first, int want_boxes, const double* bb, const Work& w,
+                 int32_t* out, unsigned grid, hipStream_t st) {
+  const bool wide = n <= kWideCells;
+  if (nb <= 4 && wide) k_small<4, 1024, 1024><<<grid, 1024, 0, st>>>(nb, cells_per_leaf, first, want_boxes, bb, w, out);
+  else if (nb <= 8 && wide) k_small<8, 1024, 1024><<<grid, 1024, 0, st>>>(nb, cells_per_leaf, first, want_boxes, bb, w, out);
+  else if (nb <= 4) k_small<4, 1024, 512><<<grid, 512, 0, st>>>(nb, cells_per_leaf, first, want_boxes, bb, w, out);
   else if (nb <= 8) k_small<8, 1024, 512><<<grid, 512, 0, st>>>(nb, cells_per_leaf, first, want_boxes, bb, w, out);
   else if (nb <= 16) k_small<16, 512, 256><<<grid, 256, 0, st>>>(nb, cells_per_leaf, first, want_boxes, bb, w, out);
   else if (nb <= 32) k_small<32, 256, 256><<<grid, 256, 0, st>>>(nb, cells_per_leaf, first, want_boxes, bb, w, out);
@@ -1033,14 +1067,14 @@ int ct_build_plan(const double* bb_coords, int64_t n_elements, int32_t n_buckets
       CT_LAUNCH_CHECK();
     }
     const unsigned small_grid = (unsigned)std::min((int64_t)2048, (int64_t)n / 2 + 1);
-    rc = launch_small(nb, cpl, done_small, want_boxes, bb_coords, w, bb_indices_out, small_grid, st);
+    rc = launch_small(n, nb, cpl, done_small, want_boxes, bb_coords, w, bb_indices_out, small_grid, st);
     if (rc) return rc;
     k_top<<<1, kTopBlock, 0, st>>>(levels, want_boxes, bb_coords, w, bb_indices_out);
     CT_LAUNCH_CHECK();
     CT_HIP(hipMemcpyAsync(&h, w.head, sizeof(h), hipMemcpyDeviceToHost, st));
     CT_HIP(hipStreamSynchronize(st));
     done_small = h.n_small;
-    if (h.err != 0 || h.active[levels & 1] == 0) break;
+    if (h.err != 0 || h.level[levels & 1].active == 0) break;
     // Children are strictly smaller than their parent and a node retries once, so the loop
     // ends within 2 * n_elements levels (the length of group_end); the guard only protects it.
     batch = std::min(std::max(2 * batch, 8), 64);

@@ -140,17 +140,6 @@ __global__ void __launch_bounds__(kBlock) k_place_rows(int64_t rows, const int64
   if (xy) xy[o] = sub_xy[r];
 }
 
-// The cell of every visit number.
-__global__ void __launch_bounds__(kBlock) k_visit_cells(const ct_node* __restrict__ nodes, int64_t n_nodes,
-                                                        const int32_t* __restrict__ bb_indices, int n,
-                                                        int32_t* __restrict__ out) {
-  const int64_t x = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (x >= n_nodes) return;
-  const ct_node nd = nodes[x];
-  if (nd.child != -1) return;
-  for (int j = 0; j < nd.size; ++j) out[n - nd.ptr - nd.size + j] = bb_indices[nd.ptr + j];
-}
-
 GatherParams params(const ct_tree* tree, int64_t n, const int32_t* visit, int kind) {
   GatherParams p{};
   p.visit = visit;
@@ -244,14 +233,6 @@ int64_t ct_gather_pool_rows(int32_t kind, int64_t n) {
   if (kind == kBoxes) return std::max((int64_t)256 * n, (int64_t)kBoxHits);
   const int64_t per_wave = std::min((int64_t)kMaxPerWave, std::max((int64_t)1, n / 4096));
   return std::max((int64_t)64 * n, ((n + per_wave - 1) / per_wave * 5 / 4 + kPools) * kRowChunk);
-}
-
-int ct_visit_cells(const ct_tree* tree, int32_t* out, void* stream) {
-  CT_REQUIRE(tree && tree->nodes && tree->bb_indices && out, "bad arguments");
-  k_visit_cells<<<grid_for(tree->n_nodes), kBlock, 0, as_stream(stream)>>>(tree->nodes, tree->n_nodes, tree->bb_indices,
-                                                                         (int)tree->n_elements, out);
-  CT_LAUNCH_CHECK();
-  return CT_OK;
 }
 
 int ct_gather_count(const ct_tree* tree, int32_t kind, const double* queries, int64_t n, const int32_t* order,

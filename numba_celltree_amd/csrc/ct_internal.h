@@ -198,13 +198,6 @@ __device__ __forceinline__ bool box_contained(const Box& a, const Box& b) {
   return a.xmin >= b.xmin && a.xmax <= b.xmax && a.ymin >= b.ymin && a.ymax <= b.ymax;
 }
 
-// geometry_utils.py:72-79 polygon_length: the first fill value at position >= 3.
-__device__ __forceinline__ int poly_len(const int32_t* __restrict__ face, int nmax) {
-  for (int i = 3; i < nmax; ++i)
-    if (face[i] == kFill) return i;
-  return nmax;
-}
-
 // Loads face `f` (row of width nmax) into registers; returns its length.
 template <int MAXV>
 __device__ __forceinline__ int load_poly(const int32_t* __restrict__ faces, int nmax, int64_t f,

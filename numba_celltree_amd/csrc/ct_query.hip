@@ -507,10 +507,8 @@ int query_order(int kind, const double* q, int64_t n, const double* bbox, const 
   return CT_OK;
 }
 
-// Start-node grid (see ct_start_grid): one lane per grid cell.
-__global__ void __launch_bounds__(kBlock) k_start_grid(TreeView t, int n, int32_t* __restrict__ out) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= (int64_t)n * n) return;
+// Start-node grid (see ct_start_grid): grid cell k.
+__device__ __forceinline__ int start_cell(const TreeView& t, int n, int64_t k) {
   const int gx = (int)(k % n), gy = (int)(k / n);
   double x0, x1, y0, y1;
   grid_span(t.bbox.xmin, t.bbox.xmax, n, gx, &x0, &x1);
@@ -525,30 +523,81 @@ __global__ void __launch_bounds__(kBlock) k_start_grid(TreeView t, int n, int32_
     else if (lo > nd.Lmax && lo >= nd.Rmin) node = nd.child + 1;      // only the right child, always
     else break;
   }
-  out[k] = node;
+  return node;
 }
 
-// Leaf-ordered cell bboxes (see ct_pack_leaf_bboxes).
-__global__ void __launch_bounds__(kBlock) k_pack_leaf_bb(TreeView t, double* __restrict__ out) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= t.n_elements) return;
-  const int c = t.bb_indices[k];
-  reinterpret_cast<double4*>(out)[k] = reinterpret_cast<const double4*>(t.bb)[c];
-}
-
-// Packed leaf coordinates (see ct_pack_leaf_coords).
-__global__ void __launch_bounds__(kBlock) k_pack_leaf(TreeView t, double* __restrict__ out) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= t.n_elements) return;
-  const int c = t.bb_indices[k];
+// Row k of the packed leaf coordinates (ct_pack_leaf_coords), rows of at most MAXV vertices: the
+// indices and then the vertices all in flight.  Bound by the rows' and vertices' scattered lines: 1e6
+// cells with the boxes, visit numbers and start grid in the same launch 114 us (four launches, the
+// vertices one after the other: 181).
+template <int MAXV>
+__device__ __forceinline__ void pack_row(const TreeView& t, int64_t k, int c, double* __restrict__ out) {
   const int32_t* row = t.elements + (int64_t)c * t.nmax;
-  const int len = poly_len(row, t.nmax);
-  double2* dst = reinterpret_cast<double2*>(out) + k * t.nmax;
-  P2 v = {0.0, 0.0};
-  for (int i = 0; i < t.nmax; ++i) {
-    if (i < len) v = ld_vertex(t.vertices, row[i]);
-    dst[i] = make_double2(v.x, v.y);  // slots past the polygon repeat its last vertex
+  const int n = t.nmax;
+  int idx[MAXV], len = n;
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i) idx[i] = row[i < n ? i : n - 1];
+#pragma unroll
+  for (int i = MAXV - 1; i >= 3; --i)
+    if (i < n && idx[i] == kFill) len = i;
+  // Slots past the polygon repeat its last vertex; every load has a valid index, so none waits for
+  // a branch.
+  P2 v[MAXV];
+#pragma unroll
+  for (int i = 1; i < MAXV; ++i) idx[i] = i < len ? idx[i] : idx[i - 1];
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i) v[i] = ld_vertex(t.vertices, idx[i]);
+  double2* dst = reinterpret_cast<double2*>(out) + k * n;
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i)
+    if (i < n) dst[i] = make_double2(v[i].x, v[i].y);
+}
+
+// What queries read beside the nodes (ct_tree_layouts), one launch: workgroups [0, leaves) the rows and
+// boxes in leaf order, [leaves, leaves + nodes) the cells by visit number, then the start grid.
+struct Layouts {
+  double* coords;
+  double* boxes;
+  int32_t* visit;
+  int32_t* grid;
+  int grid_n;
+  int64_t n_nodes;
+  unsigned leaf_blocks, node_blocks;
+};
+
+template <int MAXV>
+__global__ void __launch_bounds__(kBlock) k_layouts(TreeView t, Layouts l) {
+  unsigned b = blockIdx.x;
+  if (b < l.leaf_blocks) {
+    const int64_t k = (int64_t)b * kBlock + threadIdx.x;
+    if (k >= t.n_elements) return;
+    const int c = t.bb_indices[k];
+    if (l.boxes) reinterpret_cast<double4*>(l.boxes)[k] = reinterpret_cast<const double4*>(t.bb)[c];
+    if (l.coords) pack_row<MAXV>(t, k, c, l.coords);
+    return;
   }
+  b -= l.leaf_blocks;
+  if (b < l.node_blocks) {
+    const int64_t x = (int64_t)b * kBlock + threadIdx.x;
+    if (x < l.n_nodes) put_visits(t, t.nodes[x], l.visit);
+    return;
+  }
+  b -= l.node_blocks;
+  const int64_t k = (int64_t)b * kBlock + threadIdx.x;
+  if (k < (int64_t)l.grid_n * l.grid_n) l.grid[k] = start_cell(t, l.grid_n, k);
+}
+
+int launch_layouts(const TreeView& t, int64_t n_nodes, double* coords, double* boxes, int32_t* visit, int32_t* grid,
+                   int grid_n, hipStream_t st) {
+  Layouts l{coords, boxes, visit, grid, grid_n, n_nodes, 0, 0};
+  if (coords || boxes) l.leaf_blocks = grid_for(t.n_elements);
+  if (visit) l.node_blocks = grid_for(n_nodes);
+  const unsigned blocks = l.leaf_blocks + l.node_blocks + (grid ? grid_for((int64_t)grid_n * grid_n) : 0);
+  if (blocks == 0) return CT_OK;
+  if (t.nmax <= 4) k_layouts<4><<<blocks, kBlock, 0, st>>>(t, l);
+  else k_layouts<8><<<blocks, kBlock, 0, st>>>(t, l);
+  CT_LAUNCH_CHECK();
+  return CT_OK;
 }
 
 // ----------------------------------------------------------------- boxes
@@ -1189,9 +1238,7 @@ int ct_pack_leaf_coords(const ct_tree* tree, double* out, void* stream) {
   int rc = check_tree(tree);
   if (rc) return rc;
   CT_REQUIRE(tree->n_max_vert >= 3 && tree->n_max_vert <= 8 && out, "n_max_vert must be in [3, 8]");
-  k_pack_leaf<<<grid_for(tree->n_elements), kBlock, 0, as_stream(stream)>>>(view(tree), out);
-  CT_LAUNCH_CHECK();
-  return CT_OK;
+  return launch_layouts(view(tree), 0, out, nullptr, nullptr, nullptr, 0, as_stream(stream));
 }
 
 int ct_pack_leaf_bboxes(const ct_tree* tree, double* out, void* stream) {
@@ -1199,9 +1246,7 @@ int ct_pack_leaf_bboxes(const ct_tree* tree, double* out, void* stream) {
   if (rc) return rc;
   CT_REQUIRE(out != nullptr, "null output");
   if (tree->n_elements == 0) return CT_OK;
-  k_pack_leaf_bb<<<grid_for(tree->n_elements), kBlock, 0, as_stream(stream)>>>(view(tree), out);
-  CT_LAUNCH_CHECK();
-  return CT_OK;
+  return launch_layouts(view(tree), 0, nullptr, out, nullptr, nullptr, 0, as_stream(stream));
 }
 
 int ct_start_grid(const ct_tree* tree, int32_t n, int32_t* out, void* stream) {
@@ -1210,9 +1255,24 @@ int ct_start_grid(const ct_tree* tree, int32_t n, int32_t* out, void* stream) {
   CT_REQUIRE(n >= 1 && n <= 4096 && out != nullptr, "grid size must be in [1, 4096]");
   ct_tree t = *tree;
   t.start_grid = nullptr;
-  k_start_grid<<<grid_for((int64_t)n * n), kBlock, 0, as_stream(stream)>>>(view(t), n, out);
-  CT_LAUNCH_CHECK();
-  return CT_OK;
+  return launch_layouts(view(t), 0, nullptr, nullptr, nullptr, out, n, as_stream(stream));
+}
+
+int ct_visit_cells(const ct_tree* tree, int32_t* out, void* stream) {
+  CT_REQUIRE(tree && tree->nodes && tree->bb_indices && out, "bad arguments");
+  return launch_layouts(view(tree), tree->n_nodes, nullptr, nullptr, out, nullptr, 0, as_stream(stream));
+}
+
+int ct_tree_layouts(const ct_tree* tree, double* leaf_coords, double* leaf_bb, int32_t* visit_cells, int32_t grid_n,
+                    int32_t* grid, void* stream) {
+  int rc = check_tree(tree);
+  if (rc) return rc;
+  CT_REQUIRE(!leaf_coords || (tree->n_max_vert >= 3 && tree->n_max_vert <= 8), "n_max_vert must be in [3, 8]");
+  CT_REQUIRE(!grid || (grid_n >= 1 && grid_n <= 4096), "grid size must be in [1, 4096]");
+  ct_tree t = *tree;
+  t.start_grid = nullptr;
+  return launch_layouts(view(t), tree->n_nodes, tree->n_elements ? leaf_coords : nullptr,
+                        tree->n_elements ? leaf_bb : nullptr, visit_cells, grid, grid ? grid_n : 0, as_stream(stream));
 }
 
 size_t ct_order_workspace_bytes(int64_t n) {

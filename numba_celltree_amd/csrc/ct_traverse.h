@@ -113,6 +113,13 @@ __device__ __forceinline__ int64_t query_index(const int32_t* __restrict__ order
   return order ? (int64_t)order[i] : i;
 }
 
+// A leaf's cells to their visit numbers (ct_gather.h): the places at which a walk that enters every
+// node meets them.
+__device__ __forceinline__ void put_visits(const TreeView& t, const ct_node& nd, int32_t* __restrict__ out) {
+  if (nd.child != -1) return;
+  for (int j = 0; j < nd.size; ++j) out[t.n_elements - nd.ptr - nd.size + j] = t.bb_indices[nd.ptr + j];
+}
+
 // Processing order of a query batch: lane i answers query order[i] (i when `order` is null).
 // `sorted`, when not null, holds the queries already in that order (sorted[i] =
 // queries[order[i]]), so lane i reads its query contiguously instead of gathering it.
