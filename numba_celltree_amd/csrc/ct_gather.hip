@@ -50,23 +50,25 @@ k_gather(TreeView t, const double* __restrict__ qs, const int32_t* __restrict__ 
   gather_block<KIND, MAXV>(t, qs, order, i0, (int)min((int64_t)p.per_wave, n - i0), p, pool, rows, counts, starts, tail);
 }
 
-// Output rows from the pool, 64 queries per wavefront in query order: their rows are one run of
+// Output rows from the pool, `per_wave` queries per wavefront (a power of two, at most 64; fewer when
+// there are few: 2e3 segments in 32 wavefronts took 18 us, a query each 5) in query order: their rows are one run of
 // the output, written 64 rows per step (row g's owner by a binary search over the wavefront's
 // prefix), so every output line is written whole.  kAhead steps run together: a row is a chain of two
 // or three loads.  Queries whose rows end past `capacity` are left out.
 constexpr int kAhead = 4;
+constexpr int64_t kRowWaves = 4096;
 
 template <bool SEGMENTS>
-__global__ void __launch_bounds__(kBlock) k_pool_rows(int64_t n, const int64_t* __restrict__ offsets,
+__global__ void __launch_bounds__(kBlock) k_pool_rows(int64_t n, int per_wave, const int64_t* __restrict__ offsets,
                                                       const int64_t* __restrict__ starts, Pool pool,
                                                       int64_t capacity, int64_t* __restrict__ ii, int64_t* __restrict__ jj,
                                                       double4* __restrict__ xy) {
   const int lane = lane_id();
-  const int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  const int64_t q0 = q - lane;
+  const int64_t q0 = ((int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * per_wave;
+  const int64_t q = q0 + lane;
   long long o = 0, s = 0;
   int m = 0;
-  if (q < n) {
+  if (lane < per_wave && q < n) {
     o = offsets[q];
     s = starts[q];
     const long long end = offsets[q + 1];
@@ -210,11 +212,14 @@ int launch_pool_rows(bool segments, int64_t n, const int64_t* offsets, const int
                      double* xy, hipStream_t st) {
   const Pool pool{const_cast<int32_t*>(pool_cell), reinterpret_cast<double4*>(const_cast<double*>(pool_xy)),
                   const_cast<int32_t*>(pool_src), 0, 1, 0};
-  const unsigned grid = grid_for(n);
+  int per_wave = 64;
+  while (per_wave > 1 && n < (int64_t)per_wave * kRowWaves) per_wave >>= 1;
+  const int64_t per_block = (int64_t)per_wave * (kBlock / 64);
+  const unsigned grid = (unsigned)((n + per_block - 1) / per_block);
   if (segments)
-    k_pool_rows<true><<<grid, kBlock, 0, st>>>(n, offsets, starts, pool, capacity, ii, jj, reinterpret_cast<double4*>(xy));
+    k_pool_rows<true><<<grid, kBlock, 0, st>>>(n, per_wave, offsets, starts, pool, capacity, ii, jj, reinterpret_cast<double4*>(xy));
   else
-    k_pool_rows<false><<<grid, kBlock, 0, st>>>(n, offsets, starts, pool, capacity, ii, jj, nullptr);
+    k_pool_rows<false><<<grid, kBlock, 0, st>>>(n, per_wave, offsets, starts, pool, capacity, ii, jj, nullptr);
   CT_LAUNCH_CHECK();
   return CT_OK;
 }
