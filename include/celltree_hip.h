@@ -651,7 +651,7 @@ typedef struct ct_batch {
   const int64_t* query_offsets; /* (n_trees + 1): tree m owns queries [off[m], off[m + 1]) */
   const ct_batch_tile* tiles;   /* (n_tiles), grouped by queue */
   const int32_t* queue_starts;  /* (n_queues + 1): queue r owns tiles [s[r], s[r + 1]) */
-  int32_t* counters;            /* (n_queues) scratch */
+  int32_t* counters;            /* (n_queues * max(counter_stride, 1)) scratch */
   int64_t n_tiles;
   int32_t n_trees;
   int32_t n_queues;             /* 1 .. 64; workgroup b starts on queue b % n_queues */
@@ -660,7 +660,8 @@ typedef struct ct_batch {
   int32_t stack;                /* traversal stack class, >= max_depth: 16, 24, 32, 48, 64, 128, 256 */
   int32_t n_workgroups;         /* persistent grid size */
   int32_t block;                /* workgroup size: 64, 128 or 256 */
-  int32_t reserved;
+  int32_t counter_stride;       /* int32 from one queue's counter to the next (0: 1); 32 puts each on
+                                   a line of its own */
 } ct_batch;
 
 /* locate_points for every tree's queries: out[q] = the first containing cell of q's tree

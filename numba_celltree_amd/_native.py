@@ -84,7 +84,7 @@ class CtBatch(ctypes.Structure):
         ("stack", ctypes.c_int32),
         ("n_workgroups", ctypes.c_int32),
         ("block", ctypes.c_int32),
-        ("reserved", ctypes.c_int32),
+        ("counter_stride", ctypes.c_int32),
     ]
 
 

@@ -61,6 +61,9 @@ def _cu_count() -> int:
     return int(torch.cuda.get_device_properties(D.device()).multi_processor_count)
 
 
+COUNTER_STRIDE = 32  # a 128-byte line for every queue's counter
+
+
 class TreeBatch:
     """Device descriptors of many face trees (``CellTree2d``, 3 to 8 vertices per face)."""
 
@@ -153,7 +156,7 @@ class BatchPlan:
             torch.zeros(16, dtype=torch.uint8, device=dev)
         self.d_qoff = torch.from_numpy(qoff).to(dev)
         self.d_qstart = torch.tensor(qstart, dtype=torch.int32, device=dev)
-        self.d_counters = torch.zeros(nq, dtype=torch.int32, device=dev)
+        self.d_counters = torch.zeros(nq * COUNTER_STRIDE, dtype=torch.int32, device=dev)
         s = _native.CtBatch()
         s.trees = batch.d_trees.data_ptr()
         s.tolerances = batch.d_tols.data_ptr()
@@ -164,6 +167,7 @@ class BatchPlan:
         s.n_tiles = self.n_tiles
         s.n_trees = batch.n_trees
         s.n_queues = nq
+        s.counter_stride = COUNTER_STRIDE
         s.max_n_vert = batch.max_n_vert
         s.max_depth = batch.max_depth
         s.stack = stack
