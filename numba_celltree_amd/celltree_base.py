@@ -507,6 +507,10 @@ class CellTree2dBase:
         total, *words, left = row[n: n + 10].tolist()
         if prep is not None:
             prep.check(words)
+        if 2 * left >= n:
+            # Mostly large queries: all of them as subqueries, whose rows need no second place.
+            _, ii, jj, xy = self._split_rows(kind, queries, self._order(1 if kind == 1 else 2, queries)[0])
+            return (ii, jj) if kind == 1 else (ii, jj, xy)
         if left:
             # Queries with more rows than a wavefront's lists hold, as subqueries; their counts join.
             idx = torch.nonzero(starts < 0)[:, 0]

@@ -424,6 +424,7 @@ int ct_batch_gather_edges(const ct_batch* batch, const double* segments, int64_t
     GatherParams p{};
     p.per_wave = kMaxPerWave;
     p.group = kSegGroup;
+    p.leave = 2 * kSegHits;  // one lane walks what is left: try first
     p.depth1 = batch->max_depth + 1;
     p.stack = kStack + p.depth1;
     Pool pool{pool_cell, reinterpret_cast<double4*>(pool_xy), pool_src, 0, 1, 0};

@@ -52,9 +52,6 @@ constexpr int kCands = 128;  // 63 left over + 64
 // triangles: 0.16 ms, and 0.60 with 768, most of it for the few then left to the subqueries).
 constexpr int kBoxHits = 1024, kBoxGroupHits = 768, kBoxGroup = 480;
 constexpr int kSegHits = 320, kSegGroup = 280;
-// Expected hits beyond which a query is left without a walk that would most likely be in vain.
-constexpr int kLeaveTimes = 2;
-
 // Counters for pool allocation, each on its own 128-byte line: one counter for all wavefronts
 // would serialize them (about 11 ns per atomic on one address).
 constexpr int kPools = 64, kCounterStride = 16;
@@ -103,6 +100,7 @@ struct GatherParams {
   double reach;          // largest coordinate magnitude of the tree's bbox
   int per_wave;          // positions per wavefront
   int group;             // expected hits of the queries walked together
+  int leave;             // expected hits beyond which a query is left without a walk likely in vain
   int stack;             // stack entries
   int depth1;            // tree depth + 1
 
@@ -311,7 +309,7 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
     }
     if (in) {
       weight = expected<KIND>(rec, p.cell);
-      big = weight > kLeaveTimes * kHits;
+      big = weight > p.leave;
       start = big ? -1 : 0;
       while (start >= 0) {
         const NodeLd nd = ld_node(t.nodes, start);

@@ -153,6 +153,9 @@ GatherParams params(const ct_tree* tree, int64_t n, const int32_t* visit, int ki
   p.depth1 = tree->depth + 1;
   p.stack = kStack + p.depth1;
   p.group = kind == kBoxes ? kBoxGroup : kSegGroup;
+  // The subqueries take what is left: a walk in vain costs more than leaving a query that would have
+  // fitted (3e5 boxes of 1317 hits: 16.9 ms with twice the list's length, 10.0 without such walks).
+  p.leave = kind == kBoxes ? kBoxHits : kSegHits;
   return p;
 }
 
