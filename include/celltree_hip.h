@@ -171,6 +171,12 @@ int ct_build(const double* bb_coords, int64_t n_elements, int32_t n_buckets,
 int ct_check_tree(const ct_node* nodes, int64_t n_nodes, const int32_t* bb_indices, const int32_t* elements,
                   int64_t n_elements, int32_t n_max_vert, int64_t n_vertices, int32_t allow_fill, int32_t* depth);
 
+/* Host check, no reference counterpart: *in_order = 1 when the leaves, met left child first, hold the
+ * positions 0, 1, ... n_elements - 1 of bb_indices one after the other, as every built tree's do
+ * (creation.py:365-379).  ct_gather_count, ct_batch_gather_edges and ct_visit_cells number cells by
+ * their leaf's position and need that; the other queries walk any tree that ct_check_tree accepts. */
+int ct_leaves_in_order(const ct_node* nodes, int64_t n_nodes, int64_t n_elements, int32_t* in_order);
+
 /* query.py:568-622 collect_node_bounds -> out (n_nodes, 4); bbox is a HOST array of 4;
  * parent_scratch: device int32 array of n_nodes. */
 int ct_collect_node_bounds(const ct_node* nodes, int64_t n_nodes, const double* bbox,
@@ -397,7 +403,8 @@ int ct_sort_staged_rows(const int64_t* offsets, const int64_t* query_start, cons
                         int64_t* ii, int64_t* jj, double* xy, void* stream);
 
 /* Box and segment queries by wavefronts, a few queries each (kind 1 boxes, 2 segment-face, 3
- * segment-edge; trees of depth <= CT_MAX_DEPTH), without subqueries.  ct_gather_count writes
+ * segment-edge; trees of depth <= CT_MAX_DEPTH with their leaves in order, ct_leaves_in_order),
+ * without subqueries.  ct_gather_count writes
  * counts[q] and starts[q] and keeps the rows in the caller's pool of pool_rows entries (pool_cell;
  * segments also pool_xy, 4 doubles each, and pool_src); ct_gather_pool_rows suggests a size.
  * starts[q] < 0: q is left to the caller (more rows than a wavefront's lists hold, or no room in the
@@ -695,7 +702,7 @@ int ct_batch_sort_intersections(const double* segments, int64_t n_segments, cons
                                 const int64_t* ii, const int64_t* jj, const double* xy, int64_t capacity,
                                 int32_t n_workgroups, int64_t* jj_out, double* xy_out, void* stream);
 
-/* intersect_edges for every tree's segments by wavefront walks (as ct_gather_count), in two calls with
+/* intersect_edges for every tree's segments by wavefront walks (as ct_gather_count, on the same trees), in two calls with
  * no host synchronization between them, so the sequence can be captured.  `tile`: the largest
  * tile's queries, a multiple of 64.  ct_batch_gather_edges writes counts[q] and starts[q], and keeps
  * the rows in the pool of pool_rows entries (0, or a tree of 2^26 nodes or cells or more in the batch:

@@ -173,6 +173,7 @@ SIGNATURES = {
     "ct_locate_points_ordered": (ctypes.c_int, [_TP, _P, _I64, _F64, _P, _SZ, _P, _P]),
     "ct_locate_points_in_order": (ctypes.c_int, [_TP, _P, _I64, _P, _P, _F64, _P, _P]),
     "ct_check_tree": (ctypes.c_int, [_P, _I64, _P, _P, _I64, _I32, _I64, _I32, _P]),
+    "ct_leaves_in_order": (ctypes.c_int, [_P, _I64, _I64, ctypes.POINTER(_I32)]),
     "ct_node_parents": (ctypes.c_int, [_TP, _P, _P]),
     "ct_barycentric_triangle_backward_ordered": (ctypes.c_int, [_P, _P, _P, _I64, _P, _I32, _P, _P, _P, _P, _P]),
     "ct_barycentric_wachspress_backward_ordered": (ctypes.c_int, [_P, _P, _P, _I64, _P, _I32, _P, _F64, _P, _P, _P, _P]),

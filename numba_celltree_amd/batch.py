@@ -93,7 +93,8 @@ class TreeBatch:
         self.n_cells = np.array([int(t.d_elements.shape[0]) for t in trees])
         self.n_cu = _cu_count()
         # trees the wavefront walks take (the others' segments are walked by one lane each)
-        self.gathers = all(max(int(t.n_nodes), int(t.d_elements.shape[0])) < t.GATHER_MAX_RECORDS for t in trees)
+        self.gathers = all(t.in_order and max(int(t.n_nodes), int(t.d_elements.shape[0])) < t.GATHER_MAX_RECORDS
+                           for t in trees)
 
     # --------------------------------------------------------------- planning
     def plan(self, counts: Sequence[int], config: BatchConfig, weight: float = 1.0) -> "BatchPlan":

@@ -102,11 +102,12 @@ class CellTree2dBase:
 
     def _adopt(self, vertices: torch.Tensor, elements: torch.Tensor, bb_coords: torch.Tensor,
                nodes_raw: torch.Tensor, bb_indices: torch.Tensor, n_nodes: int, depth: int,
-               n_buckets: int, cells_per_leaf: int, built=None) -> None:
+               n_buckets: int, cells_per_leaf: int, built=None, in_order: bool = True) -> None:
         """Takes a built (or imported) tree's device arrays and derives the rest: the bbox
         statistics, the ct_tree descriptor and the device-only layouts.  ``built``: the bbox
         distances, the bbox statistics and the node boxes (None: not wanted) that a build has
-        already; an imported tree's are derived here."""
+        already; an imported tree's are derived here.  ``in_order``: treeio.leaves_in_order, which
+        holds for every built tree."""
         n = int(elements.shape[0])
         st = D.stream()
         if built is not None:
@@ -119,6 +120,7 @@ class CellTree2dBase:
 
         self.n_buckets = n_buckets
         self.cells_per_leaf = cells_per_leaf
+        self.in_order = in_order
         self.d_vertices = vertices
         self.d_elements = elements
         self.d_bb_coords = bb_coords
@@ -151,7 +153,7 @@ class CellTree2dBase:
         # Leaf-ordered cell boxes: box and segment queries read a leaf's boxes directly.
         self.d_leaf_bb = D.empty((n, 4), torch.float64) if LEAF_BBOXES and n > 0 else None
         # The cells in visit order: box queries turn visit numbers into cells.
-        self.d_visit_cells = D.empty(n, torch.int32) if nmax >= 3 else None
+        self.d_visit_cells = D.empty(n, torch.int32) if nmax >= 3 and in_order else None
         # Per grid cell, the node where every point walk through it starts.
         g = start_grid_size(self.n_nodes)
         self.d_start_grid = D.empty((g, g), torch.int32) if g else None
@@ -261,7 +263,7 @@ class CellTree2dBase:
         d_nodes = D.to_dev(a["nodes"].view(np.uint8), torch.uint8)
         d_bb_indices = D.to_dev(a["bb_indices"], torch.int32)
         self._adopt(d_vertices, d_elements, d_bb, d_nodes, d_bb_indices, len(a["nodes"]), a["depth"],
-                    a["n_buckets"], a["cells_per_leaf"])
+                    a["n_buckets"], a["cells_per_leaf"], in_order=a["in_order"])
 
     def save(self, file) -> None:
         """Writes the tree to ``file`` (a path or binary file object) in the compact file form
@@ -463,9 +465,9 @@ class CellTree2dBase:
 
     def _gathers(self, n: int) -> bool:
         """Whether a batch of n box or segment queries goes through ct_gather_*: every batch on a
-        tree the stack walks take and 32-bit offsets address, unless splitting is turned off
-        (SPLIT_MAX_PARTS <= 1: whole walks)."""
-        return (n > 0 and self.depth <= _native.CT_MAX_DEPTH and int(self.SPLIT_MAX_PARTS) > 1
+        tree the stack walks take, 32-bit offsets address and whose leaves lie in order (an imported
+        tree's may not), unless splitting is turned off (SPLIT_MAX_PARTS <= 1: whole walks)."""
+        return (n > 0 and self.in_order and self.depth <= _native.CT_MAX_DEPTH and int(self.SPLIT_MAX_PARTS) > 1
                 and max(self.n_nodes, int(self.d_elements.shape[0])) < self.GATHER_MAX_RECORDS)
 
     GATHER_MAX_RECORDS = 1 << 26

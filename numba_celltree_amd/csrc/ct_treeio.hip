@@ -6,7 +6,9 @@
 // arrays describe a tree the kernels can walk: every child link points forwards and inside
 // the node array, every node but the root has exactly one parent, every node's cell range
 // lies in [0, n), bb_indices is a permutation of [0, n), and every element index addresses a
-// vertex (faces: -1 padding allowed past the first three entries).
+// vertex (faces: -1 padding allowed past the first three entries).  Leaf ranges may overlap, leave
+// cells out or lie in any order: ct_leaves_in_order tells the trees whose leaves lie as a builder
+// lays them out from the others.
 #include <cstdint>
 #include <vector>
 
@@ -85,6 +87,32 @@ int ct_check_tree(const ct_node* nodes, int64_t n_nodes, const int32_t* bb_indic
     }
   }
   *depth = deepest;
+  return CT_OK;
+}
+
+int ct_leaves_in_order(const ct_node* nodes, int64_t n_nodes, int64_t n_elements, int32_t* in_order) {
+  CT_REQUIRE(nodes && in_order, "null pointer");
+  CT_REQUIRE(n_nodes >= 1 && n_nodes < ((int64_t)1 << 31), "n_nodes must be in [1, 2**31)");
+  *in_order = 0;
+  int64_t next = 0;                       // where the next leaf's cells have to begin
+  std::vector<int32_t> stack(1, 0);
+  while (!stack.empty()) {
+    const int32_t i = stack.back();
+    stack.pop_back();
+    const ct_node& nd = nodes[i];
+    if (nd.child == -1) {
+      if (nd.size < 0 || nd.ptr != next) return CT_OK;
+      next += nd.size;
+      continue;
+    }
+    if (nd.child <= i || (int64_t)nd.child + 1 >= n_nodes) {
+      ::ct::set_error("invalid tree: node %d's child link %d points backwards or past the last node", i, nd.child);
+      return CT_ERR_ARG;
+    }
+    stack.push_back(nd.child + 1);
+    stack.push_back(nd.child);
+  }
+  *in_order = next == n_elements ? 1 : 0;
   return CT_OK;
 }
 

@@ -84,6 +84,21 @@ def check_tree(nodes: np.ndarray, bb_indices: np.ndarray, elements: np.ndarray, 
     return int(depth.value)
 
 
+def leaves_in_order(nodes: np.ndarray, n_elements: int) -> bool:
+    """Whether the leaves of a checked tree (``nodes`` NODE_RECORD), left child first, hold the
+    positions 0, 1, ... of bb_indices one after the other, as a builder lays them out
+    (creation.py:365-379).  Trees that do not are valid; the queries that number cells by their
+    leaf's position leave them to the others."""
+    import ctypes
+
+    from numba_celltree_amd import _native
+
+    out = ctypes.c_int32(0)
+    _native.call("ct_leaves_in_order", nodes.ctypes.data_as(ctypes.c_void_p), len(nodes), int(n_elements),
+                 ctypes.byref(out))
+    return bool(out.value)
+
+
 def _to_int32(a: np.ndarray, name: str) -> np.ndarray:
     if a.dtype != np.int32:
         lo, hi = (int(a.min()), int(a.max())) if a.size else (0, 0)
@@ -102,7 +117,7 @@ def _int_array(x, name: str) -> np.ndarray:
 def validate(arrays: Dict[str, np.ndarray]) -> Dict[str, np.ndarray]:
     """Checks an exported tree (either host form) and returns it in the compact form:
     vertices float64, elements int32, nodes NODE_RECORD, bb_indices int32, bb_coords (float64
-    or None), n_buckets, cells_per_leaf, kind and depth.  Raises ValueError."""
+    or None), n_buckets, cells_per_leaf, kind, depth and in_order (leaves_in_order).  Raises ValueError."""
     missing = {"vertices", "elements", "nodes", "bb_indices", "n_buckets", "cells_per_leaf", "kind"} - set(arrays)
     if missing:
         raise ValueError(f"tree arrays lack {sorted(missing)}")
@@ -154,6 +169,7 @@ def validate(arrays: Dict[str, np.ndarray]) -> Dict[str, np.ndarray]:
     return {
         "vertices": vertices, "elements": elements32, "nodes": nodes, "bb_indices": bb32, "bb_coords": bb_coords,
         "n_buckets": n_buckets, "cells_per_leaf": cells_per_leaf, "kind": kind, "depth": depth,
+        "in_order": leaves_in_order(nodes, n),
     }
 
 
