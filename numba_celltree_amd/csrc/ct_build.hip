@@ -877,6 +877,7 @@ __global__ void __launch_bounds__(THREADS) k_small(int nb, int cells_per_leaf, i
 // The large-node stage's nodes: internal nodes per subtree and tight boxes bottom-up, DFS ranks
 // top-down, by creation level.  There are about 2 n / T of them, so one workgroup does it.
 constexpr int kTopBlock = 1024;
+constexpr int kTopLevels = 64;  // batches of levels that end by here run k_top before they are read back
 
 __global__ void __launch_bounds__(kTopBlock) k_top(int levels, int want_boxes, const double* __restrict__ bb, Work w,
                                                    const int32_t* __restrict__ cells) {
@@ -1047,6 +1048,11 @@ int ct_build_plan(const double* bb_coords, int64_t n_elements, int32_t n_buckets
   CT_LAUNCH_CHECK();
 
   Header h{};
+  auto read_header = [&]() -> int {
+    CT_HIP(hipMemcpyAsync(&h, w.head, sizeof(h), hipMemcpyDeviceToHost, st));
+    CT_HIP(hipStreamSynchronize(st));
+    return CT_OK;
+  };
   int levels = 0, done_small = 0;
   // levels of a balanced tree above the subtrees, plus two; then more, in growing batches
   int batch = 0;
@@ -1069,12 +1075,25 @@ int ct_build_plan(const double* bb_coords, int64_t n_elements, int32_t n_buckets
     const unsigned small_grid = (unsigned)std::min((int64_t)2048, (int64_t)n / 2 + 1);
     rc = launch_small(n, nb, cpl, done_small, want_boxes, bb_coords, w, bb_indices_out, small_grid, st);
     if (rc) return rc;
-    k_top<<<1, kTopBlock, 0, st>>>(levels, want_boxes, bb_coords, w, bb_indices_out);
-    CT_LAUNCH_CHECK();
-    CT_HIP(hipMemcpyAsync(&h, w.head, sizeof(h), hipMemcpyDeviceToHost, st));
-    CT_HIP(hipStreamSynchronize(st));
+    // k_top goes along where this batch may be the last; it passes over all levels, so a deep chain
+    // runs it once, at the end (a fan of 200,000 triangles, 19,081 levels: 1.0 s, and 25.3 with one a batch).
+    const bool topped = levels <= kTopLevels;
+    if (topped) {
+      k_top<<<1, kTopBlock, 0, st>>>(levels, want_boxes, bb_coords, w, bb_indices_out);
+      CT_LAUNCH_CHECK();
+    }
+    rc = read_header();
+    if (rc) return rc;
     done_small = h.n_small;
-    if (h.err != 0 || h.level[levels & 1].active == 0) break;
+    if (h.err != 0) break;
+    if (h.level[levels & 1].active == 0) {
+      if (topped) break;
+      k_top<<<1, kTopBlock, 0, st>>>(levels, want_boxes, bb_coords, w, bb_indices_out);
+      CT_LAUNCH_CHECK();
+      rc = read_header();
+      if (rc) return rc;
+      break;
+    }
     // Children are strictly smaller than their parent and a node retries once, so the loop
     // ends within 2 * n_elements levels (the length of group_end); the guard only protects it.
     batch = std::min(std::max(2 * batch, 8), 64);
