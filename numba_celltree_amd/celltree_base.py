@@ -445,12 +445,10 @@ class CellTree2dBase:
 
     def _split(self, kind: int, queries: torch.Tensor, order):
         """(subqueries (m, 2) int32, part offsets (n + 1), m) for kind 1 boxes, 2 segment-face,
-        3 segment-edge, or None when the batch is not split.  Batches too small to be ordered
+        3 segment-edge (_splits).  Batches too small to be ordered
         (order None: queries in their own order) are split too: with few lanes, one long walk
         would set the call's time."""
         n = int(queries.shape[0])
-        if n == 0 or self.depth > _native.CT_MAX_DEPTH or int(self.SPLIT_MAX_PARTS) <= 1:
-            return None
         st = D.stream()
         leaf = self.SPLIT_LEAF_CELLS if kind == 1 else self.EDGE_SPLIT_LEAF_CELLS
         args = (self.tree_ref, kind, D.ptr(queries), n, D.ptr(order), int(self.SPLIT_MIN_CELLS), int(leaf),
@@ -463,14 +461,22 @@ class CellTree2dBase:
         _native.call("ct_split_queries", *args, None, D.ptr(part_offsets), D.ptr(subs), D.ptr(keep), st)
         return subs, part_offsets, m
 
+    # Batches and trees ct_gather_* takes: its launch has 64 lanes per 1 to 16 queries (a HIP launch has
+    # fewer than 2^32 lanes), its words hold 26-bit node and cell numbers.
+    GATHER_MAX_QUERIES = 1 << 29
+    GATHER_MAX_RECORDS = 1 << 26
+
     def _gathers(self, n: int) -> bool:
         """Whether a batch of n box or segment queries goes through ct_gather_*: every batch on a
         tree the stack walks take, 32-bit offsets address and whose leaves lie in order (an imported
-        tree's may not), unless splitting is turned off (SPLIT_MAX_PARTS <= 1: whole walks)."""
-        return (n > 0 and self.in_order and self.depth <= _native.CT_MAX_DEPTH and int(self.SPLIT_MAX_PARTS) > 1
+        tree's may not), unless splitting is turned off (SPLIT_MAX_PARTS <= 1: whole walks).  The
+        others are cut into subqueries."""
+        return (0 < n <= self.GATHER_MAX_QUERIES and self.in_order and self._splits(n)
                 and max(self.n_nodes, int(self.d_elements.shape[0])) < self.GATHER_MAX_RECORDS)
 
-    GATHER_MAX_RECORDS = 1 << 26
+    def _splits(self, n: int) -> bool:
+        """Whether a batch of n box or segment queries can be cut into subqueries."""
+        return n > 0 and self.depth <= _native.CT_MAX_DEPTH and int(self.SPLIT_MAX_PARTS) > 1
 
     @staticmethod
     def _pool(rows: int, widths):
@@ -600,6 +606,8 @@ class CellTree2dBase:
         if self._gathers(n):
             return self._gather(2 if kind == 1 else 3, edge_coords, self._gather_order(4, edge_coords))
         order, srt = self._order(2, edge_coords)
+        if self._splits(n):
+            return self._split_rows(2 if kind == 1 else 3, edge_coords, order)[1:]
         counts = D.empty(n, torch.int64)
         hits, slots = self._hit_record(n, self.EDGE_HIT_SLOTS, self.EDGE_HIT_BUDGET)
         _native.call(
