@@ -92,7 +92,8 @@ class TreeBatch:
         self.depths = np.array([int(t.depth) for t in trees])
         self.n_cells = np.array([int(t.d_elements.shape[0]) for t in trees])
         self.n_cu = _cu_count()
-        # trees the wavefront walks take (the others' segments are walked by one lane each)
+        # whether the wavefront walks take every tree (CellTree2dBase._gathers); if not, all segments
+        # are walked by one lane each
         self.gathers = all(t.in_order and max(int(t.n_nodes), int(t.d_elements.shape[0])) < t.GATHER_MAX_RECORDS
                            for t in trees)
 
@@ -248,7 +249,9 @@ def concat_queries(sets: Sequence, width: int) -> Tuple[torch.Tensor, np.ndarray
 
 # Row pool of the batched segment walks: at most EDGE_HIT_SLOTS rows per segment on average and
 # EDGE_HIT_BUDGET int32 words (8 GiB, 2.8% of a 288 GB device; a row takes 10).  Segments that find it
-# used up are walked by one lane each.
+# used up are walked by one lane each.  Batches that the wavefront walks do not take have a hit record
+# instead (as CellTree2d's): up to EDGE_HIT_SLOTS cells per segment within the same budget (slot-major,
+# so only slots in use are written), from which the write pass takes rows without a second walk.
 EDGE_HIT_SLOTS = 256
 EDGE_HIT_BUDGET = 1 << 31
 POOL_WAVES = 4096  # wavefronts of a walk, each taking up to POOL_CHUNK rows at a time
@@ -258,10 +261,16 @@ POOL_GUESS = 64    # rows per segment where their number is not known yet
 
 class EdgeBuffers:
     """Device buffers of a batched segment pass with room for `capacity` rows, and its row pool for
-    about `expected` rows (default: `capacity`; record=False: no pool)."""
+    about `expected` rows (default: `capacity`), or its hit record (gathers=False: TreeBatch.gathers).
+    record=False: neither."""
 
-    def __init__(self, n_queries: int, capacity: int, record: bool = True, expected: Optional[int] = None):
+    def __init__(self, n_queries: int, capacity: int, record: bool = True, expected: Optional[int] = None,
+                 gathers: bool = True):
         self.n_queries = n_queries
+        self.hits, self.slots = None, 0
+        if record and n_queries and not gathers:
+            # Fewer slots (down to none) when the device cannot hold the full record.
+            self.hits, self.slots = CellTree2dBase._hit_record(n_queries, EDGE_HIT_SLOTS, EDGE_HIT_BUDGET)
         self.counts = D.empty(n_queries, torch.int64)
         self.starts = D.empty(n_queries, torch.int64)
         self.offsets = D.empty(n_queries + 1, torch.int64)
@@ -269,7 +278,7 @@ class EdgeBuffers:
         self.tail = D.empty(int(_native.lib().ct_gather_tail_words()), torch.int64)
         expected = int(capacity) if expected is None else int(expected)
         rows = 0
-        if record and n_queries:
+        if record and n_queries and gathers:
             # a quarter more, since a wavefront drops the end of a chunk that is too short for its
             # next segments; and a chunk at hand per wavefront
             rows = expected + expected // 4 + POOL_CHUNK * min(POOL_WAVES, n_queries)
@@ -293,20 +302,28 @@ def gather_edges(plan: BatchPlan, segments: torch.Tensor, buf: EdgeBuffers) -> N
     n = plan.n_queries
     st = D.stream()
     _check(segments, (n, 2, 2), torch.float64)
-    if not plan.batch.gathers:
-        buf.pool_rows = 0
-    _native.call("ct_batch_gather_edges", plan.ref, D.ptr(segments), n, int(plan.config.tile), buf.pool_rows,
-                 *(D.ptr(a) for a in buf.pool), D.ptr(buf.counts), D.ptr(buf.starts), D.ptr(buf.tail), st)
+    if plan.batch.gathers:
+        _native.call("ct_batch_gather_edges", plan.ref, D.ptr(segments), n, int(plan.config.tile), buf.pool_rows,
+                     *(D.ptr(a) for a in buf.pool), D.ptr(buf.counts), D.ptr(buf.starts), D.ptr(buf.tail), st)
+    else:
+        plan.edges_count(segments, buf.counts, buf.hits, buf.slots)
     _native.call("ct_exclusive_scan", D.ptr(buf.counts), n, D.ptr(buf.offsets), D.ptr(buf.scan_ws),
                  buf.scan_ws.numel(), st)
 
 
 def gather_rows(plan: BatchPlan, segments: torch.Tensor, buf: EdgeBuffers, sort_workgroups: int) -> None:
     """The rows of gather_edges within the buffers' capacity, enqueued."""
-    _native.call("ct_batch_gather_rows", plan.ref, D.ptr(segments), plan.n_queries, D.ptr(buf.offsets),
-                 D.ptr(buf.starts), D.ptr(buf.tail), *(D.ptr(a) for a in buf.pool), buf.capacity,
-                 int(sort_workgroups), D.ptr(buf.ii), D.ptr(buf.jj), D.ptr(buf.xy), D.ptr(buf.jj_sorted),
-                 D.ptr(buf.xy_sorted), D.stream())
+    n = plan.n_queries
+    st = D.stream()
+    if plan.batch.gathers:
+        _native.call("ct_batch_gather_rows", plan.ref, D.ptr(segments), n, D.ptr(buf.offsets),
+                     D.ptr(buf.starts), D.ptr(buf.tail), *(D.ptr(a) for a in buf.pool), buf.capacity,
+                     int(sort_workgroups), D.ptr(buf.ii), D.ptr(buf.jj), D.ptr(buf.xy), D.ptr(buf.jj_sorted),
+                     D.ptr(buf.xy_sorted), st)
+        return
+    plan.edges_write(segments, buf.offsets, buf.capacity, buf.ii, buf.jj, buf.xy, buf.hits, buf.slots)
+    _native.call("ct_batch_sort_intersections", D.ptr(segments), n, D.ptr(buf.offsets), D.ptr(buf.ii), D.ptr(buf.jj),
+                 D.ptr(buf.xy), buf.capacity, int(sort_workgroups), D.ptr(buf.jj_sorted), D.ptr(buf.xy_sorted), st)
 
 
 def run_edges(plan: BatchPlan, segments: torch.Tensor, buf: EdgeBuffers, sort_workgroups: int) -> None:
@@ -362,11 +379,12 @@ class BatchGraph:
         self.buf = None
         if self.eplan is not None:
             if capacity is None:
-                probe = EdgeBuffers(self.eplan.n_queries, 0, expected=POOL_GUESS * self.eplan.n_queries)
+                probe = EdgeBuffers(self.eplan.n_queries, 0, expected=POOL_GUESS * self.eplan.n_queries,
+                                    record=batch.gathers)
                 gather_edges(self.eplan, segments, probe)
                 capacity = int(probe.offsets[-1].item())
                 del probe
-            self.buf = EdgeBuffers(self.eplan.n_queries, capacity)
+            self.buf = EdgeBuffers(self.eplan.n_queries, capacity, gathers=batch.gathers)
         # warm up once eagerly on the capture stream, then capture
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
@@ -425,7 +443,7 @@ def intersect_edges(batch: TreeBatch, segment_sets: Sequence, config: BatchConfi
     segs = segs.reshape(-1, 2, 2)
     plan = batch.plan(counts, config)
     n = plan.n_queries
-    buf = EdgeBuffers(n, 0, expected=POOL_GUESS * n)
+    buf = EdgeBuffers(n, 0, expected=POOL_GUESS * n, gathers=batch.gathers)
     gather_edges(plan, segs, buf)
     buf.room(int(buf.offsets[-1].item()))
     gather_rows(plan, segs, buf, 4 * batch.n_cu)
