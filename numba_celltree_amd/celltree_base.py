@@ -475,8 +475,10 @@ class CellTree2dBase:
                 and max(self.n_nodes, int(self.d_elements.shape[0])) < self.GATHER_MAX_RECORDS)
 
     def _splits(self, n: int) -> bool:
-        """Whether a batch of n box or segment queries can be cut into subqueries."""
-        return n > 0 and self.depth <= _native.CT_MAX_DEPTH and int(self.SPLIT_MAX_PARTS) > 1
+        """Whether a batch of n box or segment queries can be cut into subqueries (frontier entries
+        hold 28-bit node numbers)."""
+        return (n > 0 and self.depth <= _native.CT_MAX_DEPTH and int(self.SPLIT_MAX_PARTS) > 1
+                and self.n_nodes < 1 << 28)
 
     @staticmethod
     def _pool(rows: int, widths):

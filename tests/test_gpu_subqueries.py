@@ -25,6 +25,8 @@ def test_routes_by_size():
         assert not t._gathers(n) and t._splits(n)
     t.n_nodes = 1 << 26
     assert not t._gathers(5) and t._splits(5)
+    t.n_nodes = 1 << 28
+    assert not t._gathers(5) and not t._splits(5)
     t.n_nodes, t.in_order = 1 << 20, False
     assert not t._gathers(5) and t._splits(5)
     t.in_order, t.depth = True, _native.CT_MAX_DEPTH + 1
