@@ -305,7 +305,7 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
       rec.prune = KIND == kFaces && t.nbox != nullptr && isfinite(mseg) && isfinite(rec.mm) && isfinite(rec.dx) &&
                   isfinite(rec.dy);
       P2 c0, d0;
-      in = cohen_sutherland(a, b, t.bbox, &c0, &d0);
+      in = cohen_sutherland<true>(a, b, t.bbox, &c0, &d0);
     }
     if (in) {
       weight = expected<KIND>(rec, p.cell);
@@ -375,7 +375,7 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
           c = t.bb_indices[k];
           const P2 a = {d.x, d.y}, b = {d.z, d.w};
           const Box bb = leaf_box(t, k, c);
-          hit = cohen_sutherland(a, b, bb, &cc, &dd);
+          hit = cohen_sutherland<true>(a, b, bb, &cc, &dd);
           if (hit) {
             if (t.leaf != nullptr) hit = edge_face_clip_row<MAXV>(t, k, c, a, b, &cc, &dd);
             else hit = edge_face_clip<MAXV>(t, c, bb, a, b, &cc, &dd);

@@ -247,6 +247,12 @@ __device__ __forceinline__ int cs_code(P2 a, const Box& b) {
 // cohen_sutherland.py:36-101.  The reference's loop is unbounded; in exact arithmetic
 // it ends within four clips.  The device loop stops after 64 (a clip that has not
 // converged by then reports no intersection instead of spinning).
+//
+// SHARED: the four bounds' expressions as one on selected operands, so that lanes at different bounds
+// share its division: for wavefronts whose lanes all clip at once.  Where most lanes of a wavefront are
+// elsewhere, the selects cost more than they save: 3e5 segments of 180 cell sides by subqueries on
+// 20,000 cells 9.85 ms shared, 8.87 with a branch per bound.
+template <bool SHARED = false>
 __device__ __forceinline__ bool cohen_sutherland(P2 a, P2 b, const Box& box, P2* c, P2* d) {
   double dx = b.x - a.x, dy = b.y - a.y;
   if (dx == 0.0 && dy == 0.0) return false;
@@ -254,14 +260,28 @@ __device__ __forceinline__ bool cohen_sutherland(P2 a, P2 b, const Box& box, P2*
   for (int iter = 0; (k1 | k2) != 0; ++iter) {
     if ((k1 & k2) != 0 || iter >= 64) return false;
     const int opt = k1 ? k1 : k2;
-    // x = a.x + dx * (bound - a.y) / dy at a y bound, y = a.y + dy * (bound - a.x) / dx at an x bound:
-    // one expression on selected operands, so that lanes at different bounds share its division.
-    const bool at_y = (opt & 12) != 0;
-    const double bound = at_y ? ((opt & 8) ? box.ymax : box.ymin) : ((opt & 2) ? box.xmax : box.xmin);
-    const double u = at_y ? a.x : a.y, du = at_y ? dx : dy;
-    const double v = at_y ? a.y : a.x, dv = at_y ? dy : dx;
-    const double w = u + du * (bound - v) / dv;
-    const double x = at_y ? w : bound, y = at_y ? bound : w;
+    double x, y;
+    if constexpr (SHARED) {
+      const bool at_y = (opt & 12) != 0;
+      const double bound = at_y ? ((opt & 8) ? box.ymax : box.ymin) : ((opt & 2) ? box.xmax : box.xmin);
+      const double u = at_y ? a.x : a.y, du = at_y ? dx : dy;
+      const double v = at_y ? a.y : a.x, dv = at_y ? dy : dx;
+      const double w = u + du * (bound - v) / dv;
+      x = at_y ? w : bound;
+      y = at_y ? bound : w;
+    } else if (opt & 8) {
+      x = a.x + dx * (box.ymax - a.y) / dy;
+      y = box.ymax;
+    } else if (opt & 4) {
+      x = a.x + dx * (box.ymin - a.y) / dy;
+      y = box.ymin;
+    } else if (opt & 2) {
+      y = a.y + dy * (box.xmax - a.x) / dx;
+      x = box.xmax;
+    } else {
+      y = a.y + dy * (box.xmin - a.x) / dx;
+      x = box.xmin;
+    }
     if (opt == k1) {
       a = {x, y};
       k1 = cs_code(a, box);
