@@ -36,6 +36,7 @@ constexpr int kMaxPerWave = 16;
 constexpr int kOwnerShift = 27;
 constexpr uint32_t kIndexMask = (1u << kOwnerShift) - 1u;
 constexpr int64_t kMaxRecords = (int64_t)1 << 26;
+constexpr uint32_t kLargeLeaf = ~0u;  // a stack entry: the large leaf at hand
 
 // LDS list lengths.  The stack: a step of P entries needs room for P more; P shrinks as the stack
 // fills, and depth + 1 places always remain for a single entry's way down (kStack + depth + 1 in all;
@@ -43,6 +44,11 @@ constexpr int64_t kMaxRecords = (int64_t)1 << 26;
 constexpr int kStack = 320;
 constexpr int kCells = 192;  // 63 left over + 2 per lane
 constexpr int kCands = 128;  // 63 left over + 64
+// A step with a leaf of more cells than this lists one leaf, 64 cells at a time by all lanes, and puts
+// the others back: each lane listing its own leaf takes as many stores as the largest has cells, and a
+// leaf may be larger than the list.  200,000 triangles in leaves of up to 130 cells, 1e5 boxes: 481 us,
+// 771 lane by lane; of up to 64 cells, 1e5 segments: 850 lane by lane, 982 one leaf at a time.
+constexpr int kLeafCells = 64;
 // Hits a wavefront holds, and the expected hits of the queries it walks together: fewer and the steps
 // at either end of a walk (few entries on the stack) weigh more, more and LDS limits the wavefronts in
 // flight or groups overflow and are walked again one by one.  Measured, 1e6 queries, milliseconds:
@@ -65,7 +71,7 @@ struct Pool {
   int32_t* src;    // segments: rows in output order -> entry of cell / xy
   int64_t rows;    // per counter
   int counters;
-  int chunk;       // segments: rows a wavefront takes at a time, at least kSegHits
+  int chunk;       // segments: rows a wavefront takes at a time, at least (0: those it asks for)
 };
 
 // A wavefront's pool rows at hand (segments) and the counter it allocates from.
@@ -76,16 +82,17 @@ struct PoolRows {
   __device__ __forceinline__ unsigned long long* counter(int64_t* tail) const {
     return reinterpret_cast<unsigned long long*>(tail) + 1 + sub * kCounterStride;
   }
-  // The next chunk: from this wavefront's counter, or from the next that has one.
-  __device__ __forceinline__ void refill(const Pool& pool, int64_t* tail) {
+  // `want` rows or a chunk: from this wavefront's counter, or from the next that has them.
+  __device__ __forceinline__ void refill(const Pool& pool, int64_t* tail, int want) {
+    const int take = max(want, pool.chunk);
     at = end = 0;
     while (tried < pool.counters) {
       long long x = 0;
-      if (lane_id() == 0) x = (long long)atomicAdd(counter(tail), (unsigned long long)pool.chunk);
+      if (lane_id() == 0) x = (long long)atomicAdd(counter(tail), (unsigned long long)take);
       x = __shfl(x, 0);
-      if (x + pool.chunk <= pool.rows) {
+      if (x + take <= pool.rows) {
         at = (long long)sub * pool.rows + x;
-        end = at + pool.chunk;
+        end = at + take;
         return;
       }
       sub = sub + 1 == pool.counters ? 0 : sub + 1;
@@ -275,6 +282,7 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
   __shared__ Key ts[KIND == kBoxes ? 1 : kHits];           // segments: t_key
   __shared__ uint16_t byown[KIND == kBoxes ? 1 : kHits];   // segments: a grouped hit's pool row
   __shared__ int cnt[kMaxPerWave], first[kMaxPerWave + 1];
+  __shared__ uint32_t large[3];                            // a large leaf on the stack: its next cell's words, cells left
   const int lane = lane_id();
   __syncthreads();  // one wavefront: the last block's LDS reads are over
 
@@ -352,13 +360,13 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
     int room = KIND == kBoxes && g1 - g0 > 1 ? kBoxGroupHits : kHits;
     if (KIND != kBoxes && alive) {
       const int want = g1 - g0 == 1 ? kHits : min(kHits, 2 * wsum + 32);
-      if (rows.end - rows.at < want) rows.refill(pool, tail);
+      if (rows.end - rows.at < want) rows.refill(pool, tail, want);
       room = (int)min((long long)kHits, rows.end - rows.at);
     }
     __syncthreads();
     int sp = __popcll(alive), ncell = 0, ncand = 0, nhit = 0;
-    bool over = false;  // more hits than `room`, or a leaf larger than the cell list
-    while (true) {
+    bool over = KIND != kBoxes && alive && room == 0;  // more hits than `room`
+    while (!over) {
       // a full list first: each step leaves room for what the next one adds
       if (KIND == kFaces && (ncand >= 64 || (sp == 0 && ncell == 0 && ncand > 0))) {
         const int take = min(64, ncand);
@@ -436,12 +444,27 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
       if (sp == 0) break;
       // the top of the stack
       const int take = min(min(64, sp), max(1, p.stack - p.depth1 - sp));
+      uint32_t e = lane < take ? stack[sp - take + lane] : 0;
+      if ((uint32_t)__builtin_amdgcn_readlane((int)e, take - 1) == kLargeLeaf) {
+        // the next cells of a large leaf (at most 64, and 128 more fit)
+        const uint32_t at = large[0], visit = large[1], left = large[2];
+        const uint32_t m = min(64u, left);
+        __syncthreads();
+        if ((uint32_t)lane < m) cells[ncell + lane] = make_uint2(at + lane, visit + lane);
+        if (lane == 0) {
+          large[0] = at + m;
+          large[1] = visit + m;
+          large[2] = left - m;
+        }
+        ncell += m;
+        if (m == left) --sp;
+        __syncthreads();
+        continue;
+      }
       sp -= take;
       bool left = false, right = false;
-      uint32_t e = 0;
       int child = 0, ptr = 0, size = 0;
       if (lane < take) {
-        e = stack[sp + lane];
         const uint32_t x = e & kIndexMask;
         const QueryRec<KIND>& r = recs[owner(e)];
         bool here = true, by_box = false;
@@ -491,17 +514,24 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
           const int y = __shfl_up(incl, d);
           if (lane >= d) incl += y;
         }
-        const bool fits = incl <= kCells - ncell;
-        const uint64_t back = __ballot(size > 0 && !fits), put = __ballot(size > 0 && fits);
-        if (back && !put) {  // a leaf larger than the list
-          over = true;
-          break;
+        const bool fits = incl <= kCells - ncell && !__any(size > kLeafCells);
+        uint64_t back = __ballot(size > 0 && !fits);
+        const uint64_t put = __ballot(size > 0 && fits), one = put ? 0 : back & -back;
+        if (one >> lane & 1) {  // a large leaf, listed by the whole wavefront
+          large[0] = tag | (uint32_t)ptr;
+          large[1] = tag | v0;
+          large[2] = (uint32_t)size;
         }
+        back &= ~one;
         if (size > 0 && fits)
           for (int j = 0; j < size; ++j)
             cells[ncell + incl - size + j] = make_uint2(tag | (uint32_t)(ptr + j), tag | (v0 + j));
-        if (size > 0 && !fits) stack[sp + below(back)] = e;
+        if (back >> lane & 1) stack[sp + below(back)] = e;
         sp += __popcll(back);
+        if (one) {
+          if (lane == 0) stack[sp] = kLargeLeaf;
+          ++sp;
+        }
         // the listed cells: the prefix of the last lane that fits
         const int last = 63 - __clzll((unsigned long long)put);
         ncell += put ? __shfl(incl, last) : 0;
@@ -510,7 +540,7 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
     }
 
     bool left_over = over;  // the group's queries are left to the caller
-    if (over && g1 - g0 > 1 && (KIND == kBoxes || room == kHits || rows.end > rows.at)) {
+    if (over && g1 - g0 > 1 && (KIND == kBoxes || room > 0)) {
       single_until = g1;  // again, one query at a time
       continue;
     }
@@ -531,9 +561,15 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
     long long at = rows.at;
     if (!over && nhit > 0) {
       if constexpr (KIND == kBoxes) {
-        if (lane == 0) at = (long long)atomicAdd(rows.counter(tail), (unsigned long long)nhit);
-        at = __shfl(at, 0);
-        left_over = at + nhit > pool.rows;
+        left_over = true;
+        while (left_over && rows.tried < pool.counters) {
+          if (lane == 0) at = (long long)atomicAdd(rows.counter(tail), (unsigned long long)nhit);
+          at = __shfl(at, 0);
+          left_over = at + nhit > pool.rows;
+          if (!left_over) break;
+          rows.sub = rows.sub + 1 == pool.counters ? 0 : rows.sub + 1;
+          ++rows.tried;
+        }
         at += (long long)rows.sub * pool.rows;
         if (!left_over) {
           if (g1 - g0 > 1) {
