@@ -404,17 +404,24 @@ int ct_sort_staged_rows(const int64_t* offsets, const int64_t* query_start, cons
 
 /* Box and segment queries by wavefronts, a few queries each (kind 1 boxes, 2 segment-face, 3
  * segment-edge; trees of depth <= CT_MAX_DEPTH with their leaves in order, ct_leaves_in_order),
- * without subqueries.  ct_gather_count writes
- * counts[q] and starts[q] and keeps the rows in the caller's pool of pool_rows entries (pool_cell;
- * segments also pool_xy, 4 doubles each, and pool_src); ct_gather_pool_rows suggests a size.
- * starts[q] < 0: q is left to the caller (more rows than a wavefront's lists hold, or no room in the
- * pool), counts[q] = 0.  tail: ct_gather_tail_words() int64 of working words; tail[0] = the number of
- * queries left.  visit_cells (boxes; ct_visit_cells): (n_elements) the cells in the order in which a
- * walk that enters every node meets them.  After an exclusive scan of the counts (with those of the
- * queries left filled in) into offsets (n + 1), ct_gather_rows writes the rows kept at their
- * offsets: boxes (ii, jj) in DFS order within a query, segments (ii, jj, xy) by t
- * (geometry_utils.py:564-574); ct_place_rows writes those of the queries left: row r of sub-query
- * s = sub_ii[r] (query idx[s]) to offsets[idx[s]] + r - sub_offsets[s]. */
+ * without subqueries.  ct_gather_count writes counts[q] and starts[q] and keeps the rows in the
+ * caller's pool of pool_rows entries (pool_cell; segments also pool_xy, 4 doubles each, and
+ * pool_src); ct_gather_pool_rows suggests a size.  starts[q] < 0: q is left to the caller (more rows
+ * than a wavefront's lists hold, or no room in the pool), counts[q] = 0.  tail:
+ * ct_gather_tail_words() int64 of working words; tail[0] = the number of queries left.  visit_cells
+ * (boxes; ct_visit_cells): (n_elements) the cells in the order in which a walk that enters every
+ * node meets them.  After an exclusive scan of the counts (with those of the queries left filled in)
+ * into offsets (n + 1), ct_gather_rows writes the rows kept at their offsets: boxes (ii, jj) in DFS
+ * order within a query, segments (ii, jj, xy) by t (geometry_utils.py:564-574).
+ *
+ * ct_gather_left lists the n_left = tail[0] queries left (found: a working word).  At most
+ * CT_LONG_MAX of them can be walked by a wavefront each: ct_long_count writes their counts[q] (and
+ * for segments left_counts, in list order); boxes may find room in the same pool after all
+ * (starts[q]).  Then ct_long_boxes writes the rows of the boxes still left to their offsets;
+ * ct_long_edges writes those of the segments to staging rows, left_offsets the exclusive scan of
+ * left_counts, and sets starts to what ct_sort_staged_rows takes as query_start (call ct_gather_rows
+ * before).  Or they are cut into subqueries, the list being their processing order. */
+#define CT_LONG_MAX (1 << 24)
 int64_t ct_gather_tail_words(void);
 int64_t ct_gather_pool_rows(int32_t kind, int64_t n);
 int ct_visit_cells(const ct_tree* tree, int32_t* out, void* stream);
@@ -425,9 +432,18 @@ int ct_gather_count(const ct_tree* tree, int32_t kind, const double* queries, in
 int ct_gather_rows(int32_t kind, int64_t n, const int64_t* offsets, const int64_t* starts,
                    const int32_t* pool_cell, const double* pool_xy, const int32_t* pool_src,
                    int64_t* ii, int64_t* jj, double* xy, void* stream);
-int ct_place_rows(int64_t rows, const int64_t* idx, const int64_t* sub_offsets,
-                  const int64_t* offsets, const int64_t* sub_ii, const int64_t* sub_jj,
-                  const double* sub_xy, int64_t* ii, int64_t* jj, double* xy, void* stream);
+int ct_gather_left(int64_t n, const int64_t* starts, int64_t n_left, int32_t* left, int64_t* found,
+                   void* stream);
+int ct_long_count(const ct_tree* tree, int32_t kind, const double* queries, int64_t n,
+                  const int32_t* left, int64_t n_left, int64_t pool_rows, int32_t* pool_cell,
+                  int64_t* counts, int64_t* starts, int64_t* left_counts, int64_t* tail, void* stream);
+int ct_long_boxes(const ct_tree* tree, const double* boxes, int64_t n, const int32_t* left,
+                  int64_t n_left, const int64_t* offsets, const int64_t* starts, int64_t* ii,
+                  int64_t* jj, void* stream);
+int ct_long_edges(const ct_tree* tree, int32_t kind, const double* segments, int64_t n,
+                  const int32_t* left, int64_t n_left, const int64_t* left_offsets, int64_t* starts,
+                  int32_t* rows_query, int32_t* rows_cell, double* rows_xy, double* rows_t,
+                  void* stream);
 
 /* geometry_utils.py:564-574 sort_intersections_by_edge on grouped output (ii ascending, the
  * rows of segment s in [offsets[s], offsets[s+1])): writes jj and xy (n_rows, 2, 2) stably

@@ -193,7 +193,10 @@ SIGNATURES = {
     "ct_visit_cells": (ctypes.c_int, [_TP, _P, _P]),
     "ct_gather_count": (ctypes.c_int, [_TP, _I32, _P, _I64, _P, _P, _I64, _P, _P, _P, _P, _P, _P, _P]),
     "ct_gather_rows": (ctypes.c_int, [_I32, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
-    "ct_place_rows": (ctypes.c_int, [_I64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
+    "ct_gather_left": (ctypes.c_int, [_I64, _P, _I64, _P, _P, _P]),
+    "ct_long_count": (ctypes.c_int, [_TP, _I32, _P, _I64, _P, _I64, _I64, _P, _P, _P, _P, _P, _P]),
+    "ct_long_boxes": (ctypes.c_int, [_TP, _P, _I64, _P, _I64, _P, _P, _P, _P, _P]),
+    "ct_long_edges": (ctypes.c_int, [_TP, _I32, _P, _I64, _P, _I64, _P, _P, _P, _P, _P, _P, _P]),
     "ct_locate_points_ordered_noalloc": (ctypes.c_int, [_TP, _P, _I64, _F64, _P, _P]),
     "ct_locate_points_on_edge": (ctypes.c_int, [_TP, _P, _I64, _F64, _P, _P]),
     "ct_order_workspace_bytes": (_SZ, [_I64]),

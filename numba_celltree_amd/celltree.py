@@ -120,7 +120,7 @@ class CellTree2d(CellTree2dBase):
         if prep is not None:
             prep.check(prep.checks[:3].tolist())
         if self._splits(n):
-            return self._split_rows(1, d_boxes, order)[1:3]
+            return self._split_rows(1, d_boxes, order)[:2]
         counts = D.empty(n, torch.int64)
         hits, slots = self._hit_record(n, self.BOX_HIT_SLOTS, self.BOX_HIT_BUDGET)
         _native.call("ct_locate_boxes_count_rec", self.tree_ref, D.ptr(d_boxes), n, D.ptr(order), D.ptr(srt),

@@ -399,7 +399,7 @@ class CellTree2dBase:
     # first EDGE_XY_SLOTS hits (32 bytes each, within EDGE_XY_BUDGET bytes), so that the write
     # pass copies the rows of a subquery whose hits all fit instead of clipping its cells again.
     EDGE_XY_SLOTS = 32
-    EDGE_XY_BUDGET = 1 << 31
+    EDGE_XY_BUDGET = 1 << 32
 
     BOX_HIT_SLOTS = 1024
     BOX_HIT_BUDGET = 1 << 30
@@ -443,12 +443,12 @@ class CellTree2dBase:
     EDGE_SPLIT_LEAF_CELLS = 64
     SPLIT_MAX_PARTS = 16
 
-    def _split(self, kind: int, queries: torch.Tensor, order):
+    def _split(self, kind: int, queries: torch.Tensor, order, n: Optional[int] = None):
         """(subqueries (m, 2) int32, part offsets (n + 1), m) for kind 1 boxes, 2 segment-face,
-        3 segment-edge (_splits).  Batches too small to be ordered
-        (order None: queries in their own order) are split too: with few lanes, one long walk
-        would set the call's time."""
-        n = int(queries.shape[0])
+        3 segment-edge (_splits) of the n queries ``order`` lists (default: all).  Batches too small
+        to be ordered (order None: queries in their own order) are split too: with few lanes, one
+        long walk would set the call's time."""
+        n = int(queries.shape[0]) if n is None else n
         st = D.stream()
         leaf = self.SPLIT_LEAF_CELLS if kind == 1 else self.EDGE_SPLIT_LEAF_CELLS
         args = (self.tree_ref, kind, D.ptr(queries), n, D.ptr(order), int(self.SPLIT_MIN_CELLS), int(leaf),
@@ -493,10 +493,14 @@ class CellTree2dBase:
                 rows //= 2
         return 0, [None for _ in widths]
 
+    # At most this many queries that a wavefront walk leaves over are walked by a wavefront each
+    # (ct_long_*); more fill the device as subqueries.
+    LONG_MAX = 1 << 20
+
     def _gather(self, kind: int, queries: torch.Tensor, order, prep=None):
         """Rows of a box (kind 1), segment-face (2) or segment-edge (3) batch: (ii, jj) or
         (ii, jj, xy).  One readback: the row total, the queries left over, and the index checks of
-        ``prep``."""
+        ``prep``; another one or two where queries are left over."""
         n = int(queries.shape[0])
         st = D.stream()
         L = _native.lib()
@@ -505,91 +509,145 @@ class CellTree2dBase:
             rows, (cell,) = self._pool(min(rows, int(self.BOX_HIT_BUDGET)), [(torch.int32, 1)])
             pxy = src = None
         else:
-            rows, (cell, pxy, src) = self._pool(min(rows, int(self.EDGE_HIT_BUDGET)),
+            rows, (cell, pxy, src) = self._pool(min(rows, int(self.EDGE_HIT_BUDGET) // 2, int(self.EDGE_XY_BUDGET) // 32),
                                                 [(torch.int32, 1), (torch.float64, 4), (torch.int32, 1)])
         pool = (D.ptr(cell), D.ptr(pxy), D.ptr(src))
         counts = D.empty(n, torch.int64)
         starts = D.empty(n, torch.int64)
         row = D.gather_row(n) if prep is None else prep.row  # offsets, check words, working words
+        tail = row[n + 9:]
         _native.call("ct_gather_count", self.tree_ref, kind, D.ptr(queries), n, D.ptr(order),
-                     D.ptr(self.d_visit_cells), rows, *pool, D.ptr(counts), D.ptr(starts), D.ptr(row[n + 9:]), st)
+                     D.ptr(self.d_visit_cells), rows, *pool, D.ptr(counts), D.ptr(starts), D.ptr(tail), st)
         D.exclusive_scan(counts, total=False, offsets=row)
         total, *words, left = row[n: n + 10].tolist()
         if prep is not None:
             prep.check(words)
-        if 2 * left >= n:
-            # Mostly large queries: all of them as subqueries, whose rows need no second place.
-            _, ii, jj, xy = self._split_rows(kind, queries, self._order(1 if kind == 1 else 2, queries)[0])
-            return (ii, jj) if kind == 1 else (ii, jj, xy)
+        write = None
         if left:
-            # Queries with more rows than a wavefront's lists hold, as subqueries; their counts join.
-            idx = torch.nonzero(starts < 0)[:, 0]
-            big = queries[idx].contiguous()
-            sub = self._split_rows(kind, big, self._order(1 if kind == 1 else 2, big)[0])
-            counts[idx] = torch.diff(sub[0])
-            _, total = D.exclusive_scan(counts, offsets=row)
+            many = left > int(self.LONG_MAX)
+            if left == n and (many or kind != 1):  # nothing is in the pool, or will be
+                cell = pxy = src = None
+                pool = (0, 0, 0)
+            ids = None
+            if left < n:
+                ids, found = D.empty(left, torch.int32), D.empty(1, torch.int64)
+                _native.call("ct_gather_left", n, D.ptr(starts), left, D.ptr(ids), D.ptr(found), st)
+            if many:
+                write = self._count_subs(kind, queries, self._left_order(kind, queries, ids), left, counts)
+            else:
+                if ids is None:
+                    ids = torch.arange(n, dtype=torch.int32, device=queries.device)
+                write = self._count_long(kind, queries, ids, left, rows, cell if kind == 1 else None, counts, starts,
+                                         tail)
+            _, all_rows = D.exclusive_scan(counts, offsets=row)
+            left_rows, total = all_rows - total, all_rows
         ii = D.empty(total, torch.int64)
         jj = D.empty(total, torch.int64)
         xy = None if kind == 1 else D.empty((total, 2, 2), torch.float64)
         _native.call("ct_gather_rows", kind, n, D.ptr(row), D.ptr(starts), *pool, D.ptr(ii), D.ptr(jj), D.ptr(xy), st)
-        if left and int(sub[1].numel()):
-            _native.call("ct_place_rows", int(sub[1].numel()), D.ptr(idx), D.ptr(sub[0]), D.ptr(row), D.ptr(sub[1]),
-                         D.ptr(sub[2]), D.ptr(sub[3]), D.ptr(ii), D.ptr(jj), D.ptr(xy), st)
+        if write is not None:
+            write(row, left_rows, ii, jj, xy)
         return (ii, jj) if kind == 1 else (ii, jj, xy)
 
-    def _split_rows(self, kind: int, queries: torch.Tensor, order):
-        """(offsets, ii, jj, xy or None) of a batch through subqueries by subtree (ct_split_queries):
-        the queries with too many rows for one wavefront."""
+    def _left_order(self, kind: int, queries: torch.Tensor, ids):
+        """The processing order of the queries ``ids`` (None: all) as subqueries."""
+        if ids is None:
+            return self._order(1 if kind == 1 else 2, queries)[0]
+        if int(ids.shape[0]) < self.ORDER_MIN:
+            return ids
+        order = self._order(1 if kind == 1 else 2, queries[ids.long()].contiguous())[0]
+        return ids[order.long()].contiguous()
+
+    def _count_long(self, kind: int, queries, ids, m: int, pool_rows: int, pool_cell, counts, starts, tail):
+        """Counts the rows of the m queries ``ids``, walked by a wavefront each; returns what writes
+        them: write(offsets, their rows, ii, jj, xy), after ct_gather_rows."""
         n = int(queries.shape[0])
         st = D.stream()
-        subs, part_offsets, m = self._split(kind, queries, order)
-        counts = D.empty(max(m, 1), torch.int64)
+        per_query = None if kind == 1 else D.empty(m, torch.int64)
+        _native.call("ct_long_count", self.tree_ref, kind, D.ptr(queries), n, D.ptr(ids), m,
+                     pool_rows if pool_cell is not None else 0, D.ptr(pool_cell), D.ptr(counts), D.ptr(starts),
+                     D.ptr(per_query), D.ptr(tail), st)
+        if kind == 1:
+            def write_boxes(offsets, rows, ii, jj, xy):
+                _native.call("ct_long_boxes", self.tree_ref, D.ptr(queries), n, D.ptr(ids), m, D.ptr(offsets),
+                             D.ptr(starts), D.ptr(ii), D.ptr(jj), st)
+
+            return write_boxes
+        left_offsets, _ = D.exclusive_scan(per_query, total=False)
+
+        def write_edges(offsets, rows, ii, jj, xy):
+            if rows == 0:
+                return
+            staged = self._staging(rows)
+            _native.call("ct_long_edges", self.tree_ref, kind, D.ptr(queries), n, D.ptr(ids), m, D.ptr(left_offsets),
+                         D.ptr(starts), *(D.ptr(t) for t in staged), st)
+            _native.call("ct_sort_staged_rows", D.ptr(offsets), D.ptr(starts), *(D.ptr(t) for t in staged), rows,
+                         D.ptr(ii), D.ptr(jj), D.ptr(xy), st)
+
+        return write_edges
+
+    @staticmethod
+    def _staging(rows: int):
+        """Staging rows of segments: query, cell, piece, t."""
+        return (D.empty(rows, torch.int32), D.empty(rows, torch.int32), D.empty((rows, 4), torch.float64),
+                D.empty(rows, torch.float64))
+
+    def _count_subs(self, kind: int, queries: torch.Tensor, order, n: int, counts: torch.Tensor):
+        """Counts the rows of the n queries ``order`` (None: all) cut into subqueries by subtree
+        (ct_split_queries) into ``counts``; returns what writes them: write(offsets, their rows, ii,
+        jj, xy)."""
+        st = D.stream()
+        subs, part_offsets, m = self._split(kind, queries, order, n)
+        sub_counts = D.empty(max(m, 1), torch.int64)
         if kind == 1:
             hits, slots = self._hit_record(m, self.BOX_HIT_SLOTS, self.BOX_HIT_BUDGET)
-            _native.call("ct_locate_boxes_count_sub", self.tree_ref, D.ptr(queries), D.ptr(subs), m, D.ptr(counts),
-                         D.ptr(hits), slots, st)
-            offsets, total = self._sub_offsets(order, n, part_offsets, counts)
-            ii = D.empty(total, torch.int64)
-            jj = D.empty(total, torch.int64)
-            _native.call("ct_locate_boxes_write_sub", self.tree_ref, D.ptr(queries), D.ptr(subs), m, D.ptr(offsets),
-                         D.ptr(counts), D.ptr(hits), slots, D.ptr(ii), D.ptr(jj), st)
-            return offsets, ii, jj, None
+            _native.call("ct_locate_boxes_count_sub", self.tree_ref, D.ptr(queries), D.ptr(subs), m,
+                         D.ptr(sub_counts), D.ptr(hits), slots, st)
+            # prefixes within each query
+            _native.call("ct_subquery_offsets", D.ptr(order), n, D.ptr(part_offsets), D.ptr(sub_counts),
+                         D.ptr(counts), st)
+
+            def write_boxes(offsets, rows, ii, jj, xy):
+                _native.call("ct_locate_boxes_write_sub", self.tree_ref, D.ptr(queries), D.ptr(subs), m,
+                             D.ptr(offsets), D.ptr(sub_counts), D.ptr(hits), slots, D.ptr(ii), D.ptr(jj), st)
+
+            return write_boxes
         edges = 1 if kind == 2 else 0  # the C ABI's kind of a segment query
         hits, slots = self._hit_record(m, self.EDGE_HIT_SLOTS, self.EDGE_HIT_BUDGET)
         hit_xy, xy_slots = (None, 0) if hits is None else self._xy_record(m, slots, self.EDGE_XY_SLOTS,
-                                                                          self.EDGE_XY_BUDGET)
+                                                                          int(self.EDGE_XY_BUDGET) // 2)
         _native.call("ct_locate_edges_count_sub", self.tree_ref, D.ptr(queries), D.ptr(subs), m, edges,
-                     D.ptr(counts), D.ptr(hits), slots, D.ptr(hit_xy), xy_slots, st)
+                     D.ptr(sub_counts), D.ptr(hits), slots, D.ptr(hit_xy), xy_slots, st)
         # staging rows in processing order, then the per-segment sort into the output rows
-        sub_offsets, total = D.exclusive_scan(counts[:m])
-        per_query = D.empty(n, torch.int64)
-        query_start = D.empty(n, torch.int64)
-        _native.call("ct_subquery_spans", D.ptr(order), n, D.ptr(part_offsets), D.ptr(sub_offsets),
-                     D.ptr(per_query), D.ptr(query_start), st)
-        offsets, _ = D.exclusive_scan(per_query, total=False)
+        sub_offsets, _ = D.exclusive_scan(sub_counts[:m], total=False)
+        query_start = D.empty(int(queries.shape[0]), torch.int64)
+        _native.call("ct_subquery_spans", D.ptr(order), n, D.ptr(part_offsets), D.ptr(sub_offsets), D.ptr(counts),
+                     D.ptr(query_start), st)
+
+        def write_edges(offsets, rows, ii, jj, xy):
+            if rows == 0:
+                return
+            staged = self._staging(rows)
+            _native.call("ct_locate_edges_write_sub", self.tree_ref, D.ptr(queries), D.ptr(subs), m, edges,
+                         D.ptr(sub_offsets), D.ptr(hits), slots, D.ptr(hit_xy), xy_slots,
+                         *(D.ptr(t) for t in staged), st)
+            _native.call("ct_sort_staged_rows", D.ptr(offsets), D.ptr(query_start), *(D.ptr(t) for t in staged), rows,
+                         D.ptr(ii), D.ptr(jj), D.ptr(xy), st)
+
+        return write_edges
+
+    def _split_rows(self, kind: int, queries: torch.Tensor, order):
+        """(ii, jj, xy or None) of a batch through subqueries: those that the wavefront walks do not
+        take."""
+        n = int(queries.shape[0])
+        counts = D.empty(n, torch.int64)
+        write = self._count_subs(kind, queries, order, n, counts)
+        offsets, total = D.exclusive_scan(counts)
         ii = D.empty(total, torch.int64)
         jj = D.empty(total, torch.int64)
-        xy = D.empty((total, 2, 2), torch.float64)
-        if total == 0:
-            return offsets, ii, jj, xy
-        rows_query = D.empty(total, torch.int32)
-        rows_cell = D.empty(total, torch.int32)
-        rows_xy = D.empty((total, 4), torch.float64)
-        rows_t = D.empty(total, torch.float64)
-        _native.call("ct_locate_edges_write_sub", self.tree_ref, D.ptr(queries), D.ptr(subs), m, edges,
-                     D.ptr(sub_offsets), D.ptr(hits), slots, D.ptr(hit_xy), xy_slots, D.ptr(rows_query),
-                     D.ptr(rows_cell), D.ptr(rows_xy), D.ptr(rows_t), st)
-        _native.call("ct_sort_staged_rows", D.ptr(offsets), D.ptr(query_start), D.ptr(rows_query),
-                     D.ptr(rows_cell), D.ptr(rows_xy), D.ptr(rows_t), total, D.ptr(ii), D.ptr(jj), D.ptr(xy), st)
-        return offsets, ii, jj, xy
-
-    def _sub_offsets(self, order, n: int, part_offsets, counts):
-        """Turns per-subquery counts into prefixes within each query; returns the query offsets
-        (n + 1) and the row total."""
-        per_query = D.empty(n, torch.int64)
-        _native.call("ct_subquery_offsets", D.ptr(order), n, D.ptr(part_offsets), D.ptr(counts), D.ptr(per_query),
-                     D.stream())
-        return D.exclusive_scan(per_query)
+        xy = None if kind == 1 else D.empty((total, 2, 2), torch.float64)
+        write(offsets, total, ii, jj, xy)
+        return ii, jj, xy
 
     def _sort_edges(self, edge_coords, offsets, ii, jj, xy, total):
         jj_sorted = torch.empty_like(jj)
@@ -609,7 +667,7 @@ class CellTree2dBase:
             return self._gather(2 if kind == 1 else 3, edge_coords, self._gather_order(4, edge_coords))
         order, srt = self._order(2, edge_coords)
         if self._splits(n):
-            return self._split_rows(2 if kind == 1 else 3, edge_coords, order)[1:]
+            return self._split_rows(2 if kind == 1 else 3, edge_coords, order)
         counts = D.empty(n, torch.int64)
         hits, slots = self._hit_record(n, self.EDGE_HIT_SLOTS, self.EDGE_HIT_BUDGET)
         _native.call(

@@ -17,6 +17,8 @@
 #ifndef CT_GATHER_H
 #define CT_GATHER_H
 
+#include <algorithm>
+
 #include "ct_internal.h"
 #include "ct_primitives.h"
 #include "ct_traverse.h"
@@ -36,18 +38,16 @@ constexpr int kMaxPerWave = 16;
 constexpr int kOwnerShift = 27;
 constexpr uint32_t kIndexMask = (1u << kOwnerShift) - 1u;
 constexpr int64_t kMaxRecords = (int64_t)1 << 26;
-constexpr uint32_t kLargeLeaf = ~0u;  // a stack entry: the large leaf at hand
 
 // LDS list lengths.  The stack: a step of P entries needs room for P more; P shrinks as the stack
-// fills, and depth + 1 places always remain for a single entry's way down (kStack + depth + 1 in all;
-// 512 instead of 320 costs boxes two wavefronts a CU, 1.28 instead of 1.22 ms, and 256 nothing).
+// fills, and depth + 1 places always remain for a single entry's way down (kStack + depth + 1 in all).
 constexpr int kStack = 320;
 constexpr int kCells = 192;  // 63 left over + 2 per lane
 constexpr int kCands = 128;  // 63 left over + 64
 // A step with a leaf of more cells than this lists one leaf, 64 cells at a time by all lanes, and puts
 // the others back: each lane listing its own leaf takes as many stores as the largest has cells, and a
-// leaf may be larger than the list.  200,000 triangles in leaves of up to 130 cells, 1e5 boxes: 481 us,
-// 771 lane by lane; of up to 64 cells, 1e5 segments: 850 lane by lane, 982 one leaf at a time.
+// leaf may be larger than the list.  200,000 triangles in leaves of up to 130 cells, 1e5 boxes: 514 us,
+// 771 lane by lane; of up to 64 cells, 1e5 segments: 857 lane by lane, 982 one leaf at a time.
 constexpr int kLeafCells = 64;
 // Hits a wavefront holds, and the expected hits of the queries it walks together: fewer and the steps
 // at either end of a walk (few entries on the stack) weigh more, more and LDS limits the wavefronts in
@@ -55,7 +55,7 @@ constexpr int kLeafCells = 64;
 // boxes 768/384 1.27, 768/480 1.22, 768/576 1.27, 512/384 1.91, 640/640 1.59;
 // segments 256/160 2.67, 256/224 2.55, 320/280 2.50, 384/336 2.65, 512/448 2.77.
 // A box walked alone may have kBoxHits: boxes of 20 cell widths have 900 (8e3 of them on 20,000
-// triangles: 0.16 ms, and 0.60 with 768, most of it for the few then left to the subqueries).
+// triangles: 0.16 ms, and 0.60 with 768).
 constexpr int kBoxHits = 1024, kBoxGroupHits = 768, kBoxGroup = 480;
 constexpr int kSegHits = 320, kSegGroup = 280;
 // Counters for pool allocation, each on its own 128-byte line: one counter for all wavefronts
@@ -243,6 +243,48 @@ __device__ __forceinline__ int expected(const QueryRec<KIND>& r, double cell) {
   return e > 1.0 ? (e < 1e6 ? (int)e : 1000000) : 1;
 }
 
+// Query q's record; whether it meets the tree's bbox.
+template <int KIND>
+__device__ __forceinline__ bool load_query(const TreeView& t, const double* __restrict__ qs, int64_t q, double reach,
+                                           QueryRec<KIND>* rec) {
+  rec->d = reinterpret_cast<const double4*>(qs)[q];
+  if constexpr (KIND == kBoxes) {
+    return boxes_intersect(Box{rec->d.x, rec->d.y, rec->d.z, rec->d.w}, t.bbox);
+  } else {
+    const P2 a = {rec->d.x, rec->d.y}, b = {rec->d.z, rec->d.w};
+    rec->dx = b.x - a.x;
+    rec->dy = b.y - a.y;
+    rec->ax2 = 2.0 * a.x;
+    rec->ay2 = 2.0 * a.y;
+    const double mseg = pmax(pmax(fabs(a.x), fabs(a.y)), pmax(fabs(b.x), fabs(b.y)));
+    const double m = 1e-9 * pmax(mseg, reach);
+    rec->sx0 = pmin(a.x, b.x) - m;
+    rec->sx1 = pmax(a.x, b.x) + m;
+    rec->sy0 = pmin(a.y, b.y) - m;
+    rec->sy1 = pmax(a.y, b.y) + m;
+    rec->mm = 2.0 * m * (fabs(rec->dx) + fabs(rec->dy));
+    rec->prune = KIND == kFaces && t.nbox != nullptr && isfinite(mseg) && isfinite(rec->mm) && isfinite(rec->dx) &&
+                 isfinite(rec->dy);
+    P2 c0, d0;
+    return cohen_sutherland<true>(a, b, t.bbox, &c0, &d0);
+  }
+}
+
+// Down from the root while a single child is viable; -1: none is.
+template <int KIND>
+__device__ __forceinline__ int first_fork(const TreeView& t, const QueryRec<KIND>& rec) {
+  int node = 0;
+  while (true) {
+    const NodeLd nd = ld_node(t.nodes, node);
+    if (nd.child == -1) return node;
+    bool left, right;
+    slab<KIND>(rec, nd, &left, &right);
+    if (left && right) return node;
+    if (!left && !right) return -1;
+    node = nd.child + (right ? 1 : 0);
+  }
+}
+
 // Whether a listed cell goes on: a box's whole test; a segment-edge pair's whole test; for a segment
 // and a face what is cheap and rejects nearly all that Cohen-Sutherland rejects (its trivial
 // rejection and seg_near): the exact test runs with the clip, where its loop diverges less.
@@ -282,7 +324,7 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
   __shared__ Key ts[KIND == kBoxes ? 1 : kHits];           // segments: t_key
   __shared__ uint16_t byown[KIND == kBoxes ? 1 : kHits];   // segments: a grouped hit's pool row
   __shared__ int cnt[kMaxPerWave], first[kMaxPerWave + 1];
-  __shared__ uint32_t large[3];                            // a large leaf on the stack: its next cell's words, cells left
+  __shared__ uint32_t leaf_done;                           // cells listed of the large leaf on top of the stack
   const int lane = lane_id();
   __syncthreads();  // one wavefront: the last block's LDS reads are over
 
@@ -293,44 +335,10 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
   if (lane < nq) {
     q = query_index(order, i0 + lane);
     QueryRec<KIND> rec;
-    rec.d = reinterpret_cast<const double4*>(qs)[q];
-    bool in;
-    if constexpr (KIND == kBoxes) {
-      in = boxes_intersect(Box{rec.d.x, rec.d.y, rec.d.z, rec.d.w}, t.bbox);
-    } else {
-      const P2 a = {rec.d.x, rec.d.y}, b = {rec.d.z, rec.d.w};
-      rec.dx = b.x - a.x;
-      rec.dy = b.y - a.y;
-      rec.ax2 = 2.0 * a.x;
-      rec.ay2 = 2.0 * a.y;
-      const double mseg = pmax(pmax(fabs(a.x), fabs(a.y)), pmax(fabs(b.x), fabs(b.y)));
-      const double m = 1e-9 * pmax(mseg, p.reach);
-      rec.sx0 = pmin(a.x, b.x) - m;
-      rec.sx1 = pmax(a.x, b.x) + m;
-      rec.sy0 = pmin(a.y, b.y) - m;
-      rec.sy1 = pmax(a.y, b.y) + m;
-      rec.mm = 2.0 * m * (fabs(rec.dx) + fabs(rec.dy));
-      rec.prune = KIND == kFaces && t.nbox != nullptr && isfinite(mseg) && isfinite(rec.mm) && isfinite(rec.dx) &&
-                  isfinite(rec.dy);
-      P2 c0, d0;
-      in = cohen_sutherland<true>(a, b, t.bbox, &c0, &d0);
-    }
-    if (in) {
+    if (load_query<KIND>(t, qs, q, p.reach, &rec)) {
       weight = expected<KIND>(rec, p.cell);
       big = weight > p.leave;
-      start = big ? -1 : 0;
-      while (start >= 0) {
-        const NodeLd nd = ld_node(t.nodes, start);
-        if (nd.child == -1) break;
-        bool left, right;
-        slab<KIND>(rec, nd, &left, &right);
-        if (left && right) break;
-        if (!left && !right) {
-          start = -1;
-          break;
-        }
-        start = nd.child + (right ? 1 : 0);
-      }
+      start = big ? -1 : first_fork<KIND>(t, rec);
     }
     recs[lane] = rec;
   }
@@ -354,12 +362,13 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
     auto owner = [](uint32_t w) { return (int)(w >> kOwnerShift); };
     __syncthreads();  // one wavefront: orders LDS accesses
     if (lane < kMaxPerWave) cnt[lane] = 0;
+    if (lane == 0) leaf_done = 0;
     if (mine && start >= 0)
       stack[below(alive)] = (uint32_t)lane << kOwnerShift | (uint32_t)start;
     // Hits this group may have: the lists' length, and the pool rows at hand (segments).
     int room = KIND == kBoxes && g1 - g0 > 1 ? kBoxGroupHits : kHits;
     if (KIND != kBoxes && alive) {
-      const int want = g1 - g0 == 1 ? kHits : min(kHits, 2 * wsum + 32);
+      const int want = min(kHits, wsum + wsum / 2 + 32);
       if (rows.end - rows.at < want) rows.refill(pool, tail, want);
       room = (int)min((long long)kHits, rows.end - rows.at);
     }
@@ -445,22 +454,6 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
       // the top of the stack
       const int take = min(min(64, sp), max(1, p.stack - p.depth1 - sp));
       uint32_t e = lane < take ? stack[sp - take + lane] : 0;
-      if ((uint32_t)__builtin_amdgcn_readlane((int)e, take - 1) == kLargeLeaf) {
-        // the next cells of a large leaf (at most 64, and 128 more fit)
-        const uint32_t at = large[0], visit = large[1], left = large[2];
-        const uint32_t m = min(64u, left);
-        __syncthreads();
-        if ((uint32_t)lane < m) cells[ncell + lane] = make_uint2(at + lane, visit + lane);
-        if (lane == 0) {
-          large[0] = at + m;
-          large[1] = visit + m;
-          large[2] = left - m;
-        }
-        ncell += m;
-        if (m == left) --sp;
-        __syncthreads();
-        continue;
-      }
       sp -= take;
       bool left = false, right = false;
       int child = 0, ptr = 0, size = 0;
@@ -516,25 +509,33 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
         }
         const bool fits = incl <= kCells - ncell && !__any(size > kLeafCells);
         uint64_t back = __ballot(size > 0 && !fits);
-        const uint64_t put = __ballot(size > 0 && fits), one = put ? 0 : back & -back;
-        if (one >> lane & 1) {  // a large leaf, listed by the whole wavefront
-          large[0] = tag | (uint32_t)ptr;
-          large[1] = tag | v0;
-          large[2] = (uint32_t)size;
+        const uint64_t put = __ballot(size > 0 && fits);
+        if (!put) {  // the top leaf's next 64 cells; it stays on top until they are all listed
+          const int top = 63 - __clzll((unsigned long long)back);
+          const uint32_t done = leaf_done, cell0 = __shfl(tag | (uint32_t)ptr, top) + done;
+          const uint32_t visit0 = __shfl(tag | v0, top) + done, rest = (uint32_t)__shfl(size, top) - done;
+          __syncthreads();
+          if ((uint32_t)lane < min(64u, rest)) cells[ncell + lane] = make_uint2(cell0 + lane, visit0 + lane);
+          ncell += (int)min(64u, rest);
+          if (lane == 0) leaf_done = rest > 64u ? done + 64u : 0u;
+          back &= ~(1ull << top);
+          if (back >> lane & 1) stack[sp + below(back)] = e;
+          sp += __popcll(back);
+          if (rest > 64u) {
+            if (lane == top) stack[sp] = e;
+            ++sp;
+          }
+          __syncthreads();
+          continue;
         }
-        back &= ~one;
         if (size > 0 && fits)
           for (int j = 0; j < size; ++j)
             cells[ncell + incl - size + j] = make_uint2(tag | (uint32_t)(ptr + j), tag | (v0 + j));
         if (back >> lane & 1) stack[sp + below(back)] = e;
         sp += __popcll(back);
-        if (one) {
-          if (lane == 0) stack[sp] = kLargeLeaf;
-          ++sp;
-        }
         // the listed cells: the prefix of the last lane that fits
         const int last = 63 - __clzll((unsigned long long)put);
-        ncell += put ? __shfl(incl, last) : 0;
+        ncell += __shfl(incl, last);
       }
       __syncthreads();
     }
@@ -574,7 +575,7 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
         if (!left_over) {
           if (g1 - g0 > 1) {
             if (nhit <= 256) group_by_owner<4, false>(hits, nullptr, nullptr, nhit, lane, first, cnt);
-            else group_by_owner<kBoxGroupHits / 64, false>(hits, nullptr, nullptr, nhit, lane, first, cnt);
+            else group_by_owner<(kBoxGroupHits + 63) / 64, false>(hits, nullptr, nullptr, nhit, lane, first, cnt);
           }
           // as many owners at a time as 64 words hold, or one larger owner
           for (int o = g0; o < g1;) {
@@ -594,7 +595,7 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
         }
       } else {
         const bool grouped = g1 - g0 > 1;
-        if (grouped) group_by_owner<kSegHits / 64, true>(hits, ts, byown, nhit, lane, first, cnt);
+        if (grouped) group_by_owner<(kSegHits + 63) / 64, true>(hits, ts, byown, nhit, lane, first, cnt);
         // geometry_utils.py:564-574: by t (NaN last), then in the walk's order
         for (int s = lane; s < nhit; s += 64) {
           const uint32_t wi = hits[s];
@@ -621,6 +622,45 @@ __device__ __forceinline__ void gather_block(const TreeView& t, const double* __
     }
     g0 = g1;
   }
+}
+
+// ------------------------------------------------------------------ launches
+constexpr int kRowChunk = 64;  // pool rows a wavefront takes at a time, at least (segments)
+
+inline GatherParams gather_params(const ct_tree* tree, int64_t n, const int32_t* visit, int kind) {
+  GatherParams p{};
+  p.visit = visit;
+  p.scale(view(tree));
+  // Few queries: fewer per wavefront, so that at least 4096 wavefronts share the work (256 CUs hold
+  // about 4000 of them); many: 16 (8 per wavefront: 1e6 boxes 1.41 instead of 1.22
+  // ms, 1e6 segments 2.74 instead of 2.67: too few entries on the stack to fill the lanes).
+  p.per_wave = (int)std::min((int64_t)kMaxPerWave, std::max((int64_t)1, n / 4096));
+  p.depth1 = tree->depth + 1;
+  p.stack = kStack + p.depth1;
+  p.group = kind == kBoxes ? kBoxGroup : kSegGroup;
+  // A walk in vain costs more than leaving a query that would have fitted.
+  p.leave = kind == kBoxes ? kBoxHits : kSegHits;
+  return p;
+}
+
+inline Pool gather_pool(int64_t rows, int64_t n, int per_wave, int32_t* cell, double* xy, int32_t* src) {
+  const int64_t waves = (n + per_wave - 1) / per_wave;
+  Pool pool{cell, reinterpret_cast<double4*>(xy), src, 0, 1, kRowChunk};
+  pool.counters = (int)std::min((int64_t)kPools, std::max((int64_t)1, waves / 64));
+  pool.rows = rows / pool.counters;
+  return pool;
+}
+
+inline int check_gather(const ct_tree* tree, int32_t kind, int64_t n) {
+  CT_REQUIRE(tree != nullptr && tree->nodes && tree->bb_indices && tree->elements && tree->vertices && tree->bb_coords,
+             "incomplete tree");
+  CT_REQUIRE(tree->depth >= 0 && tree->depth <= CT_MAX_DEPTH, "trees of depth <= %d", CT_MAX_DEPTH);
+  CT_REQUIRE(tree->n_nodes < kMaxRecords && tree->n_elements < kMaxRecords, "trees of fewer than 2^26 nodes and cells");
+  CT_REQUIRE(kind >= kBoxes && kind <= kEdges, "kind must be 1 (boxes), 2 (segment-face) or 3 (segment-edge)");
+  CT_REQUIRE(kind == kEdges ? tree->n_max_vert == 2 : (kind == kBoxes || tree->n_max_vert >= 3),
+             "kind does not match the tree");
+  CT_REQUIRE(n >= 0 && n < ((int64_t)1 << 31), "n must be in [0, 2^31)");
+  return CT_OK;
 }
 
 }  // namespace

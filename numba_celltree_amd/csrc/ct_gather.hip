@@ -9,7 +9,7 @@
 // Rows go to a pool (each wavefront allocates from one of several counters); an exclusive scan of
 // the counts gives the output offsets, and the copy kernels write whole output lines in query order.
 // A query with more hits than the LDS lists hold, or that the pool has no room for, is left to the
-// caller (starts[q] = -1): the subquery path (ct_split.hip) takes it.
+// caller (starts[q] = -1): few go to ct_long.hip, a wavefront each, many to the subqueries (ct_split.hip).
 #include <algorithm>
 #include <cmath>
 
@@ -17,8 +17,6 @@
 
 namespace ct {
 namespace {
-
-constexpr int kRowChunk = 512;  // pool rows a wavefront takes at a time (segments)
 
 // Workgroups go round-robin over the 8 XCDs (workgroup b runs on XCD b % 8).  Workgroup b takes block
 // block_of(b): every XCD sweeps whole chunks of kXcdChunk consecutive blocks, chunk c on XCD c % 8, so
@@ -48,6 +46,20 @@ k_gather(TreeView t, const double* __restrict__ qs, const int32_t* __restrict__ 
   PoolRows rows;
   rows.sub = (int)(blockIdx.x % (unsigned)pool.counters);
   gather_block<KIND, MAXV>(t, qs, order, i0, (int)min((int64_t)p.per_wave, n - i0), p, pool, rows, counts, starts, tail);
+}
+
+// The queries left to the caller (starts < 0), one list entry each; the lanes of a wavefront in order.
+__global__ void __launch_bounds__(kBlock) k_left(int64_t n, const int64_t* __restrict__ starts, int32_t* __restrict__ left,
+                                                 int64_t room, unsigned long long* __restrict__ found) {
+  const int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const bool is = q < n && starts[q] < 0;
+  const uint64_t mask = __ballot(is);
+  if (!mask) return;
+  const int lead = __ffsll((unsigned long long)mask) - 1;
+  unsigned long long at = 0;
+  if (lane_id() == lead) at = atomicAdd(found, (unsigned long long)__popcll(mask));
+  at = __shfl(at, lead) + below(mask);
+  if (is && (int64_t)at < room) left[at] = (int32_t)q;
 }
 
 // Output rows from the pool, `per_wave` queries per wavefront (a power of two, at most 64; fewer when
@@ -125,60 +137,6 @@ __global__ void __launch_bounds__(kBlock) k_pool_rows(int64_t n, int per_wave, c
   }
 }
 
-// The rows of a batch of left-over queries (sub-query s of them is query idx[s]; its rows at
-// sub_offsets[s]) to their places among all rows.
-__global__ void __launch_bounds__(kBlock) k_place_rows(int64_t rows, const int64_t* __restrict__ idx,
-                                                       const int64_t* __restrict__ sub_offsets,
-                                                       const int64_t* __restrict__ offsets,
-                                                       const int64_t* __restrict__ sub_ii,
-                                                       const int64_t* __restrict__ sub_jj,
-                                                       const double4* __restrict__ sub_xy, int64_t* __restrict__ ii,
-                                                       int64_t* __restrict__ jj, double4* __restrict__ xy) {
-  const int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (r >= rows) return;
-  const int64_t s = sub_ii[r], q = idx[s], o = offsets[q] + (r - sub_offsets[s]);
-  ii[o] = q;
-  jj[o] = sub_jj[r];
-  if (xy) xy[o] = sub_xy[r];
-}
-
-GatherParams params(const ct_tree* tree, int64_t n, const int32_t* visit, int kind) {
-  GatherParams p{};
-  p.visit = visit;
-  p.scale(view(tree));
-  // Few queries: fewer per wavefront, so that at least 4096 wavefronts share the work (256 CUs hold
-  // about 4000 of them); many: 16 (8 per wavefront: 1e6 boxes 1.41 instead of 1.22
-  // ms, 1e6 segments 2.74 instead of 2.67: too few entries on the stack to fill the lanes).
-  p.per_wave = (int)std::min((int64_t)kMaxPerWave, std::max((int64_t)1, n / 4096));
-  p.depth1 = tree->depth + 1;
-  p.stack = kStack + p.depth1;
-  p.group = kind == kBoxes ? kBoxGroup : kSegGroup;
-  // The subqueries take what is left: a walk in vain costs more than leaving a query that would have
-  // fitted (3e5 boxes of 1317 hits: 16.9 ms with twice the list's length, 10.0 without such walks).
-  p.leave = kind == kBoxes ? kBoxHits : kSegHits;
-  return p;
-}
-
-Pool make_pool(int64_t rows, int64_t n, int per_wave, int32_t* cell, double* xy, int32_t* src) {
-  const int64_t waves = (n + per_wave - 1) / per_wave;
-  Pool pool{cell, reinterpret_cast<double4*>(xy), src, 0, 1, kRowChunk};
-  pool.counters = (int)std::min((int64_t)kPools, std::max((int64_t)1, waves / 64));
-  pool.rows = rows / pool.counters;
-  return pool;
-}
-
-int check_gather(const ct_tree* tree, int32_t kind, int64_t n) {
-  CT_REQUIRE(tree != nullptr && tree->nodes && tree->bb_indices && tree->elements && tree->vertices && tree->bb_coords,
-             "incomplete tree");
-  CT_REQUIRE(tree->depth >= 0 && tree->depth <= CT_MAX_DEPTH, "trees of depth <= %d", CT_MAX_DEPTH);
-  CT_REQUIRE(tree->n_nodes < kMaxRecords && tree->n_elements < kMaxRecords, "trees of fewer than 2^26 nodes and cells");
-  CT_REQUIRE(kind >= kBoxes && kind <= kEdges, "kind must be 1 (boxes), 2 (segment-face) or 3 (segment-edge)");
-  CT_REQUIRE(kind == kEdges ? tree->n_max_vert == 2 : (kind == kBoxes || tree->n_max_vert >= 3),
-             "kind does not match the tree");
-  CT_REQUIRE(n >= 0 && n < ((int64_t)1 << 31), "n must be in [0, 2^31)");
-  return CT_OK;
-}
-
 struct GatherArgs {
   const ct_tree* tree;
   const double* qs;
@@ -237,10 +195,11 @@ int64_t ct_gather_tail_words(void) { return kTailWords; }
 
 int64_t ct_gather_pool_rows(int32_t kind, int64_t n) {
   if (n <= 0) return 0;
-  // boxes: 256 hits per query; segments: 64 per query, at least a chunk per wavefront
-  if (kind == kBoxes) return std::max((int64_t)256 * n, (int64_t)kBoxHits);
-  const int64_t per_wave = std::min((int64_t)kMaxPerWave, std::max((int64_t)1, n / 4096));
-  return std::max((int64_t)64 * n, ((n + per_wave - 1) / per_wave * 5 / 4 + kPools) * kRowChunk);
+  // Boxes (4 bytes a row): every list full, and room for a box of ct_long.hip.  Segments (40 bytes): what
+  // a group takes (half more rows than expected) if every list is full, as far as 2^26 rows go, and of
+  // more than a million segments 64 each.
+  if (kind == kBoxes) return std::max((int64_t)2 * kBoxHits * n, (int64_t)1 << 22);
+  return std::max((int64_t)64 * n, std::min((int64_t)384 * n, (int64_t)1 << 26));
 }
 
 int ct_gather_count(const ct_tree* tree, int32_t kind, const double* queries, int64_t n, const int32_t* order,
@@ -261,8 +220,8 @@ int ct_gather_count(const ct_tree* tree, int32_t kind, const double* queries, in
   a.qs = queries;
   a.order = order;
   a.n = n;
-  a.p = params(tree, n, visit_cells, kind);
-  a.pool = make_pool(pool_rows, n, a.p.per_wave, pool_cell, pool_xy, pool_src);
+  a.p = gather_params(tree, n, visit_cells, kind);
+  a.pool = gather_pool(pool_rows, n, a.p.per_wave, pool_cell, pool_xy, pool_src);
   a.counts = counts;
   a.starts = starts;
   a.tail = tail;
@@ -278,15 +237,13 @@ int ct_gather_rows(int32_t kind, int64_t n, const int64_t* offsets, const int64_
                           as_stream(stream));
 }
 
-int ct_place_rows(int64_t rows, const int64_t* idx, const int64_t* sub_offsets, const int64_t* offsets,
-                  const int64_t* sub_ii, const int64_t* sub_jj, const double* sub_xy, int64_t* ii, int64_t* jj,
-                  double* xy, void* stream) {
-  CT_REQUIRE(rows >= 0 && (rows == 0 || (idx && sub_offsets && offsets && sub_ii && sub_jj && ii && jj)), "bad arguments");
-  CT_REQUIRE((sub_xy == nullptr) == (xy == nullptr), "sub_xy and xy go together");
-  if (rows == 0) return CT_OK;
-  k_place_rows<<<grid_for(rows), kBlock, 0, as_stream(stream)>>>(rows, idx, sub_offsets, offsets, sub_ii, sub_jj,
-                                                               reinterpret_cast<const double4*>(sub_xy), ii, jj,
-                                                               reinterpret_cast<double4*>(xy));
+int ct_gather_left(int64_t n, const int64_t* starts, int64_t n_left, int32_t* left, int64_t* found, void* stream) {
+  CT_REQUIRE(n >= 0 && n < ((int64_t)1 << 31) && n_left >= 0 && found && (n == 0 || starts) && (n_left == 0 || left),
+             "bad arguments");
+  hipStream_t st = as_stream(stream);
+  const int rc = fill<int64_t>(found, 1, 0, st);
+  if (rc || n == 0) return rc;
+  k_left<<<grid_for(n), kBlock, 0, st>>>(n, starts, left, n_left, reinterpret_cast<unsigned long long*>(found));
   CT_LAUNCH_CHECK();
   return CT_OK;
 }
