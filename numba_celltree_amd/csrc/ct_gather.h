@@ -41,7 +41,7 @@ constexpr int64_t kMaxRecords = (int64_t)1 << 26;
 
 // LDS list lengths.  The stack: a step of P entries needs room for P more; P shrinks as the stack
 // fills, and depth + 1 places always remain for a single entry's way down (kStack + depth + 1 in all).
-constexpr int kStack = 320;
+constexpr int kStack = 240;
 constexpr int kCells = 192;  // 63 left over + 2 per lane
 constexpr int kCands = 128;  // 63 left over + 64
 // A step with a leaf of more cells than this lists one leaf, 64 cells at a time by all lanes, and puts
@@ -53,11 +53,13 @@ constexpr int kLeafCells = 64;
 // at either end of a walk (few entries on the stack) weigh more, more and LDS limits the wavefronts in
 // flight or groups overflow and are walked again one by one.  Measured, 1e6 queries, milliseconds:
 // boxes 768/384 1.27, 768/480 1.22, 768/576 1.27, 512/384 1.91, 640/640 1.59;
-// segments 256/160 2.67, 256/224 2.55, 320/280 2.50, 384/336 2.65, 512/448 2.77.
+// segments 256/160 2.67, 256/224 2.55, 320/280 2.50, 384/336 2.65, 512/448 2.77.  With 310/270 and the
+// stack above, a segment wavefront's LDS is 10,240 bytes up to a depth of 43, and 16 of them fit a CU
+// instead of 15: 2.55 -> 2.41.
 // A box walked alone may have kBoxHits: boxes of 20 cell widths have 900 (8e3 of them on 20,000
 // triangles: 0.16 ms, and 0.60 with 768).
 constexpr int kBoxHits = 1024, kBoxGroupHits = 768, kBoxGroup = 480;
-constexpr int kSegHits = 320, kSegGroup = 280;
+constexpr int kSegHits = 310, kSegGroup = 270;
 // Counters for pool allocation, each on its own 128-byte line: one counter for all wavefronts
 // would serialize them (about 11 ns per atomic on one address).
 constexpr int kPools = 64, kCounterStride = 16;
