@@ -82,7 +82,7 @@ def barycentric_weights(tree, points: torch.Tensor, vertices: Optional[torch.Ten
     at = points.detach().contiguous()
     n = int(at.shape[0])
     order = None
-    if tree.orders_points(n) or (vertices.requires_grad and n >= tree.ORDERED_GRAD_MIN):
+    if tree.orders_points(n, vertex_gradients=vertices.requires_grad):
         order = tree._point_order(at)
     face = tree._locate_points_dev(at, float(tolerance), order)
     w = BarycentricFunction.apply(points, vertices, tree.d_elements, face, float(tolerance), k > 3, order)

@@ -68,7 +68,8 @@ class CellTree2d(CellTree2dBase):
     # points; what it saves grows with the points and with what of the tree does not fit the L2s.  In
     # order / as they come, microseconds: 20,000 triangles, 2.6e5 points 79 / 33, 4e6 333 / 266;
     # 200,000 cells, 1e6 146 / 125, 4e6 359 / 414; a million cells, 2.6e5 96 / 61, 1e6 155 / 173,
-    # 4e6 384 / 627.
+    # 4e6 384 / 627.  ORDERED_MIN None: no batch is ordered; any other value than the default: it
+    # alone decides.
     ORDERED_MIN = 3 << 18
     ORDERED_WORK = 1 << 40
     # Points whose gradients go to the vertices are put in order from this size on: it also lets the
@@ -84,10 +85,13 @@ class CellTree2d(CellTree2dBase):
         out = self._locate_points_dev(pts, float(tolerance))
         return io.out(out)
 
-    def orders_points(self, n: int) -> bool:
-        """Whether a batch of n points is located in Morton order."""
-        return (self.ORDERED_MIN is not None and n >= self.ORDERED_MIN
-                and n * int(self.d_elements.numel()) >= self.ORDERED_WORK)
+    def orders_points(self, n: int, vertex_gradients: bool = False) -> bool:
+        """Whether a batch of n points is located in Morton order (``vertex_gradients``: as points
+        whose weights take gradients to the vertices)."""
+        if self.ORDERED_MIN is None or self.ORDERED_MIN != _ORDERED_MIN:
+            return self.ORDERED_MIN is not None and n >= self.ORDERED_MIN
+        return (n >= self.ORDERED_MIN and n * int(self.d_elements.numel()) >= self.ORDERED_WORK
+                or vertex_gradients and n >= self.ORDERED_GRAD_MIN)
 
     def _point_order(self, pts: torch.Tensor):
         """The Morton order of a point batch.  The order alone: writing the points in sorted order
@@ -255,3 +259,6 @@ class CellTree2d(CellTree2dBase):
             D.ptr(face), D.ptr(w), D.stream(),
         )
         return io.out(face), io.out(w)
+
+
+_ORDERED_MIN = CellTree2d.ORDERED_MIN
