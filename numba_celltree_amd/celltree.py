@@ -72,6 +72,13 @@ class CellTree2d(CellTree2dBase):
     # alone decides.
     ORDERED_MIN = 3 << 18
     ORDERED_WORK = 1 << 40
+    # Leaves of many cells: neighbours also share those, and points in no order leave the lanes of a
+    # wavefront at different lengths of them, so from ORDERED_LEAF cells on the points and the cells of
+    # a leaf decide, whatever the tree's size.  20,000 triangles, 8 cells a leaf, 2e6 216 / 213, 4e6
+    # 355 / 377; 16 a leaf, 1e6 187 / 192, 1e7 886 / 1313; 130 a leaf, 2.7e5 329 / 366, 3e6 886 / 1750.
+    ORDERED_LEAF = 8
+    ORDERED_LEAF_MIN = 1 << 18
+    ORDERED_LEAF_WORK = 1 << 24
     # Points whose gradients go to the vertices are put in order from this size on: it also lets the
     # backward add a face's points before it adds them to memory (1e6 points: 79 instead of 258 us).
     ORDERED_GRAD_MIN = 1 << 18
@@ -90,7 +97,9 @@ class CellTree2d(CellTree2dBase):
         whose weights take gradients to the vertices)."""
         if self.ORDERED_MIN is None or self.ORDERED_MIN != _ORDERED_MIN:
             return self.ORDERED_MIN is not None and n >= self.ORDERED_MIN
+        leaf = int(self.cells_per_leaf)
         return (n >= self.ORDERED_MIN and n * int(self.d_elements.numel()) >= self.ORDERED_WORK
+                or leaf >= self.ORDERED_LEAF and n >= self.ORDERED_LEAF_MIN and n * leaf >= self.ORDERED_LEAF_WORK
                 or vertex_gradients and n >= self.ORDERED_GRAD_MIN)
 
     def _point_order(self, pts: torch.Tensor):
