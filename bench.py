@@ -377,7 +377,7 @@ def batch_extras(args):
     out["batch_config_points"] = cfg_p.__dict__
     out["batch_config_edges"] = cfg_e.__dict__
     out["batch_autotune_points_ms"] = {"best": min(ms for _, ms in tp), "worst": max(ms for _, ms in tp)}
-    out["batch_autotune_edges_count_ms"] = {"best": min(ms for _, ms in te), "worst": max(ms for _, ms in te)}
+    out["batch_autotune_edges_ms"] = {"best": min(ms for _, ms in te), "worst": max(ms for _, ms in te)}
     graphs = {
         "batch_graph_points_ms": B.BatchGraph(tb, pts, pc, points_config=cfg_p),
         "batch_graph_edges_ms": B.BatchGraph(tb, segments=segs, segment_counts=sc, edges_config=cfg_e),

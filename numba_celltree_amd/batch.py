@@ -453,7 +453,9 @@ def intersect_edges(batch: TreeBatch, segment_sets: Sequence, config: BatchConfi
 
 
 # -------------------------------------------------------------------- autotuner
-def default_candidates(batch: TreeBatch) -> List[BatchConfig]:
+def default_candidates(batch: TreeBatch, kind: str = "points") -> List[BatchConfig]:
+    if _walks(batch, kind):
+        return [BatchConfig(tile=tile, n_queues=q) for tile, q in itertools.product((64, 128, 256, 512, 1024), (8, 16, 32))]
     base = stack_class(batch.max_depth)
     stacks = [base] + [s for s in STACK_CLASSES if s > base][:1]
     out = []
@@ -462,19 +464,25 @@ def default_candidates(batch: TreeBatch) -> List[BatchConfig]:
     return out
 
 
+def _walks(batch: TreeBatch, kind: str) -> bool:
+    """Whether the batch goes through wavefront walks, which take only the tiles and queues of a config."""
+    return kind == "edges" and batch.gathers
+
+
 _TUNED: Dict[Tuple, BatchConfig] = {}
 
 
 def autotune(batch: TreeBatch, kind: str, queries: torch.Tensor, counts: Sequence[int],
              candidates: Optional[Sequence[BatchConfig]] = None, reps: int = 3,
              cache_path: Optional[str] = None) -> Tuple[BatchConfig, List[Tuple[BatchConfig, float]]]:
-    """Time every candidate config on this batch (kind "points" or "edges": the one-lane count pass;
-    wavefront walks take only the tiles and queues of a config) and return the fastest, with all (config, ms) timings.  Results are
-    kept per (kind, tree count, query count, depth, vertex class), in memory and, with
-    `cache_path`, in a JSON file."""
+    """Time every candidate config on this batch (kind "points" or "edges": the walks of
+    intersect_edges and BatchGraph, gather_edges) and return the fastest, with all (config, ms)
+    timings.  Results are kept per (kind, tree count, query count, depth, vertex class), in memory
+    and, with `cache_path`, in a JSON file; "edges" by wavefront walks under a kind of their own."""
     if kind not in ("points", "edges"):
         raise ValueError("kind must be 'points' or 'edges'")
-    key = (kind, batch.n_trees, int(np.sum(counts)), batch.max_depth, batch.max_n_vert)
+    walks = _walks(batch, kind)
+    key = ("edges-by-wavefronts" if walks else kind, batch.n_trees, int(np.sum(counts)), batch.max_depth, batch.max_n_vert)
     skey = json.dumps(key)
     if key in _TUNED:
         return _TUNED[key], []
@@ -485,9 +493,9 @@ def autotune(batch: TreeBatch, kind: str, queries: torch.Tensor, counts: Sequenc
             cfg = BatchConfig(**saved[skey])
             _TUNED[key] = cfg
             return cfg, []
-    candidates = list(candidates or default_candidates(batch))
+    candidates = list(candidates or default_candidates(batch, kind))
     n = int(np.sum(counts))
-    out = D.empty(n, torch.int64)
+    out = D.empty(n, torch.int64) if kind == "points" else EdgeBuffers(n, 0, expected=POOL_GUESS * n, gathers=walks)
     timings = []
     tiled: Dict[Tuple[int, int], BatchPlan] = {}  # plans differ only in tiles and queues
     for cfg in candidates:
@@ -500,7 +508,7 @@ def autotune(batch: TreeBatch, kind: str, queries: torch.Tensor, counts: Sequenc
             if kind == "points":
                 plan.locate_points(queries, out)
             else:
-                plan.edges_count(queries, out)
+                gather_edges(plan, queries, out)
 
         step()
         ev0 = torch.cuda.Event(enable_timing=True)
