@@ -35,32 +35,6 @@ __device__ __forceinline__ T block_exclusive_scan(T v, T* lds, T* total) {
   return before + x - v;
 }
 
-// Segmented (by equal consecutive key) min/max reduction across a wavefront of
-// order-preserving FP64 keys; the last lane of each run applies one pair of atomics.
-// Runs must be contiguous in lane order; key < 0 marks an inactive lane.
-__device__ __forceinline__ void wave_run_minmax(int key, unsigned long long lo,
-                                                unsigned long long hi,
-                                                unsigned long long* __restrict__ out_lo,
-                                                unsigned long long* __restrict__ out_hi) {
-  const int lane = lane_id();
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int k2 = __shfl_up(key, d, 64);
-    const unsigned long long lo2 = __shfl_up(lo, d, 64);
-    const unsigned long long hi2 = __shfl_up(hi, d, 64);
-    if (lane >= d && k2 == key) {
-      lo = lo2 < lo ? lo2 : lo;
-      hi = hi2 > hi ? hi2 : hi;
-    }
-  }
-  const int knext = __shfl_down(key, 1, 64);
-  const bool tail = (lane == 63) || (knext != key);
-  if (key >= 0 && tail) {
-    atomicMin(out_lo + key, lo);
-    atomicMax(out_hi + key, hi);
-  }
-}
-
 // Ascending bitonic sort of 64 * R words, word r * 64 + lane in v[r] of the lane.
 template <int R>
 __device__ __forceinline__ void wave_sort(uint32_t (&v)[R], int lane) {
