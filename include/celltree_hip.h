@@ -597,7 +597,7 @@ typedef struct ct_regrid_topology {
  * ascending), src_tgt = tt[perm_by_src], the corners face * n_max + slot of every vertex ascending
  * (offsets n_vertices + 1; corners with room for n * n_max) and rest_targets (room for n_tgt, in no
  * order).  info (device, 3): the rest targets, the target and the source corners.  Fewer than
- * 2^32 - 1 pairs and corners together.  No synchronization. */
+ * 2^31 pairs, target corners and source corners each.  No synchronization. */
 size_t ct_regrid_lists_workspace_bytes(const ct_regrid_topology* topo);
 int ct_regrid_lists(const ct_regrid_topology* topo, void* workspace, size_t workspace_bytes,
                     int64_t* tgt_offsets, int64_t* src_offsets, int64_t* perm_by_src, int64_t* src_tgt,

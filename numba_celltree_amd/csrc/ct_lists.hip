@@ -25,6 +25,7 @@ constexpr int kHugeLds = 8192;  // items sorted in LDS; longer lists stream over
 constexpr int kHugeStream = 8;  // items a lane takes at a time then
 
 constexpr uint32_t kNone = ~0u;
+constexpr int64_t kItemsPerLaunch = (int64_t)1 << 31;  // a HIP launch has fewer than 2^32 lanes
 
 struct Lists {
   const int64_t* ss;
@@ -39,8 +40,8 @@ struct Lists {
   int64_t* starts;            // their scan, keys + 1
   uint32_t* unsorted;         // by start: a key's items in arrival order
   uint32_t* rank;             // by item: arrival among its key's, kNone: no key
-  int32_t* longer;            // keys of more than kCompare items
-  int32_t* huge;              // keys of more than kWaveMax
+  uint32_t* longer;           // keys of more than kCompare items
+  uint32_t* huge;             // keys of more than kWaveMax
   int32_t* n_longer;          // [0] longer, [1] huge
 };
 
@@ -55,8 +56,8 @@ __device__ __forceinline__ int64_t key_of(const Lists& l, int g, int64_t id) {
   return v < 0 ? -1 : l.keys[g] + v;
 }
 
-__global__ void __launch_bounds__(kBlock) k_list_count(Lists l) {
-  const int64_t x = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+__global__ void __launch_bounds__(kBlock) k_list_count(Lists l, int64_t x0) {
+  const int64_t x = x0 + (int64_t)blockIdx.x * kBlock + threadIdx.x;
   int64_t key = -1;
   if (x < l.items[kGroups]) {
     const int g = group_of(l.items, x);
@@ -78,8 +79,8 @@ __global__ void __launch_bounds__(kBlock) k_list_count(Lists l) {
   if (x < l.items[kGroups]) l.rank[x] = r;
 }
 
-__global__ void __launch_bounds__(kBlock) k_list_place(Lists l) {
-  const int64_t x = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+__global__ void __launch_bounds__(kBlock) k_list_place(Lists l, int64_t x0) {
+  const int64_t x = x0 + (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (x >= l.items[kGroups]) return;
   const uint32_t r = l.rank[x];
   if (r == kNone) return;
@@ -95,8 +96,8 @@ __device__ __forceinline__ void put(const Lists& l, int g, int64_t at, int64_t i
 
 // info: [0] rest targets (k_targets), [1] target corners, [2] source corners.
 // Offsets of every key, and the place of every item of a key with at most kCompare.
-__global__ void __launch_bounds__(kBlock) k_list_rank(Lists l, int64_t* info) {
-  const int64_t x = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+__global__ void __launch_bounds__(kBlock) k_list_rank(Lists l, int64_t x0, int64_t* info) {
+  const int64_t x = x0 + (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (x == 0) {
     info[1] = l.starts[l.keys[2]] - l.starts[l.keys[1]];
     info[2] = l.starts[l.keys[3]] - l.starts[l.keys[2]];
@@ -116,8 +117,8 @@ __global__ void __launch_bounds__(kBlock) k_list_rank(Lists l, int64_t* info) {
   const int m = (int)(l.starts[key + 1] - b);
   if (m > kCompare) {
     if (arrival == 0) {
-      if (m > kWaveMax) l.huge[atomicAdd(l.n_longer + 1, 1)] = (int)key;
-      else l.longer[atomicAdd(l.n_longer, 1)] = (int)key;
+      if (m > kWaveMax) l.huge[atomicAdd(l.n_longer + 1, 1)] = (uint32_t)key;
+      else l.longer[atomicAdd(l.n_longer, 1)] = (uint32_t)key;
     }
     return;
   }
@@ -281,7 +282,10 @@ int ct_regrid_lists(const ct_regrid_topology* topo, void* workspace, size_t work
                  (topo->n_tgt == 0 || tgt_vertex_corners),
              "null outputs");
   const ListWs w = carve_lists(topo);
-  CT_REQUIRE(w.items < (int64_t)kNone && w.keys < ((int64_t)1 << 31), "fewer than 2^32 - 1 pairs and corners");
+  // an item's number within its group, its rank and a list's length are 32-bit words
+  CT_REQUIRE(topo->n_pairs < ((int64_t)1 << 31) && topo->n_tgt * topo->n_max_t < ((int64_t)1 << 31) &&
+                 topo->n_src * topo->n_max_s < ((int64_t)1 << 31) && w.keys < (int64_t)kNone,
+             "fewer than 2^31 pairs, target corners and source corners each");
   if (workspace_bytes < w.total) {
     set_error("list workspace too small: %zu < %zu", workspace_bytes, w.total);
     return CT_ERR_WORKSPACE;
@@ -309,8 +313,8 @@ int ct_regrid_lists(const ct_regrid_topology* topo, void* workspace, size_t work
   l.starts = reinterpret_cast<int64_t*>(ws + w.starts);
   l.unsorted = reinterpret_cast<uint32_t*>(ws + w.unsorted);
   l.rank = reinterpret_cast<uint32_t*>(ws + w.rank);
-  l.longer = reinterpret_cast<int32_t*>(ws + w.longer);
-  l.huge = reinterpret_cast<int32_t*>(ws + w.huge);
+  l.longer = reinterpret_cast<uint32_t*>(ws + w.longer);
+  l.huge = reinterpret_cast<uint32_t*>(ws + w.huge);
   int rc = fill<int64_t>(l.counts, w.clear, 0, st);
   if (!rc) rc = fill<int64_t>(info, 3, 0, st);
   // a group without keys writes no offset by k_list_rank
@@ -318,12 +322,16 @@ int ct_regrid_lists(const ct_regrid_topology* topo, void* workspace, size_t work
   if (rc) return rc;
   k_targets<<<grid_for(topo->n_tgt + 1), kBlock, 0, st>>>(topo->tt, topo->n_pairs, topo->n_tgt, tgt_offsets, rest_targets,
                                                         reinterpret_cast<unsigned long long*>(info));
-  k_list_count<<<grid_for(w.items), kBlock, 0, st>>>(l);
+  auto grid = [](int64_t all, int64_t x0) { return grid_for(std::min(all - x0, kItemsPerLaunch)); };
+  for (int64_t x0 = 0; x0 < w.items; x0 += kItemsPerLaunch)
+    k_list_count<<<grid(w.items, x0), kBlock, 0, st>>>(l, x0);
   CT_LAUNCH_CHECK();
   rc = exclusive_scan(l.counts, w.keys, l.starts, ws + w.scan, ct_scan_workspace_bytes(w.keys), st);
   if (rc) return rc;
-  k_list_place<<<grid_for(w.items), kBlock, 0, st>>>(l);
-  k_list_rank<<<grid_for(std::max(w.items, w.keys)), kBlock, 0, st>>>(l, info);
+  for (int64_t x0 = 0; x0 < w.items; x0 += kItemsPerLaunch)
+    k_list_place<<<grid(w.items, x0), kBlock, 0, st>>>(l, x0);
+  for (int64_t x0 = 0; x0 < std::max(w.items, w.keys); x0 += kItemsPerLaunch)
+    k_list_rank<<<grid(std::max(w.items, w.keys), x0), kBlock, 0, st>>>(l, x0, info);
   k_list_longer<<<1024, kBlock, 0, st>>>(l);
   k_list_huge<<<256, kHugeBlock, 0, st>>>(l);
   CT_LAUNCH_CHECK();
