@@ -499,12 +499,22 @@ class CellTree2dBase:
 
     def _gather(self, kind: int, queries: torch.Tensor, order, prep=None):
         """Rows of a box (kind 1), segment-face (2) or segment-edge (3) batch: (ii, jj) or
-        (ii, jj, xy).  One readback: the row total, the queries left over, and the index checks of
-        ``prep``; another one or two where queries are left over."""
+        (ii, jj, xy).  Where the device holds the pool but not the rows beside it, again without a
+        pool: memory pressure costs a second walk, not the call."""
+        try:
+            return self._gather_rows(kind, queries, order, prep, True)
+        except torch.cuda.OutOfMemoryError:
+            pass  # the failed call's arrays are released with its traceback, at the end of this block
+        torch.cuda.empty_cache()
+        return self._gather_rows(kind, queries, order, prep, False)
+
+    def _gather_rows(self, kind: int, queries: torch.Tensor, order, prep, pooled: bool):
+        """_gather with or without a row pool.  One readback: the row total, the queries left over, and
+        the index checks of ``prep``; another one or two where queries are left over."""
         n = int(queries.shape[0])
         st = D.stream()
         L = _native.lib()
-        rows = int(L.ct_gather_pool_rows(kind, n))
+        rows = int(L.ct_gather_pool_rows(kind, n)) if pooled else 0
         if kind == 1:
             rows, (cell,) = self._pool(min(rows, int(self.BOX_HIT_BUDGET)), [(torch.int32, 1)])
             pxy = src = None
