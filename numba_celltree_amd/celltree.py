@@ -75,9 +75,10 @@ class CellTree2d(CellTree2dBase):
     # Leaves of many cells: neighbours also share those, and points in no order leave the lanes of a
     # wavefront at different lengths of them, so from ORDERED_LEAF cells on the points and the cells of
     # a leaf decide, whatever the tree's size.  20,000 triangles, 8 cells a leaf, 2e6 216 / 213, 4e6
-    # 355 / 377; 16 a leaf, 1e6 187 / 192, 1e7 886 / 1313; 130 a leaf, 2.7e5 329 / 366, 3e6 886 / 1750.
+    # 355 / 377; 16 a leaf, 1e6 187 / 192, 1e7 886 / 1313; 64 a leaf, 2.7e5 218 / 226, 5e5 276 / 305
+    # (a million cells 349 / 320 and 388 / 415); 130 a leaf, 2.7e5 329 / 366, 3e6 886 / 1750.
     ORDERED_LEAF = 8
-    ORDERED_LEAF_MIN = 1 << 18
+    ORDERED_LEAF_MIN = 3 << 17       # half as many points where the product is twice as large
     ORDERED_LEAF_WORK = 1 << 24
     # Points whose gradients go to the vertices are put in order from this size on: it also lets the
     # backward add a face's points before it adds them to memory (1e6 points: 79 instead of 258 us).
@@ -98,8 +99,9 @@ class CellTree2d(CellTree2dBase):
         if self.ORDERED_MIN is None or self.ORDERED_MIN != _ORDERED_MIN:
             return self.ORDERED_MIN is not None and n >= self.ORDERED_MIN
         leaf = int(self.cells_per_leaf)
+        in_leaves = n * leaf // self.ORDERED_LEAF_WORK  # 0: too little, 2 and more: also for fewer points
         return (n >= self.ORDERED_MIN and n * int(self.d_elements.numel()) >= self.ORDERED_WORK
-                or leaf >= self.ORDERED_LEAF and n >= self.ORDERED_LEAF_MIN and n * leaf >= self.ORDERED_LEAF_WORK
+                or leaf >= self.ORDERED_LEAF and in_leaves > 0 and n >= self.ORDERED_LEAF_MIN // min(in_leaves, 2)
                 or vertex_gradients and n >= self.ORDERED_GRAD_MIN)
 
     def _point_order(self, pts: torch.Tensor):

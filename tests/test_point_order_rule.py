@@ -16,6 +16,7 @@ def test_default_rule():
     assert not any(small.orders_points(n) for n in (1, 10**6, 10**7))
     assert [large.orders_points(n) for n in (500_000, 10**6, 10**7)] == [False, True, True]
     assert [tree(2000, 16).orders_points(n) for n in (10**6, 1 << 20, 10**7)] == [False, True, True]
+    assert [tree(20_000, 64).orders_points(n) for n in (390_000, 400_000)] == [False, True]
     assert [tree(20_000, 130).orders_points(n) for n in (250_000, 270_000)] == [False, True]
     assert not tree(20_000, 7).orders_points(10**7) and tree(20_000, 8).orders_points(10**7)
     assert small.orders_points(1 << 18, vertex_gradients=True)
