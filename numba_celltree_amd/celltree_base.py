@@ -496,6 +496,9 @@ class CellTree2dBase:
     # At most this many queries that a wavefront walk leaves over are walked by a wavefront each
     # (ct_long_*); more fill the device as subqueries.
     LONG_MAX = 1 << 20
+    # Pool rows (4 bytes) a few boxes may have, so that boxes over much of a mesh are walked once (20 boxes
+    # over a million cells: 204 ms, 395 with a second walk to write the rows).
+    LONG_BOX_ROWS = 1 << 27
 
     def _gather(self, kind: int, queries: torch.Tensor, order, prep=None):
         """Rows of a box (kind 1), segment-face (2) or segment-edge (3) batch: (ii, jj) or
@@ -516,6 +519,8 @@ class CellTree2dBase:
         L = _native.lib()
         rows = int(L.ct_gather_pool_rows(kind, n)) if pooled else 0
         if kind == 1:
+            if pooled:  # few boxes: room for any number of cells each
+                rows = max(rows, min(n * int(self.d_elements.shape[0]), int(self.LONG_BOX_ROWS)))
             rows, (cell,) = self._pool(min(rows, int(self.BOX_HIT_BUDGET)), [(torch.int32, 1)])
             pxy = src = None
         else:

@@ -195,10 +195,10 @@ int64_t ct_gather_tail_words(void) { return kTailWords; }
 
 int64_t ct_gather_pool_rows(int32_t kind, int64_t n) {
   if (n <= 0) return 0;
-  // Boxes (4 bytes a row): every list full, and room for a box of ct_long.hip.  Segments (40 bytes): what
+  // Boxes (4 bytes a row): every list full, and as much for the boxes of ct_long.hip.  Segments (40 bytes): what
   // a group takes (half more rows than expected) if every list is full, as far as 2^26 rows go, and of
   // more than a million segments 64 each.
-  if (kind == kBoxes) return std::max((int64_t)2 * kBoxHits * n, (int64_t)1 << 22);
+  if (kind == kBoxes) return (int64_t)2 * kBoxHits * n;
   return std::max((int64_t)64 * n, std::min((int64_t)384 * n, (int64_t)1 << 26));
 }
 

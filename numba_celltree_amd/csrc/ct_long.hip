@@ -192,7 +192,7 @@ k_long_count(TreeView t, const double* __restrict__ qs, const int32_t* __restric
       rows.sub = (int)(blockIdx.x % (unsigned)pool.counters);
       rows.tried = max(0, pool.counters - kLongTries);
       const int e = expected<KIND>(rec, p.cell);
-      rows.refill(pool, tail, e + e / 4 + 64);
+      rows.refill(pool, tail, (int)min((int64_t)e + e / 4 + 64, t.n_elements));
       at = rows.at;
       room = rows.end - rows.at;
     }

@@ -160,6 +160,35 @@ def test_equal_queries_up_to_the_lists_are_kept(monkeypatch, n):
     assert not seen["long"] and not seen["subs"]
 
 
+def test_few_boxes_over_all_cells_are_walked_once(monkeypatch):
+    """Boxes whose expected number of rows is more than the mesh has cells, one and several."""
+    from numba_celltree_amd import _native
+
+    tree, oracle, f = trees("mixed")
+    written = []
+    call = _native.call
+    monkeypatch.setattr(_native, "call", lambda name, *a: written.append(name) or call(name, *a))
+    for n in (1, 7):
+        boxes = np.tile([[-3.0 * L, 4.0 * L, -1.0, L + 1.0]], (n, 1))
+        ii, jj = tree.locate_boxes(boxes)
+        oi, oj = oracle.locate_boxes(boxes)
+        assert np.array_equal(ii, oi) and np.array_equal(jj, oj) and len(ii) == n * len(f)
+    assert "ct_long_count" in written
+    # every box is in the pool after its first walk
+    import torch
+
+    starts = []
+    long_boxes = type(tree)._count_long
+
+    def keep(self, k, q, ids, m, rows, cell, counts, st, tail):
+        starts.append(st)
+        return long_boxes(self, k, q, ids, m, rows, cell, counts, st, tail)
+
+    monkeypatch.setattr(type(tree), "_count_long", keep)
+    tree.locate_boxes(torch.from_numpy(boxes).cuda())
+    assert bool((starts[0] >= 0).all())
+
+
 def test_pool_stays_within_the_budgets():
     """Two int32 and 32 bytes of a piece per row, whatever the batch asks for."""
     import torch
