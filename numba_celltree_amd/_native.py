@@ -19,6 +19,7 @@ CT_ERR_DEPTH = -4
 CT_ERR_WORKSPACE = -5
 CT_MAX_N_VERTEX = 32
 CT_MAX_DEPTH = 254
+CT_LONG_MAX = 1 << 24
 CT_NOALLOC_MAX_POINTS = 1 << 21
 
 

@@ -539,7 +539,7 @@ class CellTree2dBase:
             prep.check(words)
         write = None
         if left:
-            many = left > int(self.LONG_MAX)
+            many = left > min(int(self.LONG_MAX), _native.CT_LONG_MAX)
             if left == n and (many or kind != 1):  # nothing is in the pool, or will be
                 cell = pxy = src = None
                 pool = (0, 0, 0)
