@@ -171,8 +171,7 @@ __device__ __forceinline__ P2 mean_vertex(const P2 (&poly)[CAP], int len) {
 // loops would run to 32+ slots; faces of more than 8 vertices are rare.  Same operations in
 // the same order as sh_stage.
 template <int MA, int MB>
-__device__ __forceinline__ double clip_area_indexed(const P2 (&subj)[MA], int ls, const P2 (&clip)[MB], int lc,
-                                                    P2* centre) {
+__device__ __forceinline__ double clip_area_indexed(const P2 (&subj)[MA], int ls, const P2 (&clip)[MB], int lc) {
   constexpr int CAP = MA + MB;
   P2 outp[CAP], inp[CAP];
   for (int i = 0; i < CAP; ++i) outp[i] = (i < MA) ? subj[i < MA ? i : 0] : P2{0.0, 0.0};
@@ -219,13 +218,13 @@ __device__ __forceinline__ double clip_area_indexed(const P2 (&subj)[MA], int ls
     }
     r = s;
   }
-  if (centre != nullptr) *centre = mean_vertex<CAP>(outp, n_out);
   return polygon_area<CAP>(outp, n_out);
 }
 
 // sutherland_hodgman.py:84-148 polygon_polygon_clip_area.  `row` is the lane's clip row of
 // clip_row_cap<MA, MB>() slots (CT_CLIP_ROWS); the indexed path for the large classes does
-// not use it.  centre (may be null): the mean of the clipped polygon's vertices, when it has an area.
+// not use it.  centre (may be null; up to 16 vertices together): the mean of the clipped polygon's
+// vertices, when it has an area.
 template <int MA, int MB>
 constexpr int clip_row_cap() {
   return MA + MB > 16 ? 1 : MA + MB;
@@ -236,7 +235,7 @@ __device__ __forceinline__ double clip_area(const P2 (&subj)[MA], int ls, const 
                                             const Row& row, P2* centre = nullptr) {
   constexpr int CAP = MA + MB;
   if constexpr (CAP > 16) {
-    return clip_area_indexed<MA, MB>(subj, ls, clip, lc, centre);
+    return clip_area_indexed<MA, MB>(subj, ls, clip, lc);
   } else {
     static_assert(Row::kLds + Row::kExtra == CAP, "clip row of the wrong capacity");
     P2 poly[CAP];
