@@ -36,9 +36,11 @@ inline unsigned gather_grid(int64_t blocks) {
   return (unsigned)((blocks + round - 1) / round * round);
 }
 
-// One block of queries per workgroup, one wavefront each: the hardware's scheduler balances them.
+// One block of queries per workgroup, one wavefront each: the hardware's scheduler balances them.  Faces of
+// more than 8 vertices: two wavefronts a SIMD, with spills (1e5 segments on 12-gons 1008 us with one and
+// none, 660 with two; on 24-gons 1461 and 1041).
 template <int KIND, int MAXV>
-__global__ void __launch_bounds__(64, MAXV <= 8 ? 4 : 1)
+__global__ void __launch_bounds__(64, MAXV <= 8 ? 4 : 2)
 k_gather(TreeView t, const double* __restrict__ qs, const int32_t* __restrict__ order, int64_t n, GatherParams p,
          Pool pool, int64_t* __restrict__ counts, int64_t* __restrict__ starts, int64_t* tail) {
   const int64_t i0 = block_of(blockIdx.x) * p.per_wave;

@@ -177,7 +177,7 @@ __device__ __forceinline__ int begin(const TreeView& t, const double* __restrict
 // counts[q] of the queries in the list; boxes whose rows fit what they reserved of the pool are kept there
 // (starts[q]), segments have their counts in list order too.
 template <int KIND, int MAXV>
-__global__ void __launch_bounds__(64, MAXV <= 8 ? 4 : 1)
+__global__ void __launch_bounds__(64, MAXV <= 8 ? 4 : 2)
 k_long_count(TreeView t, const double* __restrict__ qs, const int32_t* __restrict__ left, GatherParams p, Pool pool,
              int64_t* __restrict__ counts, int64_t* __restrict__ starts, int64_t* __restrict__ left_counts,
              int64_t* tail) {
@@ -225,7 +225,7 @@ k_long_boxes(TreeView t, const double* __restrict__ boxes, const int32_t* __rest
 
 // The rows of the segments in the list into staging, in list order; starts[q]: the first.
 template <int KIND, int MAXV>
-__global__ void __launch_bounds__(64, MAXV <= 8 ? 4 : 1)
+__global__ void __launch_bounds__(64, MAXV <= 8 ? 4 : 2)
 k_long_edges(TreeView t, const double* __restrict__ segs, const int32_t* __restrict__ left, GatherParams p,
              const int64_t* __restrict__ left_offsets, int64_t* __restrict__ starts, StagedRows rows) {
   extern __shared__ uint32_t stack[];
