@@ -384,8 +384,9 @@ class CellTree2dBase:
         _native.call(fn, self.tree_ref, D.ptr(pts), n, float(tolerance), D.ptr(out), D.stream())
         return io.out(out)
 
-    # Rows of box and segment batches.  Wavefront walks (_gather) keep them in a pool of at most
-    # EDGE_HIT_BUDGET (40 bytes each) or BOX_HIT_BUDGET rows (4 bytes).  Subqueries and whole walks
+    # Rows of box and segment batches.  Wavefront walks (_gather) keep them in a pool: boxes at most
+    # BOX_HIT_BUDGET rows (4 bytes each), segments (two int32 and 32 bytes) EDGE_HIT_BUDGET // 2 and
+    # EDGE_XY_BUDGET // 32, whichever is less (2^27 rows: 5.4 GB).  Subqueries and whole walks
     # record hit cells per query in the count pass (slot-major, so only slots in use are touched),
     # up to EDGE_HIT_SLOTS or BOX_HIT_SLOTS (wide boxes have hundreds of hits) within the same
     # budgets as int32 entries; queries with at most that many hits are written from the record
@@ -396,7 +397,7 @@ class CellTree2dBase:
     EDGE_HIT_BUDGET = 1 << 28
 
     # With the cells, the count pass of split segment queries keeps the clipped segments of the
-    # first EDGE_XY_SLOTS hits (32 bytes each, within EDGE_XY_BUDGET bytes), so that the write
+    # first EDGE_XY_SLOTS hits (32 bytes each, within half of EDGE_XY_BUDGET bytes), so that the write
     # pass copies the rows of a subquery whose hits all fit instead of clipping its cells again.
     EDGE_XY_SLOTS = 32
     EDGE_XY_BUDGET = 1 << 32
@@ -433,8 +434,8 @@ class CellTree2dBase:
                 xs //= 2
         return None, 0
 
-    # Work splitting of the queries a wavefront walk leaves over (ct_split_queries): a query expected
-    # to meet more than SPLIT_MIN_CELLS cells is cut into at most SPLIT_MAX_PARTS subqueries by
+    # Work splitting of trees and batches that wavefront walks do not take, and of more than LONG_MAX
+    # queries that these leave over (ct_split_queries): a query expected to meet more than SPLIT_MIN_CELLS cells is cut into at most SPLIT_MAX_PARTS subqueries by
     # subtree, expanding subtrees of more than SPLIT_LEAF_CELLS (boxes) or EDGE_SPLIT_LEAF_CELLS
     # (segments) cells; results are identical.  Segments take larger leaves: fewer subqueries
     # keep their hit records small.

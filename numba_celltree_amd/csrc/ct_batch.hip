@@ -33,7 +33,8 @@ constexpr int kWave = 64;
 constexpr int kBatchMaxBlock = 256;
 static_assert(kBatchMaxBlock == kStackStride, "batch workgroups are at most kStackStride lanes");
 
-// Wavefronts of a segment walk (what 256 CUs hold at once), and the most pool rows one takes at a time.
+// Wavefronts of a segment walk (what 256 CUs hold at once by LDS, in trees of a depth up to 43; the few
+// more than that in deeper ones start as others end), and the most pool rows one takes at a time.
 constexpr int kGatherWaves = 4096, kGatherChunk = 2048;
 
 struct BatchArgs {
@@ -117,7 +118,7 @@ __global__ void __launch_bounds__(kBatchMaxBlock) k_batch_points(BatchArgs a, co
 
 // Segment-face queries by wavefront walks (ct_gather.h).  One lane per query left most of a wavefront
 // idle, in the count pass and again in the write pass; bound by the latency of a step's loads, as
-// k_gather.  32 meshes of 1e3 to 2e5 cells, 4.6e5 segments, count, write and sort 11.4 ms, now walks 1.14
+// k_gather.  32 meshes of 1e3 to 2e5 cells, 4.6e5 segments, count, write and sort 11.4 ms, now walks 1.09
 // and rows 0.13 ms.  A wavefront pulls kMaxPerWave queries of a tile at a time: whole tiles are too few to
 // balance (64 to 1024 queries each, some 4000 wavefronts).  Rows stay in the pool; a segment with
 // more hits than a wavefront's lists hold, or that finds the pool used up, is left (starts[q] = -1,
@@ -418,7 +419,7 @@ int ct_batch_gather_edges(const ct_batch* batch, const double* segments, int64_t
   if (pool_rows < kSegHits || batch->n_tiles * units >= ((int64_t)1 << 31)) {
     k_leave_all<<<grid_for(n_queries), kBlock, 0, st>>>(n_queries, counts, starts, tail);
   } else {
-    // As many wavefronts as the device holds at once (16 a CU by LDS), or as there is work for.
+    // As many wavefronts as the device holds at once, or as there is work for.
     const int64_t all = batch->n_tiles * units;
     const unsigned grid = (unsigned)std::min(all, (int64_t)kGatherWaves);
     GatherParams p{};

@@ -21,7 +21,7 @@
 // anything back (an idle level costs three empty launches), and synchronizes once.  With a
 // sequence of 11 kernels and a host synchronization for each of the 22 levels, and the node boxes
 // in one launch a level, the constructor took 5.78 ms for 999,941 cells and 1.67 ms for 20,000;
-// now 1.14 and 0.31 ms.
+// now 1.14 and 0.33 ms.
 //
 // The stable partition is the order sort_bbox_indices (:54-151) produces with its repeated
 // stable_partition.  Per node as in the reference: special case (:312-320), empty-bucket merge

@@ -1,10 +1,10 @@
 // ct_gather.hip -- box and segment queries, one wavefront for a few queries (ct_gather.h has the walk).
 //
 // What bounds it: the latency of a step's loads (a node record, a cell box, a clip's vertices), hidden by
-// the 15 to 20 wavefronts a CU holds (LDS, registers); the FP64 arithmetic of the segment tests is
+// the 16 to 20 wavefronts a CU holds (LDS, registers); the FP64 arithmetic of the segment tests is
 // about half of the segments' time.  1e6 queries on a million-cell mesh, before (subqueries, one lane
-// each, and their replay and sort kernels) and now, whole calls: boxes (31.6e6 rows) 1.94 and 1.22 ms,
-// segments (13.6e6 rows) 3.50 and 2.50 ms; 2e3 segments 560 and 119 us.
+// each, and their replay and sort kernels) and now, whole calls: boxes (31.6e6 rows) 1.94 and 1.20 ms,
+// segments (13.6e6 rows) 3.50 and 2.40 ms; 2e3 segments 560 and 100 us.
 //
 // Rows go to a pool (each wavefront allocates from one of several counters); an exclusive scan of
 // the counts gives the output offsets, and the copy kernels write whole output lines in query order.
